@@ -24,7 +24,36 @@
 #include <type_traits>
 
 namespace wol {
+
+// A GEMM call on its way from the entry points to the kernels of its element
+// type, which are compiled as two translation units side by side: this file
+// for bf16, and through wol_linear_gemm_f16.hip for fp16.
+struct GemmArgs {
+  const void* x; const void* codes; const void* bias; const void* scale; void* out;
+  int M, K, N, gshift, out_f32;
+  void* ws; size_t ws_bytes;  // scratch for split-K partial sums, may be null
+  hipStream_t stream;
+  int act;
+};
+
+// One product of moe_ffn (see MoeLaunch below).
+struct MoeGemmArgs {
+  const void* x; const int* table; int max_tiles, bm, ns, experts; int64_t rows; float* partial; const int64_t* valid_rows;
+  const void* codes; const void* bias; const void* scale; int64_t K, N; void* out; hipStream_t stream; bool swiglu;
+};
+
+void gemm_bf16(const GemmArgs& a, int bits);
+void gemm_f16(const GemmArgs& a, int bits);
+void swiglu_gemm_bf16(const GemmArgs& a, int bits);
+void swiglu_gemm_f16(const GemmArgs& a, int bits);
+void moe_gemm_bf16(const MoeGemmArgs& a, int bits);
+void moe_gemm_f16(const MoeGemmArgs& a, int bits);
+
 namespace {
+
+#ifndef WOL_GEMM_DTYPE
+#define WOL_GEMM_DTYPE WOL_DTYPE_BF16
+#endif
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
@@ -137,11 +166,6 @@ __device__ inline void tile_of_block(int id, int nbx, int nby, int* bx, int* by)
 // and each owns nby/rg row blocks x nbx/(8/rg) column blocks, the shape that
 // makes the sum of the A rows and B columns an L2 has to fetch smallest
 // (plan_xcd_rows on the host).  rg == 0: plain order.
-// rg < 0 (the grouped GEMM over experts; nby a multiple of 8 * -rg): runs of
-// -rg consecutive row tiles -- one expert's, when the experts have about that
-// many -- go to one XCD with all their column tiles, column tile by column
-// tile, so that the row tiles of an expert meet its weights in one L2 while
-// they are there, and no other XCD fetches them.
 __device__ inline void tile_of_block_2d(int id, int nbx, int nby, int rg, int* bx, int* by) {
   if (rg == 0) {
     *by = id % nby;
@@ -149,13 +173,6 @@ __device__ inline void tile_of_block_2d(int id, int nbx, int nby, int rg, int* b
     return;
   }
   constexpr int kXcd = 8;
-  if (rg < 0) {
-    const int tpe = -rg, x = id % kXcd, i = id / kXcd;
-    const int per = tpe * nbx, gi = i / per, w = i % per;
-    *by = (gi * kXcd + x) * tpe + w % tpe;
-    *bx = w / tpe;
-    return;
-  }
   const int x = id % kXcd, i = id / kXcd;
   const int r = nby / rg, c = nbx / (kXcd / rg);
   *by = (x % rg) * r + i % r;
@@ -430,7 +447,9 @@ struct MoeTile {
   int expert;  // -1: the tile is not used
   int row0;    // first row of the tile in the permuted input
   int rows;    // rows of the tile that exist (1 .. tile height)
-  int pad;
+  int first;   // gemm_experts_kernel: first row tile of the tile's expert ...
+  int count;   // ... and how many it has
+  int pad[3];
 };
 
 // Fast path: K a multiple of the tile depth.
@@ -494,10 +513,21 @@ struct MoeTile {
 // tile (for its own tile loads, then for the workgroup) and around the
 // epilogue, and leaves the sums in p.stamps.  The reads sit where the
 // wavefront has just waited for all its LDS traffic anyway.
-template <int DT, int BITS, int G, int OFFS, int WM, int WN, int TM, int TN, int STAGES, int SWI = 0, bool RESC = false,
-          bool STAMP = false>
-__global__ __launch_bounds__(64 * WM * WN) void gemm_dma_kernel(const DmaParams p) {
-#if defined(__HIP_DEVICE_COMPILE__)  // the host pass only needs the launch stub
+// The work of one workgroup is a device function (dma_tile) of where its tile
+// lies: gemm_dma_kernel below calls it for the one tile height it is built
+// for, gemm_experts_kernel picks the height of every tile at run time.
+struct TilePlace {
+  int bx;      // column tile of the launch
+  int m0;      // first row of the tile, counted from x and out
+  int split;   // run of k tiles
+  int expert;  // >= 0: the tile lies in this expert's rows
+  int row0;    // expert >= 0: the tile's first row in x and out
+  int rows;    // expert >= 0: rows of the tile that exist
+};
+
+template <int DT, int BITS, int G, int OFFS, int WM, int WN, int TM, int TN, int STAGES, int SWI, bool RESC, bool STAMP>
+__device__ __forceinline__ void dma_tile(const DmaParams& p, unsigned char* smem, const TilePlace at) {
+#if defined(__HIP_DEVICE_COMPILE__)  // the host pass only needs the launch stubs
   constexpr int NW = WM * WN;
   constexpr int BM = WM * TM * 32, BN = WN * TN * 32;
   constexpr int TK = BITS == 8 ? 64 : 128;       // k per 16-byte lane load of B
@@ -533,7 +563,6 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_dma_kernel(const DmaParams 
   constexpr bool kPair = SWI != 0 && TN == 1;
   static_assert(OFFS != 2 || G == 0, "row sums by dot products are taken out once, in the epilogue");
   static_assert(!RESC || (G != 0 && OFFS == 0), "rescaled sums are for group-wise scales and the exact dequantisers");
-  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   unsigned long long st_entry = 0, st_prev = 0, st_work = 0, st_loads = 0, st_bar = 0, st_loop0 = 0;
   if (STAMP) st_entry = __builtin_readcyclecounter();
 
@@ -548,23 +577,18 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_dma_kernel(const DmaParams 
   const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave / WN, wn = wave % WN;
   const int j = lane & 15, sp = (lane >> 4) & 1, b = lane >> 5, r32 = lane & 31;
-  const int ntiles = p.nbx * p.nby;
-  const int split = blockIdx.x / ntiles;
-  int bx, by;
-  tile_of_block_2d(blockIdx.x - split * ntiles, p.nbx, p.nby, p.xcd_rows, &bx, &by);
-  int m0 = by * BM;
-  if (p.moe_table != nullptr) {
-    // this row tile belongs to one expert: shift every base to that expert and
-    // to the tile's first row, and let M be the rows that exist
-    const MoeTile t = reinterpret_cast<const MoeTile*>(p.moe_table)[by];
-    if (t.expert < 0) return;
-    x += static_cast<int64_t>(t.row0) * K;
-    if (p.nsplit > 1) outp = static_cast<float*>(outp) + static_cast<int64_t>(t.row0) * N;  // partial sums
-    else outp = static_cast<uint16_t*>(outp) + static_cast<int64_t>(t.row0) * (SWI ? N / 2 : N);
-    codes += static_cast<int64_t>(t.expert) * p.moe_codes_stride;
-    scale += static_cast<int64_t>(t.expert) * N;
-    if (bias != nullptr) bias += static_cast<int64_t>(t.expert) * N;
-    M = t.rows;
+  const int bx = at.bx, split = at.split;
+  int m0 = at.m0;
+  if (at.expert >= 0) {
+    // this tile belongs to one expert: shift every base to that expert and to
+    // the tile's first row, and let M be the rows that exist
+    x += static_cast<int64_t>(at.row0) * K;
+    if (p.nsplit > 1) outp = static_cast<float*>(outp) + static_cast<int64_t>(at.row0) * N;  // partial sums
+    else outp = static_cast<uint16_t*>(outp) + static_cast<int64_t>(at.row0) * (SWI ? N / 2 : N);
+    codes += static_cast<int64_t>(at.expert) * p.moe_codes_stride;
+    scale += static_cast<int64_t>(at.expert) * N;
+    if (bias != nullptr) bias += static_cast<int64_t>(at.expert) * N;
+    M = at.rows;
     m0 = 0;
   }
   // SWI: a workgroup takes BN / 2 gate columns and the BN / 2 up columns that go with them
@@ -968,7 +992,7 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_dma_kernel(const DmaParams 
     // partial sums are kept compact: row length = the columns of this launch
     const int64_t ld = p.nsplit > 1 ? static_cast<int64_t>(p.strip_hi - p.strip_lo) * kStripCols : N;
     const int ncol0 = p.nsplit > 1 ? p.strip_lo * kStripCols : 0;
-    const int64_t run_rows = p.moe_table != nullptr ? p.moe_rows : M;  // rows of one run's partial sums
+    const int64_t run_rows = at.expert >= 0 ? p.moe_rows : M;  // rows of one run's partial sums
     float* outf = static_cast<float*>(outp) + (p.nsplit > 1 ? static_cast<int64_t>(split) * run_rows * ld : 0);
 #pragma unroll
     for (int a = 0; a < TM; ++a)
@@ -1062,6 +1086,69 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_dma_kernel(const DmaParams 
   }
   leave_stamps();
 #endif
+}
+
+template <int DT, int BITS, int G, int OFFS, int WM, int WN, int TM, int TN, int STAGES, int SWI = 0, bool RESC = false,
+          bool STAMP = false>
+__global__ __launch_bounds__(64 * WM * WN) void gemm_dma_kernel(const DmaParams p) {
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  const int ntiles = p.nbx * p.nby;
+  TilePlace at;
+  at.split = blockIdx.x / ntiles;
+  int by;
+  tile_of_block_2d(blockIdx.x - at.split * ntiles, p.nbx, p.nby, p.xcd_rows, &at.bx, &by);
+  at.m0 = by * (WM * TM * 32);
+  at.expert = -1;
+  at.row0 = at.rows = 0;
+  if (p.moe_table != nullptr) {
+    const MoeTile t = reinterpret_cast<const MoeTile*>(p.moe_table)[by];
+    if (t.expert < 0) return;
+    at.expert = t.expert;
+    at.row0 = t.row0;
+    at.rows = t.rows;
+  }
+  dma_tile<DT, BITS, G, OFFS, WM, WN, TM, TN, STAGES, SWI, RESC, STAMP>(p, smem, at);
+}
+
+// The grouped GEMM over experts with many rows each: row tiles of up to four
+// 64-row units (256 rows), as many units as the tile has rows for.  A tile's
+// MFMAs, activation loads and operand reads follow its height, so an expert
+// whose row count is no multiple of the tile pays for 64-row padding only.
+// Workgroups are handed out expert by expert, column tile by column tile, all
+// row tiles of the expert next to each other, and that sequence is cut into
+// eight equal pieces, one per XCD: an expert's row tiles meet its weights in
+// one L2 while they are there, and the XCDs stay evenly loaded however the
+// rows are spread over the experts.
+// moe_ffn, 8 experts, hidden 4096, fc1 width 28672, rows spread unequally,
+// whole call, against whole tiles of 256 or 128 rows in runs of the average
+// expert's tiles per XCD: 4096 rows int4 2264 -> 1684 us, int8 2090 -> 1551;
+// 2048 rows int4 1311 -> 966, int8 1325 -> 892; 1024 rows 651 -> 591 and 666 ->
+// 552; 4 experts, width 14336, 4096 rows 1130 -> 789.
+template <int DT, int BITS, int OFFS, int TN, int STAGES, int SWI>
+__global__ __launch_bounds__(512) void gemm_experts_kernel(const DmaParams p) {
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  const MoeTile* table = reinterpret_cast<const MoeTile*>(p.moe_table);
+  const int total = table[0].expert * p.nbx;  // the header holds the number of row tiles
+  constexpr int kXcd = 8;
+  const int per = (total + kXcd - 1) / kXcd;
+  const int slot = blockIdx.x / kXcd, pos = (blockIdx.x % kXcd) * per + slot;
+  if (slot >= per || pos >= total) return;
+  // position / column tiles = some row tile of the position's expert
+  const MoeTile any = table[1 + pos / p.nbx];
+  const int w = pos - any.first * p.nbx;
+  const MoeTile t = table[1 + any.first + w % any.count];
+  TilePlace at;
+  at.bx = w / any.count;
+  at.m0 = 0;
+  at.split = 0;
+  at.expert = t.expert;
+  at.row0 = t.row0;
+  at.rows = t.rows;
+  const int units = (t.rows + 63) / 64;
+  if (units >= 4) dma_tile<DT, BITS, 0, OFFS, 2, 4, 4, TN, STAGES, SWI, false, false>(p, smem, at);
+  else if (units == 3) dma_tile<DT, BITS, 0, OFFS, 2, 4, 3, TN, STAGES, SWI, false, false>(p, smem, at);
+  else if (units == 2) dma_tile<DT, BITS, 0, OFFS, 2, 4, 2, TN, STAGES, SWI, false, false>(p, smem, at);
+  else dma_tile<DT, BITS, 0, OFFS, 2, 4, 1, TN, STAGES, SWI, false, false>(p, smem, at);
 }
 
 // out[m, col0 + c] = T( sum over the runs of part[run][m][c] + bias[col0 + c] ) for the ncols
@@ -1165,13 +1252,7 @@ __global__ __launch_bounds__(256) void reduce_partials_swiglu_kernel(
   }
 }
 
-struct Args {
-  const void* x; const void* codes; const void* bias; const void* scale; void* out;
-  int M, K, N, gshift, out_f32;
-  void* ws; size_t ws_bytes;  // scratch for split-K partial sums, may be null
-  hipStream_t stream;
-  int act;
-};
+typedef GemmArgs Args;
 
 // Raises a kernel's dynamic LDS limit once per device (the attribute belongs to
 // the device's copy of the function); safe to call from several threads.
@@ -1483,17 +1564,23 @@ void launch_fast(const Args& a) {
 #undef WOL_HALF
 }
 
-// Row-tile table of a grouped launch with tiles of `bm` rows.  cum[e] is the
-// number of rows of experts 0 .. e (the inclusive running total that the
-// reference's moe_dispatch returns as token_nums_per_expert,
+// Row-tile table of a grouped launch.  cum[e] is the number of rows of experts
+// 0 .. e (the inclusive running total that the reference's moe_dispatch returns
+// as token_nums_per_expert,
 // paddle/phi/kernels/fusion/cutlass/moe_dispatch.cu:174-182): expert e owns
-// rows cum[e-1] .. cum[e]-1 and ceil(rows / bm) tiles.  One workgroup; the
-// table has max_tiles entries, unused ones marked -1.
+// rows cum[e-1] .. cum[e]-1 and ceil(rows / bm) tiles.  One workgroup.
+// header == 0: tiles of bm rows, max_tiles entries, unused ones marked -1.
+// header == 1 (gemm_experts_kernel): entry 0 holds the number of tiles, and an
+// expert's rows are shared out in 64-row units as evenly as its ceil(rows /
+// bm) tiles allow (three tiles of 192 rows rather than two of 256 and one of
+// 64: the weight side of a tile costs the same whatever its height).
 __global__ __launch_bounds__(256) void moe_plan_kernel(const int64_t* __restrict__ cum, int num_experts, int bm,
-                                                       int max_tiles, int64_t rows, MoeTile* __restrict__ table) {
+                                                       int max_tiles, int64_t rows, int header,
+                                                       MoeTile* __restrict__ table) {
   __shared__ int first_tile[1025];  // exclusive running total of tiles, by expert
   __shared__ int row_end[1025];     // end of expert e's rows is row_end[e + 1]; row_end[0] = 0
-  for (int i = threadIdx.x; i < max_tiles; i += 256) table[i] = MoeTile{-1, 0, 0, 0};
+  if (header == 0)
+    for (int i = threadIdx.x; i < max_tiles; i += 256) table[i] = MoeTile{-1, 0, 0, 0, 0, {0, 0, 0}};
   if (threadIdx.x == 0) {
     // The running totals come from the device and are not trusted: each is
     // clamped to [previous total, rows], so an expert's count is never negative
@@ -1510,34 +1597,36 @@ __global__ __launch_bounds__(256) void moe_plan_kernel(const int64_t* __restrict
       row_end[e + 1] = static_cast<int>(end);
     }
     first_tile[num_experts] = acc;
+    if (header != 0) table[0] = MoeTile{acc < max_tiles ? acc : max_tiles, 0, 0, 0, 0, {0, 0, 0}};
   }
   __syncthreads();
   for (int e = threadIdx.x; e < num_experts; e += 256) {
     const int r0 = row_end[e], r1 = row_end[e + 1];
     const int t0 = first_tile[e], nt = first_tile[e + 1] - t0;
+    const int units = (r1 - r0 + 63) / 64;
+    int row = r0;
     for (int t = 0; t < nt && t0 + t < max_tiles; ++t) {
-      const int row = r0 + t * bm;
       const int left = r1 - row;
-      table[t0 + t] = MoeTile{e, row, left < bm ? left : bm, 0};
+      int h = bm;
+      if (header != 0) h = (units / nt + (t < units % nt ? 1 : 0)) * 64;
+      table[header + t0 + t] = MoeTile{e, row, left < h ? left : h, t0, nt, {0, 0, 0}};
+      row += h;
     }
   }
 }
 
 // Rows of a grouped launch's tiles, by the average number of rows per expert
-// (the host knows the total only; the per-expert counts stay on the device):
-// 128 x 256 tiles, or the small-M configurations' 64 x 256 (32 x 256 for int4)
-// when the experts have few rows each -- a decode step of a mixture of
-// experts -- where the large tile would do up to eight times the MFMA work
-// and hold one workgroup per CU where three fit.
-// From 512 rows per expert on, the 256 x 256 tile of the ungrouped prefill
-// launch (more MFMAs per dequantised fragment; a partial last tile per expert
-// then weighs little).
+// (the host knows the total only; the per-expert counts stay on the device).
+// Up to 64 rows each -- a decode step of a mixture of experts -- the small-M
+// configurations' 64 x 256 (32 x 256 for int4) tiles: a taller one would do up
+// to eight times the MFMA work and hold one workgroup per CU where three fit.
+// Above, gemm_experts_kernel with tiles of up to 256 rows.
+constexpr int kExpertsRows = 256;
 inline int moe_tile_rows(int64_t rows, int num_experts, int bits) {
   const int64_t avg = rows / (num_experts > 0 ? num_experts : 1);
   if (avg <= 32 && bits == 4) return 32;
   if (avg <= 64) return 64;
-  if (avg >= 512) return 256;
-  return 128;
+  return kExpertsRows;
 }
 
 // What a grouped launch needs besides the problem: the row-tile table, and
@@ -1546,25 +1635,22 @@ inline int moe_tile_rows(int64_t rows, int num_experts, int bits) {
 // of rows that belong to an expert.
 struct MoeLaunch {
   const int* table;
-  int max_tiles, bm, ns;
+  int max_tiles, bm, ns, experts;
   int64_t rows;
   float* partial;
   const int64_t* valid_rows;
-  int tiles_per_expert = 0;  // > 0: row tiles an expert has on average; its tiles then share an XCD (max_tiles a multiple of 8 x this)
 };
 
 // One grouped GEMM: every expert's rows against that expert's weights, tiles
 // of WM * TM * 32 rows x 256 columns, per-channel scales, out [rows, N] T.
-// SWI = 2: the swiglu of the fc1 output is formed in the epilogue and out is
-// [rows, N / 2] (the configurations with two blocks per wavefront).
-template <int DT, int BITS, int OFFS, int WM, int WN, int TM, int TN, int STAGES, int SWI = 0>
+template <int DT, int BITS, int OFFS, int WM, int WN, int TM, int TN, int STAGES>
 void launch_moe_gemm_cfg(const void* x, const MoeLaunch& ml, const void* codes, const void* bias,
                          const void* scale, int64_t K, int64_t N, void* out, hipStream_t stream) {
   const int* table = ml.table;
   const int max_tiles = ml.max_tiles;
-  constexpr int BN = (SWI ? 1 : TN) * WN * 32;  // output columns of a tile
+  constexpr int BN = TN * WN * 32;  // output columns of a tile
   constexpr size_t lds = dma_lds_bytes<BITS, 0, WM, WN, TM, TN, STAGES>();
-  auto kern = gemm_dma_kernel<DT, BITS, 0, OFFS, WM, WN, TM, TN, STAGES, SWI>;
+  auto kern = gemm_dma_kernel<DT, BITS, 0, OFFS, WM, WN, TM, TN, STAGES>;
   static std::atomic<uint32_t> configured{0};
   allow_lds(reinterpret_cast<const void*>(kern), lds, configured);
   DmaParams p;
@@ -1573,15 +1659,13 @@ void launch_moe_gemm_cfg(const void* x, const MoeLaunch& ml, const void* codes, 
   p.bias = static_cast<const uint16_t*>(bias);
   p.scale = static_cast<const uint16_t*>(scale);
   const int tiles = static_cast<int>(K / (BITS == 8 ? 64 : 128));
-  const int ns = !SWI && bias == nullptr && ml.partial != nullptr ? ml.ns : 1;
+  const int ns = bias == nullptr && ml.partial != nullptr ? ml.ns : 1;
   p.M = WM * TM * 32; p.K = static_cast<int>(K); p.N = static_cast<int>(N);
   p.out_f32 = 0;
-  const int64_t out_cols = SWI ? N / 2 : N;
-  p.strip_lo = 0; p.strip_hi = static_cast<int>(out_cols / kStripCols);
-  p.nbx = static_cast<int>((out_cols + BN - 1) / BN);
+  p.strip_lo = 0; p.strip_hi = static_cast<int>(N / kStripCols);
+  p.nbx = static_cast<int>((N + BN - 1) / BN);
   p.nby = max_tiles;
   p.xcd_rows = 0;
-  if (ml.tiles_per_expert > 0 && max_tiles % (8 * ml.tiles_per_expert) == 0) p.xcd_rows = -ml.tiles_per_expert;
   p.tiles_per_split = (tiles + ns - 1) / ns;
   p.nsplit = (tiles + p.tiles_per_split - 1) / p.tiles_per_split;
   p.out = p.nsplit > 1 ? static_cast<void*>(ml.partial) : out;
@@ -1599,22 +1683,68 @@ void launch_moe_gemm_cfg(const void* x, const MoeLaunch& ml, const void* codes, 
   }
 }
 
-// Whether the grouped GEMM with tiles of bm rows forms the swiglu of its output itself.
-inline bool moe_fuses_swiglu(int bm) { return bm >= 128; }
+// The grouped GEMM on tiles of up to 256 rows x 256 (TN = 2) or 128 (TN = 1)
+// columns.  SWI = 2: the swiglu of the product is formed in the epilogue, out
+// is [rows, N / 2] and a tile has half as many output columns.
+template <int DT, int BITS, int TN, int SWI>
+void launch_experts_cfg(const void* x, const MoeLaunch& ml, const void* codes, const void* bias, const void* scale,
+                        int64_t K, int64_t N, void* out, hipStream_t stream) {
+  // as the ungrouped launch chooses: int4 under bf16 takes the offset dequantiser with row sums by dot products;
+  // two stages of 128-deep int4 tiles fill the LDS
+  constexpr int kOffs = BITS == 4 && DT == WOL_DTYPE_BF16 ? 2 : 0;
+  constexpr int kStages = BITS == 8 ? 3 : 2;
+  constexpr int BN = (SWI ? 1 : TN) * 128;  // output columns of a tile
+  constexpr size_t lds = dma_lds_bytes<BITS, 0, 2, 4, 4, TN, kStages>();
+  auto kern = gemm_experts_kernel<DT, BITS, kOffs, TN, kStages, SWI>;
+  static std::atomic<uint32_t> configured{0};
+  allow_lds(reinterpret_cast<const void*>(kern), lds, configured);
+  DmaParams p;
+  p.x = static_cast<const uint16_t*>(x);
+  p.codes = static_cast<const uint8_t*>(codes);
+  p.bias = static_cast<const uint16_t*>(bias);
+  p.scale = static_cast<const uint16_t*>(scale);
+  p.out = out;
+  p.M = kExpertsRows; p.K = static_cast<int>(K); p.N = static_cast<int>(N);
+  p.out_f32 = 0;
+  const int64_t out_cols = SWI ? N / 2 : N;
+  p.strip_lo = 0; p.strip_hi = static_cast<int>(out_cols / kStripCols);
+  p.nbx = static_cast<int>((out_cols + BN - 1) / BN);
+  p.nby = ml.max_tiles;
+  p.nsplit = 1;
+  p.tiles_per_split = static_cast<int>(K / (BITS == 8 ? 64 : 128));
+  p.xcd_rows = 0;
+  p.act = WOL_ACT_NONE;
+  p.moe_table = ml.table;
+  p.moe_codes_stride = K * N * BITS / 8;
+  p.moe_rows = static_cast<int>(ml.rows);
+  p.stamps = nullptr;
+  const int64_t blocks = (static_cast<int64_t>(p.nbx) * p.nby + 7) / 8 * 8;  // the XCDs' shares are rounded up
+  kern<<<dim3(static_cast<unsigned>(blocks)), dim3(512), lds, stream>>>(p);
+}
+
+// Whether a grouped product of N columns takes 128-column tiles instead of 256:
+// only where the 256-column ones would leave CUs without work and twice as
+// many still run in about one round.  The number of row tiles is not known on
+// the host; an expert with a rows on average has max(1, a / 256 + 0.4).
+// (K = 14336, N = 4096, 8 experts, int4 / int8, 256 against 128 columns: whole
+// call at 600 rows 419 / 445 against 366 / 419 us, 1024 rows 674 / 591 against
+// 591 / 552, 1500 rows at K = 7168 387 / 348 against 338 / 328, 2048 rows
+// 966 / 892 against 1091 / 977; level at 4096.)
+inline bool experts_narrow(int64_t rows, int num_experts, int64_t N) {
+  const double avg = static_cast<double>(rows) / num_experts;
+  const double tiles = num_experts * (avg > 0.6 * 256 ? avg / 256 + 0.4 : 1.0);
+  return tiles * static_cast<double>((N + 255) / 256) <= 0.62 * num_cus();
+}
 
 // ml.bm: the tile rows the table was built for (moe_tile_rows).  swiglu: out is
-// [rows, N / 2], the swiglu of the product (only where moe_fuses_swiglu(ml.bm)).
+// [rows, N / 2], the swiglu of the product (tiles of 256 rows only).
 template <int DT, int BITS>
 void launch_moe_gemm(const void* x, const MoeLaunch& ml, const void* codes, const void* bias,
                      const void* scale, int64_t K, int64_t N, void* out, hipStream_t stream, bool swiglu = false) {
-  constexpr bool kOffs = BITS == 4 && DT == WOL_DTYPE_BF16;  // as the ungrouped launch chooses
-  constexpr int kBigOffs = kOffs ? 2 : 0;           // the 256-row tile: row sums by dot products
-  constexpr int kBigStages = BITS == 8 ? 3 : 2;     // 128-deep int4 tiles: two stages fill the LDS
-  if (swiglu) {
-    if (ml.bm == 256)
-      launch_moe_gemm_cfg<DT, BITS, kBigOffs, 2, 4, 4, 2, kBigStages, 2>(x, ml, codes, bias, scale, K, N, out, stream);
-    else
-      launch_moe_gemm_cfg<DT, BITS, kOffs, 2, 4, 2, 2, 3, 2>(x, ml, codes, bias, scale, K, N, out, stream);
+  if (ml.bm == kExpertsRows) {
+    if (swiglu) launch_experts_cfg<DT, BITS, 2, 2>(x, ml, codes, bias, scale, K, N, out, stream);
+    else if (experts_narrow(ml.rows, ml.experts, N)) launch_experts_cfg<DT, BITS, 1, 0>(x, ml, codes, bias, scale, K, N, out, stream);
+    else launch_experts_cfg<DT, BITS, 2, 0>(x, ml, codes, bias, scale, K, N, out, stream);
     return;
   }
   if constexpr (BITS == 4) {
@@ -1623,21 +1753,14 @@ void launch_moe_gemm(const void* x, const MoeLaunch& ml, const void* codes, cons
       return;
     }
   }
-  if (ml.bm == 256) {
-    launch_moe_gemm_cfg<DT, BITS, kBigOffs, 2, 4, 4, 2, kBigStages>(x, ml, codes, bias, scale, K, N, out, stream);
-    return;
-  }
-  if (ml.bm == 64)
-    launch_moe_gemm_cfg<DT, BITS, false, 1, 8, 2, 1, 2>(x, ml, codes, bias, scale, K, N, out, stream);
-  else
-    launch_moe_gemm_cfg<DT, BITS, kOffs, 2, 4, 2, 2, 3>(x, ml, codes, bias, scale, K, N, out, stream);
+  launch_moe_gemm_cfg<DT, BITS, false, 1, 8, 2, 1, 2>(x, ml, codes, bias, scale, K, N, out, stream);
 }
 
 // K runs of a grouped launch with small tiles: as many as bring the workgroups
 // (column tiles x row tiles x runs) to the CU count, at most 4, each of at
 // least 8 k tiles.  The large tile is not split.
 inline int moe_runs(int64_t K, int64_t N, int bits, int bm, int max_tiles) {
-  if (bm >= 128) return 1;
+  if (bm == kExpertsRows) return 1;
   const int64_t tiles = K / (bits == 8 ? 64 : 128), wgs = (N + 255) / 256 * max_tiles;
   int ns = static_cast<int>((num_cus() + wgs - 1) / wgs);
   ns = ns > 4 ? 4 : ns;
@@ -1662,7 +1785,60 @@ void launch_cfg(const Args& a) {
   }
 }
 
+// out [M, N / 2] = T(swiglu(x . W + bias)) in one launch
+template <int DT, int BITS, int G>
+void launch_swiglu_gemm(const Args& a) {
+  const int gate_strips = a.N / 2 / kStripCols;
+  if constexpr (G != 0) {
+    // group-wise scales: the tiles with two blocks per wavefront and rescaled sums
+    if constexpr (BITS == 8) {
+      if (a.M >= 192) launch_dma<DT, 8, G, 0, 2, 4, 4, 2, 3, 1, true>(a, 0, gate_strips, 1);
+      else launch_dma<DT, 8, G, 0, 2, 4, 2, 2, 3, 1, true>(a, 0, gate_strips, 1);
+    } else {
+      // (256 x 128 tiles: gate and up blocks in neighbouring wavefronts)
+      if (tall_half_tile(a.M)) launch_dma<DT, 4, G, 0, 2, 4, 4, 1, 2, 1, true>(a, 0, gate_strips, 1);
+      else launch_dma<DT, 4, G, 0, 2, 4, 2, 2, 2, 1, true>(a, 0, gate_strips, 1);
+    }
+  } else if constexpr (BITS == 8) {
+    if (a.M >= 192) launch_dma<DT, 8, 0, false, 2, 4, 4, 2, 3, 1>(a, 0, gate_strips, 1);
+    else launch_dma<DT, 8, 0, false, 2, 4, 2, 2, 3, 1>(a, 0, gate_strips, 1);
+  } else {
+    if (a.M >= 192) launch_dma<DT, 4, 0, DT == WOL_DTYPE_BF16 ? 2 : 0, 2, 4, 4, 2, 2, 1>(a, 0, gate_strips, 1);
+    else launch_dma<DT, 4, 0, DT == WOL_DTYPE_BF16 ? 1 : 0, 2, 4, 2, 2, 3, 1>(a, 0, gate_strips, 1);
+  }
+}
+template <int DT, int BITS>
+void launch_swiglu_gemm_g(const Args& a) {
+  if (a.gshift < 0) launch_swiglu_gemm<DT, BITS, 0>(a);
+  else if (a.gshift == 6) launch_swiglu_gemm<DT, BITS, 64>(a);
+  else launch_swiglu_gemm<DT, BITS, 128>(a);
+}
+
 }  // namespace
+
+#define WOL_CAT_(a, b) a##b
+#define WOL_CAT(a, b) WOL_CAT_(a, b)
+#if defined(WOL_GEMM_F16_UNIT)
+#define WOL_TYPED(name) WOL_CAT(name, _f16)
+#else
+#define WOL_TYPED(name) WOL_CAT(name, _bf16)
+#endif
+
+void WOL_TYPED(gemm)(const GemmArgs& a, int bits) {
+  if (bits == 8) launch_cfg<WOL_GEMM_DTYPE, 8>(a); else launch_cfg<WOL_GEMM_DTYPE, 4>(a);
+}
+
+void WOL_TYPED(swiglu_gemm)(const GemmArgs& a, int bits) {
+  if (bits == 8) launch_swiglu_gemm_g<WOL_GEMM_DTYPE, 8>(a); else launch_swiglu_gemm_g<WOL_GEMM_DTYPE, 4>(a);
+}
+
+void WOL_TYPED(moe_gemm)(const MoeGemmArgs& a, int bits) {
+  const MoeLaunch ml{a.table, a.max_tiles, a.bm, a.ns, a.experts, a.rows, a.partial, a.valid_rows};
+  if (bits == 8) launch_moe_gemm<WOL_GEMM_DTYPE, 8>(a.x, ml, a.codes, a.bias, a.scale, a.K, a.N, a.out, a.stream, a.swiglu);
+  else launch_moe_gemm<WOL_GEMM_DTYPE, 4>(a.x, ml, a.codes, a.bias, a.scale, a.K, a.N, a.out, a.stream, a.swiglu);
+}
+
+#if !defined(WOL_GEMM_F16_UNIT)
 
 int launch_reduce_partials(const float* part, int nsplit, const void* bias, int dtype, void* out,
                            bool out_f32, int64_t M, int64_t N, int act, hipStream_t stream) {
@@ -1750,37 +1926,6 @@ bool linear_gemm_fuses_swiglu(int64_t M, int64_t K, int64_t N, int bits, int gro
                      group_size > 0 ? group_size : 0, SIZE_MAX).ns > 1;
 }
 
-namespace {
-// out [M, N / 2] = T(swiglu(x . W + bias)) in one launch
-template <int DT, int BITS, int G>
-void launch_swiglu_gemm(const Args& a) {
-  const int gate_strips = a.N / 2 / kStripCols;
-  if constexpr (G != 0) {
-    // group-wise scales: the tiles with two blocks per wavefront and rescaled sums
-    if constexpr (BITS == 8) {
-      if (a.M >= 192) launch_dma<DT, 8, G, 0, 2, 4, 4, 2, 3, 1, true>(a, 0, gate_strips, 1);
-      else launch_dma<DT, 8, G, 0, 2, 4, 2, 2, 3, 1, true>(a, 0, gate_strips, 1);
-    } else {
-      // (256 x 128 tiles: gate and up blocks in neighbouring wavefronts)
-      if (tall_half_tile(a.M)) launch_dma<DT, 4, G, 0, 2, 4, 4, 1, 2, 1, true>(a, 0, gate_strips, 1);
-      else launch_dma<DT, 4, G, 0, 2, 4, 2, 2, 2, 1, true>(a, 0, gate_strips, 1);
-    }
-  } else if constexpr (BITS == 8) {
-    if (a.M >= 192) launch_dma<DT, 8, 0, false, 2, 4, 4, 2, 3, 1>(a, 0, gate_strips, 1);
-    else launch_dma<DT, 8, 0, false, 2, 4, 2, 2, 3, 1>(a, 0, gate_strips, 1);
-  } else {
-    if (a.M >= 192) launch_dma<DT, 4, 0, DT == WOL_DTYPE_BF16 ? 2 : 0, 2, 4, 4, 2, 2, 1>(a, 0, gate_strips, 1);
-    else launch_dma<DT, 4, 0, DT == WOL_DTYPE_BF16 ? 1 : 0, 2, 4, 2, 2, 3, 1>(a, 0, gate_strips, 1);
-  }
-}
-template <int DT, int BITS>
-void launch_swiglu_gemm_g(const Args& a) {
-  if (a.gshift < 0) launch_swiglu_gemm<DT, BITS, 0>(a);
-  else if (a.gshift == 6) launch_swiglu_gemm<DT, BITS, 64>(a);
-  else launch_swiglu_gemm<DT, BITS, 128>(a);
-}
-}  // namespace
-
 // f.act == WOL_ACT_SWIGLU (only where linear_gemm_fuses_swiglu): out is [M, N / 2] T.
 int launch_linear_gemm(const void* x, const void* codes, const void* bias, const void* scale,
                        int dtype, int64_t M, int64_t K, int64_t N, int bits, int group_size,
@@ -1795,18 +1940,10 @@ int launch_linear_gemm(const void* x, const void* codes, const void* bias, const
     if (workspace == nullptr || workspace_bytes < linear_gemm_workspace(M, K, N, bits, group_size)) return WOL_ERR_WORKSPACE;
   } else if (f.act == WOL_ACT_SWIGLU) {
     if (out_f32 || !linear_gemm_fuses_swiglu(M, K, N, bits, group_size)) return WOL_ERR_BAD_SHAPE;
-    if (dtype == WOL_DTYPE_BF16) {
-      if (bits == 8) launch_swiglu_gemm_g<WOL_DTYPE_BF16, 8>(a); else launch_swiglu_gemm_g<WOL_DTYPE_BF16, 4>(a);
-    } else {
-      if (bits == 8) launch_swiglu_gemm_g<WOL_DTYPE_F16, 8>(a); else launch_swiglu_gemm_g<WOL_DTYPE_F16, 4>(a);
-    }
+    if (dtype == WOL_DTYPE_BF16) swiglu_gemm_bf16(a, bits); else swiglu_gemm_f16(a, bits);
     return check_launch();
   }
-  if (dtype == WOL_DTYPE_BF16) {
-    if (bits == 8) launch_cfg<WOL_DTYPE_BF16, 8>(a); else launch_cfg<WOL_DTYPE_BF16, 4>(a);
-  } else {
-    if (bits == 8) launch_cfg<WOL_DTYPE_F16, 8>(a); else launch_cfg<WOL_DTYPE_F16, 4>(a);
-  }
+  if (dtype == WOL_DTYPE_BF16) gemm_bf16(a, bits); else gemm_f16(a, bits);
   return check_launch();
 }
 
@@ -1824,7 +1961,7 @@ static int moe_max_tiles(int64_t rows, int num_experts, int bm) {
 size_t moe_ffn_workspace(int64_t rows, int64_t hidden, int64_t inter, int num_experts) {
   // (the table at its longest: 32-row tiles; the runs' sums whenever either bit width would use small tiles)
   const bool small = moe_tile_rows(rows, num_experts, 4) < 128;
-  return moe_up(static_cast<size_t>(moe_max_tiles(rows, num_experts, 32)) * sizeof(MoeTile)) +
+  return moe_up((static_cast<size_t>(moe_max_tiles(rows, num_experts, 32)) + 1) * sizeof(MoeTile)) +
          moe_up(static_cast<size_t>(rows) * inter * 2) + moe_up(static_cast<size_t>(rows) * (inter / 2) * 2) +
          (small ? moe_up(static_cast<size_t>(kMoeMaxRuns) * rows * hidden * sizeof(float)) : 0);
 }
@@ -1835,42 +1972,27 @@ int launch_moe_ffn(const void* x, const int64_t* rows_before_expert, const void*
                    int num_experts, int bits, void* out, void* workspace, hipStream_t stream) {
   unsigned char* ws = static_cast<unsigned char*>(workspace);
   const int bm = moe_tile_rows(rows, num_experts, bits);
-  int max_tiles = moe_max_tiles(rows, num_experts, bm);
-  // large tiles (one workgroup per CU): an expert's row tiles and all their column tiles on one XCD.  The
-  // table (sized for 32-row tiles) has room for the padding of its length to a multiple of 8 experts' tiles.
-  int tpe = 0;
-  if (bm >= 128) {
-    tpe = static_cast<int>((rows / (num_experts > 0 ? num_experts : 1) + bm - 1) / bm);
-    tpe = tpe < 1 ? 1 : tpe;
-    const int padded = (max_tiles + 8 * tpe - 1) / (8 * tpe) * (8 * tpe);
-    if (padded <= moe_max_tiles(rows, num_experts, 32)) max_tiles = padded; else tpe = 0;
-  }
+  const int max_tiles = moe_max_tiles(rows, num_experts, bm);
+  const bool experts = bm == kExpertsRows;
   MoeTile* table = reinterpret_cast<MoeTile*>(ws);
-  unsigned char* fc1 = ws + moe_up(static_cast<size_t>(moe_max_tiles(rows, num_experts, 32)) * sizeof(MoeTile));
+  unsigned char* fc1 = ws + moe_up((static_cast<size_t>(moe_max_tiles(rows, num_experts, 32)) + 1) * sizeof(MoeTile));
   unsigned char* act = fc1 + moe_up(static_cast<size_t>(rows) * inter * 2);
   float* partial = reinterpret_cast<float*>(act + moe_up(static_cast<size_t>(rows) * (inter / 2) * 2));
-  // the second GEMM has hidden / 256 column tiles only: K (= inter / 2) in runs when the tiles are small
-  const MoeLaunch l1{reinterpret_cast<const int*>(table), max_tiles, bm, 1, rows, nullptr, nullptr, tpe};
-  const MoeLaunch l2{reinterpret_cast<const int*>(table), max_tiles, bm, moe_runs(inter / 2, hidden, bits, bm, max_tiles),
-                     rows, bm < 128 ? partial : nullptr, rows_before_expert + (num_experts - 1), tpe};
-  moe_plan_kernel<<<dim3(1), dim3(256), 0, stream>>>(rows_before_expert, num_experts, bm, max_tiles, rows, table);
-#define WOL_MOE(DT, B)                                                                                        \
-  do {                                                                                                        \
-    if (moe_fuses_swiglu(bm)) {                                                                               \
-      launch_moe_gemm<DT, B>(x, l1, ffn1_codes, ffn1_bias, ffn1_scale, hidden, inter, act, stream, true);     \
-    } else {                                                                                                  \
-      launch_moe_gemm<DT, B>(x, l1, ffn1_codes, ffn1_bias, ffn1_scale, hidden, inter, fc1, stream);           \
-      const int rc = launch_swiglu_t(fc1, dtype, rows, inter, act, stream);                                   \
-      if (rc != WOL_OK) return rc;                                                                            \
-    }                                                                                                         \
-    launch_moe_gemm<DT, B>(act, l2, ffn2_codes, nullptr, ffn2_scale, inter / 2, hidden, out, stream); \
-  } while (0)
-  if (dtype == WOL_DTYPE_BF16) {
-    if (bits == 8) WOL_MOE(WOL_DTYPE_BF16, 8); else WOL_MOE(WOL_DTYPE_BF16, 4);
-  } else {
-    if (bits == 8) WOL_MOE(WOL_DTYPE_F16, 8); else WOL_MOE(WOL_DTYPE_F16, 4);
+  moe_plan_kernel<<<dim3(1), dim3(256), 0, stream>>>(rows_before_expert, num_experts, bm, max_tiles, rows, experts ? 1 : 0, table);
+  const auto product = [&](const MoeGemmArgs& a) {
+    if (dtype == WOL_DTYPE_BF16) moe_gemm_bf16(a, bits); else moe_gemm_f16(a, bits);
+  };
+  const int* tab = reinterpret_cast<const int*>(table);
+  product(MoeGemmArgs{x, tab, max_tiles, bm, 1, num_experts, rows, nullptr, nullptr, ffn1_codes, ffn1_bias, ffn1_scale,
+                      hidden, inter, experts ? act : fc1, stream, experts});
+  if (!experts) {
+    const int rc = launch_swiglu_t(fc1, dtype, rows, inter, act, stream);
+    if (rc != WOL_OK) return rc;
   }
-#undef WOL_MOE
+  // the second product has hidden / 256 column tiles only: K (= inter / 2) in runs when the tiles are small
+  product(MoeGemmArgs{act, tab, max_tiles, bm, moe_runs(inter / 2, hidden, bits, bm, max_tiles), num_experts, rows,
+                      experts ? nullptr : partial, rows_before_expert + (num_experts - 1), ffn2_codes, nullptr, ffn2_scale,
+                      inter / 2, hidden, out, stream, false});
   return check_launch();
 }
 
@@ -2089,5 +2211,7 @@ int launch_mfma_probe(int variant, const void* ops, int workgroups, int iters, f
   }
   return check_launch();
 }
+
+#endif  // !WOL_GEMM_F16_UNIT
 
 }  // namespace wol

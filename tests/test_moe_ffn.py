@@ -127,3 +127,36 @@ def test_moe_ffn_equals_per_expert_calls(device):
         Q.moe_ffn(x, cum, q1, q2, None, s1, s2, "None")
     with pytest.raises(ValueError):
         Q.moe_ffn(x, cum.int(), q1, q2, None, s1, s2, "weight_only_int8")
+
+
+@pytest.mark.parametrize("dt", [H.F16, H.BF16])
+@pytest.mark.parametrize("bits", [8, 4])
+@pytest.mark.parametrize("hidden", [256, 4096])  # second product on 128-column and on 256-column tiles
+def test_moe_ffn_tile_heights(device, dt, bits, hidden):
+    # experts with many rows take row tiles of one to four 64-row units: row counts on both sides of every
+    # unit and of one and two whole tiles, an expert without rows, and rows behind the last expert's
+    import torch
+    from paddle_amd.nn import quant as Q
+
+    inter = 512
+    per = [1, 63, 64, 65, 128, 129, 192, 0, 193, 256, 257, 320, 511, 513]
+    E, T = len(per), torch.bfloat16 if dt == H.BF16 else torch.float16
+    gen = torch.Generator(device="cuda").manual_seed(11)
+    algo, wd = ("weight_only_int8", "int8") if bits == 8 else ("weight_only_int4", "int4")
+    q1, s1 = Q.moe_quantize_experts((torch.randn(E, hidden, inter, device="cuda", generator=gen) * 0.02).to(T), algo)
+    q2, s2 = Q.moe_quantize_experts((torch.randn(E, inter // 2, hidden, device="cuda", generator=gen) * 0.02).to(T), algo)
+    b1 = torch.randn(E, inter, device="cuda", generator=gen).to(T)
+    cum = torch.tensor(np.cumsum(per), dtype=torch.int64, device="cuda")
+    x = torch.randn(sum(per) + 5, hidden, device="cuda", generator=gen).to(T)
+    out = Q.moe_ffn(x, cum, q1, q2, b1, s1, s2, algo)
+    prev = 0
+    for e, n in enumerate(per):
+        if n:
+            fc1 = Q.weight_only_linear(x[prev:prev + n], q1[e], b1[e], s1[e], wd)
+            act = (torch.nn.functional.silu(fc1[:, : inter // 2].float()) * fc1[:, inter // 2:].float()).to(T)
+            ref = Q.weight_only_linear(act, q2[e], None, s2[e], wd)
+            # same fp32 sums to their order, rounded to T in the same places: only roundings that fall the other
+            # way differ, each by a T ulp (2^-8 bf16, 2^-11 f16), in a few percent of the elements at most
+            err = float((out[prev:prev + n].float() - ref.float()).norm() / ref.float().norm())
+            assert err <= (2e-3 if dt == H.BF16 else 2.5e-4), (e, n, err)
+        prev += n
