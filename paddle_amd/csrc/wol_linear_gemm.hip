@@ -516,6 +516,15 @@ struct MoeTile {
 // The work of one workgroup is a device function (dma_tile) of where its tile
 // lies: gemm_dma_kernel below calls it for the one tile height it is built
 // for, gemm_experts_kernel picks the height of every tile at run time.
+// kHalfDeep (STAGES = kHalfDeepStages + 3; int4): three stages of 64-deep tiles
+// of activations (and scales) where two 128-deep ones would overflow the LDS.
+// The packed weight still arrives in its 128-deep tiles of 16 bytes per lane:
+// they have two buffers of their own, an odd k tile's loads bring the first half
+// (by strips) of the next raw tile and the even one's the second, and the codes
+// of a raw tile are read into registers once for both k tiles.  Every stage has
+// the same number of loads, so the counted waits are those of the other forms.
+constexpr int kHalfDeepStages = 10;
+
 struct TilePlace {
   int bx;      // column tile of the launch
   int m0;      // first row of the tile, counted from x and out
@@ -530,17 +539,23 @@ __device__ __forceinline__ void dma_tile(const DmaParams& p, unsigned char* smem
 #if defined(__HIP_DEVICE_COMPILE__)  // the host pass only needs the launch stubs
   constexpr int NW = WM * WN;
   constexpr int BM = WM * TM * 32, BN = WN * TN * 32;
-  constexpr int TK = BITS == 8 ? 64 : 128;       // k per 16-byte lane load of B
+  constexpr bool kHalfDeep = STAGES > kHalfDeepStages;  // int4, 64-deep k tiles: see the comment above
+  static_assert(!kHalfDeep || (BITS == 4 && STAGES == kHalfDeepStages + 3), "half-deep tiles: int4, three stages");
+  constexpr int TK = BITS == 8 || kHalfDeep ? 64 : 128;  // k per tile
   constexpr int kDw = BITS == 8 ? 2 : 1;         // dwords per 8 codes
   constexpr int C = TK / 8;                      // 16-byte pieces per A row
   constexpr int kABytes = BM * TK * 2;           // one A tile
   constexpr int kBBytes = (BN / 16) * 1024;      // one raw B tile (all strips of the workgroup)
   constexpr int kSBytes = G == 0 ? 0 : NW * 256;  // the tile's group scales: 128 values per wavefront
-  constexpr int kStage = kABytes + kBBytes + kSBytes;
-  constexpr int kStages = STAGES;  // k tiles resident or in flight
+  constexpr int kScaleOff = kABytes + (kHalfDeep ? 0 : kBBytes);  // the scales' place in a stage
+  constexpr int kStage = kScaleOff + kSBytes;
+  constexpr int kStages = STAGES % kHalfDeepStages;  // k tiles resident or in flight
+  constexpr int kLds = kStages * kStage + (kHalfDeep ? 2 * kBBytes : 0);
   static_assert(kStages == 2 || kStages == 3, "two or three stages");
   constexpr int kALoads = kABytes / 1024 / NW;   // wave-level loads (1 KiB each) per wavefront
-  constexpr int kBLoads = BN / 16 / NW;
+  constexpr int kBSlots = BN / 16 / NW;          // wave-level loads of a raw B tile per wavefront
+  constexpr int kBLoads = kHalfDeep ? kBSlots / 2 : kBSlots;  // of them in one stage's loads
+  static_assert(!kHalfDeep || kBSlots % 2 == 0, "a raw B tile travels in two equal halves");
   static_assert(kABytes / 1024 % NW == 0 && kALoads >= 1, "A tile must split evenly over the wavefronts");
   static_assert(BN / 16 % NW == 0 && kBLoads >= 1, "B tile must split evenly over the wavefronts");
   constexpr int Q = TK / 16;  // 16-k slices (one MFMA per 32x32 block each) per tile
@@ -615,9 +630,9 @@ __device__ __forceinline__ void dma_tile(const DmaParams& p, unsigned char* smem
     m = m < M ? m : M - 1;  // rows past M are computed on valid data and never stored
     asrc[c] = x + static_cast<int64_t>(m) * K + static_cast<int64_t>(t0) * TK + cc * 8;
   }
-  const uint8_t* bsrc[kBLoads];
+  const uint8_t* bsrc[kBSlots];
 #pragma unroll
-  for (int c = 0; c < kBLoads; ++c) {
+  for (int c = 0; c < kBSlots; ++c) {
     int st = strip_blk + c * NW + wave;
     if (SWI) {
       // LDS slot L of the B tile serves wavefront column L / 4, block (L / 2) % 2, half L % 2
@@ -627,8 +642,10 @@ __device__ __forceinline__ void dma_tile(const DmaParams& p, unsigned char* smem
     st = st < nstrips ? st : nstrips - 1;  // past the last column: valid data, never stored
     if (SWI && ((c * NW + wave) / 2) % 2 == 1) st += up_strips;  // block 1: the up columns
     bsrc[c] = codes + static_cast<int64_t>(st) * strip_bytes(K, BITS) +
-              static_cast<int64_t>(t0) * 1024 + lane * 16;
+              static_cast<int64_t>(kHalfDeep ? t0 / 2 : t0) * 1024 + lane * 16;
   }
+  unsigned char* const braw_lds = smem + kStages * kStage;  // kHalfDeep: the two raw B tiles
+  const int npairs = niter / 2;                             // kHalfDeep: raw B tiles of the run
   const int swz = a_swizzle<C>(lane & 15);  // fragment rows are 32*t + r32; the swizzle has period 16
 
   // Group scales travel with the tile: value v = 2 * (64 * wave + lane) of the
@@ -647,26 +664,44 @@ __device__ __forceinline__ void dma_tile(const DmaParams& p, unsigned char* smem
   scol = scol < (SWI ? N : n_hi) ? scol : n_hi - 2;  // past the last column: valid data, never used
   // Loads lo .. hi-1 of tile `it` into its stage; a stage's loads are numbered
   // [scales,] A loads, B loads.
-  auto issue_range = [&](int it, int lo, int hi) {
+  auto issue_range = [&](int it, int lo, int hi, bool odd) {  // odd: parity of it, a constant where it is called
     const int t = tile_index(it);  // past the end: reload the last tile into a spare stage
     unsigned char* stage = smem + (it % kStages) * kStage;
     constexpr int kS = G == 0 ? 0 : 1;
     if (G != 0 && lo == 0 && hi > 0) {
       const int64_t row = (static_cast<int64_t>(t0 + t) * TK + sfold * kFoldK) >> kGShift;
       __builtin_amdgcn_global_load_lds(scale + row * N + scol,
-                                       (lds_ptr_t)(stage + kABytes + kBBytes + wave * 256), 4, 0, 0);
+                                       (lds_ptr_t)(stage + kScaleOff + wave * 256), 4, 0, 0);
     }
 #pragma unroll
     for (int c = 0; c < kALoads; ++c)
       if (kS + c >= lo && kS + c < hi)
         __builtin_amdgcn_global_load_lds(asrc[c] + t * TK, (lds_ptr_t)(stage + (c * NW + wave) * 1024), 16, 0, 0);
+    if constexpr (kHalfDeep) {
+      // tile 2T - 1 brings the first half of raw B tile T, tile 2T the second (past the end: the last one again,
+      // into a buffer that nobody reads any more)
+      const int T = (it + 1) / 2, src = T < npairs ? T : npairs - 1;
+      unsigned char* dst = braw_lds + (T & 1) * kBBytes;
+      if (odd) {
 #pragma unroll
-    for (int c = 0; c < kBLoads; ++c)
-      if (kS + kALoads + c >= lo && kS + kALoads + c < hi)
-        __builtin_amdgcn_global_load_lds(bsrc[c] + t * 1024,
-                                         (lds_ptr_t)(stage + kABytes + (c * NW + wave) * 1024), 16, 0, 0);
+        for (int c = 0; c < kBLoads; ++c)
+          if (kS + kALoads + c >= lo && kS + kALoads + c < hi)
+            __builtin_amdgcn_global_load_lds(bsrc[c] + src * 1024, (lds_ptr_t)(dst + (c * NW + wave) * 1024), 16, 0, 0);
+      } else {
+#pragma unroll
+        for (int c = 0; c < kBLoads; ++c)
+          if (kS + kALoads + c >= lo && kS + kALoads + c < hi)
+            __builtin_amdgcn_global_load_lds(bsrc[kBLoads + c] + src * 1024,
+                                             (lds_ptr_t)(dst + ((kBLoads + c) * NW + wave) * 1024), 16, 0, 0);
+      }
+    } else {
+#pragma unroll
+      for (int c = 0; c < kBLoads; ++c)
+        if (kS + kALoads + c >= lo && kS + kALoads + c < hi)
+          __builtin_amdgcn_global_load_lds(bsrc[c] + t * 1024,
+                                           (lds_ptr_t)(stage + kABytes + (c * NW + wave) * 1024), 16, 0, 0);
+    }
   };
-  auto issue = [&](int it) { issue_range(it, 0, kPerStage); };
   // With three stages the loads of tile it+3 may be issued anywhere between the
   // barrier of tile `it` (which frees their stage) and the barrier of tile it+1,
   // and still have a whole tile period to land.  They are spread over that
@@ -698,7 +733,7 @@ __device__ __forceinline__ void dma_tile(const DmaParams& p, unsigned char* smem
 #pragma unroll
         for (int c = 0; c < TN; ++c)
           dst[f][c] = *reinterpret_cast<const uint16_t*>(
-              stage + kABytes + kBBytes + (f * BN + (wn * TN + c) * 32 + r32) * 2);
+              stage + kScaleOff + (f * BN + (wn * TN + c) * 32 + r32) * 2);
     }
   };
 
@@ -726,8 +761,8 @@ __device__ __forceinline__ void dma_tile(const DmaParams& p, unsigned char* smem
 
   // byte offsets inside a stage that do not change from tile to tile
   const int a_row_off = (wm * TM * 32 + r32) * (TK * 2);
-  const int b_off = kABytes + (wn * TN * 2 + sp) * 1024 + (j + 16 * b) * 16;
-  constexpr int kValuPerMfma = ((OFFS == 2 ? 4 * TN + 4 * TM : (BITS == 8 ? 16 : 12) * TN) + TM * TN - 1) / (TM * TN) + 2;
+  const int b_off = (kHalfDeep ? 0 : kABytes) + (wn * TN * 2 + sp) * 1024 + (j + 16 * b) * 16;  // kHalfDeep: in a raw B tile
+  constexpr int kValuPerMfma = ((OFFS == 2 ? 4 * TN + 4 * TM : (BITS == 8 ? 16 : DT == WOL_DTYPE_BF16 ? 18 : 12) * TN) + TM * TN - 1) / (TM * TN) + 2;
   constexpr int kValuRescale = RESC ? 16 : 0;  // more per MFMA in the slice that starts a group
   constexpr int kHalf = (TM * TN + 1) / 2;  // MFMAs of a slice issued before the barrier
   // (With one workgroup per CU, wavefronts w and w + 4 share a SIMD and the older one wins every
@@ -834,13 +869,18 @@ __device__ __forceinline__ void dma_tile(const DmaParams& p, unsigned char* smem
     }
   };
 
-  issue(0);
-  issue(1);
-  if (kStages == 3) issue_range(2, 0, seg_lo(2));  // the rest of tile 2 goes out during tile 0
+  if constexpr (kHalfDeep) {  // the first half of raw B tile 0, which no tile before tile 0 brings
+#pragma unroll
+    for (int c = 0; c < kBLoads; ++c)
+      __builtin_amdgcn_global_load_lds(bsrc[c], (lds_ptr_t)(braw_lds + (c * NW + wave) * 1024), 16, 0, 0);
+  }
+  issue_range(0, 0, kPerStage, false);
+  issue_range(1, 0, kPerStage, true);
+  if (kStages == 3) issue_range(2, 0, seg_lo(2), false);  // the rest of tile 2 goes out during tile 0
   wait_vmcnt<(kStages - 2) * kPerStage + (kStages == 3 ? (2 * kPerStage + Q - 1) / Q : kPerStage)>();  // tile 0 has landed
   __builtin_amdgcn_s_barrier();
   if (STAMP) st_loop0 = st_prev = __builtin_readcyclecounter();
-  read_b(smem, braw[0]);
+  read_b(kHalfDeep ? braw_lds : smem, braw[0]);
   read_a(smem, af[0], 0);
   dequant(bf[0], braw[0], 0);
   // Every slice runs its MFMAs with the preparation of the next slice's
@@ -853,6 +893,10 @@ __device__ __forceinline__ void dma_tile(const DmaParams& p, unsigned char* smem
   auto tile = [&](auto odd_tile, int it, u32x4 (&raw)[TN][2], u32x4 (&raw_next)[TN][2]) {
     // RESC with groups of two tiles: the run starts on a group (launch_dma sees to it), so odd tiles continue one
     constexpr bool gstart = !(RESC && G > TK && decltype(odd_tile)::value);
+    // kHalfDeep: an odd tile consumes the second half of the raw codes and reads the next raw tile
+    constexpr bool kOdd = decltype(odd_tile)::value;
+    constexpr int q0 = kHalfDeep && kOdd ? Q : 0;
+    constexpr bool kNewB = !kHalfDeep || kOdd;
     const unsigned char* stage = smem + (it % kStages) * kStage;
     const unsigned char* next = smem + ((it + 1) % kStages) * kStage;
     read_scales(stage, sraw);  // before the stage is handed over
@@ -862,9 +906,9 @@ __device__ __forceinline__ void dma_tile(const DmaParams& p, unsigned char* smem
         const bool last = q == Q - 1;
         // this slice's share of the tile loads (segment 1 of tile it+3, or segment q+2 of tile it+2)
         const int seg = last ? 1 : q + 2;
-        if (kSpread) issue_range(last ? it + kStages : it + kStages - 1, seg_lo(seg), seg_lo(seg + 1));
+        if (kSpread) issue_range(last ? it + kStages : it + kStages - 1, seg_lo(seg), seg_lo(seg + 1), last != kOdd);
         read_a(last ? next : stage, af[(q + 1) & 1], last ? 0 : q + 1);
-        dequant(bf[(q + 1) & 1], last ? raw_next : raw, last ? 0 : q + 1);
+        dequant(bf[(q + 1) & 1], last && kNewB ? raw_next : raw, last && kNewB ? 0 : q0 + q + 1);
         mfmas(af[q & 1], bf[q & 1], q, 0, TM * TN, gstart);
 #pragma unroll
         for (int i = 0; i < TM * TN; ++i) {
@@ -904,14 +948,14 @@ __device__ __forceinline__ void dma_tile(const DmaParams& p, unsigned char* smem
           st_bar += st_c - st_b;
           st_prev = st_c;
         }
-        issue_range(it + kStages, 0, seg_lo(1));
-        read_b(next, raw_next);
-        dequant(bf[(q + 1) & 1], raw, q + 1);
+        issue_range(it + kStages, 0, seg_lo(1), !kOdd);
+        if (kNewB) read_b(kHalfDeep ? braw_lds + (((it + 1) / 2) & 1) * kBBytes : next, raw_next);
+        dequant(bf[(q + 1) & 1], raw, q0 + q + 1);
         mfmas(af[q & 1], bf[q & 1], q, kHalf, TM * TN);
 #pragma unroll
         for (int i = 0; i < TM * TN - kHalf + 1; ++i) {
           if (i < TM * TN - kHalf) __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-          if (i < 2 * TN) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+          if (kNewB && i < 2 * TN) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
           if (kSpread && i < seg_n(0)) {
             __builtin_amdgcn_sched_group_barrier(0x004, 2, 0);
             __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
@@ -922,9 +966,20 @@ __device__ __forceinline__ void dma_tile(const DmaParams& p, unsigned char* smem
       }
     }
   };
-  for (int it = 0; it < niter; it += 2) {
-    tile(std::false_type(), it, braw[0], braw[1]);
-    if (it + 1 < niter) tile(std::true_type(), it + 1, braw[1], braw[0]);
+  if constexpr (kHalfDeep) {
+    for (int it = 0; it < niter; it += 4) {  // niter is even
+      tile(std::false_type(), it, braw[0], braw[1]);
+      tile(std::true_type(), it + 1, braw[0], braw[1]);
+      if (it + 2 < niter) {
+        tile(std::false_type(), it + 2, braw[1], braw[0]);
+        tile(std::true_type(), it + 3, braw[1], braw[0]);
+      }
+    }
+  } else {
+    for (int it = 0; it < niter; it += 2) {
+      tile(std::false_type(), it, braw[0], braw[1]);
+      if (it + 1 < niter) tile(std::true_type(), it + 1, braw[1], braw[0]);
+    }
   }
   wait_vmcnt<0>();
   __builtin_amdgcn_s_barrier();  // the spare loads are done and every wavefront has stopped reading
@@ -966,7 +1021,7 @@ __device__ __forceinline__ void dma_tile(const DmaParams& p, unsigned char* smem
     // Row sums: lanes l and l + 32 hold the two halves of row r32's sum.  They
     // are added and parked in LDS (the stages are free now), from where a lane
     // takes the sums of the sixteen rows its accumulators belong to.
-    constexpr int kRsOff = kStages * kStage - NW * TM * 32 * 4;  // the end of the stages; the slabs use their start
+    constexpr int kRsOff = kLds - NW * TM * 32 * 4;  // the end of the stages; the slabs use their start
     static_assert(kRsOff >= NW * 32 * ((SWI ? 1 : TN) * 32 + 8) * 2, "row sums and slabs must not overlap");
     float* rsl = reinterpret_cast<float*>(smem + kRsOff) + wave * TM * 32;
 #pragma unroll
@@ -1013,14 +1068,14 @@ __device__ __forceinline__ void dma_tile(const DmaParams& p, unsigned char* smem
   uint16_t* out = static_cast<uint16_t*>(outp);
   constexpr int kOutBlocks = SWI ? 1 : TN;        // 32-column blocks a wavefront writes
   constexpr int kSlabRow = kOutBlocks * 32 + 8;   // padded, in elements
-  static_assert(NW * 32 * kSlabRow * 2 <= kStages * kStage, "slabs must fit in the stage buffers");
+  static_assert(NW * 32 * kSlabRow * 2 <= kLds, "slabs must fit in the stage buffers");
   uint16_t* slab = reinterpret_cast<uint16_t*>(smem) + wave * 32 * kSlabRow;
   constexpr int kPieces = 32 * (kOutBlocks * 32 / 8);
   const int ld_out = SWI ? N / 2 : N;             // row length of the output
   if constexpr (kPair) {
     // behind the slabs: one block of fp32 sums per pair of wavefronts
     constexpr int kXOff = (NW * 32 * kSlabRow * 2 + 255) / 256 * 256;
-    static_assert(kXOff + NW / 2 * 4096 <= kStages * kStage, "slabs and handed-over sums must fit in the stage buffers");
+    static_assert(kXOff + NW / 2 * 4096 <= kLds, "slabs and handed-over sums must fit in the stage buffers");
     float* xbuf = reinterpret_cast<float*>(smem + kXOff) + (wave / 2) * 1024;
 #pragma unroll
     for (int a = 0; a < TM; ++a) {
@@ -1308,6 +1363,9 @@ inline int plan_xcd_rows(int nbx, int nby, int a_bytes, int b_bytes) {
 
 template <int BITS, int G, int WM, int WN, int TM, int TN, int STAGES = 3>
 constexpr size_t dma_lds_bytes() {
+  if (STAGES > kHalfDeepStages)
+    return STAGES % kHalfDeepStages * (static_cast<size_t>(WM * TM * 32) * 64 * 2 + (G == 0 ? 0 : WM * WN * 256)) +
+           2 * (WN * TN * 32 / 16) * 1024;
   return STAGES * (static_cast<size_t>(WM * TM * 32) * (BITS == 8 ? 64 : 128) * 2 +
               (WN * TN * 32 / 16) * 1024 + (G == 0 ? 0 : WM * WN * 256));
 }
@@ -1317,7 +1375,9 @@ constexpr size_t dma_lds_bytes() {
 // SWI != 0 (swiglu epilogue): the strips are those of the gate half, [0, N / 32), a.out is [M, N / 2].
 template <int DT, int BITS, int G, int OFFS, int WM, int WN, int TM, int TN, int STAGES = 3, int SWI = 0, bool RESC = false>
 void launch_dma(const Args& a, int strip_lo, int strip_hi, int nsplit) {
-  constexpr int BM = WM * TM * 32, BN = (SWI ? TN * WN * 16 : TN * WN * 32), TK = BITS == 8 ? 64 : 128;  // BN: output columns
+  constexpr int BM = WM * TM * 32, BN = (SWI ? TN * WN * 16 : TN * WN * 32);  // BN: output columns
+  constexpr bool half_deep = STAGES > kHalfDeepStages;
+  constexpr int TK = BITS == 8 || half_deep ? 64 : 128;
   if (strip_hi <= strip_lo) return;
   if (SWI) nsplit = 1;
   constexpr size_t lds = dma_lds_bytes<BITS, G, WM, WN, TM, TN, STAGES>();
@@ -1341,7 +1401,7 @@ void launch_dma(const Args& a, int strip_lo, int strip_hi, int nsplit) {
   p.nby = (a.M + BM - 1) / BM;
   const int tiles = a.K / TK;
   p.tiles_per_split = (tiles + nsplit - 1) / nsplit;
-  if (RESC && G > TK) p.tiles_per_split = (p.tiles_per_split + 1) & ~1;  // every run starts on a group of two tiles
+  if ((RESC && G > TK) || half_deep) p.tiles_per_split = (p.tiles_per_split + 1) & ~1;  // every run starts on a group (a raw B tile) of two tiles
   p.nsplit = (tiles + p.tiles_per_split - 1) / p.tiles_per_split;
   p.xcd_rows = plan_xcd_rows(p.nbx, p.nby, BM * 2, WN * TN * 32 * BITS / 8);
   p.act = a.act;
@@ -1375,20 +1435,32 @@ inline bool tall_half_tile(int M) {
 }
 
 // Number of 256-column tiles given to the 256-row kernel; the remaining
-// columns run with 128-row tiles.  Cost model: a workgroup owns its CU, so a
+// columns run with half-size tiles.  Cost model: a workgroup owns its CU, so a
 // launch takes ceil(tiles / CUs) tile times; a half-size tile costs kSmall of a
-// full one (a little more than half).
-inline int plan_big_columns(int M, int N, bool tall_ok = true) {
+// full one (a little more than half).  int4 with group-wise scales: half-size
+// tiles cost more (their 128-deep k tiles run in two stages), and a last partial
+// round of them that plan_tail cuts into K runs costs the share of a round that
+// a run is plus the partial sums' way through memory (K = 4096, N = 12288, 700
+// rows, all on half-size tiles / all on full ones: bf16 g128 105 / 108 us, g64
+// 112 / 121; 1024 rows 129 / 113 and 137 / 125).
+inline int plan_big_columns(int M, int K, int N, int bits, int group) {
   const int cus = num_cus();
-  constexpr double kSmall = 0.55;
+  const bool g4 = bits == 4 && group != 0;
+  const double kSmall = g4 ? 0.58 : 0.55;
+  constexpr double kRuns = 0.25;
   const int nbx = (N + 255) / 256, nby_big = (M + 255) / 256, nby_small = (M + 127) / 128;
-  const bool tall = tall_ok && tall_half_tile(M);  // half tiles of 256 x 128 instead of 128 x 256
+  const bool tall = (bits == 8 || g4) && tall_half_tile(M);  // half tiles of 256 x 128 instead of 128 x 256
   int best = nbx;
   double best_t = 1e30;
   for (int c = nbx; c >= 0; --c) {
     const int small = tall ? 2 * (nbx - c) * nby_big : (nbx - c) * nby_small;
-    const double t = static_cast<double>((c * nby_big + cus - 1) / cus) +
-                     kSmall * static_cast<double>((small + cus - 1) / cus);
+    double t = static_cast<double>((c * nby_big + cus - 1) / cus);
+    const int rest = small % cus;
+    int runs = g4 && rest > 0 ? cus / rest : 1;
+    runs = runs > 4 ? 4 : runs;
+    while (runs > 1 && K / 128 / runs < 8) --runs;
+    if (runs > 1) t += kSmall * (small / cus) + kSmall / runs + kRuns;
+    else t += kSmall * static_cast<double>((small + cus - 1) / cus);
     if (t < best_t - 1e-9) { best_t = t; best = c; }
   }
   return best;
@@ -1455,14 +1527,10 @@ inline SkinnyPlan plan_skinny(int M, int K, int N, int bits, int group, size_t w
 
 // Tile of the configuration launch_fast gives the columns that do not get
 // 256 x 256 tiles (above 64 rows), and the first strip of those columns.
-inline void half_tile_config(int M, int N, int bits, int group, int* bm, int* bn, int* strip_lo) {
-  *strip_lo = 0;
-  // 256 x 256 tiles on whole rounds of the CUs (int4 with group-wise scales has none:
-  // two stages of its 128-deep tiles and their scales do not fit the LDS)
-  if (group == 0 || bits == 8) {
-    const int c = plan_big_columns(M, N, bits == 8) * 16, nstrips = N / kStripCols;
-    *strip_lo = c < nstrips ? c : nstrips;
-  }
+inline void half_tile_config(int M, int K, int N, int bits, int group, int* bm, int* bn, int* strip_lo) {
+  // 256 x 256 tiles on whole rounds of the CUs
+  const int c = plan_big_columns(M, K, N, bits, group) * 16, nstrips = N / kStripCols;
+  *strip_lo = c < nstrips ? c : nstrips;
   if (bits == 8 || group != 0) {
     *bm = tall_half_tile(M) ? 256 : 128;
     *bn = tall_half_tile(M) ? 128 : 256;
@@ -1521,7 +1589,7 @@ void launch_fast(const Args& a) {
   }
   constexpr int TK = BITS == 8 ? 64 : 128;
   int bm = 0, bn = 0, lo = 0;
-  half_tile_config(a.M, a.N, BITS, G, &bm, &bn, &lo);
+  half_tile_config(a.M, a.K, a.N, BITS, G, &bm, &bn, &lo);
   const TailPlan t = plan_tail(a.M, a.K, (nstrips - lo) * kStripCols, bm, bn, TK, a.ws != nullptr ? a.ws_bytes : 0);
   const int mid = lo + t.full_tiles * (bn / kStripCols);  // strips [lo, mid) unsplit, [mid, nstrips) in t.ns runs
   // launches a half-size configuration on both parts
@@ -1545,9 +1613,13 @@ void launch_fast(const Args& a) {
     if (bm == 256) WOL_HALF(0, 2, 4, 4, 1, 3, 0, true);
     else WOL_HALF(0, 2, 4, 2, 2, 3, 0, true);
   } else if constexpr (G != 0) {
-    // int4 with group-wise scales: the same, on 256 x 128 tiles where the rows
-    // fill them (four A blocks share every dequantised B block, and the exact
-    // int4 dequantiser is the expensive part), 128 x 256 otherwise
+    // int4 with group-wise scales: the same, the whole tiles on 64-deep k tiles
+    // (two 128-deep stages and their scales would need 164 KiB of LDS).  Against
+    // 256 x 128 tiles alone, M = 8192, K = N = 4096: bf16 g128 297 -> 249 us
+    // (1.11 PFLOP/s), g64 322 -> 273, fp16 g128 283 -> 237; M = 2048, N = 12288
+    // g128 223 -> 201.  The half-size tiles are 256 x 128 where the rows fill
+    // them (four A blocks share every dequantised B block), else 128 x 256.
+    launch_dma<DT, BITS, G, 0, 2, 4, 4, 2, kHalfDeepStages + 3, 0, true>(a, 0, lo, 1);
     if (bm == 256) WOL_HALF(0, 2, 4, 4, 1, 2, 0, true);
     else WOL_HALF(0, 2, 4, 2, 2, 2, 0, true);
   } else if constexpr (DT == WOL_DTYPE_BF16) {
@@ -1795,8 +1867,16 @@ void launch_swiglu_gemm(const Args& a) {
       if (a.M >= 192) launch_dma<DT, 8, G, 0, 2, 4, 4, 2, 3, 1, true>(a, 0, gate_strips, 1);
       else launch_dma<DT, 8, G, 0, 2, 4, 2, 2, 3, 1, true>(a, 0, gate_strips, 1);
     } else {
-      // (256 x 128 tiles: gate and up blocks in neighbouring wavefronts)
-      if (tall_half_tile(a.M)) launch_dma<DT, 4, G, 0, 2, 4, 4, 1, 2, 1, true>(a, 0, gate_strips, 1);
+      // whole tiles, or half-size ones (256 x 128: gate and up blocks in neighbouring wavefronts) where their
+      // rounds, at 0.65 of a whole tile's, are done sooner: K = 4096, N = 22016, bf16 g128, whole / half-size
+      // tiles, 256 rows 109 / 70 us, 400 rows 110 / 142, 1024 rows 231 / 224, 1237 rows 242 / 298, 2048 rows
+      // 370 / 447, 4096 rows 729 / 846
+      const bool tall = tall_half_tile(a.M);
+      const int cus = num_cus(), cols = (a.N + 255) / 256, big = cols * ((a.M + 255) / 256);
+      const int half = tall ? 2 * big : cols * ((a.M + 127) / 128);
+      if ((big + cus - 1) / cus < 0.65 * ((half + cus - 1) / cus))
+        launch_dma<DT, 4, G, 0, 2, 4, 4, 2, kHalfDeepStages + 3, 1, true>(a, 0, gate_strips, 1);
+      else if (tall) launch_dma<DT, 4, G, 0, 2, 4, 4, 1, 2, 1, true>(a, 0, gate_strips, 1);
       else launch_dma<DT, 4, G, 0, 2, 4, 2, 2, 2, 1, true>(a, 0, gate_strips, 1);
     }
   } else if constexpr (BITS == 8) {
@@ -1873,7 +1953,7 @@ size_t linear_gemm_workspace(int64_t M, int64_t K, int64_t N, int bits, int grou
   if (M > kSkinnyMaxM) {
     int bm = 0, bn = 0, lo = 0;
     const int g = group_size > 0 ? group_size : 0;
-    half_tile_config(static_cast<int>(M), static_cast<int>(N), bits, g, &bm, &bn, &lo);
+    half_tile_config(static_cast<int>(M), static_cast<int>(K), static_cast<int>(N), bits, g, &bm, &bn, &lo);
     const int ncols = static_cast<int>(N) - lo * kStripCols;
     const TailPlan t = plan_tail(static_cast<int>(M), static_cast<int>(K), ncols, bm, bn, tk, SIZE_MAX);
     return t.ns > 1 ? static_cast<size_t>(t.ns) * M * (ncols - t.full_tiles * bn) * sizeof(float) : 0;
@@ -1900,7 +1980,7 @@ void describe_linear_gemm(int64_t M, int64_t K, int64_t N, int bits, int group_s
     return;
   }
   int bm = 0, bn = 0, lo = 0;
-  half_tile_config(static_cast<int>(M), static_cast<int>(N), bits, g, &bm, &bn, &lo);
+  half_tile_config(static_cast<int>(M), static_cast<int>(K), static_cast<int>(N), bits, g, &bm, &bn, &lo);
   const int nstrips = static_cast<int>(N / kStripCols);
   const TailPlan t = plan_tail(static_cast<int>(M), static_cast<int>(K), (nstrips - lo) * kStripCols, bm, bn, tk, ws_bytes);
   const int mid = lo + t.full_tiles * (bn / kStripCols);

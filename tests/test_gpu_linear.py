@@ -905,6 +905,25 @@ def test_group_wise_gemm_keeps_its_sums_in_units_of_the_group_scale(G, oracle, d
     assert (errp[ref > 0] / ref[ref > 0]).max() < 2e-5
 
 
+@pytest.mark.parametrize("dt", [H.BF16, H.F16])
+@pytest.mark.parametrize("g,M,K,N", [
+    (128, 300, 256, 24016),   # two raw weight tiles, the fewest; a last column tile of 208 columns
+    (64, 512, 384, 24016),    # an odd number of raw tiles; whole row tiles
+    (64, 1100, 1152, 12304),  # more tiles than stages; 9 raw tiles
+    (128, 770, 2048, 16368),  # a row tile of two rows
+])
+def test_int4_group_wise_whole_tiles(G, oracle, dt, g, M, K, N):
+    # int4 with group-wise scales on 256 x 256 tiles: 64-deep k tiles of activations over
+    # raw weight tiles of 128 k, whose halves travel with the k tiles on either side
+    import ctypes
+    from paddle_amd import _lib
+
+    buf = ctypes.create_string_buffer(512)
+    _lib.check(_lib.lib.wol_linear_plan(M, K, N, 4, g, 1 << 40, buf, len(buf)))
+    assert b"256x256 tiles" in buf.value, buf.value
+    check_sampled(G, oracle, dt, 4, g, M, K, N)
+
+
 def test_call_log_names_the_kernel(device):
     # WOL_LOG=1: one line per call on stderr with the problem and the kernel taken
     # (read once per process, hence a child process)

@@ -184,6 +184,34 @@ def test_swiglu_in_the_gemm_epilogue(device, oracle, dt, bits, g):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("dt", [H.F16, H.BF16])
+@pytest.mark.parametrize("bits,g,M,K,N", [
+    (4, 128, 300, 384, 22048),  # 261 half-size tiles against 174 whole ones: whole tiles
+    (4, 64, 520, 256, 17504),
+])
+def test_swiglu_epilogue_on_whole_tiles(device, oracle, dt, bits, g, M, K, N):
+    # 256 x 256 tiles where half-size ones would need twice the rounds; the last column tile is partial.
+    # The oracle multiplies the first, a middle and the last 32 gate columns with their up columns.
+    import torch
+    from paddle_amd.nn import quant as Q
+
+    gen = torch.Generator(device="cuda").manual_seed(K + N)
+    w = (torch.randn(K, N, device="cuda", generator=gen) * 0.02).to(H.torch_dtype(dt))
+    codes, scale = Q.weight_quantize(w, algo="weight_only_int%d" % bits, group_size=g)
+    xb, bb = H.make_act(M, K, dt, seed=M), H.make_bias(N, dt, seed=7)
+    got = _fused_dev(H.bits_to_torch(xb, dt, "cuda:0"), None, codes, H.bits_to_torch(bb, dt, "cuda:0"), scale, dt, N,
+                     bits, g, 2)
+    assert bool(torch.isfinite(got.float()).all())
+    for c0 in (0, N // 4 // 16 * 16, N // 2 - 32):
+        cols = np.r_[c0:c0 + 32, N // 2 + c0:N // 2 + c0 + 32]
+        oc, osc = oracle.weight_quantize(H.torch_to_bits(w[:, torch.from_numpy(cols).cuda()].contiguous()), dt, bits, g)
+        _, wantT = oracle.linear_fused(xb, None, oc, osc, bb[cols], dt, bits, g, 2)
+        part = got[:, c0:c0 + 32].contiguous()
+        err = H.rel_l2(H.bits_to_f32(H.torch_to_bits(part), dt), H.bits_to_f32(wantT, dt))
+        assert err <= TOL, (err, dt, bits, g, M, K, N, c0)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dt", [H.F16, H.BF16])
 @pytest.mark.parametrize("bits", [8, 4])
 @pytest.mark.parametrize("g", [-1, 128])
 def test_swiglu_in_the_streaming_kernel(device, oracle, dt, bits, g):
