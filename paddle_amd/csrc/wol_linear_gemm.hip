@@ -127,21 +127,25 @@ struct DequantExact<WOL_DTYPE_F16, 4> {
   }
 };
 
+// Each nibble pair becomes two fp16 values 1024 + 16 * nibble (one and-or), a
+// mixed-precision FMA takes the offset out and widens to fp32 in one
+// instruction, and the high halves are the bf16 codes: 19 instructions per
+// eight codes, every step exact.  (Widening two bf16 values 136 + code and
+// subtracting in fp32 takes 27.)
 template <>
 struct DequantExact<WOL_DTYPE_BF16, 4> {
-  __device__ static inline uint32_t fix(uint32_t pair) {
-    // pair = two bf16 holding 136 + code; widen, subtract, narrow (all exact)
-    const float lo = __uint_as_float(pair << 16) - 136.0f;
-    const float hi = __uint_as_float(pair & 0xFFFF0000u) - 136.0f;
-    return pack_bf16_hi(lo, hi);
+  __device__ static inline uint32_t pair(uint32_t v) {
+    const f16x2 h = __builtin_bit_cast(f16x2, (v & 0x00F000F0u) | 0x64006400u);
+    return pack_bf16_hi(__builtin_fmaf(static_cast<float>(h.x), 0.0625f, -72.0f),
+                        __builtin_fmaf(static_cast<float>(h.y), 0.0625f, -72.0f));
   }
   __device__ static inline u32x4 run(const uint32_t* w) {
     const uint32_t v = w[0];
     u32x4 o;
-    o.x = fix((v & 0x000F000Fu) | 0x43004300u);
-    o.y = fix(((v >> 4) & 0x000F000Fu) | 0x43004300u);
-    o.z = fix(((v >> 8) & 0x000F000Fu) | 0x43004300u);
-    o.w = fix(((v >> 12) & 0x000F000Fu) | 0x43004300u);
+    o.x = pair(v << 4);
+    o.y = pair(v);
+    o.z = pair(v >> 4);
+    o.w = pair(v >> 8);
     return o;
   }
 };
