@@ -1,6 +1,6 @@
 // weight_quantize, weight_dequantize and the layout re-packer for gfx950.
 //
-// All three work on blocks of 128 k x 64 n of the weight and pass the signed
+// The kernels for any layout work on blocks of 128 k x 64 n of the weight and pass the signed
 // codes of a block through LDS (stage[r][c]); the layout-specific part is how
 // the bytes of a block are enumerated in global memory (block_byte()).
 //
@@ -370,7 +370,7 @@ __global__ __launch_bounds__(kThreads) void quantize_kernel(
     store_block(st, layout, BITS, K, N, k0, n0, KR, NC, codes);
 }
 
-// out[k,n] = cast_T(float(code) * float(scale)), written as [K,N] rows.
+// out[k,n] = cast_T(float(code) * float(scale)), written as [K,N] rows; codes in the other two layouts.
 template <int DT, int BITS>
 __global__ __launch_bounds__(kThreads) void dequantize_kernel(
     const uint8_t* __restrict__ codes, int layout, const uint16_t* __restrict__ scale, int64_t K,
@@ -381,10 +381,7 @@ __global__ __launch_bounds__(kThreads) void dequantize_kernel(
   const int64_t k0 = static_cast<int64_t>(blockIdx.y) * kBlockK;
   const int KR = static_cast<int>(K - k0 < kBlockK ? K - k0 : kBlockK);
   const int NC = static_cast<int>(N - n0 < kBlockN ? N - n0 : kBlockN);
-  if (layout == WOL_LAYOUT_GFX950 && KR == kBlockK && NC == kBlockN)
-    load_block_gfx950<BITS>(st, K, k0, n0, codes);
-  else
-    load_block(st, layout, BITS, K, N, k0, n0, KR, NC, codes);
+  load_block(st, layout, BITS, K, N, k0, n0, KR, NC, codes);
   __syncthreads();
   if (tx * 8 >= NC) return;
 #pragma unroll
@@ -423,6 +420,294 @@ __global__ __launch_bounds__(kThreads) void repack_kernel(const uint8_t* __restr
     store_block(st, layout_out, BITS, K, N, k0, n0, KR, NC, out);
 }
 
+// ---------------------------------------------------------------------------
+// The GFX950 layout with scales in T: quantize_gfx950_kernel and
+// dequantize_gfx950_kernel.  A block is 128 k x 128 n, and thread (rg, cg) of 16
+// x 16 owns rows 8 rg .. 8 rg + 7 of columns 8 cg .. 8 cg + 7: eight 16-byte
+// loads (or stores) of the weight, 256 bytes of a row side by side, and for
+// every column exactly the eight consecutive k that the layout keeps together
+// -- one dword (int4) or two (int8).  So codes are packed and unpacked in
+// registers and only whole dwords go through LDS, as planes [k step][dword][k
+// octet][column] that both sides touch with consecutive lanes on consecutive
+// dwords.  Any K and N of the layout; what lies past an edge is neither read
+// nor written.
+//
+// HBM-bound: 8192 x 28672 fp16 int4 g128 quantize 219 -> 124 us, dequantize 153 ->
+// 122 us (4.8 TB/s; a copy of the fp16 weight moves 5.3); 4096 x 12288 bf16 int8
+// per channel 60 -> 47 us (amax_kernel included) and 27 -> 24
+// against the byte-wise stage above with an IEEE division per element, which
+// stays for the other layouts and for fp32 scales.
+// ---------------------------------------------------------------------------
+constexpr int kWideN = 128;
+
+// Codes of eight consecutive k of one column -> the layout's dwords, biased.
+// Signed codes are summed with their place value; the bias of all fields at
+// once turns the sum into the fields.
+template <int BITS>
+__device__ inline void pack_codes(const int (&c)[8], uint32_t* d) {
+  if (BITS == 4) {
+    uint32_t v = 0;
+#pragma unroll
+    for (int p = 7; p >= 0; --p) v = (v << 4) + static_cast<uint32_t>(c[p < 4 ? 2 * p : 2 * (p - 4) + 1]);
+    d[0] = v + 0x88888888u;
+  } else {
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      uint32_t v = 0;
+#pragma unroll
+      for (int e = 3; e >= 0; --e) v = (v << 8) + static_cast<uint32_t>(c[4 * h + e]);
+      d[h] = v + 0x80808080u;
+    }
+  }
+}
+
+// The code of w under a scale whose fp32 reciprocal is y: what quant_code()
+// gives, without the division.  w and the scale have at most 11 significant
+// bits, so w / scale is either exactly half way between two integers or at
+// least 2^-13.4 away (2^-11 above 2): adding 1/2 + 2^-14 to |w| * y, off by less
+// than 2^-15, and truncating rounds every half away from zero and nothing else.
+// (Compared with roundf(w / s) for all pairs of 11-bit and of 8-bit
+// significands and all quotients up to 400, beyond which both sides clip.)
+template <int BITS>
+__device__ inline int quant_code_rcp(float w, float y) {
+  constexpr int bound = BITS == 8 ? 127 : 7;
+  const int v = static_cast<int>(__builtin_fmaf(w, y, __builtin_copysignf(0.5f + 0x1p-14f, w)));
+  const int lo = v < bound ? v : bound;
+  return lo > -bound ? lo : -bound;
+}
+
+template <int DT, int BITS, int G>  // G: 64, 128, or 0 = a scale per column
+__global__ __launch_bounds__(kThreads) void quantize_gfx950_kernel(
+    const uint16_t* __restrict__ w, int64_t K, int64_t N, int round_mode, const uint32_t* __restrict__ amax,
+    uint8_t* __restrict__ codes, uint16_t* __restrict__ scale) {
+  constexpr int kDw = BITS == 8 ? 2 : 1;  // dwords per eight codes
+  constexpr int kGroups = G == 64 ? 2 : 1;
+  __shared__ __attribute__((aligned(16))) uint32_t plane[4][kDw][4][kWideN];
+  __shared__ __attribute__((aligned(16))) float part[G == 0 ? 1 : 16][kWideN];
+  __shared__ __attribute__((aligned(16))) float sc[kGroups][kWideN], rc[kGroups][kWideN];
+
+  const int tid = threadIdx.x, cg = tid % 16, rg = tid / 16;
+  const int64_t n0 = static_cast<int64_t>(blockIdx.x) * kWideN;
+  const int64_t k0 = static_cast<int64_t>(blockIdx.y) * kBlockK;
+  const int KR = static_cast<int>(K - k0 < kBlockK ? K - k0 : kBlockK);  // 128 or 64
+  const int NC = static_cast<int>(N - n0 < kWideN ? N - n0 : kWideN);    // a multiple of 16
+  const float bound = BITS == 8 ? 127.0f : 7.0f;
+
+  Pack8 raw[8];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) raw[i].q = make_uint4(0, 0, 0, 0);
+  if (cg * 8 < NC && rg * 8 < KR) {
+    const uint16_t* src = w + (k0 + rg * 8) * N + n0 + cg * 8;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) raw[i].q = *reinterpret_cast<const uint4*>(src + i * N);
+  }
+
+  if (G != 0) {
+#pragma unroll
+    for (int c = 0; c < 8; ++c) {
+      float m = 0.0f;
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const float a = fabsf(to_f32<DT>(raw[i].h[c]));
+        m = a > m ? a : m;  // NaN never wins
+      }
+      part[rg][cg * 8 + c] = m;
+    }
+    __syncthreads();
+  }
+  // one thread per scale of the block
+  if (tid < kGroups * kWideN) {
+    const int g = tid / kWideN, c = tid % kWideN;
+    uint16_t sb = 0;
+    if (c < NC && g * 64 < KR) {
+      float src;
+      if (G != 0) {
+        src = 0.0f;
+#pragma unroll
+        for (int r = 0; r < 16 / kGroups; ++r) {
+          const float a = part[g * 8 + r][c];
+          src = a > src ? a : src;
+        }
+      } else {
+        // the signed first element, as in quantize_kernel
+        const float v0 = to_f32<DT>(w[n0 + c]);
+        const float m = __uint_as_float(amax[n0 + c]);
+        src = (v0 != v0) ? v0 : (m == 0.0f ? (v0 < 0.0f ? m : v0) : m);
+      }
+      sb = from_f32<DT>(src / bound, round_mode);
+      if (G != 0) scale[(k0 / (G != 0 ? G : 1) + g) * N + n0 + c] = sb;
+      else if (k0 == 0) scale[n0 + c] = sb;
+    }
+    const float s = to_f32<DT>(sb);
+    sc[g][c] = s;
+    // scales whose reciprocal is no ordinary number (0, NaN, infinity, the ends of bf16's range): 0 marks them
+    rc[g][c] = s >= 0x1p-100f && s <= 0x1p100f ? 1.0f / s : 0.0f;
+  }
+  __syncthreads();
+
+  const int g = G == 64 ? rg / 8 : 0;
+  const int step = rg / 4, kb = rg % 4;
+  float y[8];
+  bool ordinary = true;
+#pragma unroll
+  for (int c = 0; c < 8; ++c) {
+    y[c] = rc[g][cg * 8 + c];
+    ordinary = ordinary && y[c] != 0.0f;
+  }
+  uint32_t d[8][kDw];
+  if (ordinary) {
+#pragma unroll
+    for (int c = 0; c < 8; ++c) {
+      int code[8];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const float f = to_f32<DT>(raw[i].h[c]);
+        code[i] = quant_code_rcp<BITS>(f, y[c]);
+        if (f != f) code[i] = BITS == 8 ? 127 : -7;  // as quant_code
+      }
+      pack_codes<BITS>(code, d[c]);
+    }
+  } else {
+#pragma unroll
+    for (int c = 0; c < 8; ++c) {
+      int code[8];
+      const float s = sc[g][cg * 8 + c];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) code[i] = quant_code<BITS>(to_f32<DT>(raw[i].h[c]), s);
+      pack_codes<BITS>(code, d[c]);
+    }
+  }
+#pragma unroll
+  for (int h = 0; h < kDw; ++h)
+#pragma unroll
+    for (int c = 0; c < 8; c += 4)
+      *reinterpret_cast<uint4*>(&plane[step][h][kb][cg * 8 + c]) = make_uint4(d[c][h], d[c + 1][h], d[c + 2][h], d[c + 3][h]);
+  __syncthreads();
+
+  // lane pieces of the layout, a wavefront one tile of a strip at a time
+  const int lane = tid % 64, j = lane % 16, b = lane / 16;
+  if (BITS == 8) {
+#pragma unroll
+    for (int p = 0; p < 4; ++p) {
+      const int u = p * 4 + tid / 64, s = u / 2, t = u % 2;  // strip of the block, 64-k tile
+      if (s * 16 >= NC || t * 64 >= KR) continue;
+      const uint4 v = make_uint4(plane[2 * t][0][b][s * 16 + j], plane[2 * t][kDw - 1][b][s * 16 + j],
+                                 plane[2 * t + 1][0][b][s * 16 + j], plane[2 * t + 1][kDw - 1][b][s * 16 + j]);
+      *reinterpret_cast<uint4*>(codes + (n0 / kStripCols + s) * strip_bytes(K, 8) + (k0 / 64 + t) * 1024 + lane * 16) = v;
+    }
+  } else {
+#pragma unroll
+    for (int p = 0; p < 2; ++p) {
+      const int s = p * 4 + tid / 64;
+      if (s * 16 >= NC) continue;
+      uint8_t* dst = codes + (n0 / kStripCols + s) * strip_bytes(K, 4) + (k0 / 128) * 1024;
+      const uint32_t v0 = plane[0][0][b][s * 16 + j], v1 = plane[1][0][b][s * 16 + j];
+      if (KR == kBlockK)
+        *reinterpret_cast<uint4*>(dst + lane * 16) = make_uint4(v0, v1, plane[2][0][b][s * 16 + j], plane[3][0][b][s * 16 + j]);
+      else
+        *reinterpret_cast<uint2*>(dst + lane * 8) = make_uint2(v0, v1);  // the half tile that ends a strip
+    }
+  }
+}
+
+// out[k,n] = cast_T(float(code) * float(scale)), the same block and thread shape.
+template <int DT, int BITS>
+__global__ __launch_bounds__(kThreads) void dequantize_gfx950_kernel(
+    const uint8_t* __restrict__ codes, const uint16_t* __restrict__ scale, int64_t K, int64_t N, int gshift,
+    uint16_t* __restrict__ out) {
+  constexpr int kDw = BITS == 8 ? 2 : 1;
+  __shared__ __attribute__((aligned(16))) uint32_t plane[4][kDw][4][kWideN];
+  const int tid = threadIdx.x, cg = tid % 16, rg = tid / 16;
+  const int64_t n0 = static_cast<int64_t>(blockIdx.x) * kWideN;
+  const int64_t k0 = static_cast<int64_t>(blockIdx.y) * kBlockK;
+  const int KR = static_cast<int>(K - k0 < kBlockK ? K - k0 : kBlockK);
+  const int NC = static_cast<int>(N - n0 < kWideN ? N - n0 : kWideN);
+  const bool mine = cg * 8 < NC && rg * 8 < KR;
+  const int64_t k = k0 + rg * 8;
+  Pack8 s;
+  s.q = make_uint4(0, 0, 0, 0);
+  if (mine) s.q = *reinterpret_cast<const uint4*>(scale + (gshift >= 0 ? (k >> gshift) * N : 0) + n0 + cg * 8);
+
+  const int lane = tid % 64, j = lane % 16, b = lane / 16;
+  if (BITS == 8) {
+#pragma unroll
+    for (int p = 0; p < 4; ++p) {
+      const int u = p * 4 + tid / 64, st = u / 2, t = u % 2;
+      if (st * 16 >= NC || t * 64 >= KR) continue;
+      const uint4 v = *reinterpret_cast<const uint4*>(codes + (n0 / kStripCols + st) * strip_bytes(K, 8) +
+                                                      (k0 / 64 + t) * 1024 + lane * 16);
+      plane[2 * t][0][b][st * 16 + j] = v.x;
+      plane[2 * t][kDw - 1][b][st * 16 + j] = v.y;
+      plane[2 * t + 1][0][b][st * 16 + j] = v.z;
+      plane[2 * t + 1][kDw - 1][b][st * 16 + j] = v.w;
+    }
+  } else {
+#pragma unroll
+    for (int p = 0; p < 2; ++p) {
+      const int st = p * 4 + tid / 64;
+      if (st * 16 >= NC) continue;
+      const uint8_t* src = codes + (n0 / kStripCols + st) * strip_bytes(K, 4) + (k0 / 128) * 1024;
+      if (KR == kBlockK) {
+        const uint4 v = *reinterpret_cast<const uint4*>(src + lane * 16);
+        plane[0][0][b][st * 16 + j] = v.x;
+        plane[1][0][b][st * 16 + j] = v.y;
+        plane[2][0][b][st * 16 + j] = v.z;
+        plane[3][0][b][st * 16 + j] = v.w;
+      } else {
+        const uint2 v = *reinterpret_cast<const uint2*>(src + lane * 8);
+        plane[0][0][b][st * 16 + j] = v.x;
+        plane[1][0][b][st * 16 + j] = v.y;
+      }
+    }
+  }
+  __syncthreads();
+  if (!mine) return;
+  uint32_t d[8][kDw];
+#pragma unroll
+  for (int h = 0; h < kDw; ++h)
+#pragma unroll
+    for (int c = 0; c < 8; c += 4) {
+      const uint4 v = *reinterpret_cast<const uint4*>(&plane[rg / 4][h][rg % 4][cg * 8 + c]);
+      // biased -> two's complement fields
+      const uint32_t flip = BITS == 8 ? 0x80808080u : 0x88888888u;
+      d[c][h] = v.x ^ flip; d[c + 1][h] = v.y ^ flip; d[c + 2][h] = v.z ^ flip; d[c + 3][h] = v.w ^ flip;
+    }
+  float sf[8];
+  bool finite = true;
+#pragma unroll
+  for (int c = 0; c < 8; ++c) {
+    sf[c] = to_f32<DT>(s.h[c]);
+    finite = finite && fabsf(sf[c]) <= 3.402823466e38f;
+  }
+  auto code = [&](int c, int i) {
+    if (BITS == 8) return static_cast<int>(static_cast<int8_t>((d[c][(i / 4) % kDw] >> (8 * (i % 4))) & 0xFFu));
+    const int p = i % 2 == 0 ? i / 2 : 4 + i / 2;
+    return static_cast<int>(d[c][0] << (28 - 4 * p)) >> 28;
+  };
+  uint16_t* dst = out + k * N + n0 + cg * 8;
+  if (finite) {  // no NaN can come up: the hardware's conversions give from_f32_rne's bits
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      Pack8 o;
+#pragma unroll
+      for (int c = 0; c < 8; ++c) o.h[c] = cast_out<DT>(static_cast<float>(code(c, i)) * sf[c]);
+      *reinterpret_cast<uint4*>(dst + i * N) = o.q;
+    }
+    return;
+  }
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    Pack8 o;
+#pragma unroll
+    for (int c = 0; c < 8; ++c) o.h[c] = from_f32_rne<DT>(static_cast<float>(code(c, i)) * sf[c]);
+    *reinterpret_cast<uint4*>(dst + i * N) = o.q;
+  }
+}
+
+inline dim3 wide_grid(int64_t K, int64_t N) {
+  return dim3(static_cast<unsigned>((N + kWideN - 1) / kWideN), static_cast<unsigned>((K + kBlockK - 1) / kBlockK));
+}
+
 inline dim3 block_grid(int64_t K, int64_t N) {
   return dim3(static_cast<unsigned>((N + kBlockN - 1) / kBlockN),
               static_cast<unsigned>((K + kBlockK - 1) / kBlockK));
@@ -444,8 +729,25 @@ int launch_quantize(const void* w, int dtype, int64_t K, int64_t N, int bits, in
     else
       amax_kernel<WOL_DTYPE_F16><<<g, dim3(kThreads), 0, stream>>>(wp, K, N, amax);
   }
-  const dim3 grid = block_grid(K, N);
   uint8_t* cp = static_cast<uint8_t*>(codes);
+  if (layout == WOL_LAYOUT_GFX950 && !scale_f32) {
+    uint16_t* sp = static_cast<uint16_t*>(scale);
+    const dim3 wide = wide_grid(K, N);
+#define WOL_QW(DT, B)                                                                                                   \
+  do {                                                                                                                  \
+    if (group_size == 64) quantize_gfx950_kernel<DT, B, 64><<<wide, dim3(kThreads), 0, stream>>>(wp, K, N, round_mode, amax, cp, sp);        \
+    else if (group_size == 128) quantize_gfx950_kernel<DT, B, 128><<<wide, dim3(kThreads), 0, stream>>>(wp, K, N, round_mode, amax, cp, sp); \
+    else quantize_gfx950_kernel<DT, B, 0><<<wide, dim3(kThreads), 0, stream>>>(wp, K, N, round_mode, amax, cp, sp);                          \
+  } while (0)
+    if (dtype == WOL_DTYPE_BF16) {
+      if (bits == 8) WOL_QW(WOL_DTYPE_BF16, 8); else WOL_QW(WOL_DTYPE_BF16, 4);
+    } else {
+      if (bits == 8) WOL_QW(WOL_DTYPE_F16, 8); else WOL_QW(WOL_DTYPE_F16, 4);
+    }
+#undef WOL_QW
+    return check_launch();
+  }
+  const dim3 grid = block_grid(K, N);
   const int sf = scale_f32 ? 1 : 0;
 #define WOL_Q(DT, B)                                                                   \
   quantize_kernel<DT, B><<<grid, dim3(kThreads), 0, stream>>>(wp, K, N, group_size,   \
@@ -498,10 +800,22 @@ int launch_quantize_static(const void* w, int dtype, int64_t K, int64_t N, int b
 
 int launch_dequantize(const void* codes, int layout, const void* scale, int dtype, int64_t K,
                       int64_t N, int bits, int group_size, void* out, hipStream_t stream) {
-  const dim3 grid = block_grid(K, N);
   const uint8_t* cp = static_cast<const uint8_t*>(codes);
   const uint16_t* sp = static_cast<const uint16_t*>(scale);
   uint16_t* op = static_cast<uint16_t*>(out);
+  if (layout == WOL_LAYOUT_GFX950) {
+    const int gshift = group_size == 64 ? 6 : (group_size == 128 ? 7 : -1);
+    const dim3 wide = wide_grid(K, N);
+#define WOL_DQW(DT, B) dequantize_gfx950_kernel<DT, B><<<wide, dim3(kThreads), 0, stream>>>(cp, sp, K, N, gshift, op)
+    if (dtype == WOL_DTYPE_BF16) {
+      if (bits == 8) WOL_DQW(WOL_DTYPE_BF16, 8); else WOL_DQW(WOL_DTYPE_BF16, 4);
+    } else {
+      if (bits == 8) WOL_DQW(WOL_DTYPE_F16, 8); else WOL_DQW(WOL_DTYPE_F16, 4);
+    }
+#undef WOL_DQW
+    return check_launch();
+  }
+  const dim3 grid = block_grid(K, N);
 #define WOL_DQ(DT, B) \
   dequantize_kernel<DT, B><<<grid, dim3(kThreads), 0, stream>>>(cp, layout, sp, K, N, group_size, op)
   if (dtype == WOL_DTYPE_BF16) {

@@ -147,6 +147,31 @@ def test_quantize_near_rounding_boundaries(G, oracle, dt, bits):
     assert (frac == 0).sum() > 300, (frac == 0).sum()
 
 
+@pytest.mark.parametrize("dt", [H.F16, H.BF16])
+@pytest.mark.parametrize("bits", [8, 4])
+@pytest.mark.parametrize("g", [-1, 64, 128])
+def test_gfx950_layout_codes_without_a_division(G, oracle, dt, bits, g):
+    # the kernel of the GFX950 layout multiplies by the scale's reciprocal: quotients on and
+    # next to every rounding boundary, scales over T's whole range (subnormal, zero, infinite
+    # and NaN ones take the division), both scale roundings; K that ends in half a block, N
+    # that ends inside one.  Codes, scales and the way back are the oracle's bit for bit.
+    K, N = 320, 176
+    wb = _near_tie_weight(dt, bits, K, N, seed=40 + bits)
+    wb[:, 3] = 0
+    wb[5, 2], wb[0, 17], wb[70, 18], wb[130, 150] = [H.f32_to_bits(np.array([v], np.float32), dt)[0]
+                                                    for v in (np.nan, np.nan, np.inf, -np.inf)]
+    wb[:, 33] = wb[:, 33] & 0x8003  # smallest magnitudes of T
+    wb[:, 34] = (wb[:, 34] & 0x83FF) | (0x7B00 if dt == H.F16 else 0x7F00)  # largest
+    for trunc in (False, True):
+        oc, osc = oracle.weight_quantize(wb, dt, bits, g, cast_mode=oracle.CAST_TRUNC if trunc else oracle.CAST_RNE)
+        want = H.gfx950_from_q(H.q_from_canonical(oc, bits), bits)
+        gc, gs = G.quantize(wb, dt, bits, g, layout=2, round_mode=1 if trunc else 0)
+        assert np.array_equal(gs, osc)
+        assert np.array_equal(gc, want), np.argwhere(gc != want)[:5]
+    _, oT = oracle.dequantize(oc, osc, dt, bits, g)
+    assert np.array_equal(G.dequantize(want, 2, osc, dt, K, N, bits, g), oT)
+
+
 @pytest.mark.parametrize("bits", [8, 4])
 def test_repack_round_trips(G, bits):
     rng = np.random.default_rng(bits)
