@@ -5,7 +5,7 @@ for quant_method "weight_only_int8" / "weight_only_int4"."""
 import torch
 
 from ... import _lib
-from .quantized_linear import _dtype_id, _require_gpu, _stream_ptr, weight_quantize
+from .quantized_linear import _dtype_id, _on_device, _require_gpu, _stream_ptr, weight_quantize
 
 
 def moe_quantize_experts(w, algo="weight_only_int8"):
@@ -56,7 +56,7 @@ def moe_ffn(permute_input, token_nums_per_expert, ffn1_weight, ffn2_weight, ffn1
     w1, w2 = ffn1_weight.contiguous(), ffn2_weight.contiguous()
     s1, s2 = ffn1_scale.contiguous(), ffn2_scale.contiguous()
     cnt = token_nums_per_expert.contiguous()
-    with torch.cuda.device(x.device):
+    with _on_device(x.device):
         _lib.check(
             _lib.lib.wol_moe_ffn(
                 x.data_ptr(), cnt.data_ptr(), w1.data_ptr(), None if b1 is None else b1.data_ptr(), s1.data_ptr(),
