@@ -25,6 +25,7 @@
 //             so the result does not depend on the cut) and applies the same
 //             epilogue.
 #include <atomic>
+#include <climits>
 
 #include "wol_common.h"
 
@@ -367,9 +368,8 @@ __device__ inline uint16_t merge_plain(int acc, float range, float ws, bool has_
 }
 
 // Eight neighbouring columns nn .. nn+7 of row m: the merge with the outlier
-// columns' product (when there are any: out of LDS if xs is given, computed on
-// the spot if wd_stride is negative, else as the outlier kernel left it in the
-// output's own place) and one 16-byte store.  ws and bias hold the eight columns' values.
+// columns' product (when there are any: out of LDS if xs is given, else as the
+// outlier kernel left it in the output's own place) and one 16-byte store.  ws and bias hold the eight columns' values.
 template <int DT>
 __device__ inline void finish8(const Epi& e, int cnt, int m, int nn, float range, i32x4 s0, i32x4 s1,
                                const float* ws, const float* bias, const float* xs, int xs_stride,
@@ -401,22 +401,6 @@ __device__ inline void finish8(const Epi& e, int cnt, int m, int nn, float range
       for (int i = 0; i < 4; ++i) {
         sub[i] += xv * w0[i];
         sub[4 + i] += xv * w1[i];
-      }
-    }
-#pragma unroll
-    for (int i = 0; i < 8; ++i) sub[i] = to_f32<DT>(cast_out<DT>(sub[i]));
-  } else if (wd_stride < 0) {
-    // very few rows: straight from x and the weight, no outlier kernel ran
-#pragma unroll
-    for (int i = 0; i < 8; ++i) sub[i] = 0.0f;
-#pragma unroll 1
-    for (int j = 0; j < cnt; ++j) {
-      const int kj = e.list[j];
-      const float xv = to_f32<DT>(e.x[static_cast<int64_t>(m) * e.K + kj]);
-#pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        const float w = static_cast<float>(e.w[static_cast<int64_t>(nn + i) * e.K + kj]);
-        sub[i] += xv * to_f32<DT>(cast_out<DT>(w * ws[i]));
       }
     }
 #pragma unroll
@@ -507,6 +491,7 @@ struct GemmParams {
   const int8_t* qx;  // [M,K]
   Epi e;
   int32_t* acc;      // [runs][M,N] int32, one slab per K run; only with K runs
+  int8_t* ow;        // [kStash][N] weight bytes of up to kStash outlier columns, for llm_merge_few_kernel; else null
   int nbx, nby;      // tiles along N and M
   int n_lo, n_hi;    // columns [n_lo, n_hi) of the output belong to this launch
   int tiles_per_run; // k tiles per K run
@@ -521,6 +506,18 @@ __device__ inline int row_swizzle(int row) {
   if (C == 8) return (row & 7) ^ ((row >> 3) & 1);                             // 128-byte rows
   return ((((row >> 1) ^ (row >> 3)) & 1) << 1) | ((row >> 2) & 1);            // 64-byte rows
 }
+
+// Outlier columns whose weight bytes the GEMM with K runs picks out of its own
+// tiles as they pass through LDS and leaves in Workspace::ow for the merge kernel
+// of up to kFewRows rows: the bytes of one k of w [N,K] lie K apart, for a K of a
+// few KiB all behind the same memory channel, and cost far more as loads of that
+// kernel's own.  Whole call, K = 4096, N = 11008, 4 rows, 3 outlier columns: 31.1
+// -> 22.9 us (28.7 before that kernel's loads went out in batches); K = 8192, N =
+// 4096, 3 rows, 20 of them: 66.6 -> 24.8.  (Without K runs the epilogue's gather
+// stays: picking was 2 % faster with 8 outlier columns, 1 % slower with none.)
+constexpr int kStash = 32;
+constexpr int kFewRows = 4;
+constexpr int stash_lds_bytes(int bn) { return 512 + kStash * bn; }  // list and count, then [kStash][bn] bytes
 
 // WM x WN wavefronts, each TM x TN blocks of 32x32; k tiles of TK bytes per row
 // (128: whole cache lines per row and load; 64 for a K that is not a multiple
@@ -607,6 +604,15 @@ __global__ __launch_bounds__(WM* WN * 64) __attribute__((amdgpu_waves_per_eu(2))
         16, 0, 0);                                                                                   \
   } while (0)
 
+  // the outlier list and count, ahead of the tiles in the same in-order stream
+  unsigned char* const lds_list = smem + kStages * kStage;
+  int8_t* const stash = reinterpret_cast<int8_t*>(lds_list + 512);
+  if (RUNS && p.ow != nullptr && wave == 0) {
+    __builtin_amdgcn_global_load_lds(reinterpret_cast<const uint8_t*>(p.e.list + lane), (lds_ptr_t)lds_list, 4, 0, 0);
+    __builtin_amdgcn_global_load_lds(reinterpret_cast<const uint8_t*>(p.e.count), (lds_ptr_t)(lds_list + 256), 4, 0, 0);
+  }
+  int my_k = INT_MAX;  // outlier column number `lane`
+
   i32x16 acc[TM][TN];
 #pragma unroll
   for (int a = 0; a < TM; ++a)
@@ -647,6 +653,23 @@ __global__ __launch_bounds__(WM* WN * 64) __attribute__((amdgpu_waves_per_eu(2))
     __builtin_amdgcn_sched_barrier(0);
     WOL_LLM_ISSUE(it + kStages - 1);  // into the stage every wavefront finished reading before the barrier
     __builtin_amdgcn_sched_barrier(0);
+    if (RUNS && it == 0 && p.ow != nullptr) {  // landed with the first tile
+      const int c = *reinterpret_cast<const int*>(lds_list + 256);
+      if (c <= kStash && lane < c) my_k = *reinterpret_cast<const int*>(lds_list + lane * 4);
+    }
+    if (RUNS) {
+      const int kt = (t0 + it) * kTK;
+      unsigned long long hit = __ballot(my_k >= kt && my_k < kt + kTK);
+      while (hit != 0) {
+        const int j = __builtin_ctzll(hit);
+        hit &= hit - 1;
+        const int kj = __builtin_amdgcn_readlane(my_k, j) - kt;
+        for (int row = tid; row < BN; row += NW * 64)
+          stash[j * BN + row] =
+              static_cast<int8_t>(stage[kABytes + row * kTK + (((kj >> 4) ^ row_swizzle<C>(row)) << 4) + (kj & 15)]);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) {
       if (ks + 1 < KS) {
@@ -700,6 +723,15 @@ __global__ __launch_bounds__(WM* WN * 64) __attribute__((amdgpu_waves_per_eu(2))
   float* xs = rng + BM;                                                  // [cnt][BM]
   float* wdl = xs + p.cap * BM;                                          // [cnt][BN]
   const bool fused = !RUNS && cnt > 0 && cnt <= p.cap;
+  if (RUNS && p.ow != nullptr) {
+    const int lo = t0 * kTK, hi = (t0 + niter) * kTK;
+    unsigned long long got = __ballot(my_k >= lo && my_k < hi);
+    for (; got != 0; got &= got - 1) {
+      const int j = __builtin_ctzll(got);
+      for (int row = tid; row < BN; row += NW * 64)
+        if (n0 + row < N) p.ow[static_cast<int64_t>(j) * N + n0 + row] = stash[j * BN + row];
+    }
+  }
   if (!RUNS) {
     // (read per row out of global memory inside the row loop they cost a
     // memory latency per row, sixteen in a row per wavefront)
@@ -758,8 +790,7 @@ __global__ __launch_bounds__(WM* WN * 64) __attribute__((amdgpu_waves_per_eu(2))
 
 // Adds the K runs' int32 sums and finishes; one thread per eight columns.
 template <int DT>
-__global__ __launch_bounds__(256) void llm_merge_kernel(const int32_t* __restrict__ acc, int runs, Epi e,
-                                                        int direct_outliers) {
+__global__ __launch_bounds__(256) void llm_merge_kernel(const int32_t* __restrict__ acc, int runs, Epi e) {
   const int64_t i = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
   const int groups = e.N / 8;
   if (i >= static_cast<int64_t>(e.M) * groups) return;
@@ -774,7 +805,57 @@ __global__ __launch_bounds__(256) void llm_merge_kernel(const int32_t* __restric
   }
   float ws[8], bias[8];
   load_ws_bias8<DT>(e, nn, ws, bias);
-  finish8<DT>(e, *e.count, m, nn, e.ranges[m], s0, s1, ws, bias, nullptr, 0, nullptr, direct_outliers ? -1 : 0);
+  finish8<DT>(e, *e.count, m, nn, e.ranges[m], s0, s1, ws, bias, nullptr, 0, nullptr, 0);
+}
+
+// The same for up to kFewRows rows, the outlier columns multiplied here (no
+// outlier kernel ran).  Latency-bound: a thread takes one column of all rows, so
+// that every weight byte is fetched once, eight of them in flight at a time.
+template <int DT>
+__global__ __launch_bounds__(64) void llm_merge_few_kernel(const int32_t* __restrict__ acc, int runs, Epi e,
+                                                           const int8_t* __restrict__ ow) {
+  const int n = blockIdx.x * 64 + threadIdx.x;
+  if (n >= e.N) return;
+  const int cnt = *e.count;
+  const int64_t slab = static_cast<int64_t>(e.M) * e.N;
+  int32_t sum[kFewRows] = {0, 0, 0, 0};
+#pragma unroll 4
+  for (int r = 0; r < runs; ++r)
+#pragma unroll
+    for (int m = 0; m < kFewRows; ++m)
+      sum[m] += acc[r * slab + static_cast<int64_t>(m < e.M ? m : e.M - 1) * e.N + n];
+  const float ws = e.wscale[n];
+  const float bias = e.bias != nullptr ? to_f32<DT>(e.bias[n]) : 0.0f;
+  const int8_t* wrow = e.w + static_cast<int64_t>(n) * e.K;
+  float sub[kFewRows] = {0.0f, 0.0f, 0.0f, 0.0f};
+  constexpr int W = 8;
+  const bool picked = cnt <= kStash;  // more than the GEMM picks: out of the weight itself
+  for (int j0 = 0; j0 < cnt; j0 += W) {  // ascending k, as everywhere
+    // every load of the batch under no condition (past the end: the last column, the last row again)
+    int k[W];
+    float w[W], xv[W][kFewRows];
+#pragma unroll
+    for (int u = 0; u < W; ++u) k[u] = e.list[j0 + u < cnt ? j0 + u : cnt - 1];
+#pragma unroll
+    for (int u = 0; u < W; ++u) {
+      const int j = j0 + u < cnt ? j0 + u : cnt - 1;
+      w[u] = static_cast<float>(picked ? ow[static_cast<int64_t>(j) * e.N + n] : wrow[k[u]]);
+#pragma unroll
+      for (int m = 0; m < kFewRows; ++m)
+        xv[u][m] = to_f32<DT>(e.x[static_cast<int64_t>(m < e.M ? m : e.M - 1) * e.K + k[u]]);
+    }
+#pragma unroll
+    for (int u = 0; u < W; ++u) {
+      const float wd = to_f32<DT>(cast_out<DT>(w[u] * ws));
+#pragma unroll
+      for (int m = 0; m < kFewRows; ++m) sub[m] = j0 + u < cnt ? sub[m] + xv[u][m] * wd : sub[m];
+    }
+  }
+#pragma unroll
+  for (int m = 0; m < kFewRows; ++m)
+    if (m < e.M)
+      e.out[static_cast<int64_t>(m) * e.N + n] = static_cast<uint16_t>(
+          merge_one<DT>(sum[m], to_f32<DT>(cast_out<DT>(sub[m])), e.ranges[m], ws, e.bias != nullptr, bias));
 }
 
 inline void allow_lds(const void* kern, size_t lds, std::atomic<uint32_t>& done) {
@@ -866,6 +947,7 @@ struct Workspace {
   int32_t* list;
   int8_t* qx;
   int32_t* acc;
+  int8_t* ow;
   int64_t bytes;
 };
 
@@ -888,6 +970,8 @@ Workspace carve(void* base, int64_t M, int64_t K, int64_t N, int runs) {
   off += align256(M * K);
   w.acc = reinterpret_cast<int32_t*>(p + off);
   off += align256(M * N * 4 * runs);
+  w.ow = reinterpret_cast<int8_t*>(p + off);
+  if (runs > 1 && M <= kFewRows) off += align256(kStash * N);
   w.bytes = off;
   return w;
 }
@@ -895,8 +979,8 @@ Workspace carve(void* base, int64_t M, int64_t K, int64_t N, int runs) {
 template <int DT, int WM, int WN, int TM, int TN, int TK, int STAGES, bool RUNS>
 int launch_gemm(const GemmParams& p, int runs, hipStream_t stream) {
   constexpr int BM = WM * TM * 32, BN = WN * TN * 32;
-  constexpr size_t lds = static_cast<size_t>(STAGES) * (BM + BN) * TK;
-  static_assert(lds >= static_cast<size_t>(WM * WN) * 32 * 40 * 4 + BM * 4,
+  constexpr size_t stages = static_cast<size_t>(STAGES) * (BM + BN) * TK, lds = stages + (RUNS ? stash_lds_bytes(BN) : 0);
+  static_assert(stages >= static_cast<size_t>(WM * WN) * 32 * 40 * 4 + BM * 4,
                 "the epilogue's slabs and row ranges must fit the stages");
   static std::atomic<uint32_t> done{0};
   auto kern = llm_gemm_kernel<DT, WM, WN, TM, TN, TK, STAGES, RUNS>;
@@ -980,6 +1064,7 @@ int run_llm_int8(const void* x, const void* weight, const void* bias, const floa
             ws.count, ws.list, static_cast<uint16_t*>(out), static_cast<int>(M), static_cast<int>(K),
             static_cast<int>(N)};
   p.acc = ws.acc;
+  p.ow = pl.runs > 1 && M <= kFewRows ? ws.ow : nullptr;
   p.n_lo = 0;
   p.n_hi = static_cast<int>(N);
   p.nbx = static_cast<int>((N + pl.bn - 1) / pl.bn);
@@ -994,7 +1079,7 @@ int run_llm_int8(const void* x, const void* weight, const void* bias, const floa
   }
   // up to four rows with K runs the merge kernel multiplies the outlier columns
   // itself (a launch costs more than that work)
-  const bool direct = pl.runs > 1 && M <= 4;
+  const bool direct = pl.runs > 1 && M <= kFewRows;
   if (!direct)
     hipLaunchKernelGGL(llm_outlier_kernel<DT>, dim3(static_cast<unsigned>(((N + 255) / 256) * ((M + 63) / 64))),
                        dim3(256), 0, stream, p.e, p.cap);
@@ -1016,9 +1101,14 @@ int run_llm_int8(const void* x, const void* weight, const void* bias, const floa
   if (pl.runs == 1) return launch_gemm_tk<DT, false>(p, pl, stream);
   const int rc = launch_gemm_tk<DT, true>(p, pl, stream);
   if (rc != WOL_OK) return rc;
+  if (direct) {
+    hipLaunchKernelGGL(llm_merge_few_kernel<DT>, dim3(static_cast<unsigned>((N + 63) / 64)), dim3(64), 0, stream,
+                       ws.acc, pl.runs, p.e, ws.ow);
+    return check_launch();
+  }
   const int64_t total = M * (N / 8);
   hipLaunchKernelGGL(llm_merge_kernel<DT>, dim3(static_cast<unsigned>((total + 255) / 256)), dim3(256), 0, stream,
-                     ws.acc, pl.runs, p.e, direct ? 1 : 0);
+                     ws.acc, pl.runs, p.e);
   return check_launch();
 }
 

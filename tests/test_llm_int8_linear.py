@@ -250,6 +250,30 @@ GPU_CASES = [  # M, K, N, kind, threshold, bias
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("dt", [H.F16, H.BF16])
+@pytest.mark.parametrize("cnt", [1, 8, 9, 32, 33])
+@pytest.mark.parametrize("M,K,N", [(3, 1024, 400), (4, 576, 272), (130, 512, 400), (300, 576, 272)])
+def test_gpu_outlier_columns_out_of_the_gemm_tiles(device, oracle, dt, cnt, M, K, N):
+    # with K runs and up to four rows the weight bytes of up to 32 outlier columns are picked out of
+    # the GEMM's own tiles: columns at the ends of K, on both sides of a k tile and spread over the
+    # runs; one more than the tiles' stash holds; and many rows, where the epilogue gathers them
+    _, w_nk, ws = _weights(K, N, dt, seed=K + N)
+    rng = np.random.default_rng(cnt)
+    cols = np.r_[[0, K - 1, 127, 128, 63, 64, 255, 256], rng.permutation(np.arange(300, K - 1))][:cnt]
+    x = np.clip(rng.standard_normal((M, K), dtype=np.float32), -5, 5)
+    x[rng.integers(0, M, cnt), cols] = 20.0 + rng.random(cnt, dtype=np.float32)
+    xb, bb = H.f32_to_bits(x, dt), H.make_bias(N, dt, seed=3, std=1.0)
+    want = oracle.llm_int8_linear(xb, w_nk, bb, ws, 6.0, dt)
+    assert want["outlier"].sum() == cnt
+    import torch
+    from paddle_amd.nn import quant as Q
+
+    got = Q.llm_int8_linear(H.bits_to_torch(xb, dt, "cuda:0"), torch.from_numpy(np.ascontiguousarray(w_nk)).to("cuda:0"),
+                            H.bits_to_torch(bb, dt, "cuda:0"), torch.from_numpy(np.asarray(ws)).to("cuda:0"), 6.0)
+    assert np.array_equal(H.torch_to_bits(got), want["out"])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dt", [H.F16, H.BF16])
 @pytest.mark.parametrize("case", GPU_CASES)
 def test_gpu_llm_int8_linear_bit_exact(device, oracle, dt, case):
     import gpu_calls as G
