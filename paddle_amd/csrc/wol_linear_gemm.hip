@@ -1159,7 +1159,8 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_dma_kernel(const DmaParams 
   at.m0 = by * (WM * TM * 32);
   at.expert = -1;
   at.row0 = at.rows = 0;
-  if (p.moe_table != nullptr) {
+  // (grouped launches of this kernel are those of small tiles: the others know at compile time that they have no expert)
+  if (WM == 1 && p.moe_table != nullptr) {
     const MoeTile t = reinterpret_cast<const MoeTile*>(p.moe_table)[by];
     if (t.expert < 0) return;
     at.expert = t.expert;
