@@ -127,13 +127,38 @@ struct DequantExact<WOL_DTYPE_F16, 4> {
   }
 };
 
-// Each nibble pair becomes two fp16 values 1024 + 16 * nibble (one and-or), a
-// mixed-precision FMA takes the offset out and widens to fp32 in one
-// instruction, and the high halves are the bf16 codes: 19 instructions per
-// eight codes, every step exact.  (Widening two bf16 values 136 + code and
-// subtracting in fp32 takes 27.)
 template <>
 struct DequantExact<WOL_DTYPE_BF16, 4> {
+  __device__ static inline uint32_t fix(uint32_t pair) {
+    // pair = two bf16 holding 136 + code; widen, subtract, narrow (all exact)
+    const float lo = __uint_as_float(pair << 16) - 136.0f;
+    const float hi = __uint_as_float(pair & 0xFFFF0000u) - 136.0f;
+    return pack_bf16_hi(lo, hi);
+  }
+  __device__ static inline u32x4 run(const uint32_t* w) {
+    const uint32_t v = w[0];
+    u32x4 o;
+    o.x = fix((v & 0x000F000Fu) | 0x43004300u);
+    o.y = fix(((v >> 4) & 0x000F000Fu) | 0x43004300u);
+    o.z = fix(((v >> 8) & 0x000F000Fu) | 0x43004300u);
+    o.w = fix(((v >> 12) & 0x000F000Fu) | 0x43004300u);
+    return o;
+  }
+};
+
+// The same codes in 19 instructions per eight instead of 27: each nibble pair
+// becomes two fp16 values 1024 + 16 * nibble (one and-or), a mixed-precision FMA
+// takes the offset out and widens to fp32 in one instruction, and the high
+// halves are the bf16 codes, every step exact.  The half-deep tiles gain 1 to 2 %
+// from it.  Elsewhere the longer form is the faster one: the FMAs keep no
+// distance to the MFMAs around them and the loop fills with waits (s_nop 41 and
+// 55 against 13 and 14 per tile of 128 x 256 x 128, g128; 200 rows, K = N = 4096:
+// 31.6 against 30.7 us; swiglu, 200 rows, K = 4096, N = 8192: 70.0 against 67.6).
+template <int DT, int BITS>
+struct DequantExactFma : DequantExact<DT, BITS> {};
+
+template <>
+struct DequantExactFma<WOL_DTYPE_BF16, 4> {
   __device__ static inline uint32_t pair(uint32_t v) {
     const f16x2 h = __builtin_bit_cast(f16x2, (v & 0x00F000F0u) | 0x64006400u);
     return pack_bf16_hi(__builtin_fmaf(static_cast<float>(h.x), 0.0625f, -72.0f),
@@ -517,9 +542,19 @@ struct MoeTile {
 // tile (for its own tile loads, then for the workgroup) and around the
 // epilogue, and leaves the sums in p.stamps.  The reads sit where the
 // wavefront has just waited for all its LDS traffic anyway.
-// The work of one workgroup is a device function (dma_tile) of where its tile
-// lies: gemm_dma_kernel below calls it for the one tile height it is built
-// for, gemm_experts_kernel picks the height of every tile at run time.
+//
+// The work of one workgroup is a device function (dma_tile): gemm_dma_kernel
+// below calls it for the one tile height it is built for and lets it find its
+// tile from the workgroup id, gemm_experts_kernel (EXPERTS) picks the height of
+// every tile at run time and says where it lies.  The form of the function is
+// the one whose inner loops the compiler orders best: for gemm_dma_kernel the
+// parameters come by value, the LDS is named inside and the tile is found after
+// the lane arithmetic.  By reference, with the LDS and the tile's place as
+// arguments, the same loops run 2 to 4 % longer (int8 g128, 256 rows, K =
+// 11008, N = 4096: 52.6 against 50.0 us; int4 per channel, 200 rows, same
+// weight: 47.3 against 45.9; per-channel int8 at 2048 rows level).  The four
+// heights of gemm_experts_kernel are 0.4 % faster by reference.
+//
 // kHalfDeep (STAGES = kHalfDeepStages + 3; int4): three stages of 64-deep tiles
 // of activations (and scales) where two 128-deep ones would overflow the LDS.
 // The packed weight still arrives in its 128-deep tiles of 16 bytes per lane:
@@ -529,17 +564,17 @@ struct MoeTile {
 // the same number of loads, so the counted waits are those of the other forms.
 constexpr int kHalfDeepStages = 10;
 
+// Where a tile of gemm_experts_kernel lies.
 struct TilePlace {
   int bx;      // column tile of the launch
-  int m0;      // first row of the tile, counted from x and out
-  int split;   // run of k tiles
-  int expert;  // >= 0: the tile lies in this expert's rows
-  int row0;    // expert >= 0: the tile's first row in x and out
-  int rows;    // expert >= 0: rows of the tile that exist
+  int expert;  // the tile lies in this expert's rows
+  int row0;    // the tile's first row in x and out
+  int rows;    // rows of the tile that exist
 };
 
-template <int DT, int BITS, int G, int OFFS, int WM, int WN, int TM, int TN, int STAGES, int SWI, bool RESC, bool STAMP>
-__device__ __forceinline__ void dma_tile(const DmaParams& p, unsigned char* smem, const TilePlace at) {
+template <int DT, int BITS, int G, int OFFS, int WM, int WN, int TM, int TN, int STAGES, int SWI, bool RESC, bool STAMP,
+          bool EXPERTS>
+__device__ __forceinline__ void dma_tile(std::conditional_t<EXPERTS, const DmaParams&, const DmaParams> p, const TilePlace at) {
 #if defined(__HIP_DEVICE_COMPILE__)  // the host pass only needs the launch stubs
   constexpr int NW = WM * WN;
   constexpr int BM = WM * TM * 32, BN = WN * TN * 32;
@@ -580,8 +615,11 @@ __device__ __forceinline__ void dma_tile(const DmaParams& p, unsigned char* smem
   // SWI with one block per wavefront: wavefront columns 2i and 2i+1 hold the gate and the up block of
   // the same 32 output columns, and the up wavefront hands its sums over through LDS in the epilogue
   constexpr bool kPair = SWI != 0 && TN == 1;
+  // the small-M tiles and the half-deep ones take the shorter int4 dequantiser (see DequantExactFma)
+  constexpr bool kFmaDequant = BITS == 4 && OFFS == 0 && (kHalfDeep || WM == 1);
   static_assert(OFFS != 2 || G == 0, "row sums by dot products are taken out once, in the epilogue");
   static_assert(!RESC || (G != 0 && OFFS == 0), "rescaled sums are for group-wise scales and the exact dequantisers");
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   unsigned long long st_entry = 0, st_prev = 0, st_work = 0, st_loads = 0, st_bar = 0, st_loop0 = 0;
   if (STAMP) st_entry = __builtin_readcyclecounter();
 
@@ -596,18 +634,37 @@ __device__ __forceinline__ void dma_tile(const DmaParams& p, unsigned char* smem
   const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave / WN, wn = wave % WN;
   const int j = lane & 15, sp = (lane >> 4) & 1, b = lane >> 5, r32 = lane & 31;
-  const int bx = at.bx, split = at.split;
-  int m0 = at.m0;
-  if (at.expert >= 0) {
+  int bx, m0 = 0, split = 0;
+  int expert = -1, row0 = 0, rows = 0;
+  if constexpr (EXPERTS) {
+    bx = at.bx;
+    expert = at.expert;
+    row0 = at.row0;
+    rows = at.rows;
+  } else {
+    const int ntiles = p.nbx * p.nby;
+    split = blockIdx.x / ntiles;
+    int by;
+    tile_of_block_2d(blockIdx.x - split * ntiles, p.nbx, p.nby, p.xcd_rows, &bx, &by);
+    m0 = by * BM;
+    if (SWI == 0 && p.moe_table != nullptr) {  // (grouped launches with a fused swiglu are gemm_experts_kernel's)
+      const MoeTile t = reinterpret_cast<const MoeTile*>(p.moe_table)[by];
+      if (t.expert < 0) return;
+      expert = t.expert;
+      row0 = t.row0;
+      rows = t.rows;
+    }
+  }
+  if (expert >= 0) {
     // this tile belongs to one expert: shift every base to that expert and to
     // the tile's first row, and let M be the rows that exist
-    x += static_cast<int64_t>(at.row0) * K;
-    if (p.nsplit > 1) outp = static_cast<float*>(outp) + static_cast<int64_t>(at.row0) * N;  // partial sums
-    else outp = static_cast<uint16_t*>(outp) + static_cast<int64_t>(at.row0) * (SWI ? N / 2 : N);
-    codes += static_cast<int64_t>(at.expert) * p.moe_codes_stride;
-    scale += static_cast<int64_t>(at.expert) * N;
-    if (bias != nullptr) bias += static_cast<int64_t>(at.expert) * N;
-    M = at.rows;
+    x += static_cast<int64_t>(row0) * K;
+    if (p.nsplit > 1) outp = static_cast<float*>(outp) + static_cast<int64_t>(row0) * N;  // partial sums
+    else outp = static_cast<uint16_t*>(outp) + static_cast<int64_t>(row0) * (SWI ? N / 2 : N);
+    codes += static_cast<int64_t>(expert) * p.moe_codes_stride;
+    scale += static_cast<int64_t>(expert) * N;
+    if (bias != nullptr) bias += static_cast<int64_t>(expert) * N;
+    M = rows;
     m0 = 0;
   }
   // SWI: a workgroup takes BN / 2 gate columns and the BN / 2 up columns that go with them
@@ -766,7 +823,7 @@ __device__ __forceinline__ void dma_tile(const DmaParams& p, unsigned char* smem
   // byte offsets inside a stage that do not change from tile to tile
   const int a_row_off = (wm * TM * 32 + r32) * (TK * 2);
   const int b_off = (kHalfDeep ? 0 : kABytes) + (wn * TN * 2 + sp) * 1024 + (j + 16 * b) * 16;  // kHalfDeep: in a raw B tile
-  constexpr int kValuPerMfma = ((OFFS == 2 ? 4 * TN + 4 * TM : (BITS == 8 ? 16 : DT == WOL_DTYPE_BF16 ? 18 : 12) * TN) + TM * TN - 1) / (TM * TN) + 2;
+  constexpr int kValuPerMfma = ((OFFS == 2 ? 4 * TN + 4 * TM : (BITS == 8 ? 16 : kFmaDequant && DT == WOL_DTYPE_BF16 ? 18 : 12) * TN) + TM * TN - 1) / (TM * TN) + 2;
   constexpr int kValuRescale = RESC ? 16 : 0;  // more per MFMA in the slice that starts a group
   constexpr int kHalf = (TM * TN + 1) / 2;  // MFMAs of a slice issued before the barrier
   // (With one workgroup per CU, wavefronts w and w + 4 share a SIMD and the older one wins every
@@ -802,6 +859,7 @@ __device__ __forceinline__ void dma_tile(const DmaParams& p, unsigned char* smem
     for (int c = 0; c < TN; ++c) {
       const uint32_t w4[4] = {raw[c][h].x, raw[c][h].y, raw[c][h].z, raw[c][h].w};
       if (OFFS) dst[c] = Dequant<DT, BITS>::run(&w4[step * kDw], magic);
+      else if constexpr (kFmaDequant) dst[c] = DequantExactFma<DT, BITS>::run(&w4[step * kDw]);
       else dst[c] = DequantExact<DT, BITS>::run(&w4[step * kDw]);
     }
   };
@@ -1051,7 +1109,7 @@ __device__ __forceinline__ void dma_tile(const DmaParams& p, unsigned char* smem
     // partial sums are kept compact: row length = the columns of this launch
     const int64_t ld = p.nsplit > 1 ? static_cast<int64_t>(p.strip_hi - p.strip_lo) * kStripCols : N;
     const int ncol0 = p.nsplit > 1 ? p.strip_lo * kStripCols : 0;
-    const int64_t run_rows = at.expert >= 0 ? p.moe_rows : M;  // rows of one run's partial sums
+    const int64_t run_rows = expert >= 0 ? p.moe_rows : M;  // rows of one run's partial sums
     float* outf = static_cast<float*>(outp) + (p.nsplit > 1 ? static_cast<int64_t>(split) * run_rows * ld : 0);
 #pragma unroll
     for (int a = 0; a < TM; ++a)
@@ -1150,24 +1208,7 @@ __device__ __forceinline__ void dma_tile(const DmaParams& p, unsigned char* smem
 template <int DT, int BITS, int G, int OFFS, int WM, int WN, int TM, int TN, int STAGES, int SWI = 0, bool RESC = false,
           bool STAMP = false>
 __global__ __launch_bounds__(64 * WM * WN) void gemm_dma_kernel(const DmaParams p) {
-  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-  const int ntiles = p.nbx * p.nby;
-  TilePlace at;
-  at.split = blockIdx.x / ntiles;
-  int by;
-  tile_of_block_2d(blockIdx.x - at.split * ntiles, p.nbx, p.nby, p.xcd_rows, &at.bx, &by);
-  at.m0 = by * (WM * TM * 32);
-  at.expert = -1;
-  at.row0 = at.rows = 0;
-  // (grouped launches of this kernel are those of small tiles: the others know at compile time that they have no expert)
-  if (WM == 1 && p.moe_table != nullptr) {
-    const MoeTile t = reinterpret_cast<const MoeTile*>(p.moe_table)[by];
-    if (t.expert < 0) return;
-    at.expert = t.expert;
-    at.row0 = t.row0;
-    at.rows = t.rows;
-  }
-  dma_tile<DT, BITS, G, OFFS, WM, WN, TM, TN, STAGES, SWI, RESC, STAMP>(p, smem, at);
+  dma_tile<DT, BITS, G, OFFS, WM, WN, TM, TN, STAGES, SWI, RESC, STAMP, false>(p, TilePlace{});
 }
 
 // The grouped GEMM over experts with many rows each: row tiles of up to four
@@ -1186,7 +1227,6 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_dma_kernel(const DmaParams 
 // 552; 4 experts, width 14336, 4096 rows 1130 -> 789.
 template <int DT, int BITS, int OFFS, int TN, int STAGES, int SWI>
 __global__ __launch_bounds__(512) void gemm_experts_kernel(const DmaParams p) {
-  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   const MoeTile* table = reinterpret_cast<const MoeTile*>(p.moe_table);
   const int total = table[0].expert * p.nbx;  // the header holds the number of row tiles
   constexpr int kXcd = 8;
@@ -1197,18 +1237,12 @@ __global__ __launch_bounds__(512) void gemm_experts_kernel(const DmaParams p) {
   const MoeTile any = table[1 + pos / p.nbx];
   const int w = pos - any.first * p.nbx;
   const MoeTile t = table[1 + any.first + w % any.count];
-  TilePlace at;
-  at.bx = w / any.count;
-  at.m0 = 0;
-  at.split = 0;
-  at.expert = t.expert;
-  at.row0 = t.row0;
-  at.rows = t.rows;
+  const TilePlace at{w / any.count, t.expert, t.row0, t.rows};
   const int units = (t.rows + 63) / 64;
-  if (units >= 4) dma_tile<DT, BITS, 0, OFFS, 2, 4, 4, TN, STAGES, SWI, false, false>(p, smem, at);
-  else if (units == 3) dma_tile<DT, BITS, 0, OFFS, 2, 4, 3, TN, STAGES, SWI, false, false>(p, smem, at);
-  else if (units == 2) dma_tile<DT, BITS, 0, OFFS, 2, 4, 2, TN, STAGES, SWI, false, false>(p, smem, at);
-  else dma_tile<DT, BITS, 0, OFFS, 2, 4, 1, TN, STAGES, SWI, false, false>(p, smem, at);
+  if (units >= 4) dma_tile<DT, BITS, 0, OFFS, 2, 4, 4, TN, STAGES, SWI, false, false, true>(p, at);
+  else if (units == 3) dma_tile<DT, BITS, 0, OFFS, 2, 4, 3, TN, STAGES, SWI, false, false, true>(p, at);
+  else if (units == 2) dma_tile<DT, BITS, 0, OFFS, 2, 4, 2, TN, STAGES, SWI, false, false, true>(p, at);
+  else dma_tile<DT, BITS, 0, OFFS, 2, 4, 1, TN, STAGES, SWI, false, false, true>(p, at);
 }
 
 // out[m, col0 + c] = T( sum over the runs of part[run][m][c] + bias[col0 + c] ) for the ncols
