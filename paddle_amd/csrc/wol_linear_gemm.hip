@@ -38,7 +38,7 @@ struct GemmArgs {
 
 // One product of moe_ffn (see MoeLaunch below).
 struct MoeGemmArgs {
-  const void* x; const int* table; int max_tiles, bm, ns, experts; int64_t rows; float* partial; const int64_t* valid_rows;
+  const void* x; const int* table; int max_tiles, bm, ns; bool narrow; int64_t rows; float* partial; const int64_t* valid_rows;
   const void* codes; const void* bias; const void* scale; int64_t K, N; void* out; hipStream_t stream; bool swiglu;
 };
 
@@ -1675,40 +1675,131 @@ void launch_fast(const Args& a) {
 #undef WOL_HALF
 }
 
+// How high the row tiles of gemm_experts_kernel may be.  A round of workgroups
+// takes the time of its highest tile, and a high tile costs less than its share
+// (part of a tile's time is the same for any height), so one limit of 256 rows
+// is right where tiles fill many rounds and leaves CUs idle where few tiles
+// exist or a last round is nearly empty.  The limit with the shortest estimate
+// over both products is taken:
+//   time of such a tile x sum over the products of k tiles x rounds,
+// a round being what the CUs of an XCD take of its share of the tiles.  The
+// times of 64-, 128- and 192-row tiles against 256-row ones (0.40, 0.57, 0.78 for
+// int4; 0.60, 0.70, 0.85 for int8) and of a 128-column tile against a
+// 256-column one (0.8 and 0.7) are fitted to 616 problems timed under every
+// limit (4 to 64 experts of 65 to 1000 rows, evenly and unequally loaded, hidden
+// 1024 to 4096, fc1 width 2816 to 28672): the choice is 0.9 % (int4) and 0.7 %
+// (int8) slower than the best one on average, 256 rows always 12 % and 5 %.
+// moe_ffn against the limit of 256 rows: 8 experts, hidden 1024, width 2816, 1664
+// rows, int4 64.9 -> 46.6 us, int8 53.9 -> 43.8; 4 experts, 2048, 8192, 960 rows,
+// int4 130 -> 78.
+struct MoeHeights {
+  int xcd_cus;      // CUs of an XCD
+  int min_units;    // lowest limit the launch grid has room for; 4 = 256 rows, the highest
+  int nbx1, nbx2;   // column tiles of the two products
+  float w1, w2;     // k tiles x column cost of the two products
+  float tile[4];    // time of a tile of 1 .. 4 units
+};
+constexpr int kMaxUnits = 4;
+
+__host__ __device__ inline int moe_rounds(int tiles, int nbx, int xcd_cus) {
+  constexpr int kXcd = 8;
+  const int per = (tiles * nbx + kXcd - 1) / kXcd;
+  return (per + xcd_cus - 1) / xcd_cus;
+}
+
+__host__ __device__ inline float moe_cost(const MoeHeights& h, int tiles, int units) {
+  return h.tile[units - 1] * (h.w1 * static_cast<float>(moe_rounds(tiles, h.nbx1, h.xcd_cus)) +
+                              h.w2 * static_cast<float>(moe_rounds(tiles, h.nbx2, h.xcd_cus)));
+}
+
 // Row-tile table of a grouped launch.  cum[e] is the number of rows of experts
 // 0 .. e (the inclusive running total that the reference's moe_dispatch returns
 // as token_nums_per_expert,
 // paddle/phi/kernels/fusion/cutlass/moe_dispatch.cu:174-182): expert e owns
 // rows cum[e-1] .. cum[e]-1 and ceil(rows / bm) tiles.  One workgroup.
 // header == 0: tiles of bm rows, max_tiles entries, unused ones marked -1.
-// header == 1 (gemm_experts_kernel): entry 0 holds the number of tiles, and an
+// header == 1 (gemm_experts_kernel): bm is chosen here, where the rows of every
+// expert are known (MoeHeights), entry 0 holds the number of tiles, and an
 // expert's rows are shared out in 64-row units as evenly as its ceil(rows /
 // bm) tiles allow (three tiles of 192 rows rather than two of 256 and one of
 // 64: the weight side of a tile costs the same whatever its height).
 __global__ __launch_bounds__(256) void moe_plan_kernel(const int64_t* __restrict__ cum, int num_experts, int bm,
-                                                       int max_tiles, int64_t rows, int header,
+                                                       int max_tiles, int64_t rows, int header, MoeHeights heights,
                                                        MoeTile* __restrict__ table) {
   __shared__ int first_tile[1025];  // exclusive running total of tiles, by expert
   __shared__ int row_end[1025];     // end of expert e's rows is row_end[e + 1]; row_end[0] = 0
   if (header == 0)
     for (int i = threadIdx.x; i < max_tiles; i += 256) table[i] = MoeTile{-1, 0, 0, 0, 0, {0, 0, 0}};
-  if (threadIdx.x == 0) {
-    // The running totals come from the device and are not trusted: each is
-    // clamped to [previous total, rows], so an expert's count is never negative
-    // and no tile reaches past the last row of the input.
-    int acc = 0;
-    int64_t prev = 0;
-    row_end[0] = 0;
-    for (int e = 0; e < num_experts; ++e) {
-      first_tile[e] = acc;
-      int64_t end = cum[e];
-      end = end < prev ? prev : (end > rows ? rows : end);
-      acc += static_cast<int>((end - prev + bm - 1) / bm);
-      prev = end;
-      row_end[e + 1] = static_cast<int>(end);
+  // The running totals come from the device and are not trusted: each is
+  // clamped to [previous total, rows], so an expert's count is never negative
+  // and no tile reaches past the last row of the input.
+  if (header == 0) {
+    if (threadIdx.x == 0) {
+      int acc = 0;
+      int64_t prev = 0;
+      row_end[0] = 0;
+      for (int e = 0; e < num_experts; ++e) {
+        first_tile[e] = acc;
+        int64_t end = cum[e];
+        end = end < prev ? prev : (end > rows ? rows : end);
+        acc += static_cast<int>((end - prev + bm - 1) / bm);
+        prev = end;
+        row_end[e + 1] = static_cast<int>(end);
+      }
+      first_tile[num_experts] = acc;
     }
-    first_tile[num_experts] = acc;
-    if (header != 0) table[0] = MoeTile{acc < max_tiles ? acc : max_tiles, 0, 0, 0, 0, {0, 0, 0}};
+  } else if (threadIdx.x < 64) {
+    const int lane = threadIdx.x;
+    int tiles[kMaxUnits] = {0, 0, 0, 0};  // row tiles under a limit of 1 .. 4 units
+    int carry = 0;
+    if (lane == 0) row_end[0] = 0;
+    for (int e0 = 0; e0 < num_experts; e0 += 64) {
+      const int e = e0 + lane;
+      const int64_t total = e < num_experts ? cum[e] : 0;
+      int end = static_cast<int>(total < 0 ? 0 : (total > rows ? rows : total));
+      end = end > carry ? end : carry;
+#pragma unroll
+      for (int d = 1; d < 64; d <<= 1) {
+        const int o = __shfl_up(end, d);
+        end = lane >= d && o > end ? o : end;
+      }
+      const int before = __shfl_up(end, 1);
+      const int units = (end - (lane == 0 ? carry : before) + 63) / 64;
+#pragma unroll
+      for (int u = 1; u <= kMaxUnits; ++u) tiles[u - 1] += (units + u - 1) / u;
+      if (e < num_experts) row_end[e + 1] = end;
+      carry = __shfl(end, 63);
+    }
+    float best = 0.0f;
+#pragma unroll
+    for (int u = kMaxUnits; u >= 1; --u) {
+      int n = tiles[u - 1];
+#pragma unroll
+      for (int d = 1; d < 64; d <<= 1) n += __shfl_xor(n, d);
+      const float cost = moe_cost(heights, n, u);
+      if (u == kMaxUnits || (u >= heights.min_units && n <= max_tiles && cost < best)) {
+        best = cost;
+        bm = u * 64;
+      }
+    }
+    __builtin_amdgcn_wave_barrier();  // row_end is read back by other lanes
+    int acc = 0;
+    for (int e0 = 0; e0 < num_experts; e0 += 64) {
+      const int e = e0 + lane;
+      const int nt = e < num_experts ? (row_end[e + 1] - row_end[e] + bm - 1) / bm : 0;
+      int sum = nt;
+#pragma unroll
+      for (int d = 1; d < 64; d <<= 1) {
+        const int o = __shfl_up(sum, d);
+        sum += lane >= d ? o : 0;
+      }
+      if (e < num_experts) first_tile[e] = acc + sum - nt;
+      acc += __shfl(sum, 63);
+    }
+    if (lane == 0) {
+      first_tile[num_experts] = acc;
+      table[0] = MoeTile{acc < max_tiles ? acc : max_tiles, 0, 0, 0, 0, {0, 0, 0}};
+    }
   }
   __syncthreads();
   for (int e = threadIdx.x; e < num_experts; e += 256) {
@@ -1718,8 +1809,7 @@ __global__ __launch_bounds__(256) void moe_plan_kernel(const int64_t* __restrict
     int row = r0;
     for (int t = 0; t < nt && t0 + t < max_tiles; ++t) {
       const int left = r1 - row;
-      int h = bm;
-      if (header != 0) h = (units / nt + (t < units % nt ? 1 : 0)) * 64;
+      const int h = header != 0 ? (units / nt + (t < units % nt ? 1 : 0)) * 64 : bm;
       table[header + t0 + t] = MoeTile{e, row, left < h ? left : h, t0, nt, {0, 0, 0}};
       row += h;
     }
@@ -1731,7 +1821,7 @@ __global__ __launch_bounds__(256) void moe_plan_kernel(const int64_t* __restrict
 // Up to 64 rows each -- a decode step of a mixture of experts -- the small-M
 // configurations' 64 x 256 (32 x 256 for int4) tiles: a taller one would do up
 // to eight times the MFMA work and hold one workgroup per CU where three fit.
-// Above, gemm_experts_kernel with tiles of up to 256 rows.
+// Above, gemm_experts_kernel with tiles of up to 256 rows (MoeHeights).
 constexpr int kExpertsRows = 256;
 inline int moe_tile_rows(int64_t rows, int num_experts, int bits) {
   const int64_t avg = rows / (num_experts > 0 ? num_experts : 1);
@@ -1746,7 +1836,8 @@ inline int moe_tile_rows(int64_t rows, int num_experts, int bits) {
 // of rows that belong to an expert.
 struct MoeLaunch {
   const int* table;
-  int max_tiles, bm, ns, experts;
+  int max_tiles, bm, ns;
+  bool narrow;  // gemm_experts_kernel on 128-column tiles instead of 256
   int64_t rows;
   float* partial;
   const int64_t* valid_rows;
@@ -1833,20 +1924,6 @@ void launch_experts_cfg(const void* x, const MoeLaunch& ml, const void* codes, c
   kern<<<dim3(static_cast<unsigned>(blocks)), dim3(512), lds, stream>>>(p);
 }
 
-// Whether a grouped product of N columns takes 128-column tiles instead of 256:
-// only where the 256-column ones would leave CUs without work and twice as
-// many still run in about one round.  The number of row tiles is not known on
-// the host; an expert with a rows on average has max(1, a / 256 + 0.4).
-// (K = 14336, N = 4096, 8 experts, int4 / int8, 256 against 128 columns: whole
-// call at 600 rows 419 / 445 against 366 / 419 us, 1024 rows 674 / 591 against
-// 591 / 552, 1500 rows at K = 7168 387 / 348 against 338 / 328, 2048 rows
-// 966 / 892 against 1091 / 977; level at 4096.)
-inline bool experts_narrow(int64_t rows, int num_experts, int64_t N) {
-  const double avg = static_cast<double>(rows) / num_experts;
-  const double tiles = num_experts * (avg > 0.6 * 256 ? avg / 256 + 0.4 : 1.0);
-  return tiles * static_cast<double>((N + 255) / 256) <= 0.62 * num_cus();
-}
-
 // ml.bm: the tile rows the table was built for (moe_tile_rows).  swiglu: out is
 // [rows, N / 2], the swiglu of the product (tiles of 256 rows only).
 template <int DT, int BITS>
@@ -1854,7 +1931,7 @@ void launch_moe_gemm(const void* x, const MoeLaunch& ml, const void* codes, cons
                      const void* scale, int64_t K, int64_t N, void* out, hipStream_t stream, bool swiglu = false) {
   if (ml.bm == kExpertsRows) {
     if (swiglu) launch_experts_cfg<DT, BITS, 2, 2>(x, ml, codes, bias, scale, K, N, out, stream);
-    else if (experts_narrow(ml.rows, ml.experts, N)) launch_experts_cfg<DT, BITS, 1, 0>(x, ml, codes, bias, scale, K, N, out, stream);
+    else if (ml.narrow) launch_experts_cfg<DT, BITS, 1, 0>(x, ml, codes, bias, scale, K, N, out, stream);
     else launch_experts_cfg<DT, BITS, 2, 0>(x, ml, codes, bias, scale, K, N, out, stream);
     return;
   }
@@ -1952,7 +2029,7 @@ void WOL_TYPED(swiglu_gemm)(const GemmArgs& a, int bits) {
 }
 
 void WOL_TYPED(moe_gemm)(const MoeGemmArgs& a, int bits) {
-  const MoeLaunch ml{a.table, a.max_tiles, a.bm, a.ns, a.experts, a.rows, a.partial, a.valid_rows};
+  const MoeLaunch ml{a.table, a.max_tiles, a.bm, a.ns, a.narrow, a.rows, a.partial, a.valid_rows};
   if (bits == 8) launch_moe_gemm<WOL_GEMM_DTYPE, 8>(a.x, ml, a.codes, a.bias, a.scale, a.K, a.N, a.out, a.stream, a.swiglu);
   else launch_moe_gemm<WOL_GEMM_DTYPE, 4>(a.x, ml, a.codes, a.bias, a.scale, a.K, a.N, a.out, a.stream, a.swiglu);
 }
@@ -2083,6 +2160,41 @@ static int moe_max_tiles(int64_t rows, int num_experts, int bm) {
   return static_cast<int>((rows + bm - 1) / bm) + num_experts;
 }
 
+// What the host settles of a gemm_experts_kernel call: the lowest height limit
+// the grid is laid out for, and whether the second product takes 128-column
+// tiles.  The rows of each expert are not known here: even loads are assumed,
+// and for the limit the device looks again (moe_plan_kernel).  Workgroups that
+// find no tile cost little but not nothing, so a limit below 256 rows is offered
+// only where it asks for at most twelve rounds of them.
+static MoeHeights plan_moe_heights(int64_t rows, int64_t hidden, int64_t inter, int num_experts, int bits, bool* narrow) {
+  const int cus = num_cus();
+  MoeHeights h;
+  h.xcd_cus = cus / 8 > 0 ? cus / 8 : 1;
+  h.nbx1 = static_cast<int>((inter / 2 + 127) / 128);
+  h.nbx2 = static_cast<int>((hidden + 255) / 256);
+  h.w1 = static_cast<float>(hidden);
+  h.w2 = static_cast<float>(inter / 2);
+  const float times[2][kMaxUnits] = {{0.60f, 0.70f, 0.85f, 1.0f}, {0.40f, 0.57f, 0.78f, 1.0f}};
+  for (int u = 0; u < kMaxUnits; ++u) h.tile[u] = times[bits == 4][u];
+  h.min_units = 1;
+  while (h.min_units < kMaxUnits &&
+         static_cast<int64_t>(moe_max_tiles(rows, num_experts, h.min_units * 64)) * h.nbx1 > 12 * cus)
+    ++h.min_units;
+  MoeHeights n = h;
+  n.nbx2 = static_cast<int>((hidden + 127) / 128);
+  n.w2 *= bits == 4 ? 0.8f : 0.7f;
+  const int64_t units = ((rows + num_experts - 1) / num_experts + 63) / 64;
+  float best = 0.0f, best_n = 0.0f;
+  for (int u = kMaxUnits; u >= h.min_units; --u) {
+    const int tiles = static_cast<int>((units + u - 1) / u) * num_experts;
+    const float c = moe_cost(h, tiles, u), cn = moe_cost(n, tiles, u);
+    best = u == kMaxUnits || c < best ? c : best;
+    best_n = u == kMaxUnits || cn < best_n ? cn : best_n;
+  }
+  *narrow = best_n < best;
+  return *narrow ? n : h;
+}
+
 // Scratch: [row-tile table][fc1 output rows x inter T][activation rows x inter/2 T]
 // [fp32 sums of the second GEMM's K runs, rows x hidden each, when the tiles are small]
 size_t moe_ffn_workspace(int64_t rows, int64_t hidden, int64_t inter, int num_experts) {
@@ -2099,25 +2211,27 @@ int launch_moe_ffn(const void* x, const int64_t* rows_before_expert, const void*
                    int num_experts, int bits, void* out, void* workspace, hipStream_t stream) {
   unsigned char* ws = static_cast<unsigned char*>(workspace);
   const int bm = moe_tile_rows(rows, num_experts, bits);
-  const int max_tiles = moe_max_tiles(rows, num_experts, bm);
   const bool experts = bm == kExpertsRows;
+  bool narrow = false;
+  const MoeHeights heights = plan_moe_heights(rows, hidden, inter, num_experts, bits, &narrow);
+  const int max_tiles = moe_max_tiles(rows, num_experts, experts ? heights.min_units * 64 : bm);
   MoeTile* table = reinterpret_cast<MoeTile*>(ws);
   unsigned char* fc1 = ws + moe_up((static_cast<size_t>(moe_max_tiles(rows, num_experts, 32)) + 1) * sizeof(MoeTile));
   unsigned char* act = fc1 + moe_up(static_cast<size_t>(rows) * inter * 2);
   float* partial = reinterpret_cast<float*>(act + moe_up(static_cast<size_t>(rows) * (inter / 2) * 2));
-  moe_plan_kernel<<<dim3(1), dim3(256), 0, stream>>>(rows_before_expert, num_experts, bm, max_tiles, rows, experts ? 1 : 0, table);
+  moe_plan_kernel<<<dim3(1), dim3(256), 0, stream>>>(rows_before_expert, num_experts, bm, max_tiles, rows, experts ? 1 : 0, heights, table);
   const auto product = [&](const MoeGemmArgs& a) {
     if (dtype == WOL_DTYPE_BF16) moe_gemm_bf16(a, bits); else moe_gemm_f16(a, bits);
   };
   const int* tab = reinterpret_cast<const int*>(table);
-  product(MoeGemmArgs{x, tab, max_tiles, bm, 1, num_experts, rows, nullptr, nullptr, ffn1_codes, ffn1_bias, ffn1_scale,
+  product(MoeGemmArgs{x, tab, max_tiles, bm, 1, false, rows, nullptr, nullptr, ffn1_codes, ffn1_bias, ffn1_scale,
                       hidden, inter, experts ? act : fc1, stream, experts});
   if (!experts) {
     const int rc = launch_swiglu_t(fc1, dtype, rows, inter, act, stream);
     if (rc != WOL_OK) return rc;
   }
   // the second product has hidden / 256 column tiles only: K (= inter / 2) in runs when the tiles are small
-  product(MoeGemmArgs{act, tab, max_tiles, bm, moe_runs(inter / 2, hidden, bits, bm, max_tiles), num_experts, rows,
+  product(MoeGemmArgs{act, tab, max_tiles, bm, moe_runs(inter / 2, hidden, bits, bm, max_tiles), narrow, rows,
                       experts ? nullptr : partial, rows_before_expert + (num_experts - 1), ffn2_codes, nullptr, ffn2_scale,
                       inter / 2, hidden, out, stream, false});
   return check_launch();

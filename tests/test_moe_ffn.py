@@ -33,7 +33,8 @@ def _oracle_moe(oracle, xb, cum, w1b, b1b, w2b, dt, bits):
 # and one expert far above the average (64-row tiles; 32-row tiles for int4);
 # an average of 38 rows (64-row tiles for both bit widths); many rows
 ROWS_PER_EXPERT = [[0, 5, 128, 131, 300, 0], [0, 5, 33, 64, 1, 17], [40, 64, 0, 70, 3, 50], [2, 1, 150, 0, 3, 4],
-                   [600, 256, 0, 1000, 700, 520]]  # 512 and more on average: 256-row tiles for int8
+                   [600, 256, 0, 1000, 700, 520]]
+# (the first and the last: more than 64 rows on average, tiles of up to 256 rows; the others: tiles of 32 or 64)
 
 
 @pytest.mark.parametrize("dt", [H.F16, H.BF16])
@@ -75,7 +76,8 @@ def test_moe_ffn_against_oracle(device, oracle, dt, bits, per, inter):
             prev = int(end)
 
 
-def test_moe_ffn_clamps_running_totals_it_cannot_trust(device):
+@pytest.mark.parametrize("rows,E", [(200, 5), (1000, 5), (10000, 150)])  # small tiles; one and three scans of 64 experts
+def test_moe_ffn_clamps_running_totals_it_cannot_trust(device, rows, E):
     # token_nums_per_expert comes from the device and is read there only.  Totals
     # that run backwards or past the input's rows are clamped by the table
     # builder to [previous total, rows]: the call computes what it would with
@@ -83,16 +85,21 @@ def test_moe_ffn_clamps_running_totals_it_cannot_trust(device):
     import torch
     from paddle_amd.nn import quant as Q
 
-    hidden, inter, E = 256, 512, 5
+    hidden, inter = 256, 512
     gen = torch.Generator(device="cuda").manual_seed(3)
     w1 = (torch.randn(E, hidden, inter, device="cuda", generator=gen) * 0.02).to(torch.bfloat16)
     w2 = (torch.randn(E, inter // 2, hidden, device="cuda", generator=gen) * 0.02).to(torch.bfloat16)
     q1, s1 = Q.moe_quantize_experts(w1)
     q2, s2 = Q.moe_quantize_experts(w2)
-    rows = 200
     x = torch.randn(rows, hidden, device="cuda", generator=gen).to(torch.bfloat16)
-    bad = torch.tensor([70, 30, 150, 10 ** 9, -5], dtype=torch.int64, device="cuda")   # backwards, huge, negative
-    good = torch.tensor([70, 70, 150, 200, 200], dtype=torch.int64, device="cuda")     # what the clamp makes of it
+    if E == 5:
+        bad = np.array([70, 30, 150, 10 ** 9, -5])  # backwards, huge, negative
+    else:
+        bad = np.arange(1, E + 1) * 67
+        bad[[3, 63, 64, 100, 127]] = [10, 4500, 5, -7, 9000]  # also in the first and last places of a scan
+        bad[-3:] = [2 ** 40, 12, -2 ** 40]
+    good = np.maximum.accumulate(np.clip(bad, 0, rows))  # what the clamp makes of it
+    bad, good = (torch.from_numpy(v.astype(np.int64)).cuda() for v in (bad, good))
     want = Q.moe_ffn(x, good, q1, q2, None, s1, s2, "weight_only_int8")
     got = Q.moe_ffn(x, bad, q1, q2, None, s1, s2, "weight_only_int8")
     torch.cuda.synchronize()
@@ -129,26 +136,50 @@ def test_moe_ffn_equals_per_expert_calls(device):
         Q.moe_ffn(x, cum.int(), q1, q2, None, s1, s2, "weight_only_int8")
 
 
+ANY_LOAD = [1, 63, 64, 65, 128, 129, 192, 0, 193, 256, 257, 320, 511, 513]
+
+
 @pytest.mark.parametrize("dt", [H.F16, H.BF16])
 @pytest.mark.parametrize("bits", [8, 4])
-@pytest.mark.parametrize("hidden", [256, 4096])  # second product on 128-column and on 256-column tiles
-def test_moe_ffn_tile_heights(device, dt, bits, hidden):
-    # experts with many rows take row tiles of one to four 64-row units: row counts on both sides of every
-    # unit and of one and two whole tiles, an expert without rows, and rows behind the last expert's
+@pytest.mark.parametrize("per,hidden,inter,limit", [
+    (ANY_LOAD, 256, 512, 64),      # few column tiles: the lowest tiles; second product on 128-column tiles
+    (ANY_LOAD, 4096, 512, 64),     # second product on 256-column tiles
+    (ANY_LOAD, 1152, 2048, 128),   # 128-column tiles, an odd number of them
+    (ANY_LOAD, 4224, 2048, 128),   # 256-column tiles, the last of 128 columns
+    ([192, 190, 129, 150, 0, 161, 192, 130, 175], 4224, 8192, 192),  # one tile an expert fills one round
+    ([256, 193, 250, 224, 0, 256, 240, 200, 255], 4224, 8192, 256),
+])
+def test_moe_ffn_tile_heights(device, dt, bits, per, hidden, inter, limit):
+    # experts with many rows take row tiles of one to four 64-row units, up to a limit that the number of tiles
+    # decides: row counts on both sides of every unit and of one and two whole tiles, an expert without rows.
+    # Rows behind the last expert's are left alone.
     import torch
+    from paddle_amd import _lib
     from paddle_amd.nn import quant as Q
 
-    inter = 512
-    per = [1, 63, 64, 65, 128, 129, 192, 0, 193, 256, 257, 320, 511, 513]
     E, T = len(per), torch.bfloat16 if dt == H.BF16 else torch.float16
     gen = torch.Generator(device="cuda").manual_seed(11)
     algo, wd = ("weight_only_int8", "int8") if bits == 8 else ("weight_only_int4", "int4")
-    q1, s1 = Q.moe_quantize_experts((torch.randn(E, hidden, inter, device="cuda", generator=gen) * 0.02).to(T), algo)
-    q2, s2 = Q.moe_quantize_experts((torch.randn(E, inter // 2, hidden, device="cuda", generator=gen) * 0.02).to(T), algo)
+    q1, s1 = Q.moe_quantize_experts(torch.randn(E, hidden, inter, device="cuda", generator=gen, dtype=T) * 0.02, algo)
+    q2, s2 = Q.moe_quantize_experts(torch.randn(E, inter // 2, hidden, device="cuda", generator=gen, dtype=T) * 0.02, algo)
     b1 = torch.randn(E, inter, device="cuda", generator=gen).to(T)
     cum = torch.tensor(np.cumsum(per), dtype=torch.int64, device="cuda")
-    x = torch.randn(sum(per) + 5, hidden, device="cuda", generator=gen).to(T)
-    out = Q.moe_ffn(x, cum, q1, q2, b1, s1, s2, algo)
+    rows = sum(per) + 5
+    x = torch.randn(rows, hidden, device="cuda", generator=gen).to(T)
+    out = torch.full((rows, hidden), 77.0, device="cuda", dtype=T)
+    ws_bytes = _lib.lib.wol_moe_ffn_workspace(rows, hidden, inter, E)
+    ws = torch.empty(ws_bytes, dtype=torch.uint8, device="cuda")
+    _lib.check(_lib.lib.wol_moe_ffn(
+        x.data_ptr(), cum.data_ptr(), q1.data_ptr(), b1.data_ptr(), s1.data_ptr(), q2.data_ptr(), s2.data_ptr(), dt,
+        rows, hidden, inter, E, bits, out.data_ptr(), ws.data_ptr(), ws_bytes, torch.cuda.current_stream().cuda_stream))
+    # the row-tile table at the start of the scratch, eight words an entry: the number of tiles in front, then
+    # each tile's expert, first row and rows
+    tiles = sum(-(-n // limit) for n in per)
+    table = ws[: (tiles + 1) * 32].view(torch.int32).view(-1, 8).cpu().numpy()
+    assert table[0, 0] == tiles and table[1:, 2].max() <= limit
+    assert table[1:, 2].sum() == sum(per)
+    assert torch.equal(Q.moe_ffn(x, cum, q1, q2, b1, s1, s2, algo)[: sum(per)], out[: sum(per)])
+    assert bool((out[sum(per):] == 77.0).all())
     prev = 0
     for e, n in enumerate(per):
         if n:
