@@ -2071,16 +2071,8 @@ size_t linear_gemm_workspace(int64_t M, int64_t K, int64_t N, int bits, int grou
     const int g = group_size > 0 ? group_size : 0;
     half_tile_config(static_cast<int>(M), static_cast<int>(K), static_cast<int>(N), bits, g, &bm, &bn, &lo);
     const int ncols = static_cast<int>(N) - lo * kStripCols;
-    const auto runs_bytes = [&](int cols) {
-      const TailPlan t = plan_tail(static_cast<int>(M), static_cast<int>(K), cols, bm, bn, tk, SIZE_MAX);
-      return t.ns > 1 ? static_cast<size_t>(t.ns) * M * (cols - t.full_tiles * bn) * sizeof(float) : 0;
-    };
-    const size_t need = runs_bytes(ncols);
-    if (bits != 4 || g == 0 || lo == 0) return need;
-    // int4 with group-wise scales: never less than half-size tiles on all columns ask for, so that the size a
-    // caller has laid down does not depend on which of the two tiles a launch takes
-    const size_t half = runs_bytes(static_cast<int>(N));
-    return need > half ? need : half;
+    const TailPlan t = plan_tail(static_cast<int>(M), static_cast<int>(K), ncols, bm, bn, tk, SIZE_MAX);
+    return t.ns > 1 ? static_cast<size_t>(t.ns) * M * (ncols - t.full_tiles * bn) * sizeof(float) : 0;
   }
   const int ns = plan_skinny(static_cast<int>(M), static_cast<int>(K), static_cast<int>(N), bits,
                              group_size > 0 ? group_size : 0, SIZE_MAX).ns;

@@ -69,9 +69,11 @@ def test_workspace_queries(lib):
     assert L.wol_linear_workspace(1024, 4096, 4096, 8, 64) == 2 * 1024 * 4096 * 4  # 128 tiles: two K runs
     # group-wise int8 takes 256 x 256 tiles like per-channel int8: 192 of them, one round, no K runs
     assert L.wol_linear_workspace(1024, 4096, 12288, 8, 64) == 0
-    # group-wise int4, 256 x 128 tiles, 384 of them: the 256 of the whole round run as they are, the other 128
-    # (4096 columns) in two K runs
-    assert L.wol_linear_workspace(1024, 4096, 12288, 4, 128) == 2 * 1024 * 4096 * 4
+    # group-wise int4 the same
+    assert L.wol_linear_workspace(1024, 4096, 12288, 4, 128) == 0
+    # 128 half-size tiles of 256 x 128: two K runs; 252 whole tiles and 66 of 128 x 256: three
+    assert L.wol_linear_workspace(1024, 4096, 4096, 4, 128) == 2 * 1024 * 4096 * 4
+    assert L.wol_linear_workspace(1300, 4096, 12288, 4, 128) == 3 * 1300 * 1536 * 4
     # 256 x 256 tiles on the columns of whole rounds, one 256 x 128 column tile left over: four K runs of it
     assert L.wol_linear_workspace(700, 2048, 22016, 8, 64) == 4 * 700 * 256 * 4
     # small M on the GEMM: whole fp32 [M, N] partial buffers, at most 16 of them
@@ -88,6 +90,24 @@ def test_workspace_queries(lib):
     assert L.wol_linear_workspace_for(16, 8192, 28672, 4, 128, lib.KERNEL_GEMM) > 0
     assert L.wol_linear_workspace_for(16, 4096, 11008, 4, 128, lib.KERNEL_STREAM) == 0
     assert L.wol_linear_workspace_for(16, 4160, 11008, 4, 128, lib.KERNEL_GEMM) == 0  # K not a multiple of the k tile
+
+
+@pytest.mark.parametrize("bits,g", [(8, -1), (8, 64), (4, -1), (4, 64), (4, 128)])
+def test_workspace_query_asks_for_what_the_plan_uses(lib, bits, g):
+    # above 64 rows scratch holds the sums of K runs: a plan without runs asks for none, and one with runs is the
+    # same with exactly what it asks for
+    L = lib.lib
+    buf = ctypes.create_string_buffer(512)
+
+    def plan(M, K, N, ws):
+        lib.check(L.wol_linear_plan(M, K, N, bits, g, ws, buf, len(buf)))
+        return buf.value
+
+    for M in (65, 128, 200, 300, 512, 700, 1024, 1237, 1300, 2048, 3000, 4096):
+        for K, N in ((2048, 4096), (4096, 4096), (4096, 12288), (4096, 22016), (11008, 4096), (8192, 28672), (1024, 6160)):
+            need, ample = L.wol_linear_workspace(M, K, N, bits, g), plan(M, K, N, 1 << 40)
+            assert (need > 0) == (b"K in runs" in ample), (M, K, N, need, ample)
+            assert plan(M, K, N, need) == ample, (M, K, N, need)
 
 
 def test_argument_errors_return_before_device_work(lib):
