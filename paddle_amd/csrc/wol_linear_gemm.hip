@@ -1491,9 +1491,12 @@ inline int plan_big_columns(int M, int K, int N, int bits, int group) {
   const bool tall = (bits == 8 || g4) && tall_half_tile(M);  // half tiles of 256 x 128 instead of 128 x 256
   int best = nbx;
   double best_t = 1e30;
-  for (int c = nbx; c >= 0; --c) {
+  // the estimate grows with the number of half-size tiles, so for every number of whole rounds only the most
+  // columns that fit them matter (walking all columns took 1 to 2 us of a call on a wide weight)
+  for (int c = nbx; c >= 0;) {
     const int small = tall ? 2 * (nbx - c) * nby_big : (nbx - c) * nby_small;
-    double t = static_cast<double>((c * nby_big + cus - 1) / cus);
+    const int rounds = (c * nby_big + cus - 1) / cus;
+    double t = static_cast<double>(rounds);
     const int rest = small % cus;
     int runs = g4 && rest > 0 ? cus / rest : 1;
     runs = runs > 4 ? 4 : runs;
@@ -1501,6 +1504,8 @@ inline int plan_big_columns(int M, int K, int N, int bits, int group) {
     if (runs > 1) t += kSmall * (small / cus) + kSmall / runs + kRuns;
     else t += kSmall * static_cast<double>((small + cus - 1) / cus);
     if (t < best_t - 1e-9) { best_t = t; best = c; }
+    const int fewer = rounds > 0 ? static_cast<int>(static_cast<int64_t>(rounds - 1) * cus / nby_big) : -1;
+    c = fewer < c ? fewer : c - 1;
   }
   return best;
 }
