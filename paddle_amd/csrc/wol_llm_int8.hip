@@ -523,7 +523,11 @@ constexpr int stash_lds_bytes(int bn) { return 512 + kStash * bn; }  // list and
 // (128: whole cache lines per row and load; 64 for a K that is not a multiple
 // of 128), STAGES of them in LDS.  RUNS: K is cut into runs across workgroups,
 // each leaving its sums in its slab of acc; otherwise the epilogue writes out.
-template <int DT, int WM, int WN, int TM, int TN, int TK, int STAGES, bool RUNS>
+// STASH (with RUNS): the outlier columns' weight bytes are picked out of the
+// tiles for llm_merge_few_kernel.  An instantiation of its own: as a run-time
+// switch it cost the launches without it 2 % (K = 4096, N = 11008, 65 rows, 3
+// outlier columns: 38.4 against 37.3 us).
+template <int DT, int WM, int WN, int TM, int TN, int TK, int STAGES, bool RUNS, bool STASH>
 __global__ __launch_bounds__(WM* WN * 64) __attribute__((amdgpu_waves_per_eu(2))) void llm_gemm_kernel(GemmParams p) {
   constexpr int NW = WM * WN;
   constexpr int BM = WM * TM * 32, BN = WN * TN * 32;
@@ -607,7 +611,7 @@ __global__ __launch_bounds__(WM* WN * 64) __attribute__((amdgpu_waves_per_eu(2))
   // the outlier list and count, ahead of the tiles in the same in-order stream
   unsigned char* const lds_list = smem + kStages * kStage;
   int8_t* const stash = reinterpret_cast<int8_t*>(lds_list + 512);
-  if (RUNS && p.ow != nullptr && wave == 0) {
+  if (STASH && wave == 0) {
     __builtin_amdgcn_global_load_lds(reinterpret_cast<const uint8_t*>(p.e.list + lane), (lds_ptr_t)lds_list, 4, 0, 0);
     __builtin_amdgcn_global_load_lds(reinterpret_cast<const uint8_t*>(p.e.count), (lds_ptr_t)(lds_list + 256), 4, 0, 0);
   }
@@ -653,11 +657,11 @@ __global__ __launch_bounds__(WM* WN * 64) __attribute__((amdgpu_waves_per_eu(2))
     __builtin_amdgcn_sched_barrier(0);
     WOL_LLM_ISSUE(it + kStages - 1);  // into the stage every wavefront finished reading before the barrier
     __builtin_amdgcn_sched_barrier(0);
-    if (RUNS && it == 0 && p.ow != nullptr) {  // landed with the first tile
+    if (STASH && it == 0) {  // landed with the first tile
       const int c = *reinterpret_cast<const int*>(lds_list + 256);
       if (c <= kStash && lane < c) my_k = *reinterpret_cast<const int*>(lds_list + lane * 4);
     }
-    if (RUNS) {
+    if (STASH) {
       const int kt = (t0 + it) * kTK;
       unsigned long long hit = __ballot(my_k >= kt && my_k < kt + kTK);
       while (hit != 0) {
@@ -723,7 +727,7 @@ __global__ __launch_bounds__(WM* WN * 64) __attribute__((amdgpu_waves_per_eu(2))
   float* xs = rng + BM;                                                  // [cnt][BM]
   float* wdl = xs + p.cap * BM;                                          // [cnt][BN]
   const bool fused = !RUNS && cnt > 0 && cnt <= p.cap;
-  if (RUNS && p.ow != nullptr) {
+  if (STASH) {
     const int lo = t0 * kTK, hi = (t0 + niter) * kTK;
     unsigned long long got = __ballot(my_k >= lo && my_k < hi);
     for (; got != 0; got &= got - 1) {
@@ -976,14 +980,14 @@ Workspace carve(void* base, int64_t M, int64_t K, int64_t N, int runs) {
   return w;
 }
 
-template <int DT, int WM, int WN, int TM, int TN, int TK, int STAGES, bool RUNS>
+template <int DT, int WM, int WN, int TM, int TN, int TK, int STAGES, bool RUNS, bool STASH = false>
 int launch_gemm(const GemmParams& p, int runs, hipStream_t stream) {
   constexpr int BM = WM * TM * 32, BN = WN * TN * 32;
-  constexpr size_t stages = static_cast<size_t>(STAGES) * (BM + BN) * TK, lds = stages + (RUNS ? stash_lds_bytes(BN) : 0);
+  constexpr size_t stages = static_cast<size_t>(STAGES) * (BM + BN) * TK, lds = stages + (STASH ? stash_lds_bytes(BN) : 0);
   static_assert(stages >= static_cast<size_t>(WM * WN) * 32 * 40 * 4 + BM * 4,
                 "the epilogue's slabs and row ranges must fit the stages");
   static std::atomic<uint32_t> done{0};
-  auto kern = llm_gemm_kernel<DT, WM, WN, TM, TN, TK, STAGES, RUNS>;
+  auto kern = llm_gemm_kernel<DT, WM, WN, TM, TN, TK, STAGES, RUNS, STASH>;
   allow_lds(reinterpret_cast<const void*>(kern), lds, done);
   hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(p.nbx * p.nby * runs)), dim3(WM * WN * 64), lds, stream,
                      p);
@@ -1004,7 +1008,10 @@ int launch_gemm_for(const GemmParams& p, const Plan& pl, hipStream_t stream) {
       }
       return launch_gemm<DT, 1, 4, 4, 1, TK, 3, RUNS>(p, pl.runs, stream);
     case 64: return launch_gemm<DT, 1, 4, 2, 1, TK, 3, RUNS>(p, pl.runs, stream);
-    default: return launch_gemm<DT, 1, 4, 1, 1, TK, 3, RUNS>(p, pl.runs, stream);
+    default:
+      if constexpr (RUNS)
+        if (p.ow != nullptr) return launch_gemm<DT, 1, 4, 1, 1, TK, 3, true, true>(p, pl.runs, stream);
+      return launch_gemm<DT, 1, 4, 1, 1, TK, 3, RUNS>(p, pl.runs, stream);
   }
 }
 
