@@ -464,10 +464,13 @@ __device__ inline void pack_codes(const int (&c)[8], uint32_t* d) {
 // The code of w under a scale whose fp32 reciprocal is y: what quant_code()
 // gives, without the division.  w and the scale have at most 11 significant
 // bits, so w / scale is either exactly half way between two integers or at
-// least 2^-13.4 away (2^-11 above 2): adding 1/2 + 2^-14 to |w| * y, off by less
-// than 2^-15, and truncating rounds every half away from zero and nothing else.
-// (Compared with roundf(w / s) for all pairs of 11-bit and of 8-bit
-// significands and all quotients up to 400, beyond which both sides clip.)
+// least 2^-12 away: twice the quotient is a fraction with a denominator of at
+// most 2048, so an integer or 2^-11 away from one.  |w| * y is off by less than
+// 2^-15 (up to 128; beyond, both sides clip), so adding 1/2 + 2^-14 lifts every
+// half over the next integer and brings nothing else there (2^-14 + 2^-15 <
+// 2^-12): truncating then rounds halves away from zero.  (Compared with
+// roundf(w / s) for all pairs of 11-bit and of 8-bit significands and all
+// quotients up to 400.)
 template <int BITS>
 __device__ inline int quant_code_rcp(float w, float y) {
   constexpr int bound = BITS == 8 ? 127 : 7;
@@ -518,8 +521,9 @@ __global__ __launch_bounds__(kThreads) void quantize_gfx950_kernel(
   // one thread per scale of the block
   if (tid < kGroups * kWideN) {
     const int g = tid / kWideN, c = tid % kWideN;
+    const bool exists = c < NC && g * 64 < KR;
     uint16_t sb = 0;
-    if (c < NC && g * 64 < KR) {
+    if (exists) {
       float src;
       if (G != 0) {
         src = 0.0f;
@@ -540,8 +544,9 @@ __global__ __launch_bounds__(kThreads) void quantize_gfx950_kernel(
     }
     const float s = to_f32<DT>(sb);
     sc[g][c] = s;
-    // scales whose reciprocal is no ordinary number (0, NaN, infinity, the ends of bf16's range): 0 marks them
-    rc[g][c] = s >= 0x1p-100f && s <= 0x1p100f ? 1.0f / s : 0.0f;
+    // scales whose reciprocal is no ordinary number (0, NaN, infinity, the ends of bf16's range): 0 marks them;
+    // past an edge any ordinary value, so that no wavefront takes the divisions for columns that are not there
+    rc[g][c] = !exists ? 1.0f : (s >= 0x1p-100f && s <= 0x1p100f ? 1.0f / s : 0.0f);
   }
   __syncthreads();
 
