@@ -15,16 +15,18 @@ events on the launching stream; ms_per_step is the MEDIAN replay divided by
 Beside the headline the line carries
   prefill    the compute-bound GEMM (M=2048, int8 per-channel, K=4096,
              N=12288) with an in-run ceiling: a register-only MFMA loop;
-  configs    one entry per configuration of BASELINE.json and row count, the
-             last one the 32-layer decoder stack as a sequence (decode steps
-             at M=8, one prefill chunk at M=1024);
-  llm_int8   the sibling op on the prefill shape;
   cpu_baseline  the CPU oracle (quantize, dequantize) + fp32 BLAS matmul on
              the host cores, on a bounded sample;
   parity     the measured outputs against the oracle.  A parity failure makes
-             the run exit non-zero: no throughput is published for wrong results.
+             the run exit non-zero: no throughput is published for wrong results;
+  and the figures of the further legs as plain numbers of `roofline`.  The
+legs' tables are lines on stderr: configs, one entry per workload and row
+count; the 32-layer decoder stack as a sequence (decode steps at M=8, one
+prefill chunk at M=1024); llm_int8, the sibling op on the prefill shape; the
+gradient, the mixture of experts, the fused swiglu, and the phases of a
+prefill and of a decode launch.
 
-Prints ONE JSON line.
+Prints ONE JSON line on stdout.
 """
 import argparse
 import json
@@ -976,19 +978,11 @@ def main():
                 "inner_loop_ladder_tflops": ladder,
             },
         },
-        "configs": configs,
-        "decoder_stack": stack,
-        "linear_grad": grad,
-        "moe_ffn": moe,
-        "fused_swiglu": fused,
-        "prefill_phases": phases,
-        "decode_phases": dphases,
-        "decode_rounds": drounds,
-        "llm_int8": llm,
         "cpu_baseline": cpu,
         "parity": parity,
     }
-    # every per-configuration fraction of its roofline once more as plain numbers of `roofline`
+    # the legs' figures as plain numbers of `roofline`; their tables go to stderr, a line each, so that the JSON line
+    # stays short enough to be kept whole
     flat = out["roofline"]
     for e in configs or []:
         tag = "north_star" if e["config"].startswith("north") else e["config"]
@@ -1020,6 +1014,12 @@ def main():
         flat["llm_int8_frac"] = llm["roofline"]["frac"]
     for nm, tf in (ladder or {}).items():
         flat["ladder_%s_tflops" % nm] = tf
+    legs = dict(configs=configs, decoder_stack=stack, linear_grad=grad, moe_ffn=moe, fused_swiglu=fused,
+                prefill_phases=phases, decode_phases=dphases, decode_rounds=drounds, llm_int8=llm)
+    for name, leg in legs.items():
+        if leg:
+            print("bench.py: %s: %s" % (name, json.dumps(leg)), file=sys.stderr)
+    sys.stderr.flush()
     print(json.dumps(out))
     if failures:
         print("bench.py: PARITY FAILURE: " + "; ".join(failures), file=sys.stderr)
