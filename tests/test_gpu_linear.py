@@ -864,6 +864,9 @@ def test_gemm_partial_last_round_split(G, oracle, dt, bits, g, M, K, N):
     (H.BF16, 8, 128, 300, 2048, 8192, (-100, 20)),  # scales of a column further apart than fp32 sums can span
     (H.BF16, 4, 64, 300, 4096, 4096, (-12, 4)),     # int4: 128 x 256 tiles, two groups per k tile
     (H.F16, 4, 128, 130, 2048, 4096, (-8, 3)),      # int4: 256 x 128 tiles
+    (H.BF16, 4, 128, 300, 384, 24016, (-12, 4)),    # int4 on whole tiles of 64-deep k tiles: groups of two of them
+    (H.F16, 4, 64, 512, 1152, 24016, (-8, 3)),      # ... and of one, an odd number of raw weight tiles
+    (H.BF16, 4, 128, 512, 1152, 24016, (-100, 20)),
 ])
 def test_group_wise_gemm_keeps_its_sums_in_units_of_the_group_scale(G, oracle, dt, bits, g, M, K, N, spread):
     # above 64 rows the GEMM has one set of accumulators for group-wise scales: the
@@ -872,6 +875,13 @@ def test_group_wise_gemm_keeps_its_sums_in_units_of_the_group_scale(G, oracle, d
     # inside a column, with all-zero groups (scale 0) at the start, in the middle
     # and at the end of K: every column must still match the oracle's fp32 sums,
     # column by column (a whole-matrix norm would hide the small columns).
+    if bits == 4 and N == 24016:
+        import ctypes
+        from paddle_amd import _lib
+
+        buf = ctypes.create_string_buffer(512)
+        _lib.check(_lib.lib.wol_linear_plan(M, K, N, bits, g, 1 << 40, buf, len(buf)))
+        assert b"256x256 tiles" in buf.value, buf.value
     rng = np.random.default_rng(K + N + M)
     ng = (K + g - 1) // g
     lo, hi = spread
