@@ -149,11 +149,12 @@ struct DequantExact<WOL_DTYPE_BF16, 4> {
 // The same codes in 19 instructions per eight instead of 27: each nibble pair
 // becomes two fp16 values 1024 + 16 * nibble (one and-or), a mixed-precision FMA
 // takes the offset out and widens to fp32 in one instruction, and the high
-// halves are the bf16 codes, every step exact.  The half-deep tiles gain 1 to 2 %
-// from it.  Elsewhere the longer form is the faster one: the FMAs keep no
-// distance to the MFMAs around them and the loop fills with waits (s_nop 41 and
-// 55 against 13 and 14 per tile of 128 x 256 x 128, g128; 200 rows, K = N = 4096:
-// 31.6 against 30.7 us; swiglu, 200 rows, K = 4096, N = 8192: 70.0 against 67.6).
+// halves are the bf16 codes, every step exact.  g128 with this form against the
+// other one: 128 x 256 tiles 2 to 5 % faster (100 rows, K = 11008, N = 4096: 58.4
+// against 60.7 us; swiglu, 128 rows, 3 to 5 %), half-deep and small-M tiles 1 to
+// 2 %; 256 x 128 tiles, where four A blocks share a B block, 2 to 3 % slower (200
+// rows, K = N = 4096: 31.6 against 30.7), so they keep the other.  gemm_kernel:
+// per channel 2 to 4 % faster, group-wise up to 9 % slower (K = 4544: 65 rows).
 template <int DT, int BITS>
 struct DequantExactFma : DequantExact<DT, BITS> {};
 
@@ -317,7 +318,7 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_kernel(
 #pragma unroll
         for (int s = 0; s < TN; ++s) {
           const uint32_t w[4] = {wcur[s].x, wcur[s].y, wcur[s].z, wcur[s].w};
-          bfrag[s] = DequantExact<DT, BITS>::run(&w[step * kDw]);
+          bfrag[s] = std::conditional_t<GROUPED, DequantExact<DT, BITS>, DequantExactFma<DT, BITS>>::run(&w[step * kDw]);
         }
 #pragma unroll
         for (int a = 0; a < TM; ++a) {
@@ -615,8 +616,8 @@ __device__ __forceinline__ void dma_tile(std::conditional_t<EXPERTS, const DmaPa
   // SWI with one block per wavefront: wavefront columns 2i and 2i+1 hold the gate and the up block of
   // the same 32 output columns, and the up wavefront hands its sums over through LDS in the epilogue
   constexpr bool kPair = SWI != 0 && TN == 1;
-  // the small-M tiles and the half-deep ones take the shorter int4 dequantiser (see DequantExactFma)
-  constexpr bool kFmaDequant = BITS == 4 && OFFS == 0 && (kHalfDeep || WM == 1);
+  // all tiles but those of 256 x 128 take the shorter int4 dequantiser (see DequantExactFma)
+  constexpr bool kFmaDequant = BITS == 4 && OFFS == 0 && (TN == 2 || WM == 1);
   static_assert(OFFS != 2 || G == 0, "row sums by dot products are taken out once, in the epilogue");
   static_assert(!RESC || (G != 0 && OFFS == 0), "rescaled sums are for group-wise scales and the exact dequantisers");
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
@@ -647,7 +648,11 @@ __device__ __forceinline__ void dma_tile(std::conditional_t<EXPERTS, const DmaPa
     int by;
     tile_of_block_2d(blockIdx.x - split * ntiles, p.nbx, p.nby, p.xcd_rows, &bx, &by);
     m0 = by * BM;
-    if (SWI == 0 && p.moe_table != nullptr) {  // (grouped launches with a fused swiglu are gemm_experts_kernel's)
+    // Grouped launches of this kernel are those of small tiles (launch_moe_gemm_cfg).  The larger per-channel
+    // kernels know that at compile time (int8, 1237 rows, K = N = 4096: 54.4 against 55.8 us); the group-wise ones
+    // keep the test, which no launch answers with yes, because their loops come out better ordered with it
+    // (int8 g128, 256 rows, K = 11008, N = 4096: 50.4 against 52.5 us).
+    if (SWI == 0 && (WM == 1 || RESC) && p.moe_table != nullptr) {
       const MoeTile t = reinterpret_cast<const MoeTile*>(p.moe_table)[by];
       if (t.expert < 0) return;
       expert = t.expert;
@@ -1855,6 +1860,7 @@ void launch_moe_gemm_cfg(const void* x, const MoeLaunch& ml, const void* codes, 
                          const void* scale, int64_t K, int64_t N, void* out, hipStream_t stream) {
   const int* table = ml.table;
   const int max_tiles = ml.max_tiles;
+  static_assert(WM == 1, "the larger tiles of gemm_dma_kernel do not read the expert table");
   constexpr int BN = TN * WN * 32;  // output columns of a tile
   constexpr size_t lds = dma_lds_bytes<BITS, 0, WM, WN, TM, TN, STAGES>();
   auto kern = gemm_dma_kernel<DT, BITS, 0, OFFS, WM, WN, TM, TN, STAGES>;
