@@ -1229,7 +1229,9 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_dma_kernel(const DmaParams 
 // whole call, against whole tiles of 256 or 128 rows in runs of the average
 // expert's tiles per XCD: 4096 rows int4 2264 -> 1684 us, int8 2090 -> 1551;
 // 2048 rows int4 1311 -> 966, int8 1325 -> 892; 1024 rows 651 -> 591 and 666 ->
-// 552; 4 experts, width 14336, 4096 rows 1130 -> 789.
+// 552; 4 experts, width 14336, 4096 rows 1130 -> 789.  (Limit of 256 rows throughout;
+// moe_plan_kernel has since chosen lower ones where they are faster: 2048 rows, even
+// loads, int4 805 -> 685 us, int8 772 -> 693.)
 template <int DT, int BITS, int OFFS, int TN, int STAGES, int SWI>
 __global__ __launch_bounds__(512) void gemm_experts_kernel(const DmaParams p) {
   const MoeTile* table = reinterpret_cast<const MoeTile*>(p.moe_table);
@@ -1672,8 +1674,8 @@ void launch_fast(const Args& a) {
     if (bm == 256) WOL_HALF(0, 2, 4, 4, 1, 2, 0, true);
     else WOL_HALF(0, 2, 4, 2, 2, 2, 0, true);
   } else if constexpr (DT == WOL_DTYPE_BF16) {
-    // the exact int4 -> bf16 dequantiser costs 32 VALU instructions per 8
-    // codes; the offset form is faster: with row sums by dot products on the
+    // the exact int4 -> bf16 dequantiser costs 19 VALU instructions per 8
+    // codes; the offset form is faster or level: with row sums by dot products on the
     // 256 x 256 tile (two stages of 64 + 16 KiB fill the LDS), with one
     // cancelling MFMA per A block on the 128 x 256 tiles of the remainder
     launch_dma<DT, BITS, G, 2, 2, 4, 4, 2, 2>(a, 0, lo, 1);
