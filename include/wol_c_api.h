@@ -297,10 +297,11 @@ int wol_linear_grad_f32(const void* out_grad, const void* codes,
  * ffn2_weight [E] x (K = inter/2, N = hidden), ffn2_scale [E, hidden] T.
  * Each of the two products is ONE grouped launch (tiles looked up in a
  * row-tile table that a one-workgroup kernel derives from
- * token_nums_per_expert: 128 x 256, or 64 x 256 / 32 x 256 when rows /
- * num_experts is at most 64 / 32, in which case the second product may run
- * with K cut into runs and a kernel that adds them); the swiglu between them
- * is an element-wise pass.
+ * token_nums_per_expert: tiles of 64 to 256 rows x 256 or 128 columns with the
+ * swiglu in the first product's epilogue; or, when rows / num_experts is at
+ * most 64, 64 x 256 tiles (at most 32 and int4: 32 x 256) with the swiglu as an
+ * element-wise pass, in which case the second product may run with K cut into
+ * runs and a kernel that adds them).
  * Requires hidden % 128 == 0, inter % 256 == 0, num_experts <= 1024; the
  * workspace (wol_moe_ffn_workspace bytes, 16-byte aligned) holds the table,
  * the two intermediate tensors and the runs' sums.
