@@ -1729,23 +1729,24 @@ __host__ __device__ inline float moe_cost(const MoeHeights& h, int tiles, int un
 // as token_nums_per_expert,
 // paddle/phi/kernels/fusion/cutlass/moe_dispatch.cu:174-182): expert e owns
 // rows cum[e-1] .. cum[e]-1 and ceil(rows / bm) tiles.  One workgroup.
-// header == 0: tiles of bm rows, max_tiles entries, unused ones marked -1.
-// header == 1 (gemm_experts_kernel): bm is chosen here, where the rows of every
+// EXPERTS false: tiles of bm rows, max_tiles entries, unused ones marked -1.
+// EXPERTS true (gemm_experts_kernel): bm is chosen here, where the rows of every
 // expert are known (MoeHeights), entry 0 holds the number of tiles, and an
 // expert's rows are shared out in 64-row units as evenly as its ceil(rows /
 // bm) tiles allow (three tiles of 192 rows rather than two of 256 and one of
 // 64: the weight side of a tile costs the same whatever its height).
+template <bool EXPERTS>
 __global__ __launch_bounds__(256) void moe_plan_kernel(const int64_t* __restrict__ cum, int num_experts, int bm,
-                                                       int max_tiles, int64_t rows, int header, MoeHeights heights,
+                                                       int max_tiles, int64_t rows, MoeHeights heights,
                                                        MoeTile* __restrict__ table) {
   __shared__ int first_tile[1025];  // exclusive running total of tiles, by expert
   __shared__ int row_end[1025];     // end of expert e's rows is row_end[e + 1]; row_end[0] = 0
-  if (header == 0)
+  if (!EXPERTS)
     for (int i = threadIdx.x; i < max_tiles; i += 256) table[i] = MoeTile{-1, 0, 0, 0, 0, {0, 0, 0}};
   // The running totals come from the device and are not trusted: each is
   // clamped to [previous total, rows], so an expert's count is never negative
   // and no tile reaches past the last row of the input.
-  if (header == 0) {
+  if (!EXPERTS) {
     if (threadIdx.x == 0) {
       int acc = 0;
       int64_t prev = 0;
@@ -1821,8 +1822,8 @@ __global__ __launch_bounds__(256) void moe_plan_kernel(const int64_t* __restrict
     int row = r0;
     for (int t = 0; t < nt && t0 + t < max_tiles; ++t) {
       const int left = r1 - row;
-      const int h = header != 0 ? (units / nt + (t < units % nt ? 1 : 0)) * 64 : bm;
-      table[header + t0 + t] = MoeTile{e, row, left < h ? left : h, t0, nt, {0, 0, 0}};
+      const int h = EXPERTS ? (units / nt + (t < units % nt ? 1 : 0)) * 64 : bm;
+      table[(EXPERTS ? 1 : 0) + t0 + t] = MoeTile{e, row, left < h ? left : h, t0, nt, {0, 0, 0}};
       row += h;
     }
   }
@@ -2218,13 +2219,14 @@ int launch_moe_ffn(const void* x, const int64_t* rows_before_expert, const void*
   const int bm = moe_tile_rows(rows, num_experts, bits);
   const bool experts = bm == kExpertsRows;
   bool narrow = false;
-  const MoeHeights heights = plan_moe_heights(rows, hidden, inter, num_experts, bits, &narrow);
+  const MoeHeights heights = experts ? plan_moe_heights(rows, hidden, inter, num_experts, bits, &narrow) : MoeHeights{};
   const int max_tiles = moe_max_tiles(rows, num_experts, experts ? heights.min_units * 64 : bm);
   MoeTile* table = reinterpret_cast<MoeTile*>(ws);
   unsigned char* fc1 = ws + moe_up((static_cast<size_t>(moe_max_tiles(rows, num_experts, 32)) + 1) * sizeof(MoeTile));
   unsigned char* act = fc1 + moe_up(static_cast<size_t>(rows) * inter * 2);
   float* partial = reinterpret_cast<float*>(act + moe_up(static_cast<size_t>(rows) * (inter / 2) * 2));
-  moe_plan_kernel<<<dim3(1), dim3(256), 0, stream>>>(rows_before_expert, num_experts, bm, max_tiles, rows, experts ? 1 : 0, heights, table);
+  (experts ? moe_plan_kernel<true> : moe_plan_kernel<false>)<<<dim3(1), dim3(256), 0, stream>>>(
+      rows_before_expert, num_experts, bm, max_tiles, rows, heights, table);
   const auto product = [&](const MoeGemmArgs& a) {
     if (dtype == WOL_DTYPE_BF16) moe_gemm_bf16(a, bits); else moe_gemm_f16(a, bits);
   };
