@@ -15,13 +15,7 @@
 // gemm_kernel (v_mfma_f32_16x16x32, activations staged through registers into
 // padded LDS rows, weights loaded straight into B-fragment order) takes the
 // remaining K: those that end in a partial k tile.
-#include <atomic>
-
-#include "wol_common.h"
-#include "wol_dequant.h"
-
-#include <climits>
-#include <type_traits>
+#include "wol_gemm_common.h"
 
 namespace wol {
 
@@ -54,127 +48,6 @@ namespace {
 #ifndef WOL_GEMM_DTYPE
 #define WOL_GEMM_DTYPE WOL_DTYPE_BF16
 #endif
-
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
-typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
-
-template <int DT>
-__device__ inline f32x4 mfma16(u32x4 a, u32x4 b, f32x4 c) {
-  if (DT == WOL_DTYPE_BF16)
-    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a),
-                                                   __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
-  return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a),
-                                                __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
-}
-
-__device__ inline uint32_t pack_bf16_hi(float lo, float hi) {
-  // both values are small integers, exact in bf16: keep the high halves
-  return __builtin_amdgcn_perm(__float_as_uint(hi), __float_as_uint(lo), 0x07060302u);
-}
-
-__device__ inline uint32_t f16x2_add(uint32_t v, uint32_t c) {
-  const f16x2 r = __builtin_bit_cast(f16x2, v) + __builtin_bit_cast(f16x2, c);
-  return __builtin_bit_cast(uint32_t, r);
-}
-
-// Codes of one k step (8 per lane) -> four dwords of T pairs holding the exact
-// signed code.
-template <int DT, int BITS>
-struct DequantExact;
-
-template <>
-struct DequantExact<WOL_DTYPE_BF16, 8> {
-  __device__ static inline float sbyte(uint32_t v, int i) {
-    return static_cast<float>(static_cast<int>(static_cast<int8_t>((v >> (8 * i)) & 0xFFu)));
-  }
-  __device__ static inline u32x4 run(const uint32_t* w) {
-    // stored byte = code + 128; flipping the top bit gives the two's complement code
-    const uint32_t a = w[0] ^ 0x80808080u, b = w[1] ^ 0x80808080u;
-    u32x4 o;
-    o.x = pack_bf16_hi(sbyte(a, 0), sbyte(a, 1));
-    o.y = pack_bf16_hi(sbyte(a, 2), sbyte(a, 3));
-    o.z = pack_bf16_hi(sbyte(b, 0), sbyte(b, 1));
-    o.w = pack_bf16_hi(sbyte(b, 2), sbyte(b, 3));
-    return o;
-  }
-};
-
-template <>
-struct DequantExact<WOL_DTYPE_F16, 8> {
-  __device__ static inline u32x4 run(const uint32_t* w) {
-    u32x4 o;  // byte | 0x6400 = 1024 + byte, minus 1152 = code
-    o.x = f16x2_add(__builtin_amdgcn_perm(w[0], 0x64646464u, 0x00050004u), 0xE480E480u);
-    o.y = f16x2_add(__builtin_amdgcn_perm(w[0], 0x64646464u, 0x00070006u), 0xE480E480u);
-    o.z = f16x2_add(__builtin_amdgcn_perm(w[1], 0x64646464u, 0x00050004u), 0xE480E480u);
-    o.w = f16x2_add(__builtin_amdgcn_perm(w[1], 0x64646464u, 0x00070006u), 0xE480E480u);
-    return o;
-  }
-};
-
-template <>
-struct DequantExact<WOL_DTYPE_F16, 4> {
-  __device__ static inline u32x4 run(const uint32_t* w) {
-    const uint32_t v = w[0];
-    u32x4 o;  // nibble<<4 | 0x5400 = 64 + nibble, minus 72 = code
-    o.x = f16x2_add(((v << 4) & 0x00F000F0u) | 0x54005400u, 0xD480D480u);
-    o.y = f16x2_add((v & 0x00F000F0u) | 0x54005400u, 0xD480D480u);
-    o.z = f16x2_add(((v >> 4) & 0x00F000F0u) | 0x54005400u, 0xD480D480u);
-    o.w = f16x2_add(((v >> 8) & 0x00F000F0u) | 0x54005400u, 0xD480D480u);
-    return o;
-  }
-};
-
-template <>
-struct DequantExact<WOL_DTYPE_BF16, 4> {
-  __device__ static inline uint32_t fix(uint32_t pair) {
-    // pair = two bf16 holding 136 + code; widen, subtract, narrow (all exact)
-    const float lo = __uint_as_float(pair << 16) - 136.0f;
-    const float hi = __uint_as_float(pair & 0xFFFF0000u) - 136.0f;
-    return pack_bf16_hi(lo, hi);
-  }
-  __device__ static inline u32x4 run(const uint32_t* w) {
-    const uint32_t v = w[0];
-    u32x4 o;
-    o.x = fix((v & 0x000F000Fu) | 0x43004300u);
-    o.y = fix(((v >> 4) & 0x000F000Fu) | 0x43004300u);
-    o.z = fix(((v >> 8) & 0x000F000Fu) | 0x43004300u);
-    o.w = fix(((v >> 12) & 0x000F000Fu) | 0x43004300u);
-    return o;
-  }
-};
-
-// The same codes in 19 instructions per eight instead of 27: each nibble pair
-// becomes two fp16 values 1024 + 16 * nibble (one and-or), a mixed-precision FMA
-// takes the offset out and widens to fp32 in one instruction, and the high
-// halves are the bf16 codes, every step exact.  g128 with this form against the
-// other one: 128 x 256 tiles 2 to 5 % faster (100 rows, K = 11008, N = 4096: 58.4
-// against 60.7 us; swiglu, 128 rows, 3 to 5 %), half-deep and small-M tiles 1 to
-// 2 %; 256 x 128 tiles, where four A blocks share a B block, 2 to 3 % slower (200
-// rows, K = N = 4096: 31.6 against 30.7), so they keep the other.  gemm_kernel:
-// per channel 2 to 4 % faster, group-wise up to 9 % slower (K = 4544: 65 rows).
-template <int DT, int BITS>
-struct DequantExactFma : DequantExact<DT, BITS> {};
-
-template <>
-struct DequantExactFma<WOL_DTYPE_BF16, 4> {
-  __device__ static inline uint32_t pair(uint32_t v) {
-    const f16x2 h = __builtin_bit_cast(f16x2, (v & 0x00F000F0u) | 0x64006400u);
-    return pack_bf16_hi(__builtin_fmaf(static_cast<float>(h.x), 0.0625f, -72.0f),
-                        __builtin_fmaf(static_cast<float>(h.y), 0.0625f, -72.0f));
-  }
-  __device__ static inline u32x4 run(const uint32_t* w) {
-    const uint32_t v = w[0];
-    u32x4 o;
-    o.x = pair(v << 4);
-    o.y = pair(v);
-    o.z = pair(v >> 4);
-    o.w = pair(v >> 8);
-    return o;
-  }
-};
 
 // Workgroup -> output tile.  Hardware deals consecutive workgroup ids to the
 // 8 XCDs in turn; give XCD x the ids that form a compact block of tiles so
@@ -399,36 +272,6 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_kernel(
   }
 }
 
-// s_waitcnt that only bounds the number of outstanding vector-memory loads.
-template <int N_>
-__device__ inline void wait_vmcnt() {
-  // gfx9 encoding: vmcnt = [15:14][3:0], expcnt = [6:4], lgkmcnt = [11:8]
-  __builtin_amdgcn_s_waitcnt((N_ & 0xF) | ((N_ >> 4) << 14) | (0x7 << 4) | (0xF << 8));
-}
-
-typedef __attribute__((address_space(3))) void* lds_ptr_t;
-
-// XOR applied to the 16-byte piece index of an A row in LDS (C pieces per
-// row).  A lane group reads the same piece of 16 consecutive rows; the XOR
-// spreads those reads over the banks whether the LDS serves 8 or 16 lanes of
-// a 128-bit read per cycle.
-template <int C>
-__device__ inline int a_swizzle(int row) {
-  if (C == 8) return (row & 7) ^ ((row >> 3) & 1);  // 128-byte rows
-  return row & (C - 1);                             // 256-byte rows
-}
-
-typedef float f32x16 __attribute__((ext_vector_type(16)));
-
-template <int DT>
-__device__ inline f32x16 mfma32(u32x4 a, u32x4 b, f32x16 c) {
-  if (DT == WOL_DTYPE_BF16)
-    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a),
-                                                   __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
-  return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, a),
-                                                __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
-}
-
 // acc + the sum of the eight T values of an operand fragment, in fp32 (four
 // packed dot products against (1, 1)).
 template <int DT>
@@ -445,42 +288,6 @@ __device__ inline float sum8(u32x4 v, float acc) {
   }
   return acc;
 }
-
-// What one launch of the fast kernel works on.
-struct DmaParams {
-  const uint16_t* x;
-  const uint8_t* codes;
-  const uint16_t* bias;
-  const uint16_t* scale;
-  void* out;                    // T or fp32 [M, N]; with nsplit > 1 fp32 partial sums
-                                // [nsplit][M][columns of the launch]
-  int M, K, N;
-  int out_f32;
-  int strip_lo, strip_hi;       // the launch covers the 16-column strips [strip_lo, strip_hi)
-  int nbx, nby;                 // output tiles of the launch
-  int nsplit, tiles_per_split;  // K is cut into nsplit runs of k tiles, one workgroup each
-  int xcd_rows;                 // row groups of the XCD grid (tile_of_block), 0 = plain order
-  int act;                      // WOL_ACT_NONE or WOL_ACT_GELU, applied where the final sum is formed
-  // Grouped launch (mixture of experts): row tile `by` of the launch is entry
-  // `by` of this table -- {expert, first row, rows} -- written on the device by
-  // moe_plan_kernel; an expert's rows use that expert's weights, scales and
-  // bias (consecutive tensors, the strides below apart).  Null: one problem.
-  const int* moe_table;
-  int64_t moe_codes_stride;     // bytes between two experts' packed weights
-  int moe_rows;                 // rows of the whole grouped problem (the partial sums' row count)
-  // STAMP instantiation only: six cycle counts per wavefront, [workgroup][wavefront][8] (see wol_prefill_phases)
-  unsigned long long* stamps;
-};
-
-// One entry of the row-tile table of a grouped launch.
-struct MoeTile {
-  int expert;  // -1: the tile is not used
-  int row0;    // first row of the tile in the permuted input
-  int rows;    // rows of the tile that exist (1 .. tile height)
-  int first;   // gemm_experts_kernel: first row tile of the tile's expert ...
-  int count;   // ... and how many it has
-  int pad[3];
-};
 
 // Fast path: K a multiple of the tile depth.
 //
@@ -564,14 +371,6 @@ struct MoeTile {
 // of a raw tile are read into registers once for both k tiles.  Every stage has
 // the same number of loads, so the counted waits are those of the other forms.
 constexpr int kHalfDeepStages = 10;
-
-// Where a tile of gemm_experts_kernel lies.
-struct TilePlace {
-  int bx;      // column tile of the launch
-  int expert;  // the tile lies in this expert's rows
-  int row0;    // the tile's first row in x and out
-  int rows;    // rows of the tile that exist
-};
 
 template <int DT, int BITS, int G, int OFFS, int WM, int WN, int TM, int TN, int STAGES, int SWI, bool RESC, bool STAMP,
           bool EXPERTS>
@@ -1355,28 +1154,6 @@ __global__ __launch_bounds__(256) void reduce_partials_swiglu_kernel(
 
 typedef GemmArgs Args;
 
-// Raises a kernel's dynamic LDS limit once per device (the attribute belongs to
-// the device's copy of the function); safe to call from several threads.
-inline void allow_lds(const void* kern, size_t lds, std::atomic<uint32_t>& done) {
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess) dev = 0;
-  const uint32_t bit = 1u << (dev & 31);
-  if (done.load(std::memory_order_acquire) & bit) return;
-  (void)hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds));
-  done.fetch_or(bit, std::memory_order_release);
-}
-
-inline int num_cus() {
-  static const int cus = [] {
-    int dev = 0, n = 0;
-    if (hipGetDevice(&dev) != hipSuccess ||
-        hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0)
-      n = 256;
-    return n;
-  }();
-  return cus;
-}
-
 template <int DT, int BITS, bool GROUPED, int WM, int WN, int TM, int TN>
 void launch_one(const Args& a) {
   constexpr int BM = WM * TM * 16, BN = WN * TN * 16, TK = BITS == 8 ? 64 : 128;
@@ -1471,13 +1248,40 @@ void launch_dma(const Args& a, int strip_lo, int strip_hi, int nsplit) {
   }
 }
 
-// The half-size tile of the int8 paths: 256 x 128 (four A blocks
-// share each dequantised B block: less VALU work per MFMA, 9 % faster than
-// 128 x 256 at M = 512) unless its 256-row blocks would pad M much further
-// than 128-row blocks do.
-inline bool tall_half_tile(int M) {
-  const int pad256 = (M + 255) / 256 * 256, pad128 = (M + 127) / 128 * 128;
-  return pad256 * 100 <= pad128 * 108;
+// Launches a tile of wol_linear_wide.hip on the columns of strips [strip_lo,
+// strip_hi); the rest as launch_dma.
+template <int DT>
+void launch_wide(const Args& a, int bits, int group, WideTile tile, int swi, int strip_lo, int strip_hi, int nsplit) {
+  const int bm = tile == WideTile::kHalf ? 128 : 256, bn = swi ? 128 : 256;
+  if (strip_hi <= strip_lo) return;
+  if (swi) nsplit = 1;
+  const int ncols = (strip_hi - strip_lo) * kStripCols;
+  if (nsplit > 1 && (a.ws == nullptr || a.ws_bytes < static_cast<size_t>(nsplit) * a.M * ncols * sizeof(float)))
+    nsplit = 1;  // never write past the scratch buffer
+  DmaParams p{};
+  p.x = static_cast<const uint16_t*>(a.x);
+  p.codes = static_cast<const uint8_t*>(a.codes);
+  p.bias = static_cast<const uint16_t*>(a.bias);
+  p.scale = static_cast<const uint16_t*>(a.scale);
+  p.out = nsplit > 1 ? a.ws : a.out;
+  p.M = a.M; p.K = a.K; p.N = a.N;
+  p.out_f32 = a.out_f32;
+  p.strip_lo = strip_lo; p.strip_hi = strip_hi;
+  p.nbx = (ncols + bn - 1) / bn;
+  p.nby = (a.M + bm - 1) / bm;
+  const int tiles = a.K / 64;
+  p.tiles_per_split = (tiles + nsplit - 1) / nsplit;
+  if (group == 128 || bits == 4) p.tiles_per_split = (p.tiles_per_split + 1) & ~1;  // every run starts on a group (a raw tile) of two tiles
+  p.nsplit = (tiles + p.tiles_per_split - 1) / p.tiles_per_split;
+  p.act = a.act;
+  if (DT == WOL_DTYPE_BF16) launch_wide_bf16(p, bits, group, tile, swi, a.stream);
+  else launch_wide_f16(p, bits, group, tile, swi, a.stream);
+  if (nsplit > 1) {
+    const int64_t total = static_cast<int64_t>(a.M) * ncols;
+    reduce_partials_kernel<DT><<<dim3(static_cast<unsigned>((total / 4 + 255) / 256)), dim3(256), 0, a.stream>>>(
+        static_cast<const float*>(a.ws), p.nsplit, p.bias, a.out, a.out_f32, total, a.N,
+        strip_lo * kStripCols, ncols, a.act);
+  }
 }
 
 // Number of 256-column tiles given to the 256-row kernel; the remaining
@@ -1495,13 +1299,12 @@ inline int plan_big_columns(int M, int K, int N, int bits, int group) {
   const double kSmall = g4 ? 0.58 : 0.55;
   constexpr double kRuns = 0.25;
   const int nbx = (N + 255) / 256, nby_big = (M + 255) / 256, nby_small = (M + 127) / 128;
-  const bool tall = (bits == 8 || g4) && tall_half_tile(M);  // half tiles of 256 x 128 instead of 128 x 256
   int best = nbx;
   double best_t = 1e30;
   // the estimate grows with the number of half-size tiles, so for every number of whole rounds only the most
   // columns that fit them matter (walking all columns took 1 to 2 us of a call on a wide weight)
   for (int c = nbx; c >= 0;) {
-    const int small = tall ? 2 * (nbx - c) * nby_big : (nbx - c) * nby_small;
+    const int small = (nbx - c) * nby_small;
     const int rounds = (c * nby_big + cus - 1) / cus;
     double t = static_cast<double>(rounds);
     const int rest = small % cus;
@@ -1576,19 +1379,12 @@ inline SkinnyPlan plan_skinny(int M, int K, int N, int bits, int group, size_t w
   return best;
 }
 
-// Tile of the configuration launch_fast gives the columns that do not get
-// 256 x 256 tiles (above 64 rows), and the first strip of those columns.
-inline void half_tile_config(int M, int K, int N, int bits, int group, int* bm, int* bn, int* strip_lo) {
-  // 256 x 256 tiles on whole rounds of the CUs
+// First strip of the columns that get 128 x 256 tiles (above 64 rows); those in
+// front of it get 256 x 256 tiles.
+constexpr int kHalfRows = 128, kHalfCols = 256;
+inline int half_tile_strip(int M, int K, int N, int bits, int group) {
   const int c = plan_big_columns(M, K, N, bits, group) * 16, nstrips = N / kStripCols;
-  *strip_lo = c < nstrips ? c : nstrips;
-  if (bits == 8 || group != 0) {
-    *bm = tall_half_tile(M) ? 256 : 128;
-    *bn = tall_half_tile(M) ? 128 : 256;
-  } else {
-    *bm = 128;
-    *bn = 256;
-  }
+  return c < nstrips ? c : nstrips;
 }
 
 // How a half-size configuration (one workgroup per CU) covers ncols columns:
@@ -1638,53 +1434,20 @@ void launch_fast(const Args& a) {
     launch_dma<DT, BITS, G, false, 1, 8, 2, 1, 2>(a, 0, nstrips, ns);
     return;
   }
-  constexpr int TK = BITS == 8 ? 64 : 128;
-  int bm = 0, bn = 0, lo = 0;
-  half_tile_config(a.M, a.K, a.N, BITS, G, &bm, &bn, &lo);
-  const TailPlan t = plan_tail(a.M, a.K, (nstrips - lo) * kStripCols, bm, bn, TK, a.ws != nullptr ? a.ws_bytes : 0);
-  const int mid = lo + t.full_tiles * (bn / kStripCols);  // strips [lo, mid) unsplit, [mid, nstrips) in t.ns runs
-  // launches a half-size configuration on both parts
-#define WOL_HALF(...)                                              \
-  do {                                                             \
-    launch_dma<DT, BITS, G, __VA_ARGS__>(a, lo, mid, 1);           \
-    launch_dma<DT, BITS, G, __VA_ARGS__>(a, mid, nstrips, t.ns);   \
-  } while (0)
-  if constexpr (BITS == 8 && G == 0) {
-    // 256 x 256 x 64 tiles (144 KiB of LDS, one workgroup per CU) for as many
-    // column tiles as fill whole rounds of the CUs; the rest, which would
-    // leave CUs idle for a whole tile time, goes to half-size tiles.
-    launch_dma<DT, BITS, G, false, 2, 4, 4, 2>(a, 0, lo, 1);
-    if (bm == 256) WOL_HALF(false, 2, 4, 4, 1);
-    else WOL_HALF(false, 2, 4, 2, 2);
-  } else if constexpr (BITS == 8) {
-    // group-wise scales: the sums are kept in units of the current group's
-    // scale (RESC), so one set of accumulators serves and the tiles are those
-    // of the per-channel weights
-    launch_dma<DT, BITS, G, 0, 2, 4, 4, 2, 3, 0, true>(a, 0, lo, 1);
-    if (bm == 256) WOL_HALF(0, 2, 4, 4, 1, 3, 0, true);
-    else WOL_HALF(0, 2, 4, 2, 2, 3, 0, true);
-  } else if constexpr (G != 0) {
-    // int4 with group-wise scales: the same, the whole tiles on 64-deep k tiles
-    // (two 128-deep stages and their scales would need 164 KiB of LDS).  Against
-    // 256 x 128 tiles alone, M = 8192, K = N = 4096: bf16 g128 297 -> 249 us
-    // (1.11 PFLOP/s), g64 322 -> 273, fp16 g128 283 -> 237; M = 2048, N = 12288
-    // g128 223 -> 201.  The half-size tiles are 256 x 128 where the rows fill
-    // them (four A blocks share every dequantised B block), else 128 x 256.
-    launch_dma<DT, BITS, G, 0, 2, 4, 4, 2, kHalfDeepStages + 3, 0, true>(a, 0, lo, 1);
-    if (bm == 256) WOL_HALF(0, 2, 4, 4, 1, 2, 0, true);
-    else WOL_HALF(0, 2, 4, 2, 2, 2, 0, true);
-  } else if constexpr (DT == WOL_DTYPE_BF16) {
-    // the exact int4 -> bf16 dequantiser costs 19 VALU instructions per 8
-    // codes; the offset form is faster or level: with row sums by dot products on the
-    // 256 x 256 tile (two stages of 64 + 16 KiB fill the LDS), with one
-    // cancelling MFMA per A block on the 128 x 256 tiles of the remainder
-    launch_dma<DT, BITS, G, 2, 2, 4, 4, 2, 2>(a, 0, lo, 1);
-    WOL_HALF(true, 2, 4, 2, 2);
-  } else {
-    launch_dma<DT, BITS, G, 0, 2, 4, 4, 2, 2>(a, 0, lo, 1);
-    WOL_HALF(false, 2, 4, 2, 2);
-  }
-#undef WOL_HALF
+  // 256 x 256 tiles for as many column tiles as fill whole rounds of the CUs; the
+  // rest, which would leave CUs idle for a whole tile time, goes to 128 x 256
+  // tiles.  (256 x 128 ones, four A blocks per dequantised B block in the former
+  // kernel, are nowhere faster any more: int8, 512 rows, K = 4096, N = 12288 52.6
+  // against 50.6 us; 1237 rows, K = 11008, N = 4096 116 against 112.)
+  const int lo = half_tile_strip(a.M, a.K, a.N, BITS, G);
+  const TailPlan t = plan_tail(a.M, a.K, (nstrips - lo) * kStripCols, kHalfRows, kHalfCols, BITS == 8 ? 64 : 128,
+                               a.ws != nullptr ? a.ws_bytes : 0);
+  const int mid = lo + t.full_tiles * (kHalfCols / kStripCols);  // strips [lo, mid) unsplit, [mid, nstrips) in t.ns runs
+  if constexpr (G == 0) launch_wide<DT>(a, BITS, G, WideTile::kWhole, 0, 0, lo, 1);
+  else if constexpr (BITS == 8) launch_dma<DT, BITS, G, 0, 2, 4, 4, 2, 3, 0, true>(a, 0, lo, 1);
+  else launch_dma<DT, BITS, G, 0, 2, 4, 4, 2, kHalfDeepStages + 3, 0, true>(a, 0, lo, 1);
+  launch_wide<DT>(a, BITS, G, WideTile::kHalf, 0, lo, mid, 1);
+  launch_wide<DT>(a, BITS, G, WideTile::kHalf, 0, mid, nstrips, t.ns);
 }
 
 // How high the row tiles of gemm_experts_kernel may be.  A round of workgroups
@@ -1991,31 +1754,13 @@ void launch_cfg(const Args& a) {
 template <int DT, int BITS, int G>
 void launch_swiglu_gemm(const Args& a) {
   const int gate_strips = a.N / 2 / kStripCols;
-  if constexpr (G != 0) {
-    // group-wise scales: the tiles with two blocks per wavefront and rescaled sums
-    if constexpr (BITS == 8) {
-      if (a.M >= 192) launch_dma<DT, 8, G, 0, 2, 4, 4, 2, 3, 1, true>(a, 0, gate_strips, 1);
-      else launch_dma<DT, 8, G, 0, 2, 4, 2, 2, 3, 1, true>(a, 0, gate_strips, 1);
-    } else {
-      // whole tiles, or half-size ones (256 x 128: gate and up blocks in neighbouring wavefronts) where their
-      // rounds, at 0.65 of a whole tile's, are done sooner: K = 4096, N = 22016, bf16 g128, whole / half-size
-      // tiles, 256 rows 109 / 70 us, 400 rows 110 / 142, 1024 rows 231 / 224, 1237 rows 242 / 298, 2048 rows
-      // 370 / 447, 4096 rows 729 / 846
-      const bool tall = tall_half_tile(a.M);
-      const int cus = num_cus(), cols = (a.N + 255) / 256, big = cols * ((a.M + 255) / 256);
-      const int half = tall ? 2 * big : cols * ((a.M + 127) / 128);
-      if ((big + cus - 1) / cus < 0.65 * ((half + cus - 1) / cus))
-        launch_dma<DT, 4, G, 0, 2, 4, 4, 2, kHalfDeepStages + 3, 1, true>(a, 0, gate_strips, 1);
-      else if (tall) launch_dma<DT, 4, G, 0, 2, 4, 4, 1, 2, 1, true>(a, 0, gate_strips, 1);
-      else launch_dma<DT, 4, G, 0, 2, 4, 2, 2, 2, 1, true>(a, 0, gate_strips, 1);
-    }
-  } else if constexpr (BITS == 8) {
-    if (a.M >= 192) launch_dma<DT, 8, 0, false, 2, 4, 4, 2, 3, 1>(a, 0, gate_strips, 1);
-    else launch_dma<DT, 8, 0, false, 2, 4, 2, 2, 3, 1>(a, 0, gate_strips, 1);
-  } else {
-    if (a.M >= 192) launch_dma<DT, 4, 0, DT == WOL_DTYPE_BF16 ? 2 : 0, 2, 4, 4, 2, 2, 1>(a, 0, gate_strips, 1);
-    else launch_dma<DT, 4, 0, DT == WOL_DTYPE_BF16 ? 1 : 0, 2, 4, 2, 2, 3, 1>(a, 0, gate_strips, 1);
-  }
+  // whole tiles, or half-size ones where their rounds, at 0.6 of a whole tile's, are done sooner
+  const int cus = num_cus(), cols = (a.N + 255) / 256;
+  const int big = cols * ((a.M + 255) / 256), half = cols * ((a.M + 127) / 128);
+  if ((big + cus - 1) / cus >= 0.6 * ((half + cus - 1) / cus)) launch_wide<DT>(a, BITS, G, WideTile::kHalf, 1, 0, gate_strips, 1);
+  else if constexpr (G == 0) launch_wide<DT>(a, BITS, G, WideTile::kWhole, 1, 0, gate_strips, 1);
+  else if constexpr (BITS == 8) launch_dma<DT, 8, G, 0, 2, 4, 4, 2, 3, 1, true>(a, 0, gate_strips, 1);
+  else launch_dma<DT, 4, G, 0, 2, 4, 4, 2, kHalfDeepStages + 3, 1, true>(a, 0, gate_strips, 1);
 }
 template <int DT, int BITS>
 void launch_swiglu_gemm_g(const Args& a) {
@@ -2081,12 +1826,11 @@ size_t linear_gemm_workspace(int64_t M, int64_t K, int64_t N, int bits, int grou
   const int tk = bits == 8 ? 64 : 128;
   if (K % tk != 0 || K / tk < 2) return 0;
   if (M > kSkinnyMaxM) {
-    int bm = 0, bn = 0, lo = 0;
     const int g = group_size > 0 ? group_size : 0;
-    half_tile_config(static_cast<int>(M), static_cast<int>(K), static_cast<int>(N), bits, g, &bm, &bn, &lo);
+    const int lo = half_tile_strip(static_cast<int>(M), static_cast<int>(K), static_cast<int>(N), bits, g);
     const int ncols = static_cast<int>(N) - lo * kStripCols;
-    const TailPlan t = plan_tail(static_cast<int>(M), static_cast<int>(K), ncols, bm, bn, tk, SIZE_MAX);
-    return t.ns > 1 ? static_cast<size_t>(t.ns) * M * (ncols - t.full_tiles * bn) * sizeof(float) : 0;
+    const TailPlan t = plan_tail(static_cast<int>(M), static_cast<int>(K), ncols, kHalfRows, kHalfCols, tk, SIZE_MAX);
+    return t.ns > 1 ? static_cast<size_t>(t.ns) * M * (ncols - t.full_tiles * kHalfCols) * sizeof(float) : 0;
   }
   const int ns = plan_skinny(static_cast<int>(M), static_cast<int>(K), static_cast<int>(N), bits,
                              group_size > 0 ? group_size : 0, SIZE_MAX).ns;
@@ -2109,19 +1853,18 @@ void describe_linear_gemm(int64_t M, int64_t K, int64_t N, int bits, int group_s
              bits == 4 && M <= 32 ? 32 : 64, wide ? 512 : 256, ns, ns > 1 ? " + reduce_partials_kernel" : "");
     return;
   }
-  int bm = 0, bn = 0, lo = 0;
-  half_tile_config(static_cast<int>(M), static_cast<int>(K), static_cast<int>(N), bits, g, &bm, &bn, &lo);
+  const int lo = half_tile_strip(static_cast<int>(M), static_cast<int>(K), static_cast<int>(N), bits, g);
   const int nstrips = static_cast<int>(N / kStripCols);
-  const TailPlan t = plan_tail(static_cast<int>(M), static_cast<int>(K), (nstrips - lo) * kStripCols, bm, bn, tk, ws_bytes);
-  const int mid = lo + t.full_tiles * (bn / kStripCols);
+  const TailPlan t = plan_tail(static_cast<int>(M), static_cast<int>(K), (nstrips - lo) * kStripCols, kHalfRows, kHalfCols, tk, ws_bytes);
+  const int mid = lo + t.full_tiles * (kHalfCols / kStripCols);
   int len = 0;
-  len += snprintf(buf + len, n - len, "wol::gemm_dma_kernel (v_mfma_f32_32x32x16):");
+  len += snprintf(buf + len, n - len, "wol::gemm_dma_kernel_wide (v_mfma_f32_16x16x32):");
   if (lo > 0 && len < static_cast<int>(n))
     len += snprintf(buf + len, n - len, " 256x256 tiles on columns [0,%d)", lo * kStripCols);
   if (mid > lo && len < static_cast<int>(n))
-    len += snprintf(buf + len, n - len, " %dx%d tiles on [%d,%d)", bm, bn, lo * kStripCols, mid * kStripCols);
+    len += snprintf(buf + len, n - len, " 128x256 tiles on [%d,%d)", lo * kStripCols, mid * kStripCols);
   if (nstrips > mid && len < static_cast<int>(n))
-    len += snprintf(buf + len, n - len, " %dx%d tiles on [%d,%d)%s", bm, bn, mid * kStripCols, nstrips * kStripCols,
+    len += snprintf(buf + len, n - len, " 128x256 tiles on [%d,%d)%s", mid * kStripCols, nstrips * kStripCols,
                     t.ns > 1 ? " with K in runs + reduce_partials_kernel" : "");
 }
 
@@ -2410,39 +2153,6 @@ void launch_probe(const void* ops, int wgs, int iters, float* out, hipStream_t s
 }
 
 }  // namespace
-
-// The prefill GEMM's 256 x 256 int8 per-channel bf16 launch with cycle stamps
-// (M and N multiples of 256, K a multiple of 64 and at least 192): out [M, N]
-// bf16, stamps [(M / 256) * (N / 256)][8 wavefronts][8] counts.
-int launch_prefill_phases(const void* x, const void* codes, const void* scale, int64_t M, int64_t K, int64_t N,
-                          void* out, unsigned long long* stamps, hipStream_t stream) {
-  constexpr int WM = 2, WN = 4, TM = 4, TN = 2, STAGES = 3;
-  constexpr size_t lds = dma_lds_bytes<8, 0, WM, WN, TM, TN, STAGES>();
-  auto kern = gemm_dma_kernel<WOL_DTYPE_BF16, 8, 0, 0, WM, WN, TM, TN, STAGES, 0, false, true>;
-  static std::atomic<uint32_t> configured{0};
-  allow_lds(reinterpret_cast<const void*>(kern), lds, configured);
-  DmaParams p;
-  p.x = static_cast<const uint16_t*>(x);
-  p.codes = static_cast<const uint8_t*>(codes);
-  p.bias = nullptr;
-  p.scale = static_cast<const uint16_t*>(scale);
-  p.out = out;
-  p.M = static_cast<int>(M); p.K = static_cast<int>(K); p.N = static_cast<int>(N);
-  p.out_f32 = 0;
-  p.strip_lo = 0; p.strip_hi = static_cast<int>(N / kStripCols);
-  p.nbx = static_cast<int>(N / 256);
-  p.nby = static_cast<int>(M / 256);
-  p.tiles_per_split = static_cast<int>(K / 64);
-  p.nsplit = 1;
-  p.xcd_rows = plan_xcd_rows(p.nbx, p.nby, 256 * 2, 256);
-  p.act = WOL_ACT_NONE;
-  p.moe_table = nullptr;
-  p.moe_codes_stride = 0;
-  p.moe_rows = 0;
-  p.stamps = stamps;
-  kern<<<dim3(static_cast<unsigned>(p.nbx * p.nby)), dim3(64 * WM * WN), lds, stream>>>(p);
-  return check_launch();
-}
 
 int launch_mfma_probe(int variant, const void* ops, int workgroups, int iters, float* out, hipStream_t stream) {
   switch (variant) {

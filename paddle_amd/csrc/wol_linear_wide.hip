@@ -1,0 +1,534 @@
+// The tiles of 128 and 256 rows of weight_only_linear's GEMM (more than 64 rows, K made of whole k tiles), for bf16;
+// wol_linear_wide_f16.hip compiles the same source for fp16.  This file is built with the instruction scheduler in front
+// of register allocation switched off (build.sh): the loops below give every instruction its place, and that pass, which
+// does not see why, costs up to 40 registers and then spills (int4 per channel: 240 registers without it, 256 and
+// spills with it).
+//
+// gemm_dma_kernel_wide.  A workgroup of eight wavefronts, WM x WN, computes WM*TM*16 rows x WN*TN*16 columns from
+// v_mfma_f32_16x16x32 blocks, TM x TN per wavefront.  The k tile is 64 deep; three of them are resident or in flight, all
+// through direct-to-LDS buffer loads.
+//
+// What bounds it.  With random operands the part runs into its power limit, so energy counts as much as cycles: the
+// 16x16x32 form touches its accumulators once per 32 k, 32x32x16 does every 16 k (a plain fp16 GEMM on these tiles went
+// from 1.12 to 1.26 PFLOP/s by the form alone).  In cycles: two wavefronts share a SIMD, an MFMA takes two of its
+// ~4.3-cycle issue slots and every VALU instruction one, so beside a 16-cycle MFMA two VALU instructions are free and
+// each further one lengthens the loop.  Hence WM = 1: every wavefront covers all rows of 32 columns, a weight is
+// dequantised once per workgroup (0.9 VALU instructions per MFMA for int8, 1.2 for exact int4; with two rows of
+// wavefronts twice that) at the price of one A fragment out of LDS per two MFMAs, half of what the LDS delivers.
+// int8, bf16: M = 2048, K = 4096, N = 8192 109 -> 98 us (1.40 PFLOP/s) against 32x32x16 tiles of two by four wavefronts,
+// 100 with two by four wavefronts here; M = 8192, K = N = 4096 215 -> 191; M = 4096, K = 14336, N = 4096 358 -> 319
+// (1.51).  int4 per channel M = 2048, N = 8192 112 -> 99, with the exact dequantiser where the row sums of an offset
+// form were needed.
+//
+// Order of a k tile.  Its two halves (32 k each) run TM slots of TN MFMAs, a slot per A block.  The A fragment a slot has
+// just used is read again for the next half right behind it, so A needs one set of registers; B fragments have two
+// sets, the next half's being dequantised a few instructions per slot.  The workgroup barrier sits a quarter into the
+// second half: by then the last reads of the tile have arrived, so nobody waits for LDS there, and everything the next
+// tile's first half needs is read and converted behind it.  Tile t+3's loads go out between the barriers of tiles t
+// and t+1, a few per slot.
+//
+// A fragments: rows of 128 bytes, the 16-byte piece XORed with row % 8; the sixteen lanes that a ds_read_b128 serves
+// together ({0-3, 12-15, 20-27}, ...) then cover all 64 banks.  B: lane l of a raw strip tile owns column l % 16 and, per
+// 32-k step, the eight k from 8 * (l / 16) on: the operand itself.
+//
+// int4: a raw tile holds 128 k, so it serves two k tiles.  It has two buffers of its own; an odd tile's loads bring the
+// first half (by strips) of the next raw tile and the even one's the second (128-column tiles: all of it with the odd
+// one).
+//
+// G != 0 (group-wise scales): one set of accumulators, kept in units of the current group's scale.  Where a group
+// starts the running sums are multiplied by (previous unit / new unit) and the group's MFMAs then accumulate straight
+// into them; the epilogue multiplies by the last unit.  Every rescaling rounds the sums once (2^-24 relative, a few dozen
+// times per output element), code * scale is never rounded to T.  The unit of a column follows its group scale but never
+// falls more than 2^64 below the largest scale the column has had so far (a group that small weighs nothing next to the
+// others in fp32), so the sums cannot overflow however the scales of a column differ.
+//
+// SWI: swiglu in the epilogue.  The weight is a gate | up projection, [K, N] with the gate in columns 0 .. N/2-1; half of a
+// wavefront's strips are gate columns and the other half the up columns N/2 further on, so that silu(gate) * up is formed
+// lane by lane and only [M, N/2] leaves the kernel.
+//
+// STAMP (a diagnostic instantiation, never on a product path): every wavefront reads the cycle counter at kernel entry,
+// around the two waits of every k tile (for its own tile loads, then for the workgroup) and around the epilogue, and
+// leaves the sums in p.stamps.
+#include "wol_gemm_common.h"
+
+namespace wol {
+namespace {
+
+#ifndef WOL_GEMM_DTYPE
+#define WOL_GEMM_DTYPE WOL_DTYPE_BF16
+#endif
+
+template <int BITS, int G, int WM, int WN, int TM, int TN>
+constexpr size_t wide_lds_bytes() {
+  const size_t a = static_cast<size_t>(WM) * TM * 16 * 128, b = static_cast<size_t>(WN) * TN * 1024;
+  return 3 * (a + (BITS == 8 ? b : 0) + (G == 0 ? 0 : WM * WN * 256)) + (BITS == 4 ? 2 * b : 0);
+}
+
+// Where position `pos` of a launch's tiles lies.  The sequence walks the tiles in bands of four row tiles or so, column
+// by column within a band, and every XCD works on a piece of it that hangs together: its 32 CUs then share four row
+// blocks and eight column blocks in their L2.  (A grid of XCDs that needs both tile counts to divide left ragged ones in
+// plain order, where the 32 tiles of an XCD have 32 different column blocks.)
+__device__ inline void tile_of_position(int pos, int nbx, int nby, int* bx, int* by) {
+  const int bands = nby > 5 ? (nby + 2) / 4 : 1, base = nby / bands, extra = nby % bands;
+  int rows = base + 1, lo = 0, w = pos;  // the first `extra` bands have a row tile more
+  if (w >= extra * rows * nbx) {
+    w -= extra * rows * nbx;
+    lo = extra * rows;
+    rows = base;
+  }
+  const int b = w / (rows * nbx);
+  w -= b * rows * nbx;
+  *by = lo + b * rows + w % rows;
+  *bx = w / rows;
+}
+
+// The tile and the K run of this workgroup: consecutive workgroup ids go to the 8 XCDs in turn, and XCD x takes the x-th
+// eighth of the sequence of (run, tile).
+__device__ inline void place_of_block(const DmaParams& p, int* bx, int* by, int* split) {
+  constexpr int kXcd = 8;
+  const int tiles = p.nbx * p.nby, total = tiles * p.nsplit;
+  const int x = blockIdx.x % kXcd, q = total / kXcd, r = total % kXcd;
+  const int pos = x * q + (x < r ? x : r) + blockIdx.x / kXcd;
+  *split = pos / tiles;
+  tile_of_position(pos - *split * tiles, p.nbx, p.nby, bx, by);
+}
+
+template <int DT, int BITS, int G, int WM, int WN, int TM, int TN, int SWI, bool STAMP>
+__device__ __forceinline__ void wide_tile(const DmaParams& p, int bx, int by, int split) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  constexpr int NW = WM * WN;
+  static_assert(NW == 8, "eight wavefronts");
+  constexpr int BM = WM * TM * 16, BN = WN * TN * 16, kStrips = WN * TN;
+  constexpr int kABytes = BM * 128, kBBytes = kStrips * 1024;  // an A tile, a raw B tile
+  constexpr int kSBytes = G == 0 ? 0 : NW * 256;
+  constexpr int kScaleOff = kABytes + (BITS == 8 ? kBBytes : 0);
+  constexpr int kStage = kScaleOff + kSBytes;
+  constexpr int kRawOff = 3 * kStage;  // int4: the two raw B tiles
+  constexpr int kLds = static_cast<int>(wide_lds_bytes<BITS, G, WM, WN, TM, TN>());  // what the launch asks for
+  constexpr int kALoads = kABytes / 1024 / NW, kBSlots = kStrips / NW;
+  static_assert(kABytes / 1024 % NW == 0 && kStrips % NW == 0, "the tile must split evenly over the wavefronts");
+  constexpr int kDw = BITS == 8 ? 2 : 1;  // raw dwords of a B fragment
+  static_assert(SWI == 0 || TN % 2 == 0, "gate and up strips in one wavefront");
+  // loads of a tile: [scales,] A, B; the B loads of an odd / even tile
+  constexpr int kS = G == 0 ? 0 : 1;
+  constexpr int kBOdd = BITS == 8 || kBSlots == 1 ? kBSlots : kBSlots / 2;
+  constexpr int kBEven = BITS == 8 ? kBSlots : kBSlots - kBOdd;
+  constexpr int kLoadsOdd = kS + kALoads + kBOdd, kLoadsEven = kS + kALoads + kBEven;
+  // slots of the second half before the barrier, and loads that go out between the barrier and the end of the tile
+  constexpr int B0 = TM / 4, kSpan = 2 * TM;  // kSpan: slots from barrier to barrier
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  unsigned long long st_entry = 0, st_prev = 0, st_work = 0, st_loads = 0, st_bar = 0, st_loop0 = 0;
+  if (STAMP) st_entry = __builtin_readcyclecounter();
+
+  const int tid = threadIdx.x;
+  const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = wave / WN, wn = wave % WN;
+  const int lr = lane & 15, kb = lane >> 4;
+  const int K = p.K, N = p.N;
+  const int M = p.M, m0 = by * BM;
+  const uint16_t* x = p.x;
+  const uint16_t* scale = p.scale;
+  const uint8_t* codes = p.codes;
+  // SWI: BN / 2 gate columns and the BN / 2 up columns that go with them
+  const int strip0 = p.strip_lo + bx * (SWI ? kStrips / 2 : kStrips);
+  const int up_strips = N / 2 / kStripCols;
+  const int t0 = split * p.tiles_per_split;  // this workgroup's run of k tiles
+  const int nt = (K / 64 - t0) < p.tiles_per_split ? (K / 64 - t0) : p.tiles_per_split;
+
+  const int rows = M - m0 < BM ? M - m0 : BM;
+  const int sbytes = static_cast<int>(strip_bytes(K, BITS));
+  const int left = p.strip_hi - strip0, strips = left < (SWI ? kStrips / 2 : kStrips) ? left : (SWI ? kStrips / 2 : kStrips);
+  // One descriptor per load: it starts at the load's own eight rows (its strip) and ends with the last row (strip) that
+  // exists, so edges arrive as zeros and a lane needs the same offset for every load.
+  __amdgpu_buffer_rsrc_t ra[kALoads], rb[kBSlots];
+#pragma unroll
+  for (int c = 0; c < kALoads; ++c) {
+    const int r0 = (c * NW + wave) * 8, nr = rows - r0 > 8 ? 8 : (rows > r0 ? rows - r0 : 0);
+    ra[c] = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(x + static_cast<int64_t>(nr > 0 ? m0 + r0 : m0) * K), 0, nr * K * 2, 0x00020000);
+  }
+  // SWI: LDS slot L of the B tile serves wavefront column L / TN; the first TN / 2 slots of one are its gate strips
+#pragma unroll
+  for (int c = 0; c < kBSlots; ++c) {
+    const int L = c * NW + wave;
+    const int st = SWI ? (L / TN) * (TN / 2) + L % TN % (TN / 2) : L;
+    const int64_t first = st < strips ? strip0 + st + (SWI && L % TN >= TN / 2 ? up_strips : 0) : 0;
+    rb[c] = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(codes + first * sbytes), 0, st < strips ? sbytes : 0, 0x00020000);
+  }
+  const uint32_t aoff = static_cast<uint32_t>((lane / 8) * K + ((lane ^ (lane >> 3)) & 7) * 8) * 2, boff = lane * 16;
+  // columns of this wavefront's strips
+  auto strip_col = [&](int c) {
+    if (SWI) return (strip0 + wn * (TN / 2) + c % (TN / 2)) * kStripCols + (c >= TN / 2 ? N / 2 : 0);
+    return (strip0 + wn * TN + c) * kStripCols;
+  };
+  // group scales travel with the tile: lane l brings columns 2l and 2l + 1 of its wavefront's TN * 16
+  int scol = 0;
+  if (G != 0) {
+    const int v = 2 * lane < TN * 16 ? 2 * lane : 0;
+    scol = strip_col(v / 16) + v % 16;
+    const int last = (SWI && v / 16 < TN / 2) ? N / 2 : (SWI ? N : p.strip_hi * kStripCols);
+    scol = scol < last ? scol : last - 2;  // past the last column: valid data, never used
+  }
+  constexpr int kGShift = G == 128 ? 7 : 6;
+  // load i of tile t (stage st); odd: parity of t
+  auto issue1 = [&](int t, int st, bool odd, int i) {
+    const int tt = t0 + (t < nt ? t : nt - 1);  // past the end: the last tile again, into a stage that nobody reads
+    unsigned char* s = smem + st * kStage;
+    if (G != 0 && i == 0) {
+      const int64_t row = static_cast<int64_t>(tt) * 64 >> kGShift;
+      __builtin_amdgcn_global_load_lds(scale + row * N + scol, (lds_ptr_t)(s + kScaleOff + wave * 256), 4, 0, 0);
+      return;
+    }
+    const int c = i - kS;
+    if (c < kALoads) {
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(ra[c], (lds_ptr_t)(s + (c * NW + wave) * 1024), 16, aoff, tt * 128, 0, 0);
+    } else if (BITS == 8) {
+      const int b = c - kALoads;
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rb[b], (lds_ptr_t)(s + kABytes + (b * NW + wave) * 1024), 16, boff, tt * 1024, 0, 0);
+    } else {
+      // tile 2T - 1 brings the first part of raw tile T, tile 2T the second (past the end: the last one again)
+      const int b = c - kALoads + (odd ? 0 : kBOdd), T = (t + 1) / 2, src = t0 / 2 + (2 * T < nt ? T : nt / 2 - 1);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rb[b], (lds_ptr_t)(smem + kRawOff + (T & 1) * kBBytes + (b * NW + wave) * 1024), 16, boff,
+                                               src * 1024, 0, 0);
+    }
+  };
+
+  f32x4 acc[TM][TN];
+  float unit[TN], mrun[TN];  // G != 0: what one unit of this lane's sums of strip c is worth; the largest scale so far
+#pragma unroll
+  for (int a = 0; a < TM; ++a)
+#pragma unroll
+    for (int c = 0; c < TN; ++c) acc[a][c] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int c = 0; c < TN; ++c) unit[c] = mrun[c] = 0.0f;
+  u32x4 af[TM], raw[TN], bf[2][TN];
+  const int arow = (wm * TM * 16 + lr) * 128;
+  const int apos = arow + ((kb ^ (lr & 7)) * 16);  // the second half's piece is four further on: XOR 64
+  const int bpos = (BITS == 8 ? kABytes : 0) + wn * TN * 1024 + lane * 16;
+  auto read_a = [&](const unsigned char* s, int h, int i) { af[i] = *reinterpret_cast<const u32x4*>(s + (h ? apos ^ 64 : apos) + i * 2048); };
+  auto read_b = [&](const unsigned char* s, int c) { raw[c] = *reinterpret_cast<const u32x4*>(s + bpos + c * 1024); };
+  // part d (of kDw) of B fragment c into set w: `step` is the 32-k step within the raw tile
+  auto dequant = [&](int w, int step, int c, int d) {
+    const uint32_t v = raw[c][step * kDw + d];
+    if constexpr (BITS == 8) {
+      // half a fragment: four codes, two dwords
+      const uint32_t w2[2] = {v, v};
+      const u32x4 o = DequantExact<DT, 8>::run(w2);
+      bf[w][c][d * 2] = o.x;
+      bf[w][c][d * 2 + 1] = o.y;
+    } else {
+      bf[w][c] = DequantExactFma<DT, 4>::run(&v);
+    }
+  };
+  constexpr int kUnits = TN * kDw;
+  float rho[TN];
+  // a group starts: the new unit of every column and what the sums are multiplied by (see gemm_dma_kernel)
+  auto new_units = [&](const unsigned char* s) {
+#pragma unroll
+    for (int c = 0; c < TN; ++c) {
+      const float sv = to_f32<DT>(*reinterpret_cast<const uint16_t*>(s + kScaleOff + wave * 256 + (c * 16 + lr) * 2));
+      mrun[c] = fmaxf(mrun[c], sv);
+      const float u0 = fmaxf(sv, mrun[c] * 0x1p-64f);
+      const float u = u0 < 0x1p-126f ? unit[c] : u0;
+      rho[c] = unit[c] == 0.0f ? 0.0f : (u == unit[c] ? 1.0f : unit[c] * __builtin_amdgcn_rcpf(u));
+      unit[c] = u;
+    }
+  };
+  // the MFMAs of A block a on operand set w; rescale: a group starts here
+  auto mfmas = [&](int w, int a, bool rescale) {
+#pragma unroll
+    for (int c = 0; c < TN; ++c) {
+      if (G != 0 && rescale) {
+        f32x4 t = acc[a][c];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) t[r] *= rho[c];
+        acc[a][c] = t;
+      }
+      acc[a][c] = mfma16<DT>(af[a], bf[w][c], acc[a][c]);
+    }
+  };
+
+  // ---- start: tiles 0 and 1 and the part of tile 2 that the first half below does not bring
+  constexpr int kFirst = (kLoadsEven * (kSpan - TM)) / kSpan;  // loads of a tile issued before its predecessor-but-two ends
+  if (BITS == 4) {  // the first part of raw tile 0, which no tile before tile 0 brings
+#pragma unroll
+    for (int i = 0; i < kBOdd; ++i)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rb[i], (lds_ptr_t)(smem + kRawOff + (i * NW + wave) * 1024), 16, boff, t0 / 2 * 1024, 0, 0);
+  }
+#pragma unroll
+  for (int i = 0; i < kLoadsEven; ++i) issue1(0, 0, false, i);
+#pragma unroll
+  for (int i = 0; i < kLoadsOdd; ++i) issue1(1, 1, true, i);
+#pragma unroll
+  for (int i = 0; i < kFirst; ++i) issue1(2, 2, false, i);
+  wait_vmcnt<kLoadsOdd + kFirst>();  // tile 0 has landed
+  __builtin_amdgcn_s_barrier();
+  if (STAMP) st_loop0 = st_prev = __builtin_readcyclecounter();
+#pragma unroll
+  for (int c = 0; c < TN; ++c) read_b(BITS == 8 ? smem : smem + kRawOff, c);
+#pragma unroll
+  for (int a = 0; a < TM; ++a) read_a(smem, 0, a);
+  if (G != 0) new_units(smem);
+#pragma unroll
+  for (int u = 0; u < kUnits; ++u) dequant(0, 0, u / kDw, u % kDw);
+
+  int st = 0;
+  // One k tile; ODD: its parity where that matters (int4's raw tiles, groups of 128).
+  auto tile = [&](auto odd_tile, int t) {
+    constexpr bool kOdd = decltype(odd_tile)::value;
+    // first step of this tile and of the next one within their raw tiles
+    constexpr int q0 = BITS == 4 && kOdd ? 2 : 0, q1 = BITS == 4 && !kOdd ? 2 : 0;
+    constexpr bool kNewB = BITS == 8 || kOdd;            // the next tile starts a raw tile
+    constexpr bool kGroup = G == 64 || (G == 128 && !kOdd);  // this tile starts a group
+    constexpr bool kNextGroup = G == 64 || (G == 128 && kOdd);
+    constexpr int kN2 = kOdd ? kLoadsOdd : kLoadsEven;   // loads of tile t + 2 (parity of t) ...
+    constexpr int kN3 = kOdd ? kLoadsEven : kLoadsOdd;   // ... and of tile t + 3
+    const unsigned char* s = smem + st * kStage;
+    const int st_n = st == 2 ? 0 : st + 1, st_p = st == 0 ? 2 : st - 1;
+    const unsigned char* n = smem + st_n * kStage;
+    // The loads of tile t + 3 are spread over the slots from barrier t to barrier t + 1: positions
+    // 0 .. TM - B0 - 1 behind the barrier, the others in the next tile's first half and before its barrier
+    auto share = [&](int pos, int loads) { return loads * pos / kSpan; };
+#pragma unroll
+    for (int i = 0; i < TM; ++i) {
+      __builtin_amdgcn_sched_barrier(0);
+      mfmas(0, i, kGroup);
+      read_a(s, 1, i);
+#pragma unroll
+      for (int u = kUnits * i / TM; u < kUnits * (i + 1) / TM; ++u) dequant(1, q0 + 1, u / kDw, u % kDw);
+#pragma unroll
+      for (int l = share(TM + i, kN2); l < share(i + 1 == TM ? kSpan : TM + i + 1, kN2); ++l) issue1(t + 2, st_p, kOdd, l);
+    }
+#pragma unroll
+    for (int i = 0; i < B0; ++i) {
+      __builtin_amdgcn_sched_barrier(0);
+      mfmas(1, i, false);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    unsigned long long st_a = 0, st_b = 0;
+    if (STAMP) {
+      __builtin_amdgcn_s_waitcnt(0x0070 | 0xF | (3 << 14));  // lgkmcnt(0)
+      st_a = __builtin_readcyclecounter();
+      wait_vmcnt<kN2>();
+      st_b = __builtin_readcyclecounter();
+    } else {
+      // lgkmcnt(0): this wavefront needs nothing more of the tile; tile t + 1 has landed
+      __builtin_amdgcn_s_waitcnt(0x0070 | (kN2 & 0xF) | ((kN2 >> 4) << 14));
+    }
+    __builtin_amdgcn_s_barrier();
+    if (STAMP) {
+      const unsigned long long st_c = __builtin_readcyclecounter();
+      st_work += st_a - st_prev;
+      st_loads += st_b - st_a;
+      st_bar += st_c - st_b;
+      st_prev = st_c;
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    const unsigned char* nb = BITS == 8 ? n : smem + kRawOff + (((t + 1) / 2) & 1) * kBBytes;
+    if (kNewB) {
+#pragma unroll
+      for (int c = 0; c < TN; ++c) read_b(nb, c);
+    }
+    constexpr int S = TM - B0;  // slots behind the barrier; reads and conversions from the second one on
+#pragma unroll
+    for (int i = 0; i < S; ++i) {
+      mfmas(1, B0 + i, false);
+      if (kNextGroup && i == (S > 1 ? 1 : 0)) new_units(n);
+#pragma unroll
+      for (int a = (S > 1 && i > 0 ? TM * (i - 1) / (S - 1) : 0); a < (S > 1 ? TM * i / (S - 1) : TM); ++a) read_a(n, 0, a);
+#pragma unroll
+      for (int u = (S > 1 && i > 0 ? kUnits * (i - 1) / (S - 1) : 0); u < (S > 1 ? kUnits * i / (S - 1) : kUnits); ++u) dequant(0, q1, u / kDw, u % kDw);
+#pragma unroll
+      for (int l = share(i * TM / S, kN3); l < share((i + 1) * TM / S, kN3); ++l) issue1(t + 3, st, !kOdd, l);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    st = st_n;
+  };
+  if constexpr (BITS == 4 || G == 128) {
+    for (int t = 0; t < nt; t += 2) {
+      tile(std::false_type(), t);
+      if (BITS == 4 || t + 1 < nt) tile(std::true_type(), t + 1);  // int4: K is made of whole raw tiles
+    }
+  } else {
+    for (int t = 0; t < nt; ++t) tile(std::false_type(), t);
+  }
+  __builtin_amdgcn_s_waitcnt(0x0070);
+  __builtin_amdgcn_s_barrier();  // the spare loads are done and every wavefront has stopped reading
+  unsigned long long st_loop1 = 0;
+  if (STAMP) st_loop1 = __builtin_readcyclecounter();
+
+  // ---- epilogue: scale, bias, cast; 32-row slabs leave through LDS as 16-byte stores ----
+  // accumulator element r of lane l is row 4 * (l / 16) + r, column l % 16 of its block
+  int etid = threadIdx.x;
+  asm volatile("" : "+v"(etid));  // nothing of the epilogue's addresses is kept in registers during the loop
+  const int el = etid & 63, ec = el & 15, er = (el >> 4) * 4;
+  const uint16_t* bias = p.bias;
+  const int n_hi = p.strip_hi * kStripCols;
+  float sc[TN], bv[TN];
+#pragma unroll
+  for (int c = 0; c < TN; ++c) {
+    int n = strip_col(c) + ec;
+    const int last = SWI && c >= TN / 2 ? N : n_hi;
+    n = n < last ? n : last - 1;
+    sc[c] = G != 0 ? unit[c] : to_f32<DT>(scale[n]);
+    bv[c] = bias != nullptr && p.nsplit == 1 ? to_f32<DT>(bias[n]) : 0.0f;
+  }
+  constexpr int kOut = SWI ? TN / 2 : TN;  // strips a wavefront writes
+  const int col0 = (strip0 + wn * kOut) * kStripCols;
+  const int row_w = m0 + wm * TM * 16;     // first row of this wavefront
+  constexpr int kSlabRows = TM >= 2 ? 32 : 16, kPer = kSlabRows / 16;
+  if (SWI == 0 && (p.out_f32 || p.nsplit > 1)) {
+    // fp32 results (verification mode) or the sums of this run of k tiles, kept compact: a row is as long as the
+    // launch has columns
+    const int64_t ld = p.nsplit > 1 ? static_cast<int64_t>(p.strip_hi - p.strip_lo) * kStripCols : N;
+    const int nc0 = p.nsplit > 1 ? p.strip_lo * kStripCols : 0;
+    float* outf = static_cast<float*>(p.out) + (p.nsplit > 1 ? static_cast<int64_t>(split) * M * ld : 0);
+    constexpr int kRow = TN * 16 + 4, kPieces = kSlabRows * TN * 4;
+    static_assert(NW * kSlabRows * kRow * 4 <= kLds, "slabs must fit in the stages");
+    float* slab = reinterpret_cast<float*>(smem) + wave * kSlabRows * kRow;
+#pragma unroll
+    for (int a = 0; a < TM; a += kPer) {
+#pragma unroll
+      for (int h = 0; h < kPer; ++h)
+#pragma unroll
+        for (int c = 0; c < TN; ++c)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            const float v = acc[a + h][c][r] * sc[c] + bv[c];
+            slab[(h * 16 + er + r) * kRow + c * 16 + ec] = p.nsplit > 1 ? v : act_apply(v, p.act);
+          }
+      __builtin_amdgcn_wave_barrier();
+      for (int q = el; q < kPieces; q += 64) {
+        const int r = q / (TN * 4), cc = q % (TN * 4), m = row_w + a * 16 + r, n = col0 + cc * 4;
+        const f32x4 v = *reinterpret_cast<const f32x4*>(&slab[r * kRow + cc * 4]);
+        if (m < M && n < n_hi) *reinterpret_cast<f32x4*>(outf + static_cast<int64_t>(m) * ld + (n - nc0)) = v;
+      }
+      __builtin_amdgcn_wave_barrier();
+    }
+    return;
+  }
+  uint16_t* out = static_cast<uint16_t*>(p.out);
+  constexpr int kRow = kOut * 16 + 8, kPieces = kSlabRows * kOut * 2;
+  static_assert(NW * kSlabRows * kRow * 2 <= kLds, "slabs must fit in the stages");
+  uint16_t* slab = reinterpret_cast<uint16_t*>(smem) + wave * kSlabRows * kRow;
+  const int ld = SWI ? N / 2 : N;
+#pragma unroll
+  for (int a = 0; a < TM; a += kPer) {
+#pragma unroll
+    for (int h = 0; h < kPer; ++h)
+#pragma unroll
+      for (int c = 0; c < kOut; ++c)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          float v = acc[a + h][c][r] * sc[c] + bv[c];
+          if (SWI) {
+            float u = acc[a + h][TN / 2 + c][r] * sc[TN / 2 + c] + bv[TN / 2 + c];
+            if (SWI == 2) {  // as if fc1 had been written out in T and read back
+              v = to_f32<DT>(cast_out<DT>(v));
+              u = to_f32<DT>(cast_out<DT>(u));
+            }
+            v = act_swiglu(v, u);
+          } else {
+            v = act_apply(v, p.act);
+          }
+          slab[(h * 16 + er + r) * kRow + c * 16 + ec] = cast_out<DT>(v);
+        }
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int q = el; q < kPieces; q += 64) {
+      const int r = q / (kOut * 2), cc = q % (kOut * 2), m = row_w + a * 16 + r, n = col0 + cc * 8;
+      const u32x4 v = *reinterpret_cast<const u32x4*>(&slab[r * kRow + cc * 8]);
+      if (m < M && n < n_hi) *reinterpret_cast<u32x4*>(out + static_cast<int64_t>(m) * ld + n) = v;
+    }
+    __builtin_amdgcn_wave_barrier();
+  }
+  if (STAMP && el == 0 && p.stamps != nullptr) {
+    unsigned long long* o = p.stamps + (static_cast<size_t>(blockIdx.x) * NW + wave) * 8;
+    const unsigned long long st_end = __builtin_readcyclecounter();
+    o[0] = st_loop0 - st_entry;   // entry to the first tile's barrier
+    o[1] = st_work;               // between the barriers: MFMAs and everything issued among them
+    o[2] = st_loads;              // waiting for this wavefront's own tile loads
+    o[3] = st_bar;                // waiting for the other wavefronts
+    o[4] = st_loop1 - st_prev;    // the last tile's tail and the closing barrier
+    o[5] = st_end - st_loop1;     // epilogue
+    o[6] = st_end - st_entry;     // all of it
+    o[7] = static_cast<unsigned long long>(nt);
+  }
+#endif
+}
+
+template <int DT, int BITS, int G, int WM, int WN, int TM, int TN, int SWI, bool STAMP>
+__global__ __launch_bounds__(512) void gemm_dma_kernel_wide(const DmaParams p) {
+  int bx, by, split;
+  place_of_block(p, &bx, &by, &split);
+  wide_tile<DT, BITS, G, WM, WN, TM, TN, SWI, STAMP>(p, bx, by, split);
+}
+
+// Eight wavefronts side by side, TM 16-row blocks x 32 columns each.
+template <int DT, int BITS, int G, int TM, int SWI, bool STAMP = false>
+void launch(const DmaParams& p, hipStream_t stream) {
+  constexpr size_t lds = wide_lds_bytes<BITS, G, 1, 8, TM, 2>();
+  auto kern = gemm_dma_kernel_wide<DT, BITS, G, 1, 8, TM, 2, SWI, STAMP>;
+  static std::atomic<uint32_t> configured{0};  // per instantiation
+  allow_lds(reinterpret_cast<const void*>(kern), lds, configured);
+  kern<<<dim3(static_cast<unsigned>(p.nbx * p.nby * p.nsplit)), dim3(512), lds, stream>>>(p);
+}
+
+template <int DT, int BITS, int G>
+void launch_tile(const DmaParams& p, WideTile tile, int swi, hipStream_t stream) {
+  if (tile == WideTile::kHalf) {
+    if (swi) launch<DT, BITS, G, 8, 1>(p, stream);
+    else launch<DT, BITS, G, 8, 0>(p, stream);
+    return;
+  }
+  if constexpr (G == 0) {
+    if (swi) launch<DT, BITS, G, 16, 1>(p, stream);
+    else launch<DT, BITS, G, 16, 0>(p, stream);
+  }
+}
+
+template <int DT, int BITS>
+void launch_group(const DmaParams& p, int group, WideTile tile, int swi, hipStream_t stream) {
+  if (group == 0) launch_tile<DT, BITS, 0>(p, tile, swi, stream);
+  else if (group == 64) launch_tile<DT, BITS, 64>(p, tile, swi, stream);
+  else launch_tile<DT, BITS, 128>(p, tile, swi, stream);
+}
+
+}  // namespace
+
+#if defined(WOL_GEMM_F16_UNIT)
+#define WOL_WIDE_LAUNCH launch_wide_f16
+#else
+#define WOL_WIDE_LAUNCH launch_wide_bf16
+#endif
+void WOL_WIDE_LAUNCH(const DmaParams& p, int bits, int group, WideTile tile, int swi, hipStream_t stream) {
+  if (bits == 8) launch_group<WOL_GEMM_DTYPE, 8>(p, group, tile, swi, stream);
+  else launch_group<WOL_GEMM_DTYPE, 4>(p, group, tile, swi, stream);
+}
+
+#if !defined(WOL_GEMM_F16_UNIT)
+
+// The prefill GEMM's 256 x 256 int8 per-channel bf16 launch with cycle stamps
+// (M and N multiples of 256, K a multiple of 64 and at least 192): out [M, N]
+// bf16, stamps [(M / 256) * (N / 256)][8 wavefronts][8] counts.
+int launch_prefill_phases(const void* x, const void* codes, const void* scale, int64_t M, int64_t K, int64_t N,
+                          void* out, unsigned long long* stamps, hipStream_t stream) {
+  DmaParams p{};
+  p.x = static_cast<const uint16_t*>(x);
+  p.codes = static_cast<const uint8_t*>(codes);
+  p.scale = static_cast<const uint16_t*>(scale);
+  p.out = out;
+  p.M = static_cast<int>(M); p.K = static_cast<int>(K); p.N = static_cast<int>(N);
+  p.strip_hi = static_cast<int>(N / kStripCols);
+  p.nbx = static_cast<int>(N / 256);
+  p.nby = static_cast<int>(M / 256);
+  p.tiles_per_split = static_cast<int>(K / 64);
+  p.nsplit = 1;
+  p.act = WOL_ACT_NONE;
+  p.stamps = stamps;
+  launch<WOL_DTYPE_BF16, 8, 0, 16, 0, true>(p, stream);
+  return check_launch();
+}
+
+#endif  // !WOL_GEMM_F16_UNIT
+
+}  // namespace wol
