@@ -1443,9 +1443,7 @@ void launch_fast(const Args& a) {
   const TailPlan t = plan_tail(a.M, a.K, (nstrips - lo) * kStripCols, kHalfRows, kHalfCols, BITS == 8 ? 64 : 128,
                                a.ws != nullptr ? a.ws_bytes : 0);
   const int mid = lo + t.full_tiles * (kHalfCols / kStripCols);  // strips [lo, mid) unsplit, [mid, nstrips) in t.ns runs
-  if constexpr (G == 0) launch_wide<DT>(a, BITS, G, WideTile::kWhole, 0, 0, lo, 1);
-  else if constexpr (BITS == 8) launch_dma<DT, BITS, G, 0, 2, 4, 4, 2, 3, 0, true>(a, 0, lo, 1);
-  else launch_dma<DT, BITS, G, 0, 2, 4, 4, 2, kHalfDeepStages + 3, 0, true>(a, 0, lo, 1);
+  launch_wide<DT>(a, BITS, G, WideTile::kWhole, 0, 0, lo, 1);
   launch_wide<DT>(a, BITS, G, WideTile::kHalf, 0, lo, mid, 1);
   launch_wide<DT>(a, BITS, G, WideTile::kHalf, 0, mid, nstrips, t.ns);
 }
@@ -1757,10 +1755,8 @@ void launch_swiglu_gemm(const Args& a) {
   // whole tiles, or half-size ones where their rounds, at 0.6 of a whole tile's, are done sooner
   const int cus = num_cus(), cols = (a.N + 255) / 256;
   const int big = cols * ((a.M + 255) / 256), half = cols * ((a.M + 127) / 128);
-  if ((big + cus - 1) / cus >= 0.6 * ((half + cus - 1) / cus)) launch_wide<DT>(a, BITS, G, WideTile::kHalf, 1, 0, gate_strips, 1);
-  else if constexpr (G == 0) launch_wide<DT>(a, BITS, G, WideTile::kWhole, 1, 0, gate_strips, 1);
-  else if constexpr (BITS == 8) launch_dma<DT, 8, G, 0, 2, 4, 4, 2, 3, 1, true>(a, 0, gate_strips, 1);
-  else launch_dma<DT, 4, G, 0, 2, 4, 4, 2, kHalfDeepStages + 3, 1, true>(a, 0, gate_strips, 1);
+  const WideTile tile = (big + cus - 1) / cus >= 0.6 * ((half + cus - 1) / cus) ? WideTile::kHalf : WideTile::kWhole;
+  launch_wide<DT>(a, BITS, G, tile, 1, 0, gate_strips, 1);
 }
 template <int DT, int BITS>
 void launch_swiglu_gemm_g(const Args& a) {

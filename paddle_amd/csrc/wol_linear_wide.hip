@@ -1,4 +1,5 @@
-// The tiles of 128 and 256 rows of weight_only_linear's GEMM (more than 64 rows, K made of whole k tiles), for bf16;
+// The tiles of 128 and 256 rows of weight_only_linear's GEMM (more than 64 rows, K made of whole k tiles), for bf16:
+// gemm_dma_kernel_wide and, for group-wise scales on 256 x 256 tiles, gemm_dma_kernel_tall.
 // wol_linear_wide_f16.hip compiles the same source for fp16.  This file is built with the instruction scheduler in front
 // of register allocation switched off (build.sh): the loops below give every instruction its place, and that pass, which
 // does not see why, costs up to 40 registers and then spills (int4 per channel: 240 registers without it, 256 and
@@ -456,6 +457,300 @@ __device__ __forceinline__ void wide_tile(const DmaParams& p, int bx, int by, in
 #endif
 }
 
+// gemm_dma_kernel_tall: group-wise scales on 256 x 256 tiles.  Eight wavefronts of 256 rows x 32 columns each,
+// v_mfma_f32_32x32x16, sums in units of the current group's scale as above.
+//
+// What bounds it.  Rescaling costs a VALU instruction per accumulator register and group, 4 per 32x32x16 MFMA with
+// groups of 64; with the dequantiser's 1.75 (3.5 with two rows of wavefronts) and the MFMA's own two slots that is 33
+// cycles of issue per 32-cycle MFMA.  The 16x16x32 form would need 42 for the same work, which is why this kernel keeps
+// the larger one although it burns more power per product.
+//
+// Order.  What matters is that the VALU work is even over the tile.  The B fragments of a k tile (four 16-k slices of one
+// 32-column block) stay in registers for the whole tile and A streams past them: blocks in pairs, eight MFMAs a pair,
+// and behind every MFMA the A fragment it has used is read again for the next pair, and four accumulators of the next
+// pair are rescaled.  The next tile's codes and scales are read at the start of a tile and converted during its second and
+// third pair, so they travel one tile ahead of the activations: group g of loads brings the activations of tile g and
+// the codes and scales of tile g + 1.  The barrier that frees the tile's stage sits after the second MFMA of the last
+// pair, when all of the tile's reads have long arrived.
+//
+// A rows are XORed with (row % 8) ^ (row / 8 % 2): the phases of ds_read_b128 over the 32 rows of a fragment.
+//
+// bf16: K = 4096, N = 22016, M = 2048 int8 g64 395 -> 343 us against 32x32x16 tiles of two by four wavefronts; M = 8192,
+// N = 4096 int8 g128 (fp16) 244 -> 227, int4 g128 247 -> 224 (1.23 PFLOP/s), int4 g64 278 -> 238; swiglu, M = 1237, N =
+// 22016 int8 g64 255 -> 221, int4 g128 241 -> 204.  On gemm_dma_kernel_wide's 256-row tiles: int8 g64 M = 2048, N = 8192
+// 128 against 126, swiglu 237 against 220, int4 spills.
+template <int BITS>
+constexpr size_t tall_lds_bytes() {
+  return 3 * (32768 + (BITS == 8 ? 16384 : 0) + 2048) + (BITS == 4 ? 32768 : 0);
+}
+
+template <int DT, int BITS, int G, int SWI>
+__global__ __launch_bounds__(512) void gemm_dma_kernel_tall(const DmaParams p) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  constexpr int NW = 8, BM = 256, kStrips = 16;
+  constexpr int kABytes = 32768, kBBytes = 16384;
+  constexpr int kScaleOff = kABytes + (BITS == 8 ? kBBytes : 0);
+  constexpr int kStage = kScaleOff + 2048;
+  constexpr int kRawOff = 3 * kStage;
+  constexpr int kLds = static_cast<int>(tall_lds_bytes<BITS>());
+  constexpr int kB = BITS == 8 ? 2 : 1;  // B loads of a group
+  constexpr int kLoads = 1 + 4 + kB;
+  constexpr int kFirst = 2;
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  const int tid = threadIdx.x;
+  const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int j = lane & 15, sp = (lane >> 4) & 1, b = lane >> 5, r32 = lane & 31;
+  int bx, by, split;
+  place_of_block(p, &bx, &by, &split);
+  const int K = p.K, N = p.N, M = p.M, m0 = by * BM;
+  const int strip0 = p.strip_lo + bx * (SWI ? kStrips / 2 : kStrips);
+  const int up_strips = N / 2 / kStripCols;
+  const int t0 = split * p.tiles_per_split;
+  const int nt = (K / 64 - t0) < p.tiles_per_split ? (K / 64 - t0) : p.tiles_per_split;
+  const int rows = M - m0 < BM ? M - m0 : BM;
+  const int sbytes = static_cast<int>(strip_bytes(K, BITS));
+  const int left = p.strip_hi - strip0, own = SWI ? kStrips / 2 : kStrips, strips = left < own ? left : own;
+  __amdgpu_buffer_rsrc_t ra[4], rb[2];
+#pragma unroll
+  for (int c = 0; c < 4; ++c) {
+    const int r0 = (c * NW + wave) * 8, nr = rows - r0 > 8 ? 8 : (rows > r0 ? rows - r0 : 0);
+    ra[c] = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(p.x + static_cast<int64_t>(nr > 0 ? m0 + r0 : m0) * K), 0, nr * K * 2, 0x00020000);
+  }
+#pragma unroll
+  for (int c = 0; c < 2; ++c) {
+    const int L = c * NW + wave, st = SWI ? L / 2 : L;
+    const int64_t first = st < strips ? strip0 + st + (SWI && L % 2 ? up_strips : 0) : 0;
+    rb[c] = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(p.codes + first * sbytes), 0, st < strips ? sbytes : 0, 0x00020000);
+  }
+  const uint32_t aoff = static_cast<uint32_t>((lane / 8) * K + ((lane ^ (lane >> 3) ^ (wave & 1)) & 7) * 8) * 2, boff = lane * 16;
+  // column of position v (0 .. 31) of this wavefront
+  auto column = [&](int v) {
+    return SWI ? (strip0 + wave) * kStripCols + v % 16 + (v >= 16 ? N / 2 : 0) : (strip0 + wave * 2) * kStripCols + v;
+  };
+  int scol;
+  {
+    const int v = 2 * lane < 32 ? 2 * lane : 0;
+    scol = column(v);
+    const int last = SWI ? (v < 16 ? N / 2 : N) : p.strip_hi * kStripCols;
+    scol = scol < last ? scol : last - 2;
+  }
+  constexpr int kGShift = G == 128 ? 7 : 6;
+  auto clampt = [&](int t) { return t0 + (t < nt ? t : nt - 1); };
+  auto issue_s = [&](int t, int st) {
+    const int64_t row = static_cast<int64_t>(clampt(t)) * 64 >> kGShift;
+    __builtin_amdgcn_global_load_lds(p.scale + row * N + scol, (lds_ptr_t)(smem + st * kStage + kScaleOff + wave * 256), 4, 0, 0);
+  };
+  auto issue_b = [&](int t, int st, int c) {  // int8: tile t's codes
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rb[c], (lds_ptr_t)(smem + st * kStage + kABytes + (c * NW + wave) * 1024), 16, boff, clampt(t) * 1024, 0, 0);
+  };
+  auto issue_raw = [&](int T, int c) {  // int4: half c of raw tile T
+    const int src = t0 / 2 + (2 * T < nt ? T : nt / 2 - 1);
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rb[c], (lds_ptr_t)(smem + kRawOff + (T & 1) * kBBytes + (c * NW + wave) * 1024), 16, boff, src * 1024, 0, 0);
+  };
+  // load i of group g: scales and codes of tile g + 1, activations of tile g; st: g % 3, odd: parity of g
+  auto issue = [&](int g, int st, bool odd, int i) {
+    const int st1 = st == 2 ? 0 : st + 1;
+    if (i == 0) issue_s(g + 1, st1);
+    else if (i <= 4)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(ra[i - 1], (lds_ptr_t)(smem + st * kStage + ((i - 1) * NW + wave) * 1024), 16, aoff, clampt(g) * 128, 0, 0);
+    else if (BITS == 8) issue_b(g + 1, st1, i - 5);
+    else issue_raw(odd ? (g + 1) / 2 : (g + 2) / 2, odd ? 1 : 0);
+  };
+
+  f32x16 acc[8];
+#pragma unroll
+  for (int a = 0; a < 8; ++a)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc[a][r] = 0.0f;
+  float unit = 0.0f, mrun = 0.0f, rho = 0.0f;
+  uint32_t sraw = 0;
+  u32x4 af[8], raw[2], bf[2][4];
+  const int apos = r32 * 128 + ((b ^ a_swizzle<8>(lane & 15)) * 16);
+  const int bpos = (BITS == 8 ? kABytes : 0) + (wave * 2 + sp) * 1024 + (j + 16 * b) * 16;
+  auto read_a = [&](const unsigned char* s, int blk, int i) {  // i = which * 4 + q
+    af[i] = *reinterpret_cast<const u32x4*>(s + (apos ^ ((i & 3) * 32)) + blk * 4096);
+  };
+  auto read_b = [&](const unsigned char* s) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h) raw[h] = *reinterpret_cast<const u32x4*>(s + bpos + h * 512);
+  };
+  // piece d of B fragment q of a tile (int8: halves of two) into set w; base: the tile's first 32-k step in its raw tile
+  auto dequant = [&](int w, int base, int q, int d) {
+    if constexpr (BITS == 8) {
+      const uint32_t v = raw[q & 1][(q >> 1) * 2 + d];
+      const uint32_t w2[2] = {v, v};
+      const u32x4 o = DequantExact<DT, 8>::run(w2);
+      bf[w][q][d * 2] = o.x;
+      bf[w][q][d * 2 + 1] = o.y;
+    } else {
+      const uint32_t v = raw[q & 1][base + (q >> 1)];
+      bf[w][q] = DequantExactFma<DT, 4>::run(&v);
+    }
+  };
+  auto new_unit = [&]() {
+    const float sv = to_f32<DT>(static_cast<uint16_t>(sraw));
+    mrun = fmaxf(mrun, sv);
+    const float u0 = fmaxf(sv, mrun * 0x1p-64f);
+    const float u = u0 < 0x1p-126f ? unit : u0;
+    const float ratio = unit * __builtin_amdgcn_rcpf(u);
+    rho = unit == 0.0f ? 0.0f : (u == unit ? 1.0f : ratio);
+    unit = u;
+  };
+  auto read_s = [&](int st) { sraw = *reinterpret_cast<const uint16_t*>(smem + st * kStage + kScaleOff + wave * 256 + r32 * 2); };
+
+  // ---- start: codes and scales of tile 0, groups 0 and 1
+  issue_s(0, 0);
+#pragma unroll
+  for (int c = 0; c < 2; ++c) {
+    if (BITS == 8) issue_b(0, 0, c);
+    else issue_raw(0, c);
+  }
+#pragma unroll
+  for (int i = 0; i < kLoads; ++i) issue(0, 0, false, i);
+#pragma unroll
+  for (int i = 0; i < kLoads; ++i) issue(1, 1, true, i);
+  wait_vmcnt<kLoads>();
+  __builtin_amdgcn_s_barrier();
+  read_b(BITS == 8 ? smem : smem + kRawOff);
+  read_s(0);
+#pragma unroll
+  for (int i = 0; i < 8; ++i) read_a(smem, i >> 2, i);
+  new_unit();
+#pragma unroll
+  for (int q = 0; q < 4; ++q)
+#pragma unroll
+    for (int d = 0; d < (BITS == 8 ? 2 : 1); ++d) dequant(0, 0, q, d);
+  // group 2 brings the scales and codes of tile 3 to where tile 0's lie: they have been read by everybody first
+  __builtin_amdgcn_s_waitcnt(0x0070 | 0xF | (3 << 14));  // lgkmcnt(0)
+  __builtin_amdgcn_s_barrier();
+#pragma unroll
+  for (int i = 0; i < kFirst; ++i) issue(2, 2, false, i);
+  int st = 0;
+  auto tile = [&](auto odd_tile, int t) {
+    constexpr bool kOdd = decltype(odd_tile)::value;
+    constexpr int w = kOdd ? 1 : 0;
+    constexpr bool kGroup = G == 64 || !kOdd, kNextGroup = G == 64 || kOdd;
+    constexpr bool kNewB = BITS == 8 || kOdd;
+    constexpr int base = BITS == 4 && !kOdd ? 2 : 0;  // of tile t + 1
+    const int st_n = st == 2 ? 0 : st + 1, st_p = st == 0 ? 2 : st - 1;
+    const unsigned char* s = smem + st * kStage;
+    const unsigned char* n = smem + st_n * kStage;
+#pragma unroll
+    for (int pr = 0; pr < 4; ++pr) {
+#pragma unroll
+      for (int m = 0; m < 8; ++m) {
+        const int q = m >> 1, which = m & 1, a = 2 * pr + which;
+        acc[a] = mfma32<DT>(af[which * 4 + q], bf[w][q], acc[a]);
+        if (pr < 3) read_a(s, 2 * (pr + 1) + which, which * 4 + q);
+        if (pr == 0 && m == 0) {
+          if (kNextGroup) read_s(st_n);
+          if (kNewB) read_b(BITS == 8 ? n : smem + kRawOff + (((t + 1) / 2) & 1) * kBBytes);
+        }
+        if (pr == 3 && m == 1) {
+          __builtin_amdgcn_sched_barrier(0);
+          __builtin_amdgcn_s_waitcnt(0x0070 | kLoads);  // this tile's reads are done, group t + 1 has landed
+          __builtin_amdgcn_s_barrier();
+          __builtin_amdgcn_sched_barrier(0);
+          read_a(n, 0, 0);
+          read_a(n, 1, 4);
+        }
+        if (pr == 3 && m > 1) read_a(n, which, which * 4 + q);
+        // rescale the next pair's sums, four elements per MFMA
+        if (pr < 3 ? kGroup : kNextGroup) {
+          const int na = 2 * ((pr + 1) & 3) + (m >> 2);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) acc[na][(m & 3) * 4 + e] *= rho;
+        }
+        if (kNextGroup && pr == 2 && m == 7) new_unit();
+        if (pr == 1 || pr == 2) {
+          const int k = (pr - 1) * 8 + m;  // 0 .. 15
+          if (BITS == 8 && k % 2 == 1) dequant(w ^ 1, base, k / 4, (k / 2) % 2);
+          if (BITS == 4 && k % 4 == 1) dequant(w ^ 1, base, k / 4, 0);
+        }
+        if (pr == 3 && (m == 3 || m == 6)) issue(t + 3, st, !kOdd, m / 3 - 1);
+        if (pr < 3 && m % 4 == 3 && kFirst + pr * 2 + m / 4 < kLoads) issue(t + 2, st_p, kOdd, kFirst + pr * 2 + m / 4);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+    st = st_n;
+  };
+  for (int t = 0; t < nt; t += 2) {
+    tile(std::false_type(), t);
+    if (BITS == 4 || t + 1 < nt) tile(std::true_type(), t + 1);
+  }
+  __builtin_amdgcn_s_waitcnt(0x0070);
+  __builtin_amdgcn_s_barrier();
+
+  // ---- epilogue
+  int etid = threadIdx.x;
+  asm volatile("" : "+v"(etid));
+  const int el = etid & 63, ec = el & 31, eb = el >> 5;
+  const int n_hi = p.strip_hi * kStripCols;
+  float sc, bv;
+  {
+    int n = column(ec);
+    const int last = SWI ? (ec < 16 ? N / 2 : N) : n_hi;
+    n = n < last ? n : last - 1;
+    sc = unit;
+    bv = p.bias != nullptr && p.nsplit == 1 ? to_f32<DT>(p.bias[n]) : 0.0f;
+  }
+  if (SWI == 0 && (p.out_f32 || p.nsplit > 1)) {
+    const int64_t ld = p.nsplit > 1 ? static_cast<int64_t>(p.strip_hi - p.strip_lo) * kStripCols : N;
+    const int nc0 = p.nsplit > 1 ? p.strip_lo * kStripCols : 0;
+    float* outf = static_cast<float*>(p.out) + (p.nsplit > 1 ? static_cast<int64_t>(split) * M * ld : 0);
+    constexpr int kRow = 256 + 4;
+    static_assert(128 * kRow * 4 <= kLds, "half the tile must fit in the stages");
+    float* slab = reinterpret_cast<float*>(smem);
+#pragma unroll
+    for (int hf = 0; hf < 2; ++hf) {
+      __syncthreads();
+#pragma unroll
+      for (int a = 0; a < 4; ++a)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          const float v = acc[hf * 4 + a][r] * sc + bv;
+          slab[(a * 32 + 8 * (r / 4) + 4 * eb + r % 4) * kRow + wave * 32 + ec] = p.nsplit > 1 ? v : act_apply(v, p.act);
+        }
+      __syncthreads();
+      for (int q = etid; q < 128 * 64; q += 512) {
+        const int r = q / 64, cc = q % 64, m = m0 + hf * 128 + r, n = strip0 * kStripCols + cc * 4;
+        const f32x4 v = *reinterpret_cast<const f32x4*>(&slab[r * kRow + cc * 4]);
+        if (m < M && n < n_hi) *reinterpret_cast<f32x4*>(outf + static_cast<int64_t>(m) * ld + (n - nc0)) = v;
+      }
+    }
+    return;
+  }
+  uint16_t* out = static_cast<uint16_t*>(p.out);
+  constexpr int kCols = SWI ? 128 : 256, kRow = kCols + 8;
+  static_assert(256 * kRow * 2 <= kLds, "the tile must fit in the stages");
+  uint16_t* slab = reinterpret_cast<uint16_t*>(smem);
+#pragma unroll
+  for (int a = 0; a < 8; ++a) {
+    if constexpr (SWI != 0) {
+#pragma unroll
+      for (int r = 0; r < 16; r += 2) {
+        const float u0 = acc[a][r] * sc + bv, u1 = acc[a][r + 1] * sc + bv;
+        // lanes of a gate strip take row r, those of an up strip row r + 1, gate and up of it side by side
+        const auto sw = __builtin_amdgcn_permlane16_swap(__float_as_uint(u0), __float_as_uint(u1), false, false);
+        float g = __uint_as_float(sw[0]), u = __uint_as_float(sw[1]);
+        slab[(a * 32 + 8 * (r / 4) + 4 * eb + r % 4 + ((el >> 4) & 1)) * kRow + wave * 16 + (el & 15)] = cast_out<DT>(act_swiglu(g, u));
+      }
+    } else {
+#pragma unroll
+      for (int r = 0; r < 16; ++r)
+        slab[(a * 32 + 8 * (r / 4) + 4 * eb + r % 4) * kRow + wave * 32 + ec] = cast_out<DT>(act_apply(acc[a][r] * sc + bv, p.act));
+    }
+  }
+  __syncthreads();
+  const int ld = SWI ? N / 2 : N;
+  for (int q = etid; q < 256 * kCols / 8; q += 512) {
+    const int r = q / (kCols / 8), cc = q % (kCols / 8), m = m0 + r, n = strip0 * kStripCols + cc * 8;
+    const u32x4 v = *reinterpret_cast<const u32x4*>(&slab[r * kRow + cc * 8]);
+    if (m < M && n < n_hi) *reinterpret_cast<u32x4*>(out + static_cast<int64_t>(m) * ld + n) = v;
+  }
+#endif
+}
+
 template <int DT, int BITS, int G, int WM, int WN, int TM, int TN, int SWI, bool STAMP>
 __global__ __launch_bounds__(512) void gemm_dma_kernel_wide(const DmaParams p) {
   int bx, by, split;
@@ -473,6 +768,15 @@ void launch(const DmaParams& p, hipStream_t stream) {
   kern<<<dim3(static_cast<unsigned>(p.nbx * p.nby * p.nsplit)), dim3(512), lds, stream>>>(p);
 }
 
+template <int DT, int BITS, int G, int SWI>
+void launch_tall(const DmaParams& p, hipStream_t stream) {
+  constexpr size_t lds = tall_lds_bytes<BITS>();
+  auto kern = gemm_dma_kernel_tall<DT, BITS, G, SWI>;
+  static std::atomic<uint32_t> configured{0};  // per instantiation
+  allow_lds(reinterpret_cast<const void*>(kern), lds, configured);
+  kern<<<dim3(static_cast<unsigned>(p.nbx * p.nby * p.nsplit)), dim3(512), lds, stream>>>(p);
+}
+
 template <int DT, int BITS, int G>
 void launch_tile(const DmaParams& p, WideTile tile, int swi, hipStream_t stream) {
   if (tile == WideTile::kHalf) {
@@ -483,6 +787,9 @@ void launch_tile(const DmaParams& p, WideTile tile, int swi, hipStream_t stream)
   if constexpr (G == 0) {
     if (swi) launch<DT, BITS, G, 16, 1>(p, stream);
     else launch<DT, BITS, G, 16, 0>(p, stream);
+  } else {
+    if (swi) launch_tall<DT, BITS, G, 1>(p, stream);
+    else launch_tall<DT, BITS, G, 0>(p, stream);
   }
 }
 
