@@ -66,6 +66,10 @@ enum class WideTile {
 // those of the gate half).
 void launch_wide_bf16(const DmaParams& p, int bits, int group, WideTile tile, int swi, hipStream_t stream);
 void launch_wide_f16(const DmaParams& p, int bits, int group, WideTile tile, int swi, hipStream_t stream);
+// The grouped GEMM over experts on tiles of up to 256 rows x 256 columns (narrow: 128); p.moe_table is that of
+// moe_plan_kernel<true>.  swiglu: of the product rounded to T, p.out is [rows, N / 2].
+void launch_experts_bf16(const DmaParams& p, int bits, bool narrow, bool swiglu, unsigned blocks, hipStream_t stream);
+void launch_experts_f16(const DmaParams& p, int bits, bool narrow, bool swiglu, unsigned blocks, hipStream_t stream);
 
 namespace {
 

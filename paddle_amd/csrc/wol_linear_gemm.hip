@@ -1015,42 +1015,6 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_dma_kernel(const DmaParams 
   dma_tile<DT, BITS, G, OFFS, WM, WN, TM, TN, STAGES, SWI, RESC, STAMP, false>(p, TilePlace{});
 }
 
-// The grouped GEMM over experts with many rows each: row tiles of up to four
-// 64-row units (256 rows), as many units as the tile has rows for.  A tile's
-// MFMAs, activation loads and operand reads follow its height, so an expert
-// whose row count is no multiple of the tile pays for 64-row padding only.
-// Workgroups are handed out expert by expert, column tile by column tile, all
-// row tiles of the expert next to each other, and that sequence is cut into
-// eight equal pieces, one per XCD: an expert's row tiles meet its weights in
-// one L2 while they are there, and the XCDs stay evenly loaded however the
-// rows are spread over the experts.
-// moe_ffn, 8 experts, hidden 4096, fc1 width 28672, rows spread unequally,
-// whole call, against whole tiles of 256 or 128 rows in runs of the average
-// expert's tiles per XCD: 4096 rows int4 2264 -> 1684 us, int8 2090 -> 1551;
-// 2048 rows int4 1311 -> 966, int8 1325 -> 892; 1024 rows 651 -> 591 and 666 ->
-// 552; 4 experts, width 14336, 4096 rows 1130 -> 789.  (Limit of 256 rows throughout;
-// moe_plan_kernel has since chosen lower ones where they are faster: 2048 rows, even
-// loads, int4 805 -> 685 us, int8 772 -> 693.)
-template <int DT, int BITS, int OFFS, int TN, int STAGES, int SWI>
-__global__ __launch_bounds__(512) void gemm_experts_kernel(const DmaParams p) {
-  const MoeTile* table = reinterpret_cast<const MoeTile*>(p.moe_table);
-  const int total = table[0].expert * p.nbx;  // the header holds the number of row tiles
-  constexpr int kXcd = 8;
-  const int per = (total + kXcd - 1) / kXcd;
-  const int slot = blockIdx.x / kXcd, pos = (blockIdx.x % kXcd) * per + slot;
-  if (slot >= per || pos >= total) return;
-  // position / column tiles = some row tile of the position's expert
-  const MoeTile any = table[1 + pos / p.nbx];
-  const int w = pos - any.first * p.nbx;
-  const MoeTile t = table[1 + any.first + w % any.count];
-  const TilePlace at{w / any.count, t.expert, t.row0, t.rows};
-  const int units = (t.rows + 63) / 64;
-  if (units >= 4) dma_tile<DT, BITS, 0, OFFS, 2, 4, 4, TN, STAGES, SWI, false, false, true>(p, at);
-  else if (units == 3) dma_tile<DT, BITS, 0, OFFS, 2, 4, 3, TN, STAGES, SWI, false, false, true>(p, at);
-  else if (units == 2) dma_tile<DT, BITS, 0, OFFS, 2, 4, 2, TN, STAGES, SWI, false, false, true>(p, at);
-  else dma_tile<DT, BITS, 0, OFFS, 2, 4, 1, TN, STAGES, SWI, false, false, true>(p, at);
-}
-
 // out[m, col0 + c] = T( sum over the runs of part[run][m][c] + bias[col0 + c] ) for the ncols
 // columns from col0 on; four columns per thread; total = M * ncols.  valid_rows (may be null):
 // rows from *valid_rows on were never computed and are left alone.
@@ -1660,43 +1624,33 @@ void launch_moe_gemm_cfg(const void* x, const MoeLaunch& ml, const void* codes, 
   }
 }
 
-// The grouped GEMM on tiles of up to 256 rows x 256 (TN = 2) or 128 (TN = 1)
-// columns.  SWI = 2: the swiglu of the product is formed in the epilogue, out
-// is [rows, N / 2] and a tile has half as many output columns.
-template <int DT, int BITS, int TN, int SWI>
-void launch_experts_cfg(const void* x, const MoeLaunch& ml, const void* codes, const void* bias, const void* scale,
-                        int64_t K, int64_t N, void* out, hipStream_t stream) {
-  // as the ungrouped launch chooses: int4 under bf16 takes the offset dequantiser with row sums by dot products;
-  // two stages of 128-deep int4 tiles fill the LDS
-  constexpr int kOffs = BITS == 4 && DT == WOL_DTYPE_BF16 ? 2 : 0;
-  constexpr int kStages = BITS == 8 ? 3 : 2;
-  constexpr int BN = (SWI ? 1 : TN) * 128;  // output columns of a tile
-  constexpr size_t lds = dma_lds_bytes<BITS, 0, 2, 4, 4, TN, kStages>();
-  auto kern = gemm_experts_kernel<DT, BITS, kOffs, TN, kStages, SWI>;
-  static std::atomic<uint32_t> configured{0};
-  allow_lds(reinterpret_cast<const void*>(kern), lds, configured);
-  DmaParams p;
+// The grouped GEMM on tiles of up to 256 rows x 256 (or 128) columns.  swiglu: of
+// the product is formed in the epilogue, out is [rows, N / 2] and a tile has half
+// as many output columns.
+template <int DT>
+void launch_experts(const void* x, const MoeLaunch& ml, const void* codes, const void* bias, const void* scale, int bits,
+                    int64_t K, int64_t N, void* out, hipStream_t stream, bool swiglu) {
+  const int bn = swiglu || ml.narrow ? 128 : 256;  // output columns of a tile
+  DmaParams p{};
   p.x = static_cast<const uint16_t*>(x);
   p.codes = static_cast<const uint8_t*>(codes);
   p.bias = static_cast<const uint16_t*>(bias);
   p.scale = static_cast<const uint16_t*>(scale);
   p.out = out;
   p.M = kExpertsRows; p.K = static_cast<int>(K); p.N = static_cast<int>(N);
-  p.out_f32 = 0;
-  const int64_t out_cols = SWI ? N / 2 : N;
-  p.strip_lo = 0; p.strip_hi = static_cast<int>(out_cols / kStripCols);
-  p.nbx = static_cast<int>((out_cols + BN - 1) / BN);
+  const int64_t out_cols = swiglu ? N / 2 : N;
+  p.strip_hi = static_cast<int>(out_cols / kStripCols);
+  p.nbx = static_cast<int>((out_cols + bn - 1) / bn);
   p.nby = ml.max_tiles;
   p.nsplit = 1;
-  p.tiles_per_split = static_cast<int>(K / (BITS == 8 ? 64 : 128));
-  p.xcd_rows = 0;
+  p.tiles_per_split = static_cast<int>(K / 64);
   p.act = WOL_ACT_NONE;
   p.moe_table = ml.table;
-  p.moe_codes_stride = K * N * BITS / 8;
+  p.moe_codes_stride = K * N * bits / 8;
   p.moe_rows = static_cast<int>(ml.rows);
-  p.stamps = nullptr;
-  const int64_t blocks = (static_cast<int64_t>(p.nbx) * p.nby + 7) / 8 * 8;  // the XCDs' shares are rounded up
-  kern<<<dim3(static_cast<unsigned>(blocks)), dim3(512), lds, stream>>>(p);
+  const unsigned blocks = static_cast<unsigned>((static_cast<int64_t>(p.nbx) * p.nby + 7) / 8 * 8);  // the XCDs' shares are rounded up
+  if (DT == WOL_DTYPE_BF16) launch_experts_bf16(p, bits, ml.narrow && !swiglu, swiglu, blocks, stream);
+  else launch_experts_f16(p, bits, ml.narrow && !swiglu, swiglu, blocks, stream);
 }
 
 // ml.bm: the tile rows the table was built for (moe_tile_rows).  swiglu: out is
@@ -1705,9 +1659,7 @@ template <int DT, int BITS>
 void launch_moe_gemm(const void* x, const MoeLaunch& ml, const void* codes, const void* bias,
                      const void* scale, int64_t K, int64_t N, void* out, hipStream_t stream, bool swiglu = false) {
   if (ml.bm == kExpertsRows) {
-    if (swiglu) launch_experts_cfg<DT, BITS, 2, 2>(x, ml, codes, bias, scale, K, N, out, stream);
-    else if (ml.narrow) launch_experts_cfg<DT, BITS, 1, 0>(x, ml, codes, bias, scale, K, N, out, stream);
-    else launch_experts_cfg<DT, BITS, 2, 0>(x, ml, codes, bias, scale, K, N, out, stream);
+    launch_experts<DT>(x, ml, codes, bias, scale, BITS, K, N, out, stream, swiglu);
     return;
   }
   if constexpr (BITS == 4) {

@@ -94,8 +94,8 @@ __device__ inline void place_of_block(const DmaParams& p, int* bx, int* by, int*
   tile_of_position(pos - *split * tiles, p.nbx, p.nby, bx, by);
 }
 
-template <int DT, int BITS, int G, int WM, int WN, int TM, int TN, int SWI, bool STAMP>
-__device__ __forceinline__ void wide_tile(const DmaParams& p, int bx, int by, int split) {
+template <int DT, int BITS, int G, int WM, int WN, int TM, int TN, int SWI, bool STAMP, bool EXPERTS>
+__device__ __forceinline__ void wide_tile(const DmaParams& p, const TilePlace at, int split) {
 #if defined(__HIP_DEVICE_COMPILE__)
   constexpr int NW = WM * WN;
   static_assert(NW == 8, "eight wavefronts");
@@ -105,7 +105,7 @@ __device__ __forceinline__ void wide_tile(const DmaParams& p, int bx, int by, in
   constexpr int kScaleOff = kABytes + (BITS == 8 ? kBBytes : 0);
   constexpr int kStage = kScaleOff + kSBytes;
   constexpr int kRawOff = 3 * kStage;  // int4: the two raw B tiles
-  constexpr int kLds = static_cast<int>(wide_lds_bytes<BITS, G, WM, WN, TM, TN>());  // what the launch asks for
+  constexpr int kLds = static_cast<int>(wide_lds_bytes<BITS, G, WM, WN, EXPERTS ? 16 / WM : TM, TN>());  // of the launch  // what the launch asks for
   constexpr int kALoads = kABytes / 1024 / NW, kBSlots = kStrips / NW;
   static_assert(kABytes / 1024 % NW == 0 && kStrips % NW == 0, "the tile must split evenly over the wavefronts");
   constexpr int kDw = BITS == 8 ? 2 : 1;  // raw dwords of a B fragment
@@ -126,12 +126,16 @@ __device__ __forceinline__ void wide_tile(const DmaParams& p, int bx, int by, in
   const int wm = wave / WN, wn = wave % WN;
   const int lr = lane & 15, kb = lane >> 4;
   const int K = p.K, N = p.N;
-  const int M = p.M, m0 = by * BM;
+  const int m0 = at.row0, M = EXPERTS ? at.row0 + at.rows : p.M;
   const uint16_t* x = p.x;
   const uint16_t* scale = p.scale;
   const uint8_t* codes = p.codes;
+  if (EXPERTS) {  // the rows are those of one expert: its weights and scales
+    codes += static_cast<int64_t>(at.expert) * p.moe_codes_stride;
+    scale += static_cast<int64_t>(at.expert) * N;
+  }
   // SWI: BN / 2 gate columns and the BN / 2 up columns that go with them
-  const int strip0 = p.strip_lo + bx * (SWI ? kStrips / 2 : kStrips);
+  const int strip0 = p.strip_lo + at.bx * (SWI ? kStrips / 2 : kStrips);
   const int up_strips = N / 2 / kStripCols;
   const int t0 = split * p.tiles_per_split;  // this workgroup's run of k tiles
   const int nt = (K / 64 - t0) < p.tiles_per_split ? (K / 64 - t0) : p.tiles_per_split;
@@ -363,6 +367,7 @@ __device__ __forceinline__ void wide_tile(const DmaParams& p, int bx, int by, in
   asm volatile("" : "+v"(etid));  // nothing of the epilogue's addresses is kept in registers during the loop
   const int el = etid & 63, ec = el & 15, er = (el >> 4) * 4;
   const uint16_t* bias = p.bias;
+  if (EXPERTS && bias != nullptr) bias += static_cast<int64_t>(at.expert) * N;
   const int n_hi = p.strip_hi * kStripCols;
   float sc[TN], bv[TN];
 #pragma unroll
@@ -377,7 +382,7 @@ __device__ __forceinline__ void wide_tile(const DmaParams& p, int bx, int by, in
   const int col0 = (strip0 + wn * kOut) * kStripCols;
   const int row_w = m0 + wm * TM * 16;     // first row of this wavefront
   constexpr int kSlabRows = TM >= 2 ? 32 : 16, kPer = kSlabRows / 16;
-  if (SWI == 0 && (p.out_f32 || p.nsplit > 1)) {
+  if constexpr (SWI == 0 && !EXPERTS) if (p.out_f32 || p.nsplit > 1) {
     // fp32 results (verification mode) or the sums of this run of k tiles, kept compact: a row is as long as the
     // launch has columns
     const int64_t ld = p.nsplit > 1 ? static_cast<int64_t>(p.strip_hi - p.strip_lo) * kStripCols : N;
@@ -755,7 +760,38 @@ template <int DT, int BITS, int G, int WM, int WN, int TM, int TN, int SWI, bool
 __global__ __launch_bounds__(512) void gemm_dma_kernel_wide(const DmaParams p) {
   int bx, by, split;
   place_of_block(p, &bx, &by, &split);
-  wide_tile<DT, BITS, G, WM, WN, TM, TN, SWI, STAMP>(p, bx, by, split);
+  wide_tile<DT, BITS, G, WM, WN, TM, TN, SWI, STAMP, false>(p, TilePlace{bx, 0, by * WM * TM * 16, 0}, split);
+}
+
+// The grouped GEMM over experts with many rows each: row tiles of up to four
+// 64-row units (256 rows), as many units as the tile has rows for.  A tile's
+// MFMAs, activation loads and operand reads follow its height, so an expert
+// whose row count is no multiple of the tile pays for 64-row padding only.
+// Workgroups are handed out expert by expert, column tile by column tile, all
+// row tiles of the expert next to each other, and that sequence is cut into
+// eight equal pieces, one per XCD: an expert's row tiles meet its weights in
+// one L2 while they are there, and the XCDs stay evenly loaded however the
+// rows are spread over the experts.  WM, TN: wavefronts side by side on 256
+// columns (1, 2), or two rows of them on 128 columns (2, 2), where one row would
+// read an A fragment per MFMA.
+template <int DT, int BITS, int WM, int SWI>
+__global__ __launch_bounds__(512) void gemm_experts_kernel(const DmaParams p) {
+  const MoeTile* table = reinterpret_cast<const MoeTile*>(p.moe_table);
+  const int total = table[0].expert * p.nbx;  // the header holds the number of row tiles
+  constexpr int kXcd = 8, WN = 8 / WM;
+  const int per = (total + kXcd - 1) / kXcd;
+  const int slot = blockIdx.x / kXcd, pos = (blockIdx.x % kXcd) * per + slot;
+  if (slot >= per || pos >= total) return;
+  // position / column tiles = some row tile of the position's expert
+  const MoeTile any = table[1 + pos / p.nbx];
+  const int w = pos - any.first * p.nbx;
+  const MoeTile t = table[1 + any.first + w % any.count];
+  const TilePlace at{w / any.count, t.expert, t.row0, t.rows};
+  const int units = (t.rows + 63) / 64;
+  if (units >= 4) wide_tile<DT, BITS, 0, WM, WN, 16 / WM, 2, SWI, false, true>(p, at, 0);
+  else if (units == 3) wide_tile<DT, BITS, 0, WM, WN, 12 / WM, 2, SWI, false, true>(p, at, 0);
+  else if (units == 2) wide_tile<DT, BITS, 0, WM, WN, 8 / WM, 2, SWI, false, true>(p, at, 0);
+  else wide_tile<DT, BITS, 0, WM, WN, 4 / WM, 2, SWI, false, true>(p, at, 0);
 }
 
 // Eight wavefronts side by side, TM 16-row blocks x 32 columns each.
@@ -793,6 +829,22 @@ void launch_tile(const DmaParams& p, WideTile tile, int swi, hipStream_t stream)
   }
 }
 
+template <int DT, int BITS, int WM, int SWI>
+void launch_experts_on(const DmaParams& p, unsigned blocks, hipStream_t stream) {
+  constexpr size_t lds = wide_lds_bytes<BITS, 0, WM, 8 / WM, 16 / WM, 2>();
+  auto kern = gemm_experts_kernel<DT, BITS, WM, SWI>;
+  static std::atomic<uint32_t> configured{0};  // per instantiation
+  allow_lds(reinterpret_cast<const void*>(kern), lds, configured);
+  kern<<<dim3(blocks), dim3(512), lds, stream>>>(p);
+}
+
+template <int DT, int BITS>
+void launch_experts(const DmaParams& p, bool narrow, bool swiglu, unsigned blocks, hipStream_t stream) {
+  if (swiglu) launch_experts_on<DT, BITS, 1, 2>(p, blocks, stream);
+  else if (narrow) launch_experts_on<DT, BITS, 2, 0>(p, blocks, stream);
+  else launch_experts_on<DT, BITS, 1, 0>(p, blocks, stream);
+}
+
 template <int DT, int BITS>
 void launch_group(const DmaParams& p, int group, WideTile tile, int swi, hipStream_t stream) {
   if (group == 0) launch_tile<DT, BITS, 0>(p, tile, swi, stream);
@@ -804,12 +856,18 @@ void launch_group(const DmaParams& p, int group, WideTile tile, int swi, hipStre
 
 #if defined(WOL_GEMM_F16_UNIT)
 #define WOL_WIDE_LAUNCH launch_wide_f16
+#define WOL_EXPERTS_LAUNCH launch_experts_f16
 #else
 #define WOL_WIDE_LAUNCH launch_wide_bf16
+#define WOL_EXPERTS_LAUNCH launch_experts_bf16
 #endif
 void WOL_WIDE_LAUNCH(const DmaParams& p, int bits, int group, WideTile tile, int swi, hipStream_t stream) {
   if (bits == 8) launch_group<WOL_GEMM_DTYPE, 8>(p, group, tile, swi, stream);
   else launch_group<WOL_GEMM_DTYPE, 4>(p, group, tile, swi, stream);
+}
+void WOL_EXPERTS_LAUNCH(const DmaParams& p, int bits, bool narrow, bool swiglu, unsigned blocks, hipStream_t stream) {
+  if (bits == 8) launch_experts<WOL_GEMM_DTYPE, 8>(p, narrow, swiglu, blocks, stream);
+  else launch_experts<WOL_GEMM_DTYPE, 4>(p, narrow, swiglu, blocks, stream);
 }
 
 #if !defined(WOL_GEMM_F16_UNIT)
