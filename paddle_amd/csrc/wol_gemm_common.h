@@ -224,6 +224,24 @@ __device__ inline f32x16 mfma32(u32x4 a, u32x4 b, f32x16 c) {
                                                 __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
 }
 
+// Where position `pos` of a launch's tiles lies.  The sequence walks the tiles in bands of four row tiles or so, column
+// by column within a band, and every XCD works on a piece of it that hangs together: its 32 CUs then share four row
+// blocks and eight column blocks in their L2.  (A grid of XCDs that needs both tile counts to divide left ragged ones in
+// plain order, where the 32 tiles of an XCD have 32 different column blocks.)
+__device__ inline void tile_of_position(int pos, int nbx, int nby, int* bx, int* by) {
+  const int bands = nby > 5 ? (nby + 2) / 4 : 1, base = nby / bands, extra = nby % bands;
+  int rows = base + 1, lo = 0, w = pos;  // the first `extra` bands have a row tile more
+  if (w >= extra * rows * nbx) {
+    w -= extra * rows * nbx;
+    lo = extra * rows;
+    rows = base;
+  }
+  const int b = w / (rows * nbx);
+  w -= b * rows * nbx;
+  *by = lo + b * rows + w % rows;
+  *bx = w / rows;
+}
+
 // Raises a kernel's dynamic LDS limit once per device (the attribute belongs to
 // the device's copy of the function); safe to call from several threads.
 inline void allow_lds(const void* kern, size_t lds, std::atomic<uint32_t>& done) {

@@ -65,24 +65,6 @@ constexpr size_t wide_lds_bytes() {
   return 3 * (a + (BITS == 8 ? b : 0) + (G == 0 ? 0 : WM * WN * 256)) + (BITS == 4 ? 2 * b : 0);
 }
 
-// Where position `pos` of a launch's tiles lies.  The sequence walks the tiles in bands of four row tiles or so, column
-// by column within a band, and every XCD works on a piece of it that hangs together: its 32 CUs then share four row
-// blocks and eight column blocks in their L2.  (A grid of XCDs that needs both tile counts to divide left ragged ones in
-// plain order, where the 32 tiles of an XCD have 32 different column blocks.)
-__device__ inline void tile_of_position(int pos, int nbx, int nby, int* bx, int* by) {
-  const int bands = nby > 5 ? (nby + 2) / 4 : 1, base = nby / bands, extra = nby % bands;
-  int rows = base + 1, lo = 0, w = pos;  // the first `extra` bands have a row tile more
-  if (w >= extra * rows * nbx) {
-    w -= extra * rows * nbx;
-    lo = extra * rows;
-    rows = base;
-  }
-  const int b = w / (rows * nbx);
-  w -= b * rows * nbx;
-  *by = lo + b * rows + w % rows;
-  *bx = w / rows;
-}
-
 // The tile and the K run of this workgroup: consecutive workgroup ids go to the 8 XCDs in turn, and XCD x takes the x-th
 // eighth of the sequence of (run, tile).
 __device__ inline void place_of_block(const DmaParams& p, int* bx, int* by, int* split) {

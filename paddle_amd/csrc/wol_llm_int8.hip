@@ -24,26 +24,13 @@
 //             int32 sums in a slab of its own and this kernel adds them (exact,
 //             so the result does not depend on the cut) and applies the same
 //             epilogue.
-#include <atomic>
-#include <climits>
-
-#include "wol_common.h"
+#include "wol_gemm_common.h"
 
 namespace wol {
 namespace {
 
 typedef int i32x4 __attribute__((ext_vector_type(4)));
 typedef int i32x16 __attribute__((ext_vector_type(16)));
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-typedef __attribute__((address_space(3))) void* lds_ptr_t;
-
-
-template <int N_>
-__device__ inline void wait_vmcnt() {
-  // gfx9 encoding: vmcnt = [15:14][3:0], expcnt = [6:4], lgkmcnt = [11:8]
-  __builtin_amdgcn_s_waitcnt((N_ & 0xF) | ((N_ >> 4) << 14) | (0x7 << 4) | (0xF << 8));
-}
 
 // ---------------------------------------------------------------------------
 // activation side
@@ -334,19 +321,21 @@ struct Epi {
   const int32_t* list;
   uint16_t* out;          // [M,N] T
   int M, K, N;
+  // few outlier columns, collected by the outlier kernel for the GEMM's epilogue:
+  uint16_t* xo;           // [kOutCap][ldx] x of outlier column j, by row
+  uint16_t* wo;           // [kOutCap][ldw] T(w * wscale) of outlier column j, by output column
+  int ldx, ldw;           // M and N rounded up to whole tiles
 };
+constexpr int kOutCap = 32;
 
-// v / 127, correctly rounded, in four instructions instead of the dozen of the
-// IEEE division sequence: q = v * RN(1/127), r = v - 127 q (exact in an FMA),
-// q + r * RN(1/127).  Equal to the division for every one of the 2^32 float
-// inputs (checked exhaustively on a CPU with hardware FMA); q itself is the
-// answer where r is zero or NaN (v = -0, infinities).
+// v / 127, correctly rounded, in four instructions instead of the dozen of the IEEE division sequence: q = v * RN(1/127),
+// r = v - 127 q (exact in an FMA), q + r * RN(1/127), and v_div_fixup for v = -0 and infinities, where q is already the
+// answer.  Equal to the division for every one of the 2^32 float inputs (checked exhaustively on the device).
 __device__ inline float div127(float v) {
   const float y = 1.0f / 127.0f;
   const float q = v * y;
   const float r = __builtin_fmaf(-q, 127.0f, v);
-  const float q2 = __builtin_fmaf(r, y, q);
-  return (r != 0.0f && r == r) ? q2 : q;
+  return __builtin_amdgcn_div_fixupf(__builtin_fmaf(r, y, q), 127.0f, v);
 }
 
 // DequantFunc (:172-176) and the two T additions that follow it.  The casts
@@ -444,7 +433,18 @@ template <int DT>
 __global__ __launch_bounds__(256) void llm_outlier_kernel(Epi e, int fused_cap) {
   uint16_t* sub = e.out;  // the product waits where the output will go: whoever merges element (m, n) reads it first
   const int cnt = *e.count;
-  if (cnt <= fused_cap) return;  // none, or few enough for the GEMM's epilogue to take them
+  if (cnt <= fused_cap) {
+    const int per = e.M + e.N;
+    const int64_t total = static_cast<int64_t>(cnt) * per;
+    for (int64_t i = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x; i < total; i += static_cast<int64_t>(gridDim.x) * 256) {
+      const int j = static_cast<int>(i / per), r = static_cast<int>(i - static_cast<int64_t>(j) * per), k = e.list[j];
+      if (r < e.M) e.xo[static_cast<int64_t>(j) * e.ldx + r] = e.x[static_cast<int64_t>(r) * e.K + k];
+      else
+        e.wo[static_cast<int64_t>(j) * e.ldw + (r - e.M)] =
+            cast_out<DT>(static_cast<float>(e.w[static_cast<int64_t>(r - e.M) * e.K + k]) * e.wscale[r - e.M]);
+    }
+    return;
+  }
   __shared__ __attribute__((aligned(16))) float xs[32][64];
   const int tid = threadIdx.x;
   const int nbx = (e.N + 255) / 256;
@@ -484,6 +484,22 @@ __global__ __launch_bounds__(256) void llm_outlier_kernel(Epi e, int fused_cap) 
   }
 }
 
+// What the outlier kernel has collected for a tile of BM rows from m0 and BN
+// columns from n0 on, as floats: xs [cnt][BM], wd [cnt][BN].
+template <int DT, int BM, int BN, int THREADS>
+__device__ inline void stage_outliers(const Epi& e, int cnt, int m0, int n0, int tid, float* xs, float* wd) {
+  auto rows = [&](const uint16_t* src, int64_t ld, int len, float* dst) {
+    for (int i = tid; i < cnt * len / 8; i += THREADS) {
+      const int j = i / (len / 8), r = (i - j * (len / 8)) * 8;
+      const u32x4 v = *reinterpret_cast<const u32x4*>(src + j * ld + r);
+#pragma unroll
+      for (int q = 0; q < 8; ++q) dst[j * len + r + q] = to_f32<DT>(static_cast<uint16_t>(v[q >> 1] >> (16 * (q & 1))));
+    }
+  };
+  rows(e.xo + m0, e.ldx, BM, xs);
+  rows(e.wo + n0, e.ldw, BN, wd);
+}
+
 // ---------------------------------------------------------------------------
 // int8 GEMM
 // ---------------------------------------------------------------------------
@@ -497,6 +513,8 @@ struct GemmParams {
   int tiles_per_run; // k tiles per K run
   int cap;  // outlier columns the epilogue takes through LDS itself; more come from the outlier kernel
 };
+
+constexpr int kSlabInts = 32 * 40;  // a wavefront's slab of the GEMMs' epilogues
 
 // XOR applied to the 16-byte piece index of a row in LDS (C pieces per row) so
 // that the 16 rows a quarter of a wavefront reads hit distinct LDS banks,
@@ -743,18 +761,7 @@ __global__ __launch_bounds__(WM* WN * 64) __attribute__((amdgpu_waves_per_eu(2))
     if (!fused) __syncthreads();
   }
   if (fused) {
-    for (int i = tid; i < cnt * BM; i += NW * 64) {
-      const int j = i / BM;
-      int m = m0 + i % BM;
-      m = m < M ? m : M - 1;
-      xs[i] = to_f32<DT>(e.x[static_cast<int64_t>(m) * K + e.list[j]]);
-    }
-    for (int i = tid; i < cnt * BN; i += NW * 64) {
-      const int j = i / BN;
-      int n = n0 + i % BN;
-      n = n < N ? n : N - 1;
-      wdl[i] = to_f32<DT>(cast_out<DT>(static_cast<float>(e.w[static_cast<int64_t>(n) * K + e.list[j]]) * e.wscale[n]));
-    }
+    stage_outliers<DT, BM, BN, NW * 64>(e, cnt, m0, n0, tid, xs, wdl);
     __syncthreads();
   }
 #pragma unroll
@@ -790,6 +797,259 @@ __global__ __launch_bounds__(WM* WN * 64) __attribute__((amdgpu_waves_per_eu(2))
       }
     }
   }
+}
+
+// The product of more than 128 rows for a K of whole 128-byte k tiles: 256 x 256 or 128 x 256 tiles, a workgroup of two by
+// four wavefronts of TM x 4 v_mfma_i32_16x16x64_i8 blocks each.
+//
+// What bounds it: as in the other large-tile GEMMs the matrix pipes and the power they draw, provided that nothing stands
+// between two MFMAs.  Hence the order: the fragment of A block i is read again for the next k step right behind the four
+// MFMAs that used it, the next step's B fragments arrive in a second set of registers, and the one workgroup barrier
+// of a k tile (two steps of 64 k) sits a quarter into its second step, where the tile's last reads have long arrived; the
+// next tile's first fragments are read behind it.  256 rows: two stages of 64 KiB, all loads of tile t + 2 go out right
+// behind the barrier that frees their stage; 128 rows: three stages of 48 KiB, the loads spread from barrier to barrier.
+template <int TM>
+constexpr int llm_wide_stages() { return TM == 8 ? 2 : 3; }
+template <int TM>
+constexpr size_t llm_wide_lds() { return static_cast<size_t>(llm_wide_stages<TM>()) * (TM * 32 + 256) * 128; }
+
+template <int DT, int TM>
+__global__ __launch_bounds__(512) void llm_wide_kernel(GemmParams p) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  constexpr int NW = 8, WN = 4, TN = 4;
+  constexpr int BM = TM * 32, BN = 256;
+  constexpr int kABytes = BM * 128, kStage = kABytes + BN * 128, kStages = llm_wide_stages<TM>();
+  constexpr int kALoads = BM / 64, kLoads = kALoads + 4;  // loads of a tile, per wavefront (1 KiB = 8 rows each)
+  constexpr int B0 = TM / 4, S = TM - B0;                 // slots of the second step in front of the barrier, behind it
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  const int M = p.e.M, K = p.e.K, N = p.e.N;
+  const int tid = threadIdx.x;
+  const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = wave / WN, wn = wave % WN;
+  const int lr = lane & 15, kb = lane >> 4;
+  int bx, by;
+  {  // consecutive workgroup ids go to the 8 XCDs in turn, and XCD x takes the x-th eighth of the tile sequence
+    constexpr int kXcd = 8;
+    const int total = p.nbx * p.nby, x = blockIdx.x % kXcd, q = total / kXcd, r = total % kXcd;
+    tile_of_position(x * q + (x < r ? x : r) + blockIdx.x / kXcd, p.nbx, p.nby, &bx, &by);
+  }
+  const int m0 = by * BM, n0 = p.n_lo + bx * BN;
+  const int nt = K / 128;
+
+  // One descriptor per load, over the load's own eight rows as far as they exist: what lies past M or N arrives as zeros.
+  __amdgpu_buffer_rsrc_t ra[kALoads], rb[4];
+  auto rows_desc = [&](const int8_t* base, int row0, int rows) {
+    const int nr = rows - row0 > 8 ? 8 : (rows > row0 ? rows - row0 : 0);
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<int8_t*>(base + static_cast<int64_t>(nr > 0 ? row0 : 0) * K), 0, nr * K, 0x00020000);
+  };
+#pragma unroll
+  for (int c = 0; c < kALoads; ++c) ra[c] = rows_desc(p.qx, m0 + (c * NW + wave) * 8, M);
+#pragma unroll
+  for (int c = 0; c < 4; ++c) rb[c] = rows_desc(p.e.w, n0 + (c * NW + wave) * 8, N);
+  // rows of 128 bytes in LDS, the 16-byte piece XORed with row % 8
+  const uint32_t off = static_cast<uint32_t>((lane / 8) * K + ((lane ^ (lane >> 3)) & 7) * 16);
+  auto issue = [&](int t, int st, int i) {
+    const int tt = t < nt ? t : nt - 1;  // past the end: the last tile again, into a stage that nobody reads
+    unsigned char* s = smem + st * kStage + (i < kALoads ? 0 : kABytes) + ((i < kALoads ? i : i - kALoads) * NW + wave) * 1024;
+    if (i < kALoads) __builtin_amdgcn_raw_ptr_buffer_load_lds(ra[i], (lds_ptr_t)s, 16, off, tt * 128, 0, 0);
+    else __builtin_amdgcn_raw_ptr_buffer_load_lds(rb[i - kALoads], (lds_ptr_t)s, 16, off, tt * 128, 0, 0);
+  };
+
+  i32x4 acc[TM][TN], af[TM], bf[2][TN];
+#pragma unroll
+  for (int a = 0; a < TM; ++a)
+#pragma unroll
+    for (int c = 0; c < TN; ++c) acc[a][c] = i32x4{0, 0, 0, 0};
+  const int swz = (kb ^ (lr & 7)) * 16;  // step 1's piece is four further on: XOR 64
+  const int apos = (wm * TM * 16 + lr) * 128 + swz, bpos = kABytes + (wn * TN * 16 + lr) * 128 + swz;
+  auto read_a = [&](const unsigned char* s, int h, int i) { af[i] = *reinterpret_cast<const i32x4*>(s + (h ? apos ^ 64 : apos) + i * 2048); };
+  auto read_b = [&](const unsigned char* s, int h, int c) { bf[h][c] = *reinterpret_cast<const i32x4*>(s + (h ? bpos ^ 64 : bpos) + c * 2048); };
+  auto mfmas = [&](int h, int a) {
+#pragma unroll
+    for (int c = 0; c < TN; ++c) acc[a][c] = __builtin_amdgcn_mfma_i32_16x16x64_i8(bf[h][c], af[a], acc[a][c], 0, 0, 0);
+  };
+
+#pragma unroll
+  for (int t = 0; t < kStages - 1; ++t)
+#pragma unroll
+    for (int i = 0; i < kLoads; ++i) issue(t, t, i);
+  // three stages: the part of tile 2 that the loop's first tile does not bring
+  auto share = [&](int pos) { return kLoads * pos / (2 * TM); };
+  constexpr int kFirst = kStages == 3 ? kLoads * S / (2 * TM) : kLoads;
+#pragma unroll
+  for (int i = 0; i < kFirst; ++i) issue(kStages - 1, kStages - 1, i);
+  wait_vmcnt<(kStages - 2) * kLoads + kFirst>();  // tile 0 has landed
+  __builtin_amdgcn_s_barrier();
+#pragma unroll
+  for (int c = 0; c < TN; ++c) read_b(smem, 0, c);
+#pragma unroll
+  for (int a = 0; a < TM; ++a) read_a(smem, 0, a);
+
+  int st = 0;
+  for (int t = 0; t < nt; ++t) {
+    const int st_n = st == kStages - 1 ? 0 : st + 1, st_p = st == 0 ? kStages - 1 : st - 1;
+    const unsigned char* s = smem + st * kStage;
+    const unsigned char* n = smem + st_n * kStage;
+#pragma unroll
+    for (int i = 0; i < TM; ++i) {
+      __builtin_amdgcn_sched_barrier(0);
+      mfmas(0, i);
+      __builtin_amdgcn_sched_barrier(0);
+      if (i < 2) {
+        read_b(s, 1, 2 * i);
+        read_b(s, 1, 2 * i + 1);
+      }
+      read_a(s, 1, i);
+      if (kStages == 3) {
+#pragma unroll
+        for (int l = share(S + i); l < share(S + i + 1); ++l) issue(t + 2, st_p, l);
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < B0; ++i) {
+      __builtin_amdgcn_sched_barrier(0);
+      mfmas(1, i);
+      if (kStages == 3) {
+#pragma unroll
+        for (int l = share(S + TM + i); l < share(S + TM + i + 1); ++l) issue(t + 2, st_p, l);
+      }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    // lgkmcnt(0): this wavefront needs nothing more of the tile; tile t + 1 has landed
+    __builtin_amdgcn_s_waitcnt(0x0070 | (kStages == 3 ? kLoads : 0));
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int i = 0; i < S; ++i) {
+      mfmas(1, B0 + i);
+      __builtin_amdgcn_sched_barrier(0);
+      if (i < 2) {
+        read_b(n, 0, 2 * i);
+        read_b(n, 0, 2 * i + 1);
+      }
+#pragma unroll
+      for (int a = i > 0 ? TM * (i - 1) / (S - 1) : 0; a < TM * i / (S - 1); ++a) read_a(n, 0, a);
+      if (kStages == 3) {
+#pragma unroll
+        for (int l = share(i); l < share(i + 1); ++l) issue(t + 3, st, l);
+      } else {
+#pragma unroll
+        for (int l = kLoads * i / S; l < kLoads * (i + 1) / S; ++l) issue(t + 2, st, l);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    st = st_n;
+  }
+  __builtin_amdgcn_s_waitcnt(0x0070);
+  __builtin_amdgcn_s_barrier();  // the spare loads are done and every wavefront has stopped reading
+
+  // ---- epilogue.  The weight rows were the MFMA's first operand: element r of lane l is row l % 16 of x, column
+  // 4 * (l / 16) + r of its block, so that a lane finishes four neighbouring columns, and 32 rows x 64 columns of T
+  // leave through a slab of the wavefront's own as whole cache lines.
+  const Epi& e = p.e;
+  constexpr int kRow = 64 + 8;  // elements: the sixteen rows of a store to the slab lie in different banks
+  static_assert(32 * kRow * 2 <= kSlabInts * 4, "fused_cap counts on slabs of kSlabInts");
+  int etid = threadIdx.x;
+  asm volatile("" : "+v"(etid));  // nothing of the epilogue's addresses is kept in registers during the loop
+  const int el = etid & 63, er = el & 15, ec = (el >> 4) * 4;
+  uint16_t* slab = reinterpret_cast<uint16_t*>(smem) + wave * (32 * kRow);
+  const int cnt = *e.count;
+  float* rng = reinterpret_cast<float*>(smem + NW * kSlabInts * 4);  // [BM]: the tile's row ranges
+  float* xs = rng + BM;                                              // [cnt][BM]
+  float* wdl = xs + p.cap * BM;                                      // [cnt][BN]
+  const bool fused = cnt > 0 && cnt <= p.cap;
+  for (int i = etid; i < BM; i += NW * 64) rng[i] = e.ranges[m0 + i < M ? m0 + i : M - 1];
+  if (fused) stage_outliers<DT, BM, BN, NW * 64>(e, cnt, m0, n0, etid, xs, wdl);
+  const int nw = n0 + wn * 64;  // the wavefront's first column
+  const bool has_bias = e.bias != nullptr;
+  f32x4 ws[TN], bias[TN];
+#pragma unroll
+  for (int c = 0; c < TN; ++c) {
+    const int n = nw + c * 16 < p.n_hi ? nw + c * 16 + ec : 0;
+    ws[c] = *reinterpret_cast<const f32x4*>(e.wscale + n);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) bias[c][r] = has_bias ? to_f32<DT>(e.bias[n + r]) : 0.0f;
+  }
+  __syncthreads();
+  // piece q of the slab: eight columns of one row, the wavefront's 64 lanes on eight rows
+  auto each_piece = [&](int a, auto&& f) {
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int row = q * 8 + (el >> 3), m = m0 + (wm * TM + a) * 16 + row, n = nw + (el & 7) * 8;
+      if (m < M && n < p.n_hi)
+        f(reinterpret_cast<u32x4*>(slab + row * kRow + (el & 7) * 8), reinterpret_cast<u32x4*>(e.out + static_cast<int64_t>(m) * N + n));
+    }
+  };
+  auto settle = [&]() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  };
+  auto emit = [&](int a, int h, int c, auto&& one) {  // block (a + h, c): one(r) is its element r as T
+    u32x2 o;
+    o.x = static_cast<uint32_t>(one(0)) | (static_cast<uint32_t>(one(1)) << 16);
+    o.y = static_cast<uint32_t>(one(2)) | (static_cast<uint32_t>(one(3)) << 16);
+    *reinterpret_cast<u32x2*>(slab + (h * 16 + er) * kRow + c * 16 + ec) = o;
+  };
+#pragma unroll
+  for (int a = 0; a < TM; a += 2) {
+    const int row = (wm * TM + a) * 16 + er;  // of the tile; the second block's is 16 further on
+    const float range[2] = {rng[row], rng[row + 16]};
+    if (cnt == 0) {
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int c = 0; c < TN; ++c)
+          emit(a, h, c, [&](int r) { return merge_plain<DT>(acc[a + h][c][r], range[h], ws[c][r], has_bias, bias[c][r]); });
+    } else {
+      f32x4 sub[2][TN];  // the outlier columns' product
+      if (fused) {
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+          for (int c = 0; c < TN; ++c) sub[h][c] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+        for (int j = 0; j < cnt; ++j) {
+          const float xv[2] = {xs[j * BM + row], xs[j * BM + row + 16]};
+#pragma unroll
+          for (int c = 0; c < TN; ++c) {
+            const f32x4 wd = *reinterpret_cast<const f32x4*>(wdl + j * BN + wn * 64 + c * 16 + ec);
+#pragma unroll
+            for (int h = 0; h < 2; ++h)
+#pragma unroll
+              for (int r = 0; r < 4; ++r) sub[h][c][r] += xv[h] * wd[r];
+          }
+        }
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+          for (int c = 0; c < TN; ++c)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) sub[h][c][r] = to_f32<DT>(cast_out<DT>(sub[h][c][r]));
+      } else {  // as the outlier kernel left it in the output's own place
+        each_piece(a, [&](u32x4* l, u32x4* g) { *l = *g; });
+        settle();
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+          for (int c = 0; c < TN; ++c) {
+            const u32x2 v = *reinterpret_cast<const u32x2*>(slab + (h * 16 + er) * kRow + c * 16 + ec);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) sub[h][c][r] = to_f32<DT>(static_cast<uint16_t>(v[r >> 1] >> (16 * (r & 1))));
+          }
+        settle();
+      }
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int c = 0; c < TN; ++c)
+          emit(a, h, c, [&](int r) { return static_cast<uint16_t>(merge_one<DT>(acc[a + h][c][r], sub[h][c][r], range[h], ws[c][r], has_bias, bias[c][r])); });
+    }
+    settle();
+    each_piece(a, [&](u32x4* l, u32x4* g) { *g = *l; });
+    settle();  // the rows have been read
+  }
+#endif
 }
 
 // Adds the K runs' int32 sums and finishes; one thread per eight columns.
@@ -862,15 +1122,6 @@ __global__ __launch_bounds__(64) void llm_merge_few_kernel(const int32_t* __rest
           merge_one<DT>(sum[m], to_f32<DT>(cast_out<DT>(sub[m])), e.ranges[m], ws, e.bias != nullptr, bias));
 }
 
-inline void allow_lds(const void* kern, size_t lds, std::atomic<uint32_t>& done) {
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess) dev = 0;
-  const uint32_t bit = 1u << (dev & 31);
-  if (done.load(std::memory_order_acquire) & bit) return;
-  (void)hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds));
-  done.fetch_or(bit, std::memory_order_release);
-}
-
 inline int64_t align256(int64_t v) { return (v + 255) / 256 * 256; }
 
 struct Plan {
@@ -880,17 +1131,6 @@ struct Plan {
   int runs;       // K runs (1: the GEMM writes the output itself)
   int tiles_per_run;
 };
-
-inline int num_cus() {
-  static const int cus = [] {
-    int dev = 0, n = 0;
-    if (hipGetDevice(&dev) != hipSuccess ||
-        hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0)
-      n = 256;
-    return n;
-  }();
-  return cus;
-}
 
 // Up to 128 rows: one row tile of 32, 64 or 128 rows, 128 columns wide so that
 // the column tiles spread over the CUs, and K cut into runs while CUs are
@@ -952,6 +1192,9 @@ struct Workspace {
   int8_t* qx;
   int32_t* acc;
   int8_t* ow;
+  uint16_t* xo;
+  uint16_t* wo;
+  int ldx, ldw;
   int64_t bytes;
 };
 
@@ -976,6 +1219,12 @@ Workspace carve(void* base, int64_t M, int64_t K, int64_t N, int runs) {
   off += align256(M * N * 4 * runs);
   w.ow = reinterpret_cast<int8_t*>(p + off);
   if (runs > 1 && M <= kFewRows) off += align256(kStash * N);
+  w.ldx = static_cast<int>(align256(M));  // whole tiles: 256 is a multiple of every tile's rows and columns
+  w.ldw = static_cast<int>(align256(N));
+  w.xo = reinterpret_cast<uint16_t*>(p + off);
+  if (runs == 0) off += static_cast<int64_t>(kOutCap) * w.ldx * 2;
+  w.wo = reinterpret_cast<uint16_t*>(p + off);
+  if (runs == 0) off += static_cast<int64_t>(kOutCap) * w.ldw * 2;
   w.bytes = off;
   return w;
 }
@@ -994,17 +1243,26 @@ int launch_gemm(const GemmParams& p, int runs, hipStream_t stream) {
   return check_launch();
 }
 
+template <int DT, int TM>
+int launch_wide(const GemmParams& p, hipStream_t stream) {
+  static std::atomic<uint32_t> done{0};
+  auto kern = llm_wide_kernel<DT, TM>;
+  allow_lds(reinterpret_cast<const void*>(kern), llm_wide_lds<TM>(), done);
+  hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(p.nbx * p.nby)), dim3(512), llm_wide_lds<TM>(), stream, p);
+  return check_launch();
+}
+
 template <int DT, int TK, bool RUNS>
 int launch_gemm_for(const GemmParams& p, const Plan& pl, hipStream_t stream) {
   switch (pl.bm) {
     case 256:
       if (RUNS) return WOL_ERR_BAD_SHAPE;  // make_plan cuts K only for tiles of at most 128 rows
-      if (pl.bn == 256) return launch_gemm<DT, 2, 4, 4, 2, 128, 2, false>(p, pl.runs, stream);
+      if (pl.bn == 256) return launch_wide<DT, 8>(p, stream);
       return launch_gemm<DT, 2, 2, 4, 2, 64, 3, false>(p, pl.runs, stream);
     case 128:
       if (pl.bn == 256) {
         if (RUNS || TK != 128) return WOL_ERR_BAD_SHAPE;  // make_plan: many rows, 128-deep tiles
-        return launch_gemm<DT, 2, 4, 2, 2, 128, 3, false>(p, pl.runs, stream);
+        return launch_wide<DT, 4>(p, stream);
       }
       return launch_gemm<DT, 1, 4, 4, 1, TK, 3, RUNS>(p, pl.runs, stream);
     case 64: return launch_gemm<DT, 1, 4, 2, 1, TK, 3, RUNS>(p, pl.runs, stream);
@@ -1021,14 +1279,14 @@ int launch_gemm_tk(const GemmParams& p, const Plan& pl, hipStream_t stream) {
 }
 
 // Outlier columns the GEMM's epilogue can hold in LDS behind its slabs (at most
-// 32): (rows + columns of the tile) floats each.
+// kOutCap): (rows + columns of the tile) floats each.
 int fused_cap(const Plan& pl) {
   if (pl.runs > 1) return 0;  // the merge kernel reads the outlier kernel's product
   const bool eight = pl.bn == 256;  // the configurations of eight wavefronts
   const int64_t lds = static_cast<int64_t>(pl.bm == 256 && eight ? 2 : 3) * (pl.bm + pl.bn) * pl.tk;
-  const int64_t room = lds - (eight ? 8 : 4) * 32 * 40 * 4 - pl.bm * 4;  // slabs, row ranges
+  const int64_t room = lds - (eight ? 8 : 4) * kSlabInts * 4 - pl.bm * 4;  // slabs, row ranges
   const int64_t cap = room / ((pl.bm + pl.bn) * 4);
-  return static_cast<int>(cap > 32 ? 32 : (cap < 0 ? 0 : cap));
+  return static_cast<int>(cap > kOutCap ? kOutCap : (cap < 0 ? 0 : cap));
 }
 
 template <int DT>
@@ -1069,7 +1327,7 @@ int run_llm_int8(const void* x, const void* weight, const void* bias, const floa
   p.qx = ws.qx;
   p.e = Epi{xs, static_cast<const int8_t*>(weight), wscale, ws.ranges, static_cast<const uint16_t*>(bias),
             ws.count, ws.list, static_cast<uint16_t*>(out), static_cast<int>(M), static_cast<int>(K),
-            static_cast<int>(N)};
+            static_cast<int>(N), ws.xo, ws.wo, ws.ldx, ws.ldw};
   p.acc = ws.acc;
   p.ow = pl.runs > 1 && M <= kFewRows ? ws.ow : nullptr;
   p.n_lo = 0;
