@@ -245,15 +245,12 @@ __device__ inline void sync_stage() {
   __syncthreads();
 }
 
-// XOR applied to the 16-byte piece index of a row of out_grad's tile (rows of
-// 128 bytes): a lane group reads the same piece of 16 consecutive rows.
-__device__ inline int a_swizzle(int row) { return (row & 7) ^ ((row >> 3) & 1); }
-
-// The same for the weight tile, rows k of 128 bytes: a linear map of the low
-// five bits of k to a 3-bit piece XOR, chosen so that no access of the kernel
-// has a bank conflict whether the LDS serves 128 or 256 bytes per cycle:
-//   * 128-bit operand reads: 8 (16) consecutive rows, the same logical piece ->
-//     8 distinct pieces (and 16 distinct piece/row-parity pairs);
+// XOR applied to the 16-byte piece index of a row (k) of the weight tile, rows of
+// 128 bytes: a linear map of the low five bits of k to three, chosen so that no
+// access of the kernel has a bank conflict whether the LDS serves 128 or 256
+// bytes per cycle:
+//   * 128-bit operand reads: the sixteen lanes served together ({0-3, 12-15,
+//     20-27}, ...: rows l % 16, piece l / 16) hit 8 distinct pieces per row parity;
 //   * the dword stores of one instruction: rows i + 8*kb + (j & 1), pieces
 //     2*strip + j/8 -> the 8 combinations of (j & 1, kb & 1, j / 8) (128 bytes
 //     per cycle: half a wavefront) and of (kb, j / 8) per row parity (256) all
@@ -289,7 +286,7 @@ __global__ __launch_bounds__(512) void grad_gemm_kernel(const GradParams p) {
   const int tid = threadIdx.x;
   const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave / WKW, wk = wave % WKW;
-  const int j = lane & 15, kb = lane >> 4, b = lane >> 5, r32 = lane & 31;
+  const int j = lane & 15, kb = lane >> 4;
   const int ntiles = p.nbm * p.nbk;
   const int split = blockIdx.x / ntiles, tile = blockIdx.x - split * ntiles;
   const int bm = tile % p.nbm, bk = tile / p.nbm;
@@ -300,16 +297,16 @@ __global__ __launch_bounds__(512) void grad_gemm_kernel(const GradParams p) {
   const int cbase = split * p.chunks_per_split;
   const int niter = (p.npad / kChunk - cbase) < p.chunks_per_split ? (p.npad / kChunk - cbase) : p.chunks_per_split;
 
-  // ---- out_grad's tile: sources of this lane's direct-to-LDS loads
-  const uint16_t* asrc[kALoads];
+  // ---- out_grad's tile: one descriptor per load, over the load's own eight rows as far as they exist (rows past M
+  // arrive as zeros); the 16-byte piece of a row is XORed with row % 8
+  __amdgpu_buffer_rsrc_t ra[kALoads];
 #pragma unroll
   for (int c = 0; c < kALoads; ++c) {
-    const int q = (c * NW + wave) * 64 + lane;
-    const int row = q / 8, slot = q % 8;
-    int m = m0 + row;
-    m = m < M ? m : M - 1;  // rows past M: valid data, never stored
-    asrc[c] = p.a + static_cast<int64_t>(m) * p.npad + (slot ^ a_swizzle(row)) * 8;
+    const int row0 = m0 + (c * NW + wave) * 8, nr = M - row0 > 8 ? 8 : (M > row0 ? M - row0 : 0);
+    ra[c] = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(p.a + static_cast<int64_t>(nr > 0 ? row0 : m0) * p.npad), 0,
+                                              nr * p.npad * 2, 0x00020000);
   }
+  const uint32_t aload = static_cast<uint32_t>((lane / 8) * p.npad + ((lane ^ (lane >> 3)) & 7) * 8) * 2;
 
   // ---- the weight units of this wavefront: unit u = wave * TB + c covers k
   // chunk u / 4 (64 k) of strip u % 4 of the n chunk
@@ -366,25 +363,18 @@ __global__ __launch_bounds__(512) void grad_gemm_kernel(const GradParams p) {
       }
     }
   };
-  // chunk `it` of out_grad's tile into stage it % AS; past the last chunk the
-  // last one is fetched again (into a stage nobody reads any more)
-  auto issue_a = [&](int it) {
-    unsigned char* stage = smem + (it % AS) * kABytes;
+  // load c of chunk `it` of out_grad's tile, into stage it % AS; past the last chunk the last one is fetched again (into
+  // a stage nobody reads any more)
+  auto issue_a = [&](int it, int c) {
     const int src = cbase + (it < niter ? it : niter - 1);
-#pragma unroll
-    for (int c = 0; c < kALoads; ++c)
-      __builtin_amdgcn_global_load_lds(asrc[c] + src * kChunk, (lds_ptr_t)(stage + (c * NW + wave) * 1024), 16, 0, 0);
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(ra[c], (lds_ptr_t)(smem + (it % AS) * kABytes + (c * NW + wave) * 1024), 16, aload, src * 128, 0, 0);
   };
-  // Converts pairs (2*h, 2*h+1) of k step `step` of every unit and stores them
-  // into the weight tile `tile`: a quarter of a chunk's conversion work.
-  auto store_quarter = [&](unsigned char* tile, const Raw& r, int step, int h) {
-#pragma unroll
-    for (int c = 0; c < kUnits; ++c) {
-      const _Float16 sh = __builtin_bit_cast(_Float16, r.s[c]);
-      const f16x2 s2 = {sh, sh};
-      const int piece0 = (2 * ustrip[c] + (j >> 3)) ^ wpiece_lane;
-#pragma unroll
-      for (int pr = 2 * h; pr < 2 * h + 2; ++pr) {
+  // Converts pair u % 4 of k step u / 4 % 2 of unit u / 8 and stores it into the weight tile `tile`.
+  auto store_pair = [&](unsigned char* tile, const Raw& r, int u) {
+        const int c = u / 8, step = u / 4 % 2, pr = u % 4;
+        const _Float16 sh = __builtin_bit_cast(_Float16, r.s[c]);
+        const f16x2 s2 = {sh, sh};
+        const int piece0 = (2 * ustrip[c] + (j >> 3)) ^ wpiece_lane;
         // fp16 bits of (1024 + stored code) for k = 2*pr and 2*pr + 1 of the step
         uint32_t bits2;
         f16x2 off;
@@ -410,78 +400,68 @@ __global__ __launch_bounds__(512) void grad_gemm_kernel(const GradParams p) {
         // the swizzle is linear: the pair's part is that of k = 2*pr
         const int piece = piece0 ^ b_swizzle(2 * pr);
         *reinterpret_cast<uint32_t*>(tile + ulds[c] + (32 * step + 2 * pr) * 128 + piece * 16) = d;
-      }
-    }
   };
 
-  f32x16 acc[TM][TB];
+  constexpr int A16 = 2 * TM, B16 = 2 * TB;  // 16-row and 16-column blocks of a wavefront
+  f32x4v acc[A16][B16];
 #pragma unroll
-  for (int a = 0; a < TM; ++a)
+  for (int a = 0; a < A16; ++a)
 #pragma unroll
-    for (int c = 0; c < TB; ++c)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) acc[a][c][r] = 0.0f;
+    for (int c = 0; c < B16; ++c) acc[a][c] = f32x4v{0.f, 0.f, 0.f, 0.f};
 
-  // operand reads: rows 32*t + r32 of a tile; the swizzles have period 16 (out_grad) and 32 (weight)
-  const int a_off = (wm * TM * 32 + r32) * 128;
-  const int a_swz = a_swizzle(r32 & 15);
-  const int b_off = (wk * TB * 32 + r32) * 128;
-  const int b_swz = b_swizzle(r32);
-  auto read_frags = [&](const unsigned char* at, const unsigned char* bt, u32x4 (&af)[TM], u32x4 (&bf)[TB], int q) {
+  // operand reads: lane l takes piece l / 16 (+ 4 in the second step) of row l % 16 of a block
+  const int apos = (wm * A16 * 16 + j) * 128 + ((kb ^ (j & 7)) * 16);
+  int bpos[2];  // the weight's swizzle has period 32
 #pragma unroll
-    for (int a = 0; a < TM; ++a)
-      af[a] = *reinterpret_cast<const u32x4*>(at + a_off + a * 32 * 128 + (((2 * q + b) ^ a_swz) * 16));
-#pragma unroll
-    for (int c = 0; c < TB; ++c)
-      bf[c] = *reinterpret_cast<const u32x4*>(bt + b_off + c * 32 * 128 + (((2 * q + b) ^ b_swz) * 16));
+  for (int q = 0; q < 2; ++q) bpos[q] = (wk * B16 * 16 + q * 16 + j) * 128 + ((kb ^ b_swizzle(q * 16 + j)) * 16);
+  u32x4 af[A16], bf[2][B16];
+  auto read_a = [&](const unsigned char* at, int h, int a) { af[a] = *reinterpret_cast<const u32x4*>(at + (h ? apos ^ 64 : apos) + a * 2048); };
+  auto read_b = [&](const unsigned char* bt, int h, int c) {
+    bf[h][c] = *reinterpret_cast<const u32x4*>(bt + (h ? bpos[c & 1] ^ 64 : bpos[c & 1]) + (c >> 1) * 4096);
   };
   auto chunk_of = [&](int it) { return cbase + (it < niter ? it : niter - 1); };  // past the end: the last chunk again
-  auto mfmas = [&](const u32x4 (&af)[TM], const u32x4 (&bf)[TB]) {
+  // the weight is the first operand: element r of lane l is row l % 16 of out_grad, column (k) 4 * (l / 16) + r
+  auto mfmas = [&](int h, int a) {
 #pragma unroll
-    for (int a = 0; a < TM; ++a)
-#pragma unroll
-      for (int c = 0; c < TB; ++c)
-        acc[a][c] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, af[a]),
-                                                           __builtin_bit_cast(f16x8, bf[c]), acc[a][c], 0, 0, 0);
+    for (int c = 0; c < B16; ++c)
+      acc[a][c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, bf[h][c]), __builtin_bit_cast(f16x8, af[a]),
+                                                         acc[a][c], 0, 0, 0);
   };
 
-  // Schedule.  A chunk is four slices of 16 n; operand fragments are read two
-  // slices ahead of their MFMAs, and the one workgroup barrier of a chunk sits
-  // in its middle:
-  //   first half of chunk it:   MFMAs of slices 0, 1; fragments of slices 2, 3
-  //                             are read; the codes of chunk it+1 (in registers
-  //                             since the middle of chunk it-1) are converted
-  //                             and stored into the other weight tile
-  //   middle:                   wait for out_grad's tile of chunk it+1 and for
-  //                             the stores; barrier.  Nobody reads the tiles of
-  //                             chunk it any more (their last fragments are in
-  //                             registers), so out_grad's tile of chunk it+2
-  //                             is requested into the stage of chunk it, and
-  //                             the codes of chunk it+3 into the registers
-  //                             just converted
-  //   second half:              MFMAs of slices 2, 3 while the fragments of
-  //                             slices 0, 1 of chunk it+1 are read
-  // so neither the barrier nor the LDS latency stands between two MFMAs, and
-  // two stages of each tile suffice.  Loads past the last chunk repeat it into
-  // places nobody reads any more.
-  // (With eight MFMAs per slice one slice of lead covers the LDS latency, and
-  // four sets of fragments would not fit the registers: kDeep = false reads
-  // one slice ahead and requests slice 3 just before the barrier.)
-  constexpr bool kDeep = TM * TB < 8;
+  // Schedule.  A chunk is two steps of 32 n, a step a slot of B16 MFMAs per A
+  // block.  The A fragment a slot has used is read again for the next step right
+  // behind it, the next step's B fragments arrive in a second set.
+  //   first step of chunk it:   the fragments of the second step are read; the
+  //                             codes of chunk it+1 (in registers since chunk
+  //                             it-1) are converted and stored into the other
+  //                             weight tile, a few per slot
+  //   second step:              a quarter of it later everything requested has
+  //                             arrived: wait for out_grad's tile of chunk it+1
+  //                             and for the stores; barrier.  Nobody reads the
+  //                             tiles of chunk it any more: out_grad's tile of
+  //                             chunk it+2 is requested into its stage, the
+  //                             codes of chunk it+3 into the registers just
+  //                             converted, and the fragments of chunk it+1's
+  //                             first step are read between the remaining MFMAs
+  // so neither the barrier nor the LDS latency stands between two MFMAs.
+  constexpr int B0 = A16 / 4, S = A16 - B0, kPairs = kUnits * 8;
   Raw raw[2];
-  u32x4 af[kDeep ? 4 : 2][TM], bf[kDeep ? 4 : 2][TB];  // kDeep: the fragments of slice q live in af[q], bf[q]
-  issue_a(0);
+#pragma unroll
+  for (int c = 0; c < kALoads; ++c) issue_a(0, c);
   load_units(chunk_of(0), raw[0]);
-  issue_a(1);
+#pragma unroll
+  for (int c = 0; c < kALoads; ++c) issue_a(1, c);
   load_units(chunk_of(1), raw[1]);
 #pragma unroll
-  for (int q = 0; q < 4; ++q) store_quarter(smem + kBBase, raw[0], q / 2, q % 2);
+  for (int u = 0; u < kPairs; ++u) store_pair(smem + kBBase, raw[0], u);
   load_units(chunk_of(2), raw[0]);
   wait_vmcnt<0>();
   __builtin_amdgcn_s_waitcnt(0x0070 | (0xF << 0) | (3 << 14));  // lgkmcnt(0)
   __builtin_amdgcn_s_barrier();
-  read_frags(smem, smem + kBBase, af[0], bf[0], 0);
-  if (kDeep) read_frags(smem, smem + kBBase, af[1], bf[1], 1);
+#pragma unroll
+  for (int c = 0; c < B16; ++c) read_b(smem + kBBase, 0, c);
+#pragma unroll
+  for (int a = 0; a < A16; ++a) read_a(smem, 0, a);
 
   // conv: the codes of chunk it+1; refilled with those of chunk it+3
   auto chunk = [&](int it, Raw& conv) {
@@ -489,47 +469,42 @@ __global__ __launch_bounds__(512) void grad_gemm_kernel(const GradParams p) {
     const unsigned char* bt = smem + kBBase + (it & 1) * kBBytes;
     const unsigned char* an = smem + ((it + 1) & 1) * kABytes;
     unsigned char* bn = smem + kBBase + ((it + 1) & 1) * kBBytes;
-    if (kDeep) {
-      read_frags(at, bt, af[2], bf[2], 2);
-      mfmas(af[0], bf[0]);
-      store_quarter(bn, conv, 0, 0);
-      store_quarter(bn, conv, 0, 1);
-      read_frags(at, bt, af[3], bf[3], 3);
-      mfmas(af[1], bf[1]);
-      store_quarter(bn, conv, 1, 0);
-      store_quarter(bn, conv, 1, 1);
-    } else {
-      read_frags(at, bt, af[1], bf[1], 1);
-      mfmas(af[0], bf[0]);
-      store_quarter(bn, conv, 0, 0);
-      store_quarter(bn, conv, 0, 1);
+#pragma unroll
+    for (int i = 0; i < A16; ++i) {
       __builtin_amdgcn_sched_barrier(0);
-      read_frags(at, bt, af[0], bf[0], 2);
-      mfmas(af[1], bf[1]);
-      store_quarter(bn, conv, 1, 0);
-      store_quarter(bn, conv, 1, 1);
+      mfmas(0, i);
+#pragma unroll
+      for (int c = B16 * i / 2; c < B16 * (i + 1) / 2 && c < B16; ++c) read_b(bt, 1, c);
+      read_a(at, 1, i);
+#pragma unroll
+      for (int u = kPairs * i / A16; u < kPairs * (i + 1) / A16; ++u) store_pair(bn, conv, u);
+    }
+#pragma unroll
+    for (int i = 0; i < B0; ++i) {
       __builtin_amdgcn_sched_barrier(0);
-      read_frags(at, bt, af[1], bf[1], 3);
+      mfmas(1, i);
     }
     __builtin_amdgcn_sched_barrier(0);
-    // out_grad's tile of chunk it+1 has landed (the codes requested with it may
+    // out_grad's tile of chunk it+1 has landed (the codes requested behind it may
     // still fly), this wavefront's stores and fragment reads are done
     wait_vmcnt<kCLoads>();
     __builtin_amdgcn_s_waitcnt(0x0070 | (0xF << 0) | (3 << 14));  // lgkmcnt(0)
     __builtin_amdgcn_s_barrier();
-    issue_a(it + 2);
-    load_units(chunk_of(it + 3), conv);
     __builtin_amdgcn_sched_barrier(0);
-    if (kDeep) {
-      read_frags(an, bn, af[0], bf[0], 0);
-      mfmas(af[2], bf[2]);
-      read_frags(an, bn, af[1], bf[1], 1);
-      mfmas(af[3], bf[3]);
-    } else {
-      mfmas(af[0], bf[0]);
+#pragma unroll
+    for (int i = 0; i < S; ++i) {
+      mfmas(1, B0 + i);
       __builtin_amdgcn_sched_barrier(0);
-      read_frags(an, bn, af[0], bf[0], 0);
-      mfmas(af[1], bf[1]);
+      if (i == 0) {
+#pragma unroll
+        for (int c = 0; c < kALoads; ++c) issue_a(it + 2, c);
+      }
+      if (i == 1) load_units(chunk_of(it + 3), conv);
+#pragma unroll
+      for (int c = B16 * i / 2; c < B16 * (i + 1) / 2 && c < B16; ++c) read_b(bn, 0, c);
+#pragma unroll
+      for (int a = i > 0 ? A16 * (i - 1) / (S - 1) : 0; a < A16 * i / (S - 1); ++a) read_a(an, 0, a);
+      __builtin_amdgcn_sched_barrier(0);
     }
   };
   for (int it = 0; it < niter; it += 2) {
@@ -540,48 +515,53 @@ __global__ __launch_bounds__(512) void grad_gemm_kernel(const GradParams p) {
   __builtin_amdgcn_s_waitcnt(0x0070 | (0xF << 0) | (3 << 14));  // the fragments read ahead have arrived
   __builtin_amdgcn_s_barrier();  // the spare loads are done and every wavefront has stopped reading
 
-  // ---- epilogue: 2^-e[m], cast, 32-row slabs leave through LDS as 16-byte stores
-  // accumulator element r of lane l is row 8*(r/4) + 4*(l/32) + r%4, column l%32 of its block
-  const int col0 = k0 + wk * TB * 32;
-  if (p.out_f32 || p.nsplit > 1) {  // fp32 results (verification mode) or the sums of this run: plain stores
+  // ---- epilogue: 2^-e[m], cast; a lane has four neighbouring columns of a row, 32-row slabs leave through LDS as
+  // 16-byte stores
+  int etid = threadIdx.x;
+  asm volatile("" : "+v"(etid));  // nothing of the epilogue's addresses is kept in registers during the loop
+  const int el = etid & 63, er = el & 15, ec = (el >> 4) * 4;
+  const int col0 = k0 + wk * B16 * 16, row0 = m0 + wm * A16 * 16;
+  if (p.out_f32 || p.nsplit > 1) {  // fp32 results (verification mode) or the sums of this run
     float* outf = p.nsplit > 1 ? p.partial + static_cast<int64_t>(split) * M * K : static_cast<float*>(p.out);
 #pragma unroll
-    for (int a = 0; a < TM; ++a)
+    for (int a = 0; a < A16; ++a) {
+      const int m = row0 + a * 16 + er;
+      if (m >= M) continue;
+      const float rf = p.rowf[m];
 #pragma unroll
-      for (int c = 0; c < TB; ++c)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const int m = m0 + (wm * TM + a) * 32 + 8 * (r / 4) + 4 * b + r % 4;
-          const int k = col0 + c * 32 + r32;
-          if (m < M && k < K) outf[static_cast<int64_t>(m) * K + k] = acc[a][c][r] * p.rowf[m];
-        }
+      for (int c = 0; c < B16; ++c) {
+        const int k = col0 + c * 16 + ec;
+        if (k < K) *reinterpret_cast<f32x4v*>(outf + static_cast<int64_t>(m) * K + k) = acc[a][c] * rf;
+      }
+    }
     return;
   }
   uint16_t* out = static_cast<uint16_t*>(p.out);
-  constexpr int kSlabRow = TB * 32 + 8;  // padded, in elements
+  constexpr int kSlabRow = B16 * 16 + 8;  // padded, in elements
   static_assert(NW * 32 * kSlabRow * 2 <= kLds, "slabs must fit in the stage buffers");
   uint16_t* slab = reinterpret_cast<uint16_t*>(smem) + wave * 32 * kSlabRow;
-  constexpr int kPieces = 32 * (TB * 32 / 8);
+  constexpr int kPieces = 32 * B16 * 2;
 #pragma unroll
-  for (int a = 0; a < TM; ++a) {
-    float rf[16];
+  for (int a = 0; a < A16; a += 2) {
 #pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      int m = m0 + (wm * TM + a) * 32 + 8 * (r / 4) + 4 * b + r % 4;
-      m = m < M ? m : M - 1;
-      rf[r] = p.rowf[m];
+    for (int h = 0; h < 2; ++h) {
+      const int m = row0 + (a + h) * 16 + er;
+      const float rf = p.rowf[m < M ? m : M - 1];
+#pragma unroll
+      for (int c = 0; c < B16; ++c) {
+        u32x2 o;
+#pragma unroll
+        for (int r = 0; r < 2; ++r)
+          o[r] = static_cast<uint32_t>(cast_out<DT>(acc[a + h][c][2 * r] * rf)) |
+                 (static_cast<uint32_t>(cast_out<DT>(acc[a + h][c][2 * r + 1] * rf)) << 16);
+        *reinterpret_cast<u32x2*>(slab + (h * 16 + er) * kSlabRow + c * 16 + ec) = o;
+      }
     }
-#pragma unroll
-    for (int c = 0; c < TB; ++c)
-#pragma unroll
-      for (int r = 0; r < 16; ++r)
-        slab[(8 * (r / 4) + 4 * b + r % 4) * kSlabRow + c * 32 + r32] = cast_out<DT>(acc[a][c][r] * rf[r]);
     __builtin_amdgcn_wave_barrier();
 #pragma unroll
-    for (int q = lane; q < kPieces; q += 64) {
-      const int r = q / (TB * 4), cc = q % (TB * 4);
-      const int m = m0 + (wm * TM + a) * 32 + r;
-      const int k = col0 + cc * 8;
+    for (int q = el; q < kPieces; q += 64) {
+      const int r = q / (B16 * 2), cc = q % (B16 * 2);
+      const int m = row0 + a * 16 + r, k = col0 + cc * 8;
       const u32x4 v = *reinterpret_cast<const u32x4*>(&slab[r * kSlabRow + cc * 8]);
       if (m < M && k < K) *reinterpret_cast<u32x4*>(out + static_cast<int64_t>(m) * K + k) = v;
     }
