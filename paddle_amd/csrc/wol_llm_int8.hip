@@ -13,7 +13,7 @@
 //   quant   : qx = 0 in outlier columns, else clip(round(x * 127 * (1/range)))
 //             (QuantActKernel :270-303, QuantFunc :153-164); one extra
 //             workgroup turns the mask into an ascending list of columns
-//             (one or two rows: these three as one single-workgroup kernel)
+//             (up to eight rows: these three as one kernel)
 //   outlier : sub = T(sum over the outlier columns of x * T(w * wscale)), fp32
 //             sum in ascending column order; leaves at once without outliers
 //   gemm    : acc = qx . w^T in int32 on v_mfma_i32_32x32x32_i8, both operands
@@ -149,9 +149,16 @@ __device__ inline void build_list(int nwords, F word_at, int32_t* list, int32_t*
 }
 
 // Row ranges, outlier mask and list, activation codes of up to kSmallRows rows
-// in one workgroup: the decode-sized case, where three launches cost more
-// than the work.  The mask lives in LDS (K / 32 words, dynamic).
-constexpr int kSmallRows = 2;  // beyond two rows the single workgroup takes longer than the three launches
+// in one launch: the decode-sized case, where a launch costs more than the work.
+// A workgroup per row, and one more for the list.  Which columns are outliers
+// depends on every row, so each workgroup looks through all of them (a few dozen
+// KiB out of L2) instead of waiting for the others, and finds its own row's
+// range on the way.  The mask lives in LDS (K / 32 words, dynamic).
+// Whole call, us, against three launches (one or two rows: one workgroup for
+// everything), K = 4096, N = 11008, 3 outlier columns: 1 row 20.1 -> 18.5, 4 rows
+// 23.4 -> 20.3, 8 rows 28.9 -> 26.8: the gain shrinks as every workgroup's look
+// through all rows grows, hence the limit.
+constexpr int kSmallRows = 8;
 constexpr int kSmallThreads = 1024;
 constexpr int kSmallMaxK = 65536;
 
@@ -163,65 +170,78 @@ __global__ __launch_bounds__(kSmallThreads) void llm_act_small_kernel(const uint
                                                                       int32_t* __restrict__ count,
                                                                       int32_t* __restrict__ list) {
   extern __shared__ uint32_t smask[];
-  __shared__ float part[kSmallThreads / 64][kSmallRows];
-  __shared__ float srange[kSmallRows];
-  __shared__ int scan[256];
-  __shared__ int base_s;
-  const int tid = threadIdx.x;
-  const int nwords = K / 32;
+  __shared__ float part[kSmallThreads / 64];
+  const int tid = threadIdx.x, row = blockIdx.x;
+  const int nwords = K / 32, per = K / 8;
   const float thr = to_f32<DT>(from_f32_rne<DT>(threshold));
   for (int w = tid; w < nwords; w += kSmallThreads) smask[w] = 0u;
   __syncthreads();
-  float mx[kSmallRows];
+  float mx = 0.0f;
+  // 16 bytes of a row per thread, four in flight
+  const int nvec = M * per;
+  for (int v0 = tid; v0 < nvec; v0 += 4 * kSmallThreads) {
+    u32x4 d[4];
 #pragma unroll
-  for (int r = 0; r < kSmallRows; ++r) mx[r] = 0.0f;
-  for (int k0 = tid * 8; k0 < K; k0 += kSmallThreads * 8) {
-    uint32_t bits = 0;
+    for (int u = 0; u < 4; ++u) {
+      const int v = v0 + u * kSmallThreads;
+      d[u] = *reinterpret_cast<const u32x4*>(x + static_cast<int64_t>(v < nvec ? v : v0) * 8);  // past the end: its first again
+    }
 #pragma unroll
-    for (int r = 0; r < kSmallRows; ++r) {
-      if (r < M) {
-        const u32x4 v = *reinterpret_cast<const u32x4*>(x + static_cast<int64_t>(r) * K + k0);
+    for (int u = 0; u < 4; ++u) {
+      const int v = v0 + u * kSmallThreads;
+      if (v >= nvec) break;
+      const int m = v / per, k0 = (v - m * per) * 8;
+      uint32_t bits = 0;
+      float top = 0.0f;
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
-          float a = fabsf(to_f32<DT>(static_cast<uint16_t>(v[i >> 1] >> (16 * (i & 1)))));
-          if (a > thr) {
-            bits |= 1u << i;
-            a = 0.0f;
-          }
-          mx[r] = a > mx[r] ? a : mx[r];
+      for (int i = 0; i < 8; ++i) {
+        float a = fabsf(to_f32<DT>(static_cast<uint16_t>(d[u][i >> 1] >> (16 * (i & 1)))));
+        if (a > thr) {
+          bits |= 1u << i;
+          a = 0.0f;
         }
+        top = a > top ? a : top;
       }
+      mx = m == row && top > mx ? top : mx;
+      if (bits != 0) atomicOr(&smask[k0 >> 5], bits << (k0 & 31));
     }
-    if (bits != 0) atomicOr(&smask[k0 >> 5], bits << (k0 & 31));
   }
 #pragma unroll
-  for (int r = 0; r < kSmallRows; ++r) {
-#pragma unroll
-    for (int d = 32; d > 0; d >>= 1) {
-      const float o = __shfl_xor(mx[r], d, 64);
-      mx[r] = o > mx[r] ? o : mx[r];
-    }
-    if ((tid & 63) == 0) part[tid >> 6][r] = mx[r];
+  for (int d = 32; d > 0; d >>= 1) {
+    const float o = __shfl_xor(mx, d, 64);
+    mx = o > mx ? o : mx;
   }
+  if ((tid & 63) == 0) part[tid >> 6] = mx;
   __syncthreads();
-  if (tid < M) {
-    float r = part[0][tid];
+  if (row == M) {
+    for (int w = tid; w < nwords; w += kSmallThreads) mask[w] = static_cast<int32_t>(smask[w]);  // for whoever inspects the stages
+    if (tid >= 64) return;
+    int n = 0;  // outlier columns so far
+    for (int w0 = 0; w0 < nwords; w0 += 64) {
+      uint32_t word = w0 + tid < nwords ? smask[w0 + tid] : 0u;
+      const int c = __popc(word);
+      int upto = c;  // of the words up to this lane's
 #pragma unroll
-    for (int i = 1; i < kSmallThreads / 64; ++i) r = part[i][tid] > r ? part[i][tid] : r;
-    ranges[tid] = r;
-    srange[tid] = r;
+      for (int d = 1; d < 64; d <<= 1) {
+        const int o = __shfl_up(upto, d, 64);
+        upto += tid >= d ? o : 0;
+      }
+      for (int o = n + upto - c; word != 0; word &= word - 1) list[o++] = (w0 + tid) * 32 + __ffs(word) - 1;
+      n += __shfl(upto, 63, 64);
+    }
+    if (tid == 0) *count = n;
+    return;
   }
-  for (int w = tid; w < nwords; w += kSmallThreads) mask[w] = static_cast<int32_t>(smask[w]);  // for whoever inspects the stages
-  build_list(nwords, [&](int w) { return smask[w]; }, list, count, scan, &base_s);  // its barriers also publish srange
-  const int64_t nvec = static_cast<int64_t>(M) * K / 16;
-  for (int64_t v = tid; v < nvec; v += kSmallThreads) {
-    const int64_t e = v * 16;
-    const int m = static_cast<int>(e / K);
-    const int k = static_cast<int>(e - static_cast<int64_t>(m) * K);
-    const u32x4 lo = *reinterpret_cast<const u32x4*>(x + e);
-    const u32x4 hi = *reinterpret_cast<const u32x4*>(x + e + 8);
+  float range = part[0];
+#pragma unroll
+  for (int i = 1; i < kSmallThreads / 64; ++i) range = part[i] > range ? part[i] : range;
+  const float inv = 1.0f / range;
+  const uint16_t* xrow = x + static_cast<int64_t>(row) * K;
+  for (int v = tid; v < K / 16; v += kSmallThreads) {
+    const int k = v * 16;
+    const u32x4 lo = *reinterpret_cast<const u32x4*>(xrow + k);
+    const u32x4 hi = *reinterpret_cast<const u32x4*>(xrow + k + 8);
     const uint32_t out_bits = smask[k >> 5] >> (k & 31);
-    const float inv = 1.0f / srange[m];
     u32x4 q = {0u, 0u, 0u, 0u};
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
@@ -230,8 +250,9 @@ __global__ __launch_bounds__(kSmallThreads) void llm_act_small_kernel(const uint
       const uint32_t c = (out_bits >> i) & 1u ? 0u : quant_one(xv, inv);
       q[i >> 2] |= c << (8 * (i & 3));
     }
-    *reinterpret_cast<u32x4*>(qx + e) = q;
+    *reinterpret_cast<u32x4*>(qx + static_cast<int64_t>(row) * K + k) = q;
   }
+  if (tid == 0) ranges[row] = range;
 }
 
 // ORs the row kernel's partial masks (groups rows of K / 32 words) into the
@@ -1297,7 +1318,7 @@ int run_llm_int8(const void* x, const void* weight, const void* bias, const floa
   const uint16_t* xs = static_cast<const uint16_t*>(x);
   const bool small = M <= kSmallRows && K <= kSmallMaxK;
   if (small) {
-    hipLaunchKernelGGL(llm_act_small_kernel<DT>, dim3(1), dim3(kSmallThreads), static_cast<size_t>(K / 32 * 4), stream,
+    hipLaunchKernelGGL(llm_act_small_kernel<DT>, dim3(static_cast<unsigned>(M + 1)), dim3(kSmallThreads), static_cast<size_t>(K / 32 * 4), stream,
                        xs, threshold, static_cast<int>(M), static_cast<int>(K), ws.ranges, ws.mask, ws.qx, ws.count,
                        ws.list);
   }

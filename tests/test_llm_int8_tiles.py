@@ -1,7 +1,8 @@
 """Edges of llm_int8_linear's 128- and 256-row tiles, bit for bit against the CPU
 oracle: rows and columns on both sides of a tile, one to four 128-deep k tiles,
 ragged grids over the XCDs; sums that merge to zeros of either sign and to
-infinities, whose division by 127 takes the special cases."""
+infinities, whose division by 127 takes the special cases.  And the activation
+stages of a few rows, on both sides of the one-launch form's limit."""
 import numpy as np
 import pytest
 
@@ -39,3 +40,27 @@ def test_tile_edges(device, oracle, dt, outliers, M, K, N):
     nan = np.isnan(H.bits_to_f32(want, dt))
     assert np.array_equal(np.isnan(H.bits_to_f32(g, dt)), nan)
     assert np.array_equal(g[~nan], want[~nan])
+
+
+@pytest.mark.parametrize("dt", [H.F16, H.BF16])
+@pytest.mark.parametrize("M", [1, 2, 7, 8, 9])
+@pytest.mark.parametrize("K", [64, 2112, 8256])  # one, more than one and more than four rounds of the mask's 64 words
+def test_few_rows(device, oracle, dt, M, K):
+    import gpu_calls as G
+
+    rng = np.random.default_rng(M * K)
+    N = 48
+    w = rng.integers(-127, 128, (N, K), dtype=np.int8)
+    ws = (rng.random(N, dtype=np.float32) * np.float32(1e-3) + np.float32(1e-4)).astype(np.float32)
+    x = np.clip(rng.standard_normal((M, K), dtype=np.float32), -5, 5)
+    cols = np.unique(np.r_[0, K - 1, rng.integers(0, K, 5)])
+    x[rng.integers(0, M, cols.size), cols] = 20.0
+    x[M - 1, 3], x[0, 5] = np.nan, -0.0
+    xb = H.f32_to_bits(x, dt)
+    o = oracle.llm_int8_linear(xb, w, None, ws, 6.0, dt)
+    got, st = G.llm_int8_linear(xb, w, None, ws, 6.0, dt, stages=True)
+    assert np.array_equal(st["list"], np.nonzero(o["outlier"])[0]) and st["count"] == cols.size
+    assert np.array_equal(st["outlier"], o["outlier"])
+    assert np.array_equal(st["ranges"], o["ranges"])
+    assert np.array_equal(st["qx"], o["qx"])
+    assert np.array_equal(got, o["out"])
