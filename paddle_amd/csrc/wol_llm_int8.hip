@@ -20,7 +20,7 @@
 //             through direct-to-LDS loads, two or three k tiles deep.  The
 //             epilogue is DequantMergeKernel (:415-447): out = T( sub + T(acc *
 //             range * wscale / 127) ), then T(out + bias).
-//   merge   : only when K is cut into runs (few rows): every run leaves its
+//   merge   : only when K is cut into runs (few tiles): every run leaves its
 //             int32 sums in a slab of its own and this kernel adds them (exact,
 //             so the result does not depend on the cut) and applies the same
 //             epilogue.
@@ -829,12 +829,16 @@ __global__ __launch_bounds__(WM* WN * 64) __attribute__((amdgpu_waves_per_eu(2))
 // of a k tile (two steps of 64 k) sits a quarter into its second step, where the tile's last reads have long arrived; the
 // next tile's first fragments are read behind it.  256 rows: two stages of 64 KiB, all loads of tile t + 2 go out right
 // behind the barrier that frees their stage; 128 rows: three stages of 48 KiB, the loads spread from barrier to barrier.
+// Whole call, us, against 32x32x32 blocks whose first fragments of a tile are read behind its barrier, with an epilogue
+// that passes int32 sums through LDS and stores half cache lines: 8192 x 4096 x 12288 490 -> 398 (six rounds of tiles: 50
+// in the k loop, 40 without its loads, and 11 in the epilogue each), 2048 x 4096 x 12288 132 -> 114, 300 x 4096 x 4096
+// with 20 outlier columns 61.6 -> 49.0.
 template <int TM>
 constexpr int llm_wide_stages() { return TM == 8 ? 2 : 3; }
 template <int TM>
 constexpr size_t llm_wide_lds() { return static_cast<size_t>(llm_wide_stages<TM>()) * (TM * 32 + 256) * 128; }
 
-template <int DT, int TM>
+template <int DT, int TM, bool RUNS>
 __global__ __launch_bounds__(512) void llm_wide_kernel(GemmParams p) {
 #if defined(__HIP_DEVICE_COMPILE__)
   constexpr int NW = 8, WN = 4, TN = 4;
@@ -848,14 +852,17 @@ __global__ __launch_bounds__(512) void llm_wide_kernel(GemmParams p) {
   const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave / WN, wn = wave % WN;
   const int lr = lane & 15, kb = lane >> 4;
-  int bx, by;
-  {  // consecutive workgroup ids go to the 8 XCDs in turn, and XCD x takes the x-th eighth of the tile sequence
+  int bx, by, run;
+  {  // consecutive workgroup ids go to the 8 XCDs in turn, and XCD x takes the x-th eighth of the sequence of (run, tile)
     constexpr int kXcd = 8;
-    const int total = p.nbx * p.nby, x = blockIdx.x % kXcd, q = total / kXcd, r = total % kXcd;
-    tile_of_position(x * q + (x < r ? x : r) + blockIdx.x / kXcd, p.nbx, p.nby, &bx, &by);
+    const int total = gridDim.x, x = blockIdx.x % kXcd, q = total / kXcd, r = total % kXcd;
+    const int pos = x * q + (x < r ? x : r) + blockIdx.x / kXcd;
+    run = pos / (p.nbx * p.nby);
+    tile_of_position(pos - run * (p.nbx * p.nby), p.nbx, p.nby, &bx, &by);
   }
   const int m0 = by * BM, n0 = p.n_lo + bx * BN;
-  const int nt = K / 128;
+  const int t0 = run * p.tiles_per_run;  // this workgroup's run of k tiles
+  const int nt = K / 128 - t0 < p.tiles_per_run ? K / 128 - t0 : p.tiles_per_run;
 
   // One descriptor per load, over the load's own eight rows as far as they exist: what lies past M or N arrives as zeros.
   __amdgpu_buffer_rsrc_t ra[kALoads], rb[4];
@@ -870,7 +877,7 @@ __global__ __launch_bounds__(512) void llm_wide_kernel(GemmParams p) {
   // rows of 128 bytes in LDS, the 16-byte piece XORed with row % 8
   const uint32_t off = static_cast<uint32_t>((lane / 8) * K + ((lane ^ (lane >> 3)) & 7) * 16);
   auto issue = [&](int t, int st, int i) {
-    const int tt = t < nt ? t : nt - 1;  // past the end: the last tile again, into a stage that nobody reads
+    const int tt = t0 + (t < nt ? t : nt - 1);  // past the end: the last tile again, into a stage that nobody reads
     unsigned char* s = smem + st * kStage + (i < kALoads ? 0 : kABytes) + ((i < kALoads ? i : i - kALoads) * NW + wave) * 1024;
     if (i < kALoads) __builtin_amdgcn_raw_ptr_buffer_load_lds(ra[i], (lds_ptr_t)s, 16, off, tt * 128, 0, 0);
     else __builtin_amdgcn_raw_ptr_buffer_load_lds(rb[i - kALoads], (lds_ptr_t)s, 16, off, tt * 128, 0, 0);
@@ -973,6 +980,16 @@ __global__ __launch_bounds__(512) void llm_wide_kernel(GemmParams p) {
   int etid = threadIdx.x;
   asm volatile("" : "+v"(etid));  // nothing of the epilogue's addresses is kept in registers during the loop
   const int el = etid & 63, er = el & 15, ec = (el >> 4) * 4;
+  if constexpr (RUNS) {  // this run's sums, to be added by the merge kernel
+#pragma unroll
+    for (int a = 0; a < TM; ++a)
+#pragma unroll
+      for (int c = 0; c < TN; ++c) {
+        const int m = m0 + (wm * TM + a) * 16 + er, n = n0 + wn * 64 + c * 16 + ec;
+        if (m < M && n < p.n_hi) *reinterpret_cast<i32x4*>(p.acc + (static_cast<int64_t>(run) * M + m) * N + n) = acc[a][c];
+      }
+    return;
+  }
   uint16_t* slab = reinterpret_cast<uint16_t*>(smem) + wave * (32 * kRow);
   const int cnt = *e.count;
   float* rng = reinterpret_cast<float*>(smem + NW * kSlabInts * 4);  // [BM]: the tile's row ranges
@@ -1186,6 +1203,29 @@ Plan make_plan(int64_t M, int64_t K, int64_t N) {
       }
       pl.whole_cols = static_cast<int>(best_c * 256 < N ? best_c * 256 : N);
       if (best_c == 0) pl.bm = 128;
+      // Few tiles leave CUs idle: half tiles with K cut into runs, by the estimate in us of a round (a k tile of a whole
+      // tile takes 1.7, of a half one 1.0, their starts and ends 11 and 6, 4 with sums instead of results) and of the
+      // merge launch with the sums' way through memory.  The 0.9: with runs the outlier columns' product is a pass of its
+      // own, which the estimate cannot know.  Whole call, us, one run against this: 200 x 8192 x 3008 56.0 -> 34.7, with 5
+      // outlier columns 42.0; 1024 x 11008 x 4096 102 -> 79; 300 x 4096 x 4096 with 20 outlier columns 49.0 -> 51.3.
+      const double kt = static_cast<double>(ktiles);
+      const double one = (best_c * rows256 + cus - 1) / cus * (1.7 * kt + 11) + ((cols - best_c) * rows128 + cus - 1) / cus * (1.0 * kt + 6);
+      double best = 0.9 * one;
+      int64_t best_r = 1;
+      for (int64_t r = 2; r <= 8 && ktiles / r >= 4; ++r) {
+        const int64_t per = (ktiles + r - 1) / r, eff = (ktiles + per - 1) / per;
+        const double t = static_cast<double>((cols * rows128 * eff + cus - 1) / cus) * (1.0 * per + 4) + 4 +
+                         static_cast<double>(M) * N * (8 * eff + 2) / 4.5e6;
+        if (t < best) {
+          best = t;
+          best_r = eff;
+        }
+      }
+      if (best_r > 1) {
+        pl.bm = 128;
+        pl.whole_cols = 0;
+        runs = best_r;
+      }
     }
   } else {
     pl.bm = M > 64 ? 128 : (M > 32 ? 64 : 32);
@@ -1264,12 +1304,12 @@ int launch_gemm(const GemmParams& p, int runs, hipStream_t stream) {
   return check_launch();
 }
 
-template <int DT, int TM>
-int launch_wide(const GemmParams& p, hipStream_t stream) {
+template <int DT, int TM, bool RUNS>
+int launch_wide(const GemmParams& p, int runs, hipStream_t stream) {
   static std::atomic<uint32_t> done{0};
-  auto kern = llm_wide_kernel<DT, TM>;
+  auto kern = llm_wide_kernel<DT, TM, RUNS>;
   allow_lds(reinterpret_cast<const void*>(kern), llm_wide_lds<TM>(), done);
-  hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(p.nbx * p.nby)), dim3(512), llm_wide_lds<TM>(), stream, p);
+  hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(p.nbx * p.nby * runs)), dim3(512), llm_wide_lds<TM>(), stream, p);
   return check_launch();
 }
 
@@ -1278,12 +1318,12 @@ int launch_gemm_for(const GemmParams& p, const Plan& pl, hipStream_t stream) {
   switch (pl.bm) {
     case 256:
       if (RUNS) return WOL_ERR_BAD_SHAPE;  // make_plan cuts K only for tiles of at most 128 rows
-      if (pl.bn == 256) return launch_wide<DT, 8>(p, stream);
+      if (pl.bn == 256) return launch_wide<DT, 8, false>(p, 1, stream);
       return launch_gemm<DT, 2, 2, 4, 2, 64, 3, false>(p, pl.runs, stream);
     case 128:
       if (pl.bn == 256) {
-        if (RUNS || TK != 128) return WOL_ERR_BAD_SHAPE;  // make_plan: many rows, 128-deep tiles
-        return launch_wide<DT, 4>(p, stream);
+        if (TK != 128) return WOL_ERR_BAD_SHAPE;  // make_plan: many rows, 128-deep tiles
+        return launch_wide<DT, 4, RUNS>(p, pl.runs, stream);
       }
       return launch_gemm<DT, 1, 4, 4, 1, TK, 3, RUNS>(p, pl.runs, stream);
     case 64: return launch_gemm<DT, 1, 4, 2, 1, TK, 3, RUNS>(p, pl.runs, stream);
