@@ -167,12 +167,9 @@ struct DequantExact<WOL_DTYPE_BF16, 4> {
 // The same codes in 19 instructions per eight instead of 27: each nibble pair
 // becomes two fp16 values 1024 + 16 * nibble (one and-or), a mixed-precision FMA
 // takes the offset out and widens to fp32 in one instruction, and the high
-// halves are the bf16 codes, every step exact.  g128 with this form against the
-// other one: 128 x 256 tiles 2 to 5 % faster (100 rows, K = 11008, N = 4096: 58.4
-// against 60.7 us; swiglu, 128 rows, 3 to 5 %), half-deep and small-M tiles 1 to
-// 2 %; 256 x 128 tiles, where four A blocks share a B block, 2 to 3 % slower (200
-// rows, K = N = 4096: 31.6 against 30.7), so they keep the other.  gemm_kernel:
-// per channel 2 to 4 % faster, group-wise up to 9 % slower (K = 4544: 65 rows).
+// halves are the bf16 codes, every step exact.  Against the other form the small-M
+// tiles are 1 to 2 % faster; gemm_kernel: per channel 2 to 4 % faster, group-wise
+// up to 9 % slower (K = 4544: 65 rows), so it keeps the other there.
 template <int DT, int BITS>
 struct DequantExactFma : DequantExact<DT, BITS> {};
 

@@ -1,16 +1,17 @@
 // weight_only_linear for large M (prefill): MFMA GEMMs.
 //
-// gemm_dma_kernel is the kernel that runs whenever K is made of whole k tiles
-// (64 k for int8, 128 k for int4): a workgroup of WM x WN wavefronts computes a
-// BM x BN tile of the output from TM x TN blocks of v_mfma_f32_32x32x16 per
-// wavefront.  Both operands travel global -> LDS with direct-to-LDS loads,
-// two or three k tiles deep; the packed weights land as they lie in memory and
-// are dequantised in registers to exact signed bf16/fp16 integers on their way
-// into the B operand; scales are applied to fp32 accumulators -- in the
-// epilogue (per-channel) or once per group -- so code * scale is never rounded
-// to T.  For few rows K is cut into runs across workgroups whose fp32 partial
-// sums reduce_partials_kernel adds.  Workgroups are numbered so that each XCD
-// (one L2 each) works on a compact block of neighbouring tiles.
+// For a K made of whole k tiles (64 k for int8, 128 k for int4) up to 64 rows run
+// on gemm_dma_kernel: a workgroup of eight wavefronts side by side computes a BM
+// x BN tile of the output from TM x TN blocks of v_mfma_f32_32x32x16 per
+// wavefront; more rows on the tiles of wol_linear_wide.hip, planned here.  Both
+// operands travel global -> LDS with direct-to-LDS loads; the packed weights
+// land as they lie in memory and are dequantised in registers to exact signed
+// bf16/fp16 integers on their way into the B operand; scales are applied to fp32
+// accumulators -- in the epilogue (per-channel) or once per group -- so code *
+// scale is never rounded to T.  For few rows K is cut into runs across
+// workgroups whose fp32 partial sums reduce_partials_kernel adds.  Workgroups
+// are numbered so that each XCD (one L2 each) works on a compact block of
+// neighbouring tiles.
 //
 // gemm_kernel (v_mfma_f32_16x16x32, activations staged through registers into
 // padded LDS rows, weights loaded straight into B-fragment order) takes the
@@ -272,32 +273,15 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_kernel(
   }
 }
 
-// acc + the sum of the eight T values of an operand fragment, in fp32 (four
-// packed dot products against (1, 1)).
-template <int DT>
-__device__ inline float sum8(u32x4 v, float acc) {
-  typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-  typedef _Float16 h16x2 __attribute__((ext_vector_type(2)));
-  const uint32_t w[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    if (DT == WOL_DTYPE_BF16)
-      acc = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, w[i]), __builtin_bit_cast(bf16x2, 0x3F803F80u), acc, false);
-    else
-      acc = __builtin_amdgcn_fdot2(__builtin_bit_cast(h16x2, w[i]), __builtin_bit_cast(h16x2, 0x3C003C00u), acc, false);
-  }
-  return acc;
-}
-
 // Fast path: K a multiple of the tile depth.
 //
-// v_mfma_f32_32x32x16 is the instruction that reaches the matrix cores' full
-// rate on gfx950 (the 16x16x32 form issues at half of it), so the wavefront
-// tile is built from 32 x 32 blocks: TM x TN of them.  Both operands travel
+// The wavefront tile is built from 32 x 32 blocks of v_mfma_f32_32x32x16: TM x TN
+// of them.  (wol_linear_wide.hip's 16x16x32 tiles with 64 rows, three stages deep,
+// are level here: 64 rows, K = 8192, N = 28672, int4 g128 fp16 53.3 us against 53.4
+// with K in two runs, 51.0 in four; 4096 x 11008 bf16 23.4 against 21.3.)  Both operands travel
 // global -> LDS with direct-to-LDS loads (no registers, no LDS store
-// instructions), STAGES k tiles deep: while tile `it` is consumed the loads of
-// tiles it+1 (and, with three stages, it+2) are in flight.  A lands in LDS as unpadded rows whose
-// 16-byte pieces are XOR-swizzled by row so a lane group's fragment reads
+// instructions), two k tiles deep: while tile `it` is consumed the loads of
+// tile it+1 are in flight.  A lands in LDS as unpadded rows whose 16-byte pieces are XOR-swizzled by row so a lane group's fragment reads
 // fall into distinct banks.  The raw packed B tiles land exactly as they lie
 // in memory (16-column strips in 16x16x32 order); a 32x32x16 B operand is
 // assembled by letting lane l = 32*b + 16*sp + j read the 16 bytes that lane
@@ -312,89 +296,33 @@ __device__ inline float sum8(u32x4 v, float acc) {
 //
 // OFFS selects the offset dequantiser: a fraction of the VALU work, and the
 // constant offset of every code is taken out again as -offset * (sum of the
-// row's activations).  OFFS = 1 forms that sum with one more MFMA per A
-// fragment and slice against a constant B operand (into `canc`, added when
-// the scale is applied) -- the right trade when M is small: the matrix pipe
-// idles, the VALU does not.  OFFS = 2 forms it with four packed dot products
-// per A fragment (a lane adds up the eight activations of its fragment; the
-// two lanes that share a row meet in the epilogue), which costs no MFMA and
-// no accumulators and is what lets int4 weights under bf16 activations take
-// the largest tile; per-channel scales only.
+// row's activations), which one more MFMA per A fragment and slice forms against
+// a constant B operand (into `canc`, added when the scale is applied) -- the
+// right trade when M is small: the matrix pipe idles, the VALU does not.
 //
 // With nsplit > 1 a workgroup covers only a run of k tiles and leaves its
 // fp32 sums (scaled, without bias) in a partial buffer; reduce_partials_kernel
 // adds the runs.  That is what fills the CUs when M is small.
 //
-// SWI != 0: swiglu in the epilogue (TN = 2, per-channel scales).  The weight is
-// a gate | up projection, [K, N] with the gate in columns 0 .. N/2-1; block 0
-// of every wavefront then takes 32 gate columns and block 1 the 32 up columns
-// N/2 further on, so that silu(gate) * up is formed lane by lane from the two
-// accumulators and only [M, N/2] leaves the kernel.  SWI = 1 applies it to the
-// fp32 sums (wol_linear_fused); SWI = 2 first rounds both sums to T, as a
-// separate fc1 output would have been (the mixture-of-experts FFN).
-//
-// RESC (group-wise scales): one set of accumulators instead of two.  The
-// running sums are kept in units of the current group's scale: where a group
-// starts they are multiplied by (previous unit / new unit) and the group's
-// MFMAs then accumulate straight into them; the epilogue multiplies by the last
-// unit.  Every rescaling rounds the sums once (2^-24 relative, a few dozen
-// times per output element), code * scale is still never rounded to T, and
-// the registers of the second accumulator set are free for the largest tile.
-// The unit of a column follows its group scale but never falls more than 2^64
-// below the largest scale the column has had so far (a group that small
-// weighs nothing next to the others in fp32), so the sums cannot overflow
-// however the scales of a column differ.
-//
-// STAMP (a diagnostic instantiation, never on a product path): every wavefront
-// reads the cycle counter at kernel entry, around the two waits of every k
-// tile (for its own tile loads, then for the workgroup) and around the
-// epilogue, and leaves the sums in p.stamps.  The reads sit where the
-// wavefront has just waited for all its LDS traffic anyway.
-//
-// The work of one workgroup is a device function (dma_tile): gemm_dma_kernel
-// below calls it for the one tile height it is built for and lets it find its
-// tile from the workgroup id, gemm_experts_kernel (EXPERTS) picks the height of
-// every tile at run time and says where it lies.  The form of the function is
-// the one whose inner loops the compiler orders best: for gemm_dma_kernel the
-// parameters come by value, the LDS is named inside and the tile is found after
-// the lane arithmetic.  By reference, with the LDS and the tile's place as
-// arguments, the same loops run 2 to 4 % longer (int8 g128, 256 rows, K =
-// 11008, N = 4096: 52.6 against 50.0 us; int4 per channel, 200 rows, same
-// weight: 47.3 against 45.9; per-channel int8 at 2048 rows level).  The four
-// heights of gemm_experts_kernel are 0.4 % faster by reference.
-//
-// kHalfDeep (STAGES = kHalfDeepStages + 3; int4): three stages of 64-deep tiles
-// of activations (and scales) where two 128-deep ones would overflow the LDS.
-// The packed weight still arrives in its 128-deep tiles of 16 bytes per lane:
-// they have two buffers of their own, an odd k tile's loads bring the first half
-// (by strips) of the next raw tile and the even one's the second, and the codes
-// of a raw tile are read into registers once for both k tiles.  Every stage has
-// the same number of loads, so the counted waits are those of the other forms.
-constexpr int kHalfDeepStages = 10;
-
-template <int DT, int BITS, int G, int OFFS, int WM, int WN, int TM, int TN, int STAGES, int SWI, bool RESC, bool STAMP,
-          bool EXPERTS>
-__device__ __forceinline__ void dma_tile(std::conditional_t<EXPERTS, const DmaParams&, const DmaParams> p, const TilePlace at) {
+// (A device function with the parameters by value: as the kernel's own body the
+// same loops come out in another order.)
+template <int DT, int BITS, int G, bool OFFS, int WM, int WN, int TM, int TN>
+__device__ __forceinline__ void dma_tile(const DmaParams p) {
 #if defined(__HIP_DEVICE_COMPILE__)  // the host pass only needs the launch stubs
   constexpr int NW = WM * WN;
   constexpr int BM = WM * TM * 32, BN = WN * TN * 32;
-  constexpr bool kHalfDeep = STAGES > kHalfDeepStages;  // int4, 64-deep k tiles: see the comment above
-  static_assert(!kHalfDeep || (BITS == 4 && STAGES == kHalfDeepStages + 3), "half-deep tiles: int4, three stages");
-  constexpr int TK = BITS == 8 || kHalfDeep ? 64 : 128;  // k per tile
+  constexpr int TK = BITS == 8 ? 64 : 128;       // k per tile
   constexpr int kDw = BITS == 8 ? 2 : 1;         // dwords per 8 codes
   constexpr int C = TK / 8;                      // 16-byte pieces per A row
   constexpr int kABytes = BM * TK * 2;           // one A tile
   constexpr int kBBytes = (BN / 16) * 1024;      // one raw B tile (all strips of the workgroup)
   constexpr int kSBytes = G == 0 ? 0 : NW * 256;  // the tile's group scales: 128 values per wavefront
-  constexpr int kScaleOff = kABytes + (kHalfDeep ? 0 : kBBytes);  // the scales' place in a stage
+  constexpr int kScaleOff = kABytes + kBBytes;    // the scales' place in a stage
   constexpr int kStage = kScaleOff + kSBytes;
-  constexpr int kStages = STAGES % kHalfDeepStages;  // k tiles resident or in flight
-  constexpr int kLds = kStages * kStage + (kHalfDeep ? 2 * kBBytes : 0);
-  static_assert(kStages == 2 || kStages == 3, "two or three stages");
+  constexpr int kStages = 2;                     // k tiles resident or in flight
+  constexpr int kLds = kStages * kStage;
   constexpr int kALoads = kABytes / 1024 / NW;   // wave-level loads (1 KiB each) per wavefront
-  constexpr int kBSlots = BN / 16 / NW;          // wave-level loads of a raw B tile per wavefront
-  constexpr int kBLoads = kHalfDeep ? kBSlots / 2 : kBSlots;  // of them in one stage's loads
-  static_assert(!kHalfDeep || kBSlots % 2 == 0, "a raw B tile travels in two equal halves");
+  constexpr int kBLoads = BN / 16 / NW;          // wave-level loads of a raw B tile per wavefront
   static_assert(kABytes / 1024 % NW == 0 && kALoads >= 1, "A tile must split evenly over the wavefronts");
   static_assert(BN / 16 % NW == 0 && kBLoads >= 1, "B tile must split evenly over the wavefronts");
   constexpr int Q = TK / 16;  // 16-k slices (one MFMA per 32x32 block each) per tile
@@ -410,18 +338,8 @@ __device__ __forceinline__ void dma_tile(std::conditional_t<EXPERTS, const DmaPa
   constexpr int kPerStage = kALoads + kBLoads + (G == 0 ? 0 : 1);
   static_assert(Q >= 2 && (Q - 2) % kFold != 0 && (Q - 2) % kFold != kFold - 1,
                 "the slice that holds the barrier neither starts nor ends a group");
-  static_assert(SWI == 0 || ((TN == 2 || (TN == 1 && WN % 2 == 0)) && (G == 0 || RESC)),
-                "the swiglu epilogue pairs the two blocks of a wavefront, or two neighbouring wavefronts");
-  // SWI with one block per wavefront: wavefront columns 2i and 2i+1 hold the gate and the up block of
-  // the same 32 output columns, and the up wavefront hands its sums over through LDS in the epilogue
-  constexpr bool kPair = SWI != 0 && TN == 1;
-  // all tiles but those of 256 x 128 take the shorter int4 dequantiser (see DequantExactFma)
-  constexpr bool kFmaDequant = BITS == 4 && OFFS == 0 && (TN == 2 || WM == 1);
-  static_assert(OFFS != 2 || G == 0, "row sums by dot products are taken out once, in the epilogue");
-  static_assert(!RESC || (G != 0 && OFFS == 0), "rescaled sums are for group-wise scales and the exact dequantisers");
+  constexpr bool kFmaDequant = BITS == 4 && !OFFS;  // the shorter int4 dequantiser (see DequantExactFma)
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-  unsigned long long st_entry = 0, st_prev = 0, st_work = 0, st_loads = 0, st_bar = 0, st_loop0 = 0;
-  if (STAMP) st_entry = __builtin_readcyclecounter();
 
   const uint16_t* __restrict__ x = p.x;
   const uint16_t* __restrict__ scale = p.scale;
@@ -434,48 +352,33 @@ __device__ __forceinline__ void dma_tile(std::conditional_t<EXPERTS, const DmaPa
   const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave / WN, wn = wave % WN;
   const int j = lane & 15, sp = (lane >> 4) & 1, b = lane >> 5, r32 = lane & 31;
-  int bx, m0 = 0, split = 0;
-  int expert = -1, row0 = 0, rows = 0;
-  if constexpr (EXPERTS) {
-    bx = at.bx;
-    expert = at.expert;
-    row0 = at.row0;
-    rows = at.rows;
-  } else {
-    const int ntiles = p.nbx * p.nby;
-    split = blockIdx.x / ntiles;
-    int by;
-    tile_of_block_2d(blockIdx.x - split * ntiles, p.nbx, p.nby, p.xcd_rows, &bx, &by);
-    m0 = by * BM;
-    // Grouped launches of this kernel are those of small tiles (launch_moe_gemm_cfg).  The larger per-channel
-    // kernels know that at compile time (int8, 1237 rows, K = N = 4096: 54.4 against 55.8 us); the group-wise ones
-    // keep the test, which no launch answers with yes, because their loops come out better ordered with it
-    // (int8 g128, 256 rows, K = 11008, N = 4096: 50.4 against 52.5 us).
-    if (SWI == 0 && (WM == 1 || RESC) && p.moe_table != nullptr) {
-      const MoeTile t = reinterpret_cast<const MoeTile*>(p.moe_table)[by];
-      if (t.expert < 0) return;
-      expert = t.expert;
-      row0 = t.row0;
-      rows = t.rows;
-    }
+  int bx, by, expert = -1, row0 = 0, rows = 0;
+  const int ntiles = p.nbx * p.nby;
+  const int split = blockIdx.x / ntiles;
+  tile_of_block_2d(blockIdx.x - split * ntiles, p.nbx, p.nby, p.xcd_rows, &bx, &by);
+  int m0 = by * BM;
+  if (p.moe_table != nullptr) {
+    const MoeTile t = reinterpret_cast<const MoeTile*>(p.moe_table)[by];
+    if (t.expert < 0) return;
+    expert = t.expert;
+    row0 = t.row0;
+    rows = t.rows;
   }
   if (expert >= 0) {
     // this tile belongs to one expert: shift every base to that expert and to
     // the tile's first row, and let M be the rows that exist
     x += static_cast<int64_t>(row0) * K;
     if (p.nsplit > 1) outp = static_cast<float*>(outp) + static_cast<int64_t>(row0) * N;  // partial sums
-    else outp = static_cast<uint16_t*>(outp) + static_cast<int64_t>(row0) * (SWI ? N / 2 : N);
+    else outp = static_cast<uint16_t*>(outp) + static_cast<int64_t>(row0) * N;
     codes += static_cast<int64_t>(expert) * p.moe_codes_stride;
     scale += static_cast<int64_t>(expert) * N;
     if (bias != nullptr) bias += static_cast<int64_t>(expert) * N;
     M = rows;
     m0 = 0;
   }
-  // SWI: a workgroup takes BN / 2 gate columns and the BN / 2 up columns that go with them
-  const int strip_blk = p.strip_lo + bx * (SWI ? BN / 32 : BN / 16);
+  const int strip_blk = p.strip_lo + bx * (BN / 16);
   const int nstrips = p.strip_hi;
   const int n_hi = p.strip_hi * kStripCols;
-  const int up_strips = N / 2 / kStripCols;  // SWI: strips between a gate column and its up column
   // this workgroup's run of k tiles
   const int t0 = split * p.tiles_per_split;
   const int niter = (K / TK - t0) < p.tiles_per_split ? (K / TK - t0) : p.tiles_per_split;
@@ -495,22 +398,13 @@ __device__ __forceinline__ void dma_tile(std::conditional_t<EXPERTS, const DmaPa
     m = m < M ? m : M - 1;  // rows past M are computed on valid data and never stored
     asrc[c] = x + static_cast<int64_t>(m) * K + static_cast<int64_t>(t0) * TK + cc * 8;
   }
-  const uint8_t* bsrc[kBSlots];
+  const uint8_t* bsrc[kBLoads];
 #pragma unroll
-  for (int c = 0; c < kBSlots; ++c) {
+  for (int c = 0; c < kBLoads; ++c) {
     int st = strip_blk + c * NW + wave;
-    if (SWI) {
-      // LDS slot L of the B tile serves wavefront column L / 4, block (L / 2) % 2, half L % 2
-      const int L = c * NW + wave;
-      st = strip_blk + (L / 4) * 2 + L % 2;
-    }
     st = st < nstrips ? st : nstrips - 1;  // past the last column: valid data, never stored
-    if (SWI && ((c * NW + wave) / 2) % 2 == 1) st += up_strips;  // block 1: the up columns
-    bsrc[c] = codes + static_cast<int64_t>(st) * strip_bytes(K, BITS) +
-              static_cast<int64_t>(kHalfDeep ? t0 / 2 : t0) * 1024 + lane * 16;
+    bsrc[c] = codes + static_cast<int64_t>(st) * strip_bytes(K, BITS) + static_cast<int64_t>(t0) * 1024 + lane * 16;
   }
-  unsigned char* const braw_lds = smem + kStages * kStage;  // kHalfDeep: the two raw B tiles
-  const int npairs = niter / 2;                             // kHalfDeep: raw B tiles of the run
   const int swz = a_swizzle<C>(lane & 15);  // fragment rows are 32*t + r32; the swizzle has period 16
 
   // Group scales travel with the tile: value v = 2 * (64 * wave + lane) of the
@@ -518,78 +412,34 @@ __device__ __forceinline__ void dma_tile(std::conditional_t<EXPERTS, const DmaPa
   const int sval = 2 * (wave * 64 + lane) < kGT * BN ? 2 * (wave * 64 + lane) : 0;
   const int sfold = sval / BN;
   int scol = strip_blk * kStripCols + sval % BN;
-  if (SWI) {
-    // position p of the tile's columns is column p % 32 of block (p / 32) % 2 of wavefront column p / 64:
-    // the gate columns of that wavefront column, or the up columns N / 2 further on
-    const int pcol = sval % BN;
-    scol = (strip_blk + (pcol / 64) * 2) * kStripCols + pcol % 32;
-    scol = scol < n_hi ? scol : n_hi - 2;
-    scol += ((pcol / 32) % 2) * (N / 2);
-  }
-  scol = scol < (SWI ? N : n_hi) ? scol : n_hi - 2;  // past the last column: valid data, never used
-  // Loads lo .. hi-1 of tile `it` into its stage; a stage's loads are numbered
-  // [scales,] A loads, B loads.
-  auto issue_range = [&](int it, int lo, int hi, bool odd) {  // odd: parity of it, a constant where it is called
+  scol = scol < n_hi ? scol : n_hi - 2;  // past the last column: valid data, never used
+  // The loads of tile `it` into its stage: [scales,] A loads, B loads.  They go out right behind the barrier that frees the
+  // stage.
+  auto issue = [&](int it) {
     const int t = tile_index(it);  // past the end: reload the last tile into a spare stage
     unsigned char* stage = smem + (it % kStages) * kStage;
-    constexpr int kS = G == 0 ? 0 : 1;
-    if (G != 0 && lo == 0 && hi > 0) {
+    if (G != 0) {
       const int64_t row = (static_cast<int64_t>(t0 + t) * TK + sfold * kFoldK) >> kGShift;
       __builtin_amdgcn_global_load_lds(scale + row * N + scol,
                                        (lds_ptr_t)(stage + kScaleOff + wave * 256), 4, 0, 0);
     }
 #pragma unroll
     for (int c = 0; c < kALoads; ++c)
-      if (kS + c >= lo && kS + c < hi)
-        __builtin_amdgcn_global_load_lds(asrc[c] + t * TK, (lds_ptr_t)(stage + (c * NW + wave) * 1024), 16, 0, 0);
-    if constexpr (kHalfDeep) {
-      // tile 2T - 1 brings the first half of raw B tile T, tile 2T the second (past the end: the last one again,
-      // into a buffer that nobody reads any more)
-      const int T = (it + 1) / 2, src = T < npairs ? T : npairs - 1;
-      unsigned char* dst = braw_lds + (T & 1) * kBBytes;
-      if (odd) {
+      __builtin_amdgcn_global_load_lds(asrc[c] + t * TK, (lds_ptr_t)(stage + (c * NW + wave) * 1024), 16, 0, 0);
 #pragma unroll
-        for (int c = 0; c < kBLoads; ++c)
-          if (kS + kALoads + c >= lo && kS + kALoads + c < hi)
-            __builtin_amdgcn_global_load_lds(bsrc[c] + src * 1024, (lds_ptr_t)(dst + (c * NW + wave) * 1024), 16, 0, 0);
-      } else {
-#pragma unroll
-        for (int c = 0; c < kBLoads; ++c)
-          if (kS + kALoads + c >= lo && kS + kALoads + c < hi)
-            __builtin_amdgcn_global_load_lds(bsrc[kBLoads + c] + src * 1024,
-                                             (lds_ptr_t)(dst + ((kBLoads + c) * NW + wave) * 1024), 16, 0, 0);
-      }
-    } else {
-#pragma unroll
-      for (int c = 0; c < kBLoads; ++c)
-        if (kS + kALoads + c >= lo && kS + kALoads + c < hi)
-          __builtin_amdgcn_global_load_lds(bsrc[c] + t * 1024,
-                                           (lds_ptr_t)(stage + kABytes + (c * NW + wave) * 1024), 16, 0, 0);
-    }
+    for (int c = 0; c < kBLoads; ++c)
+      __builtin_amdgcn_global_load_lds(bsrc[c] + t * 1024,
+                                       (lds_ptr_t)(stage + kABytes + (c * NW + wave) * 1024), 16, 0, 0);
   };
-  // With three stages the loads of tile it+3 may be issued anywhere between the
-  // barrier of tile `it` (which frees their stage) and the barrier of tile it+1,
-  // and still have a whole tile period to land.  They are spread over that
-  // period, a few per slice: issued in one burst right behind the barrier, the
-  // loads of all wavefronts meet in the one load path of the CU at the same
-  // moment, and a wavefront that waits there issues no MFMA.  Segment 0 is the
-  // half slice behind the barrier, segment 1 the last slice of the tile,
-  // segments 2 .. Q-1 the slices 0 .. Q-3 of the next tile.  Two stages leave
-  // no such freedom: everything goes out behind the barrier.
-  constexpr bool kSpread = kStages == 3;
-  auto seg_lo = [](int s) { return kSpread ? (s * kPerStage + Q - 1) / Q : (s > 0 ? kPerStage : 0); };
-  auto seg_n = [&](int s) { return seg_lo(s + 1) - seg_lo(s); };
 
   // columns of this lane's accumulators: block c of the wavefront, column r32
-  const int col0 = (strip_blk + (kPair ? wn / 2 : wn) * (SWI ? 1 : TN) * 2) * 16;
+  const int col0 = (strip_blk + wn * TN * 2) * 16;
   int ncol[TN];
 #pragma unroll
   for (int c = 0; c < TN; ++c) {
     const int n = col0 + c * 32 + r32;
     ncol[c] = n < n_hi ? n : n_hi - 1;
-    if (SWI && c == 1) ncol[c] = ncol[0] + N / 2;
   }
-  if (kPair && wn % 2 == 1) ncol[0] += N / 2;
   // this lane's scales of the tile in `stage`, out of LDS
   auto read_scales = [&](const unsigned char* stage, uint16_t (&dst)[kGT > 0 ? kGT : 1][TN]) {
     if (G != 0) {
@@ -603,37 +453,27 @@ __device__ __forceinline__ void dma_tile(std::conditional_t<EXPERTS, const DmaPa
   };
 
   f32x16 tot[TM][TN];
-  f32x16 part[G != 0 && !RESC ? TM : 1][G != 0 && !RESC ? TN : 1];
-  float unit[TN], mrun[TN];  // RESC: what one unit of this lane's sums of block c is worth; the largest scale so far
-#pragma unroll
-  for (int c = 0; c < TN; ++c) unit[c] = mrun[c] = 0.0f;
-  f32x16 canc[OFFS == 1 ? TM : 1];
-  float rsum[OFFS == 2 ? TM : 1];  // this lane's share of the sum of the activations of row r32 of block a
+  f32x16 part[G != 0 ? TM : 1][G != 0 ? TN : 1];
+  f32x16 canc[OFFS ? TM : 1];
 #pragma unroll
   for (int a = 0; a < TM; ++a) {
 #pragma unroll
     for (int c = 0; c < TN; ++c)
 #pragma unroll
       for (int r = 0; r < 16; ++r) tot[a][c][r] = 0.0f;
-    if (OFFS == 1) {
+    if (OFFS) {
 #pragma unroll
       for (int r = 0; r < 16; ++r) canc[a][r] = 0.0f;
     }
-    if (OFFS == 2) rsum[a] = 0.0f;
   }
   uint32_t magic = Dequant<DT, BITS>::kMagic;
   asm volatile("" : "+v"(magic));  // keep the constant in a VGPR
 
   // byte offsets inside a stage that do not change from tile to tile
   const int a_row_off = (wm * TM * 32 + r32) * (TK * 2);
-  const int b_off = (kHalfDeep ? 0 : kABytes) + (wn * TN * 2 + sp) * 1024 + (j + 16 * b) * 16;  // kHalfDeep: in a raw B tile
-  constexpr int kValuPerMfma = ((OFFS == 2 ? 4 * TN + 4 * TM : (BITS == 8 ? 16 : kFmaDequant && DT == WOL_DTYPE_BF16 ? 18 : 12) * TN) + TM * TN - 1) / (TM * TN) + 2;
-  constexpr int kValuRescale = RESC ? 16 : 0;  // more per MFMA in the slice that starts a group
+  const int b_off = kABytes + (wn * TN * 2 + sp) * 1024 + (j + 16 * b) * 16;
+  constexpr int kValuPerMfma = ((BITS == 8 ? 16 : kFmaDequant && DT == WOL_DTYPE_BF16 ? 18 : 12) * TN + TM * TN - 1) / (TM * TN) + 2;
   constexpr int kHalf = (TM * TN + 1) / 2;  // MFMAs of a slice issued before the barrier
-  // (With one workgroup per CU, wavefronts w and w + 4 share a SIMD and the older one wins every
-  // arbitration: it finishes a k tile in two thirds of the tile's time and waits out the rest at the
-  // barrier.  Handing the priority back and forth with s_setprio evens their arrival out and makes the
-  // kernel 3 % slower: the tile's period follows the sum of their work, and the switches add to it.)
 
   // The wavefront's pipeline registers: raw codes of the current and the next
   // tile, and two sets of operands -- the one the MFMAs of slice q use and the
@@ -668,50 +508,22 @@ __device__ __forceinline__ void dma_tile(std::conditional_t<EXPERTS, const DmaPa
     }
   };
   // MFMAs lo .. hi-1 (numbered a * TN + c) of slice q
-  // gstart: the tile starts a group (a group of 128 spans two int8 tiles: the second one of a pair does not)
-  auto mfmas = [&](const u32x4 (&a4)[TM], const u32x4 (&b4)[TN], int q, int lo, int hi, bool gstart = true) {
-    const bool first = q % kFold == 0 && (!RESC || gstart);
+  auto mfmas = [&](const u32x4 (&a4)[TM], const u32x4 (&b4)[TN], int q, int lo, int hi) {
+    const bool first = q % kFold == 0;
     f32x16 zero;
 #pragma unroll
     for (int r = 0; r < 16; ++r) zero[r] = 0.0f;
-    float rho[TN];
-    if (RESC && first) {
-#pragma unroll
-      for (int c = 0; c < TN; ++c) {
-        const float s = to_f32<DT>(sraw[q / kFold][c]);
-        mrun[c] = fmaxf(mrun[c], s);
-        const float u0 = fmaxf(s, mrun[c] * 0x1p-64f);
-        // a scale of zero before any other (or one in the denormal range, which the reciprocal below
-        // does not take): the unit stays what it is
-        const float u = u0 < 0x1p-126f ? unit[c] : u0;
-        // what was summed under a unit of zero (groups whose scale is zero may hold any codes) counts
-        // for nothing; inside a group, and from a group to one of the same scale, nothing changes
-        rho[c] = unit[c] == 0.0f ? 0.0f : (u == unit[c] ? 1.0f : unit[c] * __builtin_amdgcn_rcpf(u));
-        unit[c] = u;
-      }
-    }
 #pragma unroll
     for (int a = 0; a < TM; ++a)
 #pragma unroll
       for (int c = 0; c < TN; ++c)
         if (a * TN + c >= lo && a * TN + c < hi) {
-          if (OFFS == 2 && c == 0) {
-            rsum[a] = sum8<DT>(a4[a], rsum[a]);
-            // pinned to this slice: left alone the compiler sinks the sums of a
-            // whole tile behind the loop's branch and keeps every fragment alive for them
-            asm volatile("" : "+v"(rsum[a]));
-          }
-          if (OFFS == 1 && c == 0) {
+          if (OFFS && c == 0) {
             const u32x4 cb = {Dequant<DT, BITS>::kCancel, Dequant<DT, BITS>::kCancel,
                               Dequant<DT, BITS>::kCancel, Dequant<DT, BITS>::kCancel};
             canc[a] = mfma32<DT>(a4[a], cb, (G != 0 && first) ? zero : canc[a]);
           }
-          if (RESC && first) {
-            f32x16 t = tot[a][c];
-#pragma unroll
-            for (int r = 0; r < 16; ++r) t[r] *= rho[c];
-            tot[a][c] = mfma32<DT>(a4[a], b4[c], t);
-          } else if (G == 0 || RESC) {
+          if (G == 0) {
             tot[a][c] = mfma32<DT>(a4[a], b4[c], tot[a][c]);
           } else if (first) {
             part[a][c] = mfma32<DT>(a4[a], b4[c], zero);
@@ -722,7 +534,7 @@ __device__ __forceinline__ void dma_tile(std::conditional_t<EXPERTS, const DmaPa
   };
   // after the last slice of a group: tot += part * scale
   auto fold = [&](const uint16_t (&sr)[kGT > 0 ? kGT : 1][TN], int q) {
-    if (G != 0 && !RESC && q % kFold == kFold - 1) {
+    if (G != 0 && q % kFold == kFold - 1) {
 #pragma unroll
       for (int c = 0; c < TN; ++c) {
         const float sc = to_f32<DT>(sr[q / kFold][c]);
@@ -730,39 +542,26 @@ __device__ __forceinline__ void dma_tile(std::conditional_t<EXPERTS, const DmaPa
         for (int a = 0; a < TM; ++a)
 #pragma unroll
           for (int r = 0; r < 16; ++r)
-            tot[a][c][r] = fmaf(OFFS == 1 ? part[a][c][r] + canc[a][r] : part[a][c][r], sc, tot[a][c][r]);
+            tot[a][c][r] = fmaf(OFFS ? part[a][c][r] + canc[a][r] : part[a][c][r], sc, tot[a][c][r]);
       }
     }
   };
 
-  if constexpr (kHalfDeep) {  // the first half of raw B tile 0, which no tile before tile 0 brings
-#pragma unroll
-    for (int c = 0; c < kBLoads; ++c)
-      __builtin_amdgcn_global_load_lds(bsrc[c], (lds_ptr_t)(braw_lds + (c * NW + wave) * 1024), 16, 0, 0);
-  }
-  issue_range(0, 0, kPerStage, false);
-  issue_range(1, 0, kPerStage, true);
-  if (kStages == 3) issue_range(2, 0, seg_lo(2), false);  // the rest of tile 2 goes out during tile 0
-  wait_vmcnt<(kStages - 2) * kPerStage + (kStages == 3 ? (2 * kPerStage + Q - 1) / Q : kPerStage)>();  // tile 0 has landed
+  issue(0);
+  issue(1);
+  wait_vmcnt<kPerStage>();  // tile 0 has landed
   __builtin_amdgcn_s_barrier();
-  if (STAMP) st_loop0 = st_prev = __builtin_readcyclecounter();
-  read_b(kHalfDeep ? braw_lds : smem, braw[0]);
+  read_b(smem, braw[0]);
   read_a(smem, af[0], 0);
   dequant(bf[0], braw[0], 0);
   // Every slice runs its MFMAs with the preparation of the next slice's
   // operands (A fragments read from LDS, B fragments dequantised) spread
   // between them, so that the VALU work executes in the shadow of the matrix
   // pipe.  The workgroup barrier that hands the stage of tile `it` over to
-  // tile it+3 sits in the middle of the last but one slice, once the
+  // tile it+2 sits in the middle of the last but one slice, once the
   // wavefront has fetched its last operands of the tile; the raw codes of tile
   // it+1 are read right behind it and have a whole slice to arrive.
-  auto tile = [&](auto odd_tile, int it, u32x4 (&raw)[TN][2], u32x4 (&raw_next)[TN][2]) {
-    // RESC with groups of two tiles: the run starts on a group (launch_dma sees to it), so odd tiles continue one
-    constexpr bool gstart = !(RESC && G > TK && decltype(odd_tile)::value);
-    // kHalfDeep: an odd tile consumes the second half of the raw codes and reads the next raw tile
-    constexpr bool kOdd = decltype(odd_tile)::value;
-    constexpr int q0 = kHalfDeep && kOdd ? Q : 0;
-    constexpr bool kNewB = !kHalfDeep || kOdd;
+  auto tile = [&](int it, u32x4 (&raw)[TN][2], u32x4 (&raw_next)[TN][2]) {
     const unsigned char* stage = smem + (it % kStages) * kStage;
     const unsigned char* next = smem + ((it + 1) % kStages) * kStage;
     read_scales(stage, sraw);  // before the stage is handed over
@@ -770,22 +569,14 @@ __device__ __forceinline__ void dma_tile(std::conditional_t<EXPERTS, const DmaPa
     for (int q = 0; q < Q; ++q) {
       if (q != Q - 2) {
         const bool last = q == Q - 1;
-        // this slice's share of the tile loads (segment 1 of tile it+3, or segment q+2 of tile it+2)
-        const int seg = last ? 1 : q + 2;
-        if (kSpread) issue_range(last ? it + kStages : it + kStages - 1, seg_lo(seg), seg_lo(seg + 1), last != kOdd);
         read_a(last ? next : stage, af[(q + 1) & 1], last ? 0 : q + 1);
-        dequant(bf[(q + 1) & 1], last && kNewB ? raw_next : raw, last && kNewB ? 0 : q0 + q + 1);
-        mfmas(af[q & 1], bf[q & 1], q, 0, TM * TN, gstart);
+        dequant(bf[(q + 1) & 1], last ? raw_next : raw, last ? 0 : q + 1);
+        mfmas(af[q & 1], bf[q & 1], q, 0, TM * TN);
 #pragma unroll
         for (int i = 0; i < TM * TN; ++i) {
           __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);                   // one MFMA
           if (i < TM) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);       // one LDS read
-          if (kSpread && i % 2 == 1 && i / 2 < seg_n(seg)) {
-            __builtin_amdgcn_sched_group_barrier(0x004, 2, 0);                 // its LDS address into m0
-            __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);                 // one tile load
-          }
-          if (RESC && gstart && q % kFold == 0) __builtin_amdgcn_sched_group_barrier(0x002, kValuPerMfma + kValuRescale, 0);
-          else __builtin_amdgcn_sched_group_barrier(0x002, kValuPerMfma, 0);  // VALU
+          __builtin_amdgcn_sched_group_barrier(0x002, kValuPerMfma, 0);        // VALU
         }
         __builtin_amdgcn_sched_barrier(0);
         fold(sraw, q);
@@ -800,113 +591,46 @@ __device__ __forceinline__ void dma_tile(std::conditional_t<EXPERTS, const DmaPa
         __builtin_amdgcn_sched_barrier(0);
         // this wavefront needs nothing more from the tile's stage; once every
         // wavefront is there, tile it+1 (landed by now) may be read and the
-        // stage refilled with tile it+3
+        // stage refilled with tile it+2
         __builtin_amdgcn_s_waitcnt(0x0070 | (0xF << 0) | (3 << 14));  // lgkmcnt(0)
-        unsigned long long st_a = 0, st_b = 0;
-        if (STAMP) st_a = __builtin_readcyclecounter();
-        wait_vmcnt<(kStages - 2) * kPerStage>();
-        if (STAMP) st_b = __builtin_readcyclecounter();
+        wait_vmcnt<0>();
         __builtin_amdgcn_s_barrier();
-        if (STAMP) {
-          const unsigned long long st_c = __builtin_readcyclecounter();
-          st_work += st_a - st_prev;
-          st_loads += st_b - st_a;
-          st_bar += st_c - st_b;
-          st_prev = st_c;
-        }
-        issue_range(it + kStages, 0, seg_lo(1), !kOdd);
-        if (kNewB) read_b(kHalfDeep ? braw_lds + (((it + 1) / 2) & 1) * kBBytes : next, raw_next);
-        dequant(bf[(q + 1) & 1], raw, q0 + q + 1);
+        issue(it + kStages);
+        read_b(next, raw_next);
+        dequant(bf[(q + 1) & 1], raw, q + 1);
         mfmas(af[q & 1], bf[q & 1], q, kHalf, TM * TN);
 #pragma unroll
         for (int i = 0; i < TM * TN - kHalf + 1; ++i) {
           if (i < TM * TN - kHalf) __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-          if (kNewB && i < 2 * TN) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-          if (kSpread && i < seg_n(0)) {
-            __builtin_amdgcn_sched_group_barrier(0x004, 2, 0);
-            __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
-          }
+          if (i < 2 * TN) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
           __builtin_amdgcn_sched_group_barrier(0x002, 2 * kValuPerMfma, 0);
         }
         __builtin_amdgcn_sched_barrier(0);
       }
     }
   };
-  if constexpr (kHalfDeep) {
-    for (int it = 0; it < niter; it += 4) {  // niter is even
-      tile(std::false_type(), it, braw[0], braw[1]);
-      tile(std::true_type(), it + 1, braw[0], braw[1]);
-      if (it + 2 < niter) {
-        tile(std::false_type(), it + 2, braw[1], braw[0]);
-        tile(std::true_type(), it + 3, braw[1], braw[0]);
-      }
-    }
-  } else {
-    for (int it = 0; it < niter; it += 2) {
-      tile(std::false_type(), it, braw[0], braw[1]);
-      if (it + 1 < niter) tile(std::true_type(), it + 1, braw[1], braw[0]);
-    }
+  for (int it = 0; it < niter; it += 2) {
+    tile(it, braw[0], braw[1]);
+    if (it + 1 < niter) tile(it + 1, braw[1], braw[0]);
   }
   wait_vmcnt<0>();
   __builtin_amdgcn_s_barrier();  // the spare loads are done and every wavefront has stopped reading
-  unsigned long long st_loop1 = 0;
-  if (STAMP) st_loop1 = __builtin_readcyclecounter();
-  // the stamps leave at the end of the epilogue (lane 0 of every wavefront)
-  auto leave_stamps = [&]() {
-    if (STAMP && lane == 0 && p.stamps != nullptr) {
-      unsigned long long* o = p.stamps + (static_cast<size_t>(blockIdx.x) * NW + wave) * 8;
-      const unsigned long long st_end = __builtin_readcyclecounter();
-      o[0] = st_loop0 - st_entry;   // entry to the first tile's barrier
-      o[1] = st_work;               // between the barriers: MFMAs and everything issued among them
-      o[2] = st_loads;              // waiting for this wavefront's own tile loads
-      o[3] = st_bar;                // waiting for the other wavefronts
-      o[4] = st_loop1 - st_prev;    // the last tile's tail and the closing barrier
-      o[5] = st_end - st_loop1;     // epilogue
-      o[6] = st_end - st_entry;     // all of it
-      o[7] = static_cast<unsigned long long>(niter);
-    }
-  };
 
   // ---- epilogue: scale, bias, cast; 32-row slabs leave through LDS as 16-byte stores ----
   // accumulator element r of lane l is row 8*(r/4) + 4*(l/32) + r%4, column l%32 of its block
   float sc[TN], bv[TN];
 #pragma unroll
   for (int c = 0; c < TN; ++c) {
-    sc[c] = RESC ? unit[c] : (G == 0 ? to_f32<DT>(scale[ncol[c]]) : 1.0f);
+    sc[c] = G == 0 ? to_f32<DT>(scale[ncol[c]]) : 1.0f;
     bv[c] = (bias != nullptr && p.nsplit == 1) ? to_f32<DT>(bias[ncol[c]]) : 0.0f;
   }
-  if (OFFS == 1 && G == 0) {
+  if (OFFS && G == 0) {
 #pragma unroll
     for (int a = 0; a < TM; ++a)
 #pragma unroll
       for (int c = 0; c < TN; ++c)
 #pragma unroll
         for (int r = 0; r < 16; ++r) tot[a][c][r] += canc[a][r];
-  }
-  if (OFFS == 2) {
-    // Row sums: lanes l and l + 32 hold the two halves of row r32's sum.  They
-    // are added and parked in LDS (the stages are free now), from where a lane
-    // takes the sums of the sixteen rows its accumulators belong to.
-    constexpr int kRsOff = kLds - NW * TM * 32 * 4;  // the end of the stages; the slabs use their start
-    static_assert(kRsOff >= NW * 32 * ((SWI ? 1 : TN) * 32 + 8) * 2, "row sums and slabs must not overlap");
-    float* rsl = reinterpret_cast<float*>(smem + kRsOff) + wave * TM * 32;
-#pragma unroll
-    for (int a = 0; a < TM; ++a) {
-      const float other = __builtin_bit_cast(float, __builtin_amdgcn_ds_bpermute(((lane ^ 32) << 2), __builtin_bit_cast(int, rsum[a])));
-      if (b == 0) rsl[a * 32 + r32] = rsum[a] + other;
-    }
-    __builtin_amdgcn_wave_barrier();
-#pragma unroll
-    for (int a = 0; a < TM; ++a)
-#pragma unroll
-      for (int q4 = 0; q4 < 4; ++q4) {
-        const f32x4 rv = *reinterpret_cast<const f32x4*>(&rsl[a * 32 + 8 * q4 + 4 * b]);
-#pragma unroll
-        for (int c = 0; c < TN; ++c)
-#pragma unroll
-          for (int e = 0; e < 4; ++e) tot[a][c][4 * q4 + e] = fmaf(-Dequant<DT, BITS>::kOffset, rv[e], tot[a][c][4 * q4 + e]);
-      }
-    __builtin_amdgcn_wave_barrier();
   }
   if (p.out_f32 || p.nsplit > 1) {
     // fp32 results (verification mode) or partial sums of this run of k tiles: plain stores
@@ -932,87 +656,35 @@ __device__ __forceinline__ void dma_tile(std::conditional_t<EXPERTS, const DmaPa
     return;
   }
   uint16_t* out = static_cast<uint16_t*>(outp);
-  constexpr int kOutBlocks = SWI ? 1 : TN;        // 32-column blocks a wavefront writes
-  constexpr int kSlabRow = kOutBlocks * 32 + 8;   // padded, in elements
+  constexpr int kSlabRow = TN * 32 + 8;   // padded, in elements
   static_assert(NW * 32 * kSlabRow * 2 <= kLds, "slabs must fit in the stage buffers");
   uint16_t* slab = reinterpret_cast<uint16_t*>(smem) + wave * 32 * kSlabRow;
-  constexpr int kPieces = 32 * (kOutBlocks * 32 / 8);
-  const int ld_out = SWI ? N / 2 : N;             // row length of the output
-  if constexpr (kPair) {
-    // behind the slabs: one block of fp32 sums per pair of wavefronts
-    constexpr int kXOff = (NW * 32 * kSlabRow * 2 + 255) / 256 * 256;
-    static_assert(kXOff + NW / 2 * 4096 <= kLds, "slabs and handed-over sums must fit in the stage buffers");
-    float* xbuf = reinterpret_cast<float*>(smem + kXOff) + (wave / 2) * 1024;
-#pragma unroll
-    for (int a = 0; a < TM; ++a) {
-      if (wn % 2 == 1) {
-#pragma unroll
-        for (int r = 0; r < 16; ++r) xbuf[r * 64 + lane] = tot[a][0][r] * sc[0] + bv[0];
-      }
-      __syncthreads();
-      if (wn % 2 == 0) {
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          float g = tot[a][0][r] * sc[0] + bv[0], u = xbuf[r * 64 + lane];
-          if (SWI == 2) {
-            g = to_f32<DT>(cast_out<DT>(g));
-            u = to_f32<DT>(cast_out<DT>(u));
-          }
-          slab[(8 * (r / 4) + 4 * b + r % 4) * kSlabRow + r32] = cast_out<DT>(act_swiglu(g, u));
-        }
-        __builtin_amdgcn_wave_barrier();
-#pragma unroll
-        for (int q = lane; q < kPieces; q += 64) {
-          const int r = q / 4, cc = q % 4;
-          const int m = m0 + (wm * TM + a) * 32 + r;
-          const int n = col0 + cc * 8;
-          const u32x4 v = *reinterpret_cast<const u32x4*>(&slab[r * kSlabRow + cc * 8]);
-          if (m < M && n < n_hi) *reinterpret_cast<u32x4*>(out + static_cast<int64_t>(m) * ld_out + n) = v;
-        }
-      }
-      __syncthreads();  // the handed-over sums have been read
-    }
-    return;
-  }
+  constexpr int kPieces = 32 * (TN * 32 / 8);
 #pragma unroll
   for (int a = 0; a < TM; ++a) {
-    if (SWI) {
 #pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        float g = tot[a][0][r] * sc[0] + bv[0], u = tot[a][TN - 1][r] * sc[TN - 1] + bv[TN - 1];
-        if (SWI == 2) {  // as if fc1 had been written out in T and read back
-          g = to_f32<DT>(cast_out<DT>(g));
-          u = to_f32<DT>(cast_out<DT>(u));
-        }
-        slab[(8 * (r / 4) + 4 * b + r % 4) * kSlabRow + r32] = cast_out<DT>(act_swiglu(g, u));
-      }
-    } else {
+    for (int c = 0; c < TN; ++c)
 #pragma unroll
-      for (int c = 0; c < TN; ++c)
-#pragma unroll
-        for (int r = 0; r < 16; ++r)
-          slab[(8 * (r / 4) + 4 * b + r % 4) * kSlabRow + c * 32 + r32] =
-              cast_out<DT>(act_apply(tot[a][c][r] * sc[c] + bv[c], p.act));
-    }
+      for (int r = 0; r < 16; ++r)
+        slab[(8 * (r / 4) + 4 * b + r % 4) * kSlabRow + c * 32 + r32] =
+            cast_out<DT>(act_apply(tot[a][c][r] * sc[c] + bv[c], p.act));
     __builtin_amdgcn_wave_barrier();
 #pragma unroll
     for (int q = lane; q < kPieces; q += 64) {
-      const int r = q / (kOutBlocks * 4), cc = q % (kOutBlocks * 4);
+      const int r = q / (TN * 4), cc = q % (TN * 4);
       const int m = m0 + (wm * TM + a) * 32 + r;
       const int n = col0 + cc * 8;
       const u32x4 v = *reinterpret_cast<const u32x4*>(&slab[r * kSlabRow + cc * 8]);
-      if (m < M && n < n_hi) *reinterpret_cast<u32x4*>(out + static_cast<int64_t>(m) * ld_out + n) = v;
+      if (m < M && n < n_hi) *reinterpret_cast<u32x4*>(out + static_cast<int64_t>(m) * N + n) = v;
     }
     __builtin_amdgcn_wave_barrier();
   }
-  leave_stamps();
 #endif
 }
 
-template <int DT, int BITS, int G, int OFFS, int WM, int WN, int TM, int TN, int STAGES, int SWI = 0, bool RESC = false,
-          bool STAMP = false>
+template <int DT, int BITS, int G, bool OFFS, int WM, int WN, int TM, int TN>
 __global__ __launch_bounds__(64 * WM * WN) void gemm_dma_kernel(const DmaParams p) {
-  dma_tile<DT, BITS, G, OFFS, WM, WN, TM, TN, STAGES, SWI, RESC, STAMP, false>(p, TilePlace{});
+  dma_tile<DT, BITS, G, OFFS, WM, WN, TM, TN>(p);
 }
 
 // out[m, col0 + c] = T( sum over the runs of part[run][m][c] + bias[col0 + c] ) for the ncols
@@ -1148,27 +820,21 @@ inline int plan_xcd_rows(int nbx, int nby, int a_bytes, int b_bytes) {
   return best;
 }
 
-template <int BITS, int G, int WM, int WN, int TM, int TN, int STAGES = 3>
+template <int BITS, int G, int WM, int WN, int TM, int TN>
 constexpr size_t dma_lds_bytes() {
-  if (STAGES > kHalfDeepStages)
-    return STAGES % kHalfDeepStages * (static_cast<size_t>(WM * TM * 32) * 64 * 2 + (G == 0 ? 0 : WM * WN * 256)) +
-           2 * (WN * TN * 32 / 16) * 1024;
-  return STAGES * (static_cast<size_t>(WM * TM * 32) * (BITS == 8 ? 64 : 128) * 2 +
+  return 2 * (static_cast<size_t>(WM * TM * 32) * (BITS == 8 ? 64 : 128) * 2 +
               (WN * TN * 32 / 16) * 1024 + (G == 0 ? 0 : WM * WN * 256));
 }
 
 // Launches the fast kernel on the columns of strips [strip_lo, strip_hi), K
 // cut into nsplit runs (nsplit > 1 needs a.ws: nsplit x M x columns floats).
-// SWI != 0 (swiglu epilogue): the strips are those of the gate half, [0, N / 32), a.out is [M, N / 2].
-template <int DT, int BITS, int G, int OFFS, int WM, int WN, int TM, int TN, int STAGES = 3, int SWI = 0, bool RESC = false>
+template <int DT, int BITS, int G, bool OFFS, int WM, int WN, int TM, int TN>
 void launch_dma(const Args& a, int strip_lo, int strip_hi, int nsplit) {
-  constexpr int BM = WM * TM * 32, BN = (SWI ? TN * WN * 16 : TN * WN * 32);  // BN: output columns
-  constexpr bool half_deep = STAGES > kHalfDeepStages;
-  constexpr int TK = BITS == 8 || half_deep ? 64 : 128;
+  constexpr int BM = WM * TM * 32, BN = TN * WN * 32;
+  constexpr int TK = BITS == 8 ? 64 : 128;
   if (strip_hi <= strip_lo) return;
-  if (SWI) nsplit = 1;
-  constexpr size_t lds = dma_lds_bytes<BITS, G, WM, WN, TM, TN, STAGES>();
-  auto kern = gemm_dma_kernel<DT, BITS, G, OFFS, WM, WN, TM, TN, STAGES, SWI, RESC>;
+  constexpr size_t lds = dma_lds_bytes<BITS, G, WM, WN, TM, TN>();
+  auto kern = gemm_dma_kernel<DT, BITS, G, OFFS, WM, WN, TM, TN>;
   static std::atomic<uint32_t> configured{0};  // per instantiation
   allow_lds(reinterpret_cast<const void*>(kern), lds, configured);
   const int ncols = (strip_hi - strip_lo) * kStripCols;
@@ -1188,7 +854,6 @@ void launch_dma(const Args& a, int strip_lo, int strip_hi, int nsplit) {
   p.nby = (a.M + BM - 1) / BM;
   const int tiles = a.K / TK;
   p.tiles_per_split = (tiles + nsplit - 1) / nsplit;
-  if ((RESC && G > TK) || half_deep) p.tiles_per_split = (p.tiles_per_split + 1) & ~1;  // every run starts on a group (a raw B tile) of two tiles
   p.nsplit = (tiles + p.tiles_per_split - 1) / p.tiles_per_split;
   p.xcd_rows = plan_xcd_rows(p.nbx, p.nby, BM * 2, WN * TN * 32 * BITS / 8);
   p.act = a.act;
@@ -1199,7 +864,7 @@ void launch_dma(const Args& a, int strip_lo, int strip_hi, int nsplit) {
   kern<<<dim3(static_cast<unsigned>(p.nbx * p.nby * p.nsplit)), dim3(64 * WM * WN), lds, a.stream>>>(p);
   if (nsplit > 1) {
     const int64_t total = static_cast<int64_t>(a.M) * ncols;
-    if (!SWI && a.act == WOL_ACT_SWIGLU) {
+    if (a.act == WOL_ACT_SWIGLU) {
       // a gate|up projection whose runs cover all of N (the small-M configurations): the kernel
       // that adds the runs forms silu(gate) * up, out is [M, N / 2]
       reduce_partials_swiglu_kernel<DT><<<dim3(static_cast<unsigned>((total / 8 + 255) / 256)), dim3(256), 0, a.stream>>>(
@@ -1387,15 +1052,15 @@ void launch_fast(const Args& a) {
     const int ns = sp.ns;
     if constexpr (BITS == 4) {
       if (a.M <= 32) {
-        if (wide) launch_dma<DT, BITS, G, true, 1, 8, 1, 2, 2>(a, 0, nstrips, ns);
-        else launch_dma<DT, BITS, G, true, 1, 8, 1, 1, 2>(a, 0, nstrips, ns);
+        if (wide) launch_dma<DT, BITS, G, true, 1, 8, 1, 2>(a, 0, nstrips, ns);
+        else launch_dma<DT, BITS, G, true, 1, 8, 1, 1>(a, 0, nstrips, ns);
         return;
       }
     }
     if constexpr (!(BITS == 4 && G == 64)) {
-      if (wide) { launch_dma<DT, BITS, G, false, 1, 8, 2, 2, 2>(a, 0, nstrips, ns); return; }
+      if (wide) { launch_dma<DT, BITS, G, false, 1, 8, 2, 2>(a, 0, nstrips, ns); return; }
     }
-    launch_dma<DT, BITS, G, false, 1, 8, 2, 1, 2>(a, 0, nstrips, ns);
+    launch_dma<DT, BITS, G, false, 1, 8, 2, 1>(a, 0, nstrips, ns);
     return;
   }
   // 256 x 256 tiles for as many column tiles as fill whole rounds of the CUs; the
@@ -1583,15 +1248,14 @@ struct MoeLaunch {
 
 // One grouped GEMM: every expert's rows against that expert's weights, tiles
 // of WM * TM * 32 rows x 256 columns, per-channel scales, out [rows, N] T.
-template <int DT, int BITS, int OFFS, int WM, int WN, int TM, int TN, int STAGES>
+template <int DT, int BITS, bool OFFS, int WM, int WN, int TM, int TN>
 void launch_moe_gemm_cfg(const void* x, const MoeLaunch& ml, const void* codes, const void* bias,
                          const void* scale, int64_t K, int64_t N, void* out, hipStream_t stream) {
   const int* table = ml.table;
   const int max_tiles = ml.max_tiles;
-  static_assert(WM == 1, "the larger tiles of gemm_dma_kernel do not read the expert table");
   constexpr int BN = TN * WN * 32;  // output columns of a tile
-  constexpr size_t lds = dma_lds_bytes<BITS, 0, WM, WN, TM, TN, STAGES>();
-  auto kern = gemm_dma_kernel<DT, BITS, 0, OFFS, WM, WN, TM, TN, STAGES>;
+  constexpr size_t lds = dma_lds_bytes<BITS, 0, WM, WN, TM, TN>();
+  auto kern = gemm_dma_kernel<DT, BITS, 0, OFFS, WM, WN, TM, TN>;
   static std::atomic<uint32_t> configured{0};
   allow_lds(reinterpret_cast<const void*>(kern), lds, configured);
   DmaParams p;
@@ -1664,11 +1328,11 @@ void launch_moe_gemm(const void* x, const MoeLaunch& ml, const void* codes, cons
   }
   if constexpr (BITS == 4) {
     if (ml.bm == 32) {
-      launch_moe_gemm_cfg<DT, 4, true, 1, 8, 1, 1, 2>(x, ml, codes, bias, scale, K, N, out, stream);
+      launch_moe_gemm_cfg<DT, 4, true, 1, 8, 1, 1>(x, ml, codes, bias, scale, K, N, out, stream);
       return;
     }
   }
-  launch_moe_gemm_cfg<DT, BITS, false, 1, 8, 2, 1, 2>(x, ml, codes, bias, scale, K, N, out, stream);
+  launch_moe_gemm_cfg<DT, BITS, false, 1, 8, 2, 1>(x, ml, codes, bias, scale, K, N, out, stream);
 }
 
 // K runs of a grouped launch with small tiles: as many as bring the workgroups

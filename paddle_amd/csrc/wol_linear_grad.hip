@@ -3,7 +3,7 @@
 // (what paddle/phi/kernels/gpu/weight_only_linear_grad_kernel.cu:27-72
 // computes by dequantising the whole weight to T and calling a library GEMM).
 //
-// Arithmetic.  The contraction runs over n on v_mfma_f32_32x32x16_f16 with fp32
+// Arithmetic.  The contraction runs over n on v_mfma_f32_16x16x32_f16 with fp32
 // accumulation, for both element types T:
 //   c[n]    = the power of two that brings max_g |scale[g, n]| into [2^7, 2^8)
 //   s'[g,n] = scale[g, n] * 2^c[n]                 (exact: a T value fits fp16)
@@ -37,6 +37,13 @@
 // out_grad's tile goes global -> LDS with direct-to-LDS loads, as in the
 // forward GEMM.  Two stages: while chunk `it` is multiplied, chunk it+1 is
 // loaded, converted and stored; one workgroup barrier per chunk.
+//
+// What bounds it: MFMA issue and power, as in the forward's large tiles (a product
+// on 16x16x32 blocks draws less than on 32x32x16 ones), beside 96 VALU
+// instructions of conversion per wavefront and chunk.  Whole call, us, against
+// 32x32x16 blocks in four slices with a slice's conversions in one piece: 8192 x
+// 4096 x 4096 int4 g128 bf16 278 -> 264, int8 283 -> 263; 5000 x 4096 x 14336 int8
+// g64 864 -> 811; 256 x 4096 x 4096 int4 g128 33.3 -> 30.9.
 #include <atomic>
 
 #include "wol_common.h"
@@ -46,7 +53,6 @@ namespace {
 
 typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
-typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 typedef float f32x4v __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) void* lds_ptr_t;
