@@ -16,7 +16,8 @@
 //             (up to eight rows: these three as one kernel)
 //   outlier : sub = T(sum over the outlier columns of x * T(w * wscale)), fp32
 //             sum in ascending column order; leaves at once without outliers
-//   gemm    : acc = qx . w^T in int32 on v_mfma_i32_32x32x32_i8, both operands
+//   gemm    : acc = qx . w^T in int32 on v_mfma_i32_32x32x32_i8 (above 128 rows
+//             16x16x64), both operands
 //             through direct-to-LDS loads, two or three k tiles deep.  The
 //             epilogue is DequantMergeKernel (:415-447): out = T( sub + T(acc *
 //             range * wscale / 127) ), then T(out + bias).
