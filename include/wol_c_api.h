@@ -303,7 +303,7 @@ int wol_linear_grad_f32(const void* out_grad, const void* codes,
  * element-wise pass, in which case the second product may run with K cut into
  * runs and a kernel that adds them).
  * Requires hidden % 128 == 0, inter % 256 == 0, num_experts <= 1024; the
- * workspace (wol_moe_ffn_workspace bytes, 16-byte aligned) holds the table,
+ * workspace (wol_moe_ffn_workspace bytes, 16-byte aligned) holds the tables,
  * the two intermediate tensors and the runs' sums.
  */
 size_t wol_moe_ffn_workspace(int64_t rows, int64_t hidden, int64_t inter,

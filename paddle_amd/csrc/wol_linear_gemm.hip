@@ -1081,44 +1081,44 @@ void launch_fast(const Args& a) {
 // takes the time of its highest tile, and a high tile costs less than its share
 // (part of a tile's time is the same for any height), so one limit of 256 rows
 // is right where tiles fill many rounds and leaves CUs idle where few tiles
-// exist or a last round is nearly empty.  The limit with the shortest estimate
-// over both products is taken:
-//   time of such a tile x sum over the products of k tiles x rounds,
+// exist or a last round is nearly empty.  Each product, with column tiles of its
+// own number, takes the limit with the shortest estimate:
+//   time of such a tile x rounds,
 // a round being what the CUs of an XCD take of its share of the tiles.  The
-// times of 64-, 128- and 192-row tiles against 256-row ones (0.40, 0.57, 0.78 for
-// int4; 0.60, 0.70, 0.85 for int8) and of a 128-column tile against a
-// 256-column one (0.8 and 0.7) are fitted to 616 problems timed under every
-// limit (4 to 64 experts of 65 to 1000 rows, evenly and unequally loaded, hidden
-// 1024 to 4096, fc1 width 2816 to 28672): the choice is 0.9 % (int4) and 0.7 %
-// (int8) slower than the best one on average, 256 rows always 12 % and 5 %.
-// moe_ffn against the limit of 256 rows: 8 experts, hidden 1024, width 2816, 1664
-// rows, int4 64.9 -> 46.6 us, int8 53.9 -> 43.8; 4 experts, 2048, 8192, 960 rows,
-// int4 130 -> 78.
+// times of 64-, 128- and 192-row tiles against 256-row ones (0.46, 0.66, 0.85) and
+// of a 128-column tile against a 256-column one (0.7) come from 11 problems timed
+// under every pair of limits.  A limit of each product's own and these times
+// against one limit for both and the times of the former tiles, 22 problems, whole
+// call: 1.05 x on average, 0.97 to 1.25 (4 experts, hidden 4096, width 11008, 900
+// rows, int4 173 -> 138 us; 8 experts, 2048, 16384, 1500 rows, int4 228 -> 191; 8
+// experts, 4096, 28672, 4096 rows, int4 1311 -> 1283, 1024 rows int8 465 -> 477).
 struct MoeHeights {
   int xcd_cus;      // CUs of an XCD
   int min_units;    // lowest limit the launch grid has room for; 4 = 256 rows, the highest
-  int nbx1, nbx2;   // column tiles of the two products
-  float w1, w2;     // k tiles x column cost of the two products
+  int nbx;          // column tiles
   float tile[4];    // time of a tile of 1 .. 4 units
 };
 constexpr int kMaxUnits = 4;
 
-__host__ __device__ inline int moe_rounds(int tiles, int nbx, int xcd_cus) {
+__host__ __device__ inline float moe_cost(const MoeHeights& h, int tiles, int units) {
   constexpr int kXcd = 8;
-  const int per = (tiles * nbx + kXcd - 1) / kXcd;
-  return (per + xcd_cus - 1) / xcd_cus;
+  const int per = (tiles * h.nbx + kXcd - 1) / kXcd;
+  return h.tile[units - 1] * static_cast<float>((per + h.xcd_cus - 1) / h.xcd_cus);
 }
 
-__host__ __device__ inline float moe_cost(const MoeHeights& h, int tiles, int units) {
-  return h.tile[units - 1] * (h.w1 * static_cast<float>(moe_rounds(tiles, h.nbx1, h.xcd_cus)) +
-                              h.w2 * static_cast<float>(moe_rounds(tiles, h.nbx2, h.xcd_cus)));
-}
+// One product's table: where it goes and what its tiles may be.
+struct MoePlan {
+  MoeTile* table;
+  int max_tiles;
+  MoeHeights heights;
+};
 
 // Row-tile table of a grouped launch.  cum[e] is the number of rows of experts
 // 0 .. e (the inclusive running total that the reference's moe_dispatch returns
 // as token_nums_per_expert,
 // paddle/phi/kernels/fusion/cutlass/moe_dispatch.cu:174-182): expert e owns
-// rows cum[e-1] .. cum[e]-1 and ceil(rows / bm) tiles.  One workgroup.
+// rows cum[e-1] .. cum[e]-1 and ceil(rows / bm) tiles.  One workgroup;
+// EXPERTS: one per product.
 // EXPERTS false: tiles of bm rows, max_tiles entries, unused ones marked -1.
 // EXPERTS true (gemm_experts_kernel): bm is chosen here, where the rows of every
 // expert are known (MoeHeights), entry 0 holds the number of tiles, and an
@@ -1127,8 +1127,11 @@ __host__ __device__ inline float moe_cost(const MoeHeights& h, int tiles, int un
 // 64: the weight side of a tile costs the same whatever its height).
 template <bool EXPERTS>
 __global__ __launch_bounds__(256) void moe_plan_kernel(const int64_t* __restrict__ cum, int num_experts, int bm,
-                                                       int max_tiles, int64_t rows, MoeHeights heights,
-                                                       MoeTile* __restrict__ table) {
+                                                       int64_t rows, MoePlan first, MoePlan second) {
+  const MoePlan& plan = EXPERTS && blockIdx.x == 1 ? second : first;  // EXPERTS: a workgroup per product
+  const MoeHeights& heights = plan.heights;
+  const int max_tiles = plan.max_tiles;
+  MoeTile* __restrict__ table = plan.table;
   __shared__ int first_tile[1025];  // exclusive running total of tiles, by expert
   __shared__ int row_end[1025];     // end of expert e's rows is row_end[e + 1]; row_end[0] = 0
   if (!EXPERTS)
@@ -1522,46 +1525,42 @@ static int moe_max_tiles(int64_t rows, int num_experts, int bm) {
 }
 
 // What the host settles of a gemm_experts_kernel call: the lowest height limit
-// the grid is laid out for, and whether the second product takes 128-column
-// tiles.  The rows of each expert are not known here: even loads are assumed,
-// and for the limit the device looks again (moe_plan_kernel).  Workgroups that
-// find no tile cost little but not nothing, so a limit below 256 rows is offered
-// only where it asks for at most twelve rounds of them.
-static MoeHeights plan_moe_heights(int64_t rows, int64_t hidden, int64_t inter, int num_experts, int bits, bool* narrow) {
+// each product's grid is laid out for, and whether the second product takes
+// 128-column tiles.  The rows of each expert are not known here: even loads are
+// assumed, and for the limit the device looks again (moe_plan_kernel).  Workgroups
+// that find no tile cost little but not nothing, so a limit below 256 rows is
+// offered only where it asks for at most twelve rounds of them.
+static MoeHeights plan_moe_heights(int64_t rows, int64_t cols, int bn, int num_experts, float column_cost) {
   const int cus = num_cus();
   MoeHeights h;
   h.xcd_cus = cus / 8 > 0 ? cus / 8 : 1;
-  h.nbx1 = static_cast<int>((inter / 2 + 127) / 128);
-  h.nbx2 = static_cast<int>((hidden + 255) / 256);
-  h.w1 = static_cast<float>(hidden);
-  h.w2 = static_cast<float>(inter / 2);
-  const float times[2][kMaxUnits] = {{0.60f, 0.70f, 0.85f, 1.0f}, {0.40f, 0.57f, 0.78f, 1.0f}};
-  for (int u = 0; u < kMaxUnits; ++u) h.tile[u] = times[bits == 4][u];
+  h.nbx = static_cast<int>((cols + bn - 1) / bn);
+  const float times[kMaxUnits] = {0.46f, 0.66f, 0.85f, 1.0f};
+  for (int u = 0; u < kMaxUnits; ++u) h.tile[u] = times[u] * column_cost;
   h.min_units = 1;
   while (h.min_units < kMaxUnits &&
-         static_cast<int64_t>(moe_max_tiles(rows, num_experts, h.min_units * 64)) * h.nbx1 > 12 * cus)
+         static_cast<int64_t>(moe_max_tiles(rows, num_experts, h.min_units * 64)) * h.nbx > 12 * cus)
     ++h.min_units;
-  MoeHeights n = h;
-  n.nbx2 = static_cast<int>((hidden + 127) / 128);
-  n.w2 *= bits == 4 ? 0.8f : 0.7f;
-  const int64_t units = ((rows + num_experts - 1) / num_experts + 63) / 64;
-  float best = 0.0f, best_n = 0.0f;
-  for (int u = kMaxUnits; u >= h.min_units; --u) {
-    const int tiles = static_cast<int>((units + u - 1) / u) * num_experts;
-    const float c = moe_cost(h, tiles, u), cn = moe_cost(n, tiles, u);
-    best = u == kMaxUnits || c < best ? c : best;
-    best_n = u == kMaxUnits || cn < best_n ? cn : best_n;
-  }
-  *narrow = best_n < best;
-  return *narrow ? n : h;
+  return h;
 }
 
-// Scratch: [row-tile table][fc1 output rows x inter T][activation rows x inter/2 T]
+// The best estimate under any limit, the experts evenly loaded.
+static float best_moe_cost(const MoeHeights& h, int64_t rows, int num_experts) {
+  const int64_t units = ((rows + num_experts - 1) / num_experts + 63) / 64;
+  float best = 0.0f;
+  for (int u = kMaxUnits; u >= h.min_units; --u) {
+    const float c = moe_cost(h, static_cast<int>((units + u - 1) / u) * num_experts, u);
+    best = u == kMaxUnits || c < best ? c : best;
+  }
+  return best;
+}
+
+// Scratch: [row-tile tables of the two products][fc1 output rows x inter T][activation rows x inter/2 T]
 // [fp32 sums of the second GEMM's K runs, rows x hidden each, when the tiles are small]
 size_t moe_ffn_workspace(int64_t rows, int64_t hidden, int64_t inter, int num_experts) {
   // (the table at its longest: 32-row tiles; the runs' sums whenever either bit width would use small tiles)
   const bool small = moe_tile_rows(rows, num_experts, 4) < 128;
-  return moe_up((static_cast<size_t>(moe_max_tiles(rows, num_experts, 32)) + 1) * sizeof(MoeTile)) +
+  return 2 * moe_up((static_cast<size_t>(moe_max_tiles(rows, num_experts, 32)) + 1) * sizeof(MoeTile)) +
          moe_up(static_cast<size_t>(rows) * inter * 2) + moe_up(static_cast<size_t>(rows) * (inter / 2) * 2) +
          (small ? moe_up(static_cast<size_t>(kMoeMaxRuns) * rows * hidden * sizeof(float)) : 0);
 }
@@ -1573,27 +1572,36 @@ int launch_moe_ffn(const void* x, const int64_t* rows_before_expert, const void*
   unsigned char* ws = static_cast<unsigned char*>(workspace);
   const int bm = moe_tile_rows(rows, num_experts, bits);
   const bool experts = bm == kExpertsRows;
+  const size_t table_bytes = moe_up((static_cast<size_t>(moe_max_tiles(rows, num_experts, 32)) + 1) * sizeof(MoeTile));
+  MoePlan plan1{reinterpret_cast<MoeTile*>(ws), moe_max_tiles(rows, num_experts, bm), {}}, plan2 = plan1;
   bool narrow = false;
-  const MoeHeights heights = experts ? plan_moe_heights(rows, hidden, inter, num_experts, bits, &narrow) : MoeHeights{};
-  const int max_tiles = moe_max_tiles(rows, num_experts, experts ? heights.min_units * 64 : bm);
-  MoeTile* table = reinterpret_cast<MoeTile*>(ws);
-  unsigned char* fc1 = ws + moe_up((static_cast<size_t>(moe_max_tiles(rows, num_experts, 32)) + 1) * sizeof(MoeTile));
+  if (experts) {
+    plan1.heights = plan_moe_heights(rows, inter / 2, 128, num_experts, 1.0f);
+    plan2.heights = plan_moe_heights(rows, hidden, 256, num_experts, 1.0f);
+    const MoeHeights n = plan_moe_heights(rows, hidden, 128, num_experts, 0.7f);
+    narrow = best_moe_cost(n, rows, num_experts) < best_moe_cost(plan2.heights, rows, num_experts);
+    if (narrow) plan2.heights = n;
+    plan1.max_tiles = moe_max_tiles(rows, num_experts, plan1.heights.min_units * 64);
+    plan2.max_tiles = moe_max_tiles(rows, num_experts, plan2.heights.min_units * 64);
+    plan2.table = reinterpret_cast<MoeTile*>(ws + table_bytes);
+  }
+  unsigned char* fc1 = ws + 2 * table_bytes;
   unsigned char* act = fc1 + moe_up(static_cast<size_t>(rows) * inter * 2);
   float* partial = reinterpret_cast<float*>(act + moe_up(static_cast<size_t>(rows) * (inter / 2) * 2));
-  (experts ? moe_plan_kernel<true> : moe_plan_kernel<false>)<<<dim3(1), dim3(256), 0, stream>>>(
-      rows_before_expert, num_experts, bm, max_tiles, rows, heights, table);
+  (experts ? moe_plan_kernel<true> : moe_plan_kernel<false>)<<<dim3(experts ? 2 : 1), dim3(256), 0, stream>>>(
+      rows_before_expert, num_experts, bm, rows, plan1, plan2);
   const auto product = [&](const MoeGemmArgs& a) {
     if (dtype == WOL_DTYPE_BF16) moe_gemm_bf16(a, bits); else moe_gemm_f16(a, bits);
   };
-  const int* tab = reinterpret_cast<const int*>(table);
-  product(MoeGemmArgs{x, tab, max_tiles, bm, 1, false, rows, nullptr, nullptr, ffn1_codes, ffn1_bias, ffn1_scale,
+  product(MoeGemmArgs{x, reinterpret_cast<const int*>(plan1.table), plan1.max_tiles, bm, 1, false, rows, nullptr, nullptr, ffn1_codes, ffn1_bias, ffn1_scale,
                       hidden, inter, experts ? act : fc1, stream, experts});
   if (!experts) {
     const int rc = launch_swiglu_t(fc1, dtype, rows, inter, act, stream);
     if (rc != WOL_OK) return rc;
   }
   // the second product has hidden / 256 column tiles only: K (= inter / 2) in runs when the tiles are small
-  product(MoeGemmArgs{act, tab, max_tiles, bm, moe_runs(inter / 2, hidden, bits, bm, max_tiles), narrow, rows,
+  product(MoeGemmArgs{act, reinterpret_cast<const int*>(plan2.table), plan2.max_tiles, bm,
+                      moe_runs(inter / 2, hidden, bits, bm, plan2.max_tiles), narrow, rows,
                       experts ? nullptr : partial, rows_before_expert + (num_experts - 1), ffn2_codes, nullptr, ffn2_scale,
                       inter / 2, hidden, out, stream, false});
   return check_launch();
