@@ -76,6 +76,28 @@ __device__ inline void place_of_block(const DmaParams& p, int* bx, int* by, int*
   tile_of_position(pos - *split * tiles, p.nbx, p.nby, bx, by);
 }
 
+// The same for launches of short K runs (below kShortRun k tiles): every XCD takes a part of every run.  With a run, or part
+// of one, to itself an XCD reads the same less than 4 KiB of every row of x, rows that lie a power of two apart more often
+// than not, through the few channels of its L2 (256 bytes each in turn, 16 of them) that hold those.  At least as many row
+// tiles as column tiles: plain order; fewer: an eighth of the run's tiles, as above, so that the row tiles of a column stay
+// together.  us a call, (run, tile) order / plain / eighths of every run: 1300 x 2048 -> 1024 int8, four runs of 8, 22.5 /
+// 19.1 / 19.3; 1500 x 1152 -> 1536 int8 g64, two of 9, 25.7 / 22.2 / 25.1; 700 x 1152 -> 4096 int8, two of 9, 24.2 / 22.7 /
+// 21.6; 205 x 3584 -> 7904 int8, four of 14, 26.9 / 29.8 / 27.4; 700 x 11008 -> 4096 int8, two of 86, 73.6 / 77.4 / 76.0.
+// (A kernel of its own: the other instantiations lose 1 to 3 % by the code alone.)
+constexpr int kShortRun = 32;
+__device__ inline void place_in_short_run(const DmaParams& p, int* bx, int* by, int* split) {
+  constexpr int kXcd = 8;
+  const int tiles = p.nbx * p.nby, q = tiles / kXcd, r = tiles % kXcd;
+  *split = blockIdx.x / tiles;
+  const int w = blockIdx.x - *split * tiles, x = w % kXcd;
+  if (p.nby >= p.nbx) {
+    *by = w / p.nbx;
+    *bx = w - *by * p.nbx;
+  } else {
+    tile_of_position(x * q + (x < r ? x : r) + w / kXcd, p.nbx, p.nby, bx, by);
+  }
+}
+
 template <int DT, int BITS, int G, int WM, int WN, int TM, int TN, int SWI, bool STAMP, bool EXPERTS>
 __device__ __forceinline__ void wide_tile(const DmaParams& p, const TilePlace at, int split) {
 #if defined(__HIP_DEVICE_COMPILE__)
@@ -738,10 +760,11 @@ __global__ __launch_bounds__(512) void gemm_dma_kernel_tall(const DmaParams p) {
 #endif
 }
 
-template <int DT, int BITS, int G, int WM, int WN, int TM, int TN, int SWI, bool STAMP>
+template <int DT, int BITS, int G, int WM, int WN, int TM, int TN, int SWI, bool STAMP, bool SHORT_RUNS>
 __global__ __launch_bounds__(512) void gemm_dma_kernel_wide(const DmaParams p) {
   int bx, by, split;
-  place_of_block(p, &bx, &by, &split);
+  if (SHORT_RUNS) place_in_short_run(p, &bx, &by, &split);
+  else place_of_block(p, &bx, &by, &split);
   wide_tile<DT, BITS, G, WM, WN, TM, TN, SWI, STAMP, false>(p, TilePlace{bx, 0, by * WM * TM * 16, 0}, split);
 }
 
@@ -777,10 +800,10 @@ __global__ __launch_bounds__(512) void gemm_experts_kernel(const DmaParams p) {
 }
 
 // Eight wavefronts side by side, TM 16-row blocks x 32 columns each.
-template <int DT, int BITS, int G, int TM, int SWI, bool STAMP = false>
+template <int DT, int BITS, int G, int TM, int SWI, bool STAMP = false, bool SHORT_RUNS = false>
 void launch(const DmaParams& p, hipStream_t stream) {
   constexpr size_t lds = wide_lds_bytes<BITS, G, 1, 8, TM, 2>();
-  auto kern = gemm_dma_kernel_wide<DT, BITS, G, 1, 8, TM, 2, SWI, STAMP>;
+  auto kern = gemm_dma_kernel_wide<DT, BITS, G, 1, 8, TM, 2, SWI, STAMP, SHORT_RUNS>;
   static std::atomic<uint32_t> configured{0};  // per instantiation
   allow_lds(reinterpret_cast<const void*>(kern), lds, configured);
   kern<<<dim3(static_cast<unsigned>(p.nbx * p.nby * p.nsplit)), dim3(512), lds, stream>>>(p);
@@ -799,6 +822,7 @@ template <int DT, int BITS, int G>
 void launch_tile(const DmaParams& p, WideTile tile, int swi, hipStream_t stream) {
   if (tile == WideTile::kHalf) {
     if (swi) launch<DT, BITS, G, 8, 1>(p, stream);
+    else if (p.nsplit > 1 && p.tiles_per_split < kShortRun) launch<DT, BITS, G, 8, 0, false, true>(p, stream);
     else launch<DT, BITS, G, 8, 0>(p, stream);
     return;
   }

@@ -30,3 +30,20 @@ def test_whole_tile_edges(G, oracle, dt, bits, g):
     # one round of 256 x 256 tiles and some half-size ones behind it; the last row tile is partial
     for M, K, N in [(2047, 256, 8224), (1793, 128 if bits == 4 else 192, 8192)]:
         check_sampled(G, oracle, dt, bits, g, M, K, N, bias=(M % 2 == 1), seed=M)
+
+
+@pytest.mark.parametrize("dt", [H.F16, H.BF16])
+@pytest.mark.parametrize("bits", [8, 4])
+@pytest.mark.parametrize("g", [-1, 64, 128])
+@pytest.mark.parametrize("M,K,N", [
+    (300, 2048, 272),   # more row tiles than column tiles, both ragged: runs of 8 (int8) and 16 (int4) k tiles in plain order
+    (129, 2176, 784),   # fewer: two row tiles on four column tiles; a shorter last run
+    (65, 2176, 1296),   # one row tile, six column tiles, no multiple of the XCDs
+    (129, 8448, 272),   # runs of 33 and 34
+])
+def test_half_tiles_with_k_in_runs(G, oracle, dt, bits, g, M, K, N):
+    from paddle_amd import _lib
+
+    ws = _lib.lib.wol_linear_workspace(M, K, N, bits, g)
+    assert ws > 0 and "128x256 tiles on [0,%d) with K in runs" % N in G.linear_plan(M, K, N, bits, g, ws)
+    check(G, oracle, dt, bits, g, M, K, N, bias=(M % 2 == 1), seed=M)
