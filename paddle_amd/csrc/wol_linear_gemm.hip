@@ -1473,8 +1473,13 @@ void describe_linear_gemm(int64_t M, int64_t K, int64_t N, int bits, int group_s
   const TailPlan t = plan_tail(static_cast<int>(M), static_cast<int>(K), (nstrips - lo) * kStripCols, kHalfRows, kHalfCols, tk, ws_bytes);
   const int mid = lo + t.full_tiles * (kHalfCols / kStripCols);
   int len = 0;
-  len += snprintf(buf + len, n - len, "wol::gemm_dma_kernel_wide (v_mfma_f32_16x16x32):");
-  if (lo > 0 && len < static_cast<int>(n))
+  const bool tall = lo > 0 && g != 0;  // group-wise scales on whole tiles have a kernel of their own
+  if (tall)
+    len += snprintf(buf + len, n - len, "wol::gemm_dma_kernel_tall (v_mfma_f32_32x32x16): 256x256 tiles on columns [0,%d)%s",
+                    lo * kStripCols, nstrips > lo ? "; " : "");
+  if ((!tall || nstrips > lo) && len < static_cast<int>(n))
+    len += snprintf(buf + len, n - len, "%sgemm_dma_kernel_wide (v_mfma_f32_16x16x32):", tall ? "" : "wol::");
+  if (lo > 0 && !tall && len < static_cast<int>(n))
     len += snprintf(buf + len, n - len, " 256x256 tiles on columns [0,%d)", lo * kStripCols);
   if (mid > lo && len < static_cast<int>(n))
     len += snprintf(buf + len, n - len, " 128x256 tiles on [%d,%d)", lo * kStripCols, mid * kStripCols);

@@ -328,6 +328,14 @@ def test_linear_plan_names_the_kernel_per_shape(lib):
     assert "stream_kernel" in plan(8, 8192, 28672, 8, -1)   # int8 at K = 8192 does not fit its registers
     assert "gemm_dma_kernel" in plan(2048, 4096, 12288, 8, -1)
     assert "256x256" in plan(2048, 4096, 12288, 8, -1)
+    wide, tall = "gemm_dma_kernel_wide (v_mfma_f32_16x16x32): ", "gemm_dma_kernel_tall (v_mfma_f32_32x32x16): "
+    for bits, g, whole in ((8, -1, wide), (4, -1, wide), (8, 64, tall), (4, 128, tall)):
+        name = plan(8192, 4096, 4096, bits, g)
+        assert name == "wol::" + whole + "256x256 tiles on columns [0,4096)"
+        name = plan(2048, 4096, 12288, bits, g)  # whole and half-size tiles
+        assert name.startswith("wol::" + whole + "256x256 tiles on columns [0,") and "128x256 tiles on [" in name
+        assert name.count(wide) == 1
+        assert tall not in plan(128, 4096, 12288, bits, g) and wide in plan(128, 4096, 12288, bits, g)
     assert lib.lib.wol_linear_plan(4, 4096, 100, 8, -1, 0, ctypes.create_string_buffer(8), 8) == 5
 
 
