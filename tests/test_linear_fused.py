@@ -160,7 +160,7 @@ def test_swiglu_in_the_gemm_epilogue(device, oracle, dt, bits, g):
     # writes [M, N/2] itself: no fp32 sums, no extra pass (group-wise scales: the
     # tiles whose sums are kept in units of the group scale; their scales are
     # gathered from the gate and the up columns like the codes).
-    # 128-row and 256-row tiles, rows off the tile height, a gate half that ends
+    # 128-row tiles, rows off the tile height, a gate half that ends
     # inside a column tile (N/2 = 1168), with and without bias
     from paddle_amd import _lib
 
@@ -187,6 +187,12 @@ def test_swiglu_in_the_gemm_epilogue(device, oracle, dt, bits, g):
 @pytest.mark.parametrize("bits,g,M,K,N", [
     (4, 128, 300, 384, 22048),  # 261 half-size tiles against 174 whole ones: whole tiles
     (4, 64, 520, 256, 17504),
+    (4, -1, 300, 384, 22048),
+    (8, 64, 300, 320, 22048),   # an odd number of 64-deep k tiles; groups of 128: the last one is half a group
+    (8, 128, 300, 320, 22048),
+    (8, -1, 300, 320, 22048),
+    (8, 64, 520, 128, 17504),   # two k tiles
+    (8, 128, 511, 192, 22048),
 ])
 def test_swiglu_epilogue_on_whole_tiles(device, oracle, dt, bits, g, M, K, N):
     # 256 x 256 tiles where half-size ones would need twice the rounds; the last column tile is partial.
@@ -194,6 +200,10 @@ def test_swiglu_epilogue_on_whole_tiles(device, oracle, dt, bits, g, M, K, N):
     import torch
     from paddle_amd.nn import quant as Q
 
+    # launch_swiglu_gemm's choice: whole tiles unless half-size ones, at 0.6 of their time, are done in fewer rounds
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    whole, half = (-(-N // 256) * -(-M // rows) for rows in (256, 128))
+    assert -(-whole // cus) < 0.6 * -(-half // cus)
     gen = torch.Generator(device="cuda").manual_seed(K + N)
     w = (torch.randn(K, N, device="cuda", generator=gen) * 0.02).to(H.torch_dtype(dt))
     codes, scale = Q.weight_quantize(w, algo="weight_only_int%d" % bits, group_size=g)
