@@ -236,7 +236,8 @@ GPU_CASES = [  # M, K, N, kind, threshold, bias
     (5, 128, 48, "normal", 2.0, True),        # many outlier columns
     (33, 192, 80, "spiky", 6.0, False),       # 64-row tile
     (100, 320, 400, "spiky", 6.0, True),      # 128-row tile, one run
-    (130, 1024, 144, "spiky", 6.0, True),     # 256-row tile, fused epilogue, ragged in M and N
+    (130, 1024, 144, "spiky", 6.0, True),     # 128-row tiles, two runs, ragged in M and N
+    (257, 384, 400, "spiky", 6.0, True),      # 128-row tiles, the outlier columns in the epilogue, ragged in M and N
     (300, 512, 1040, "normal", 3.0, False),   # several row tiles, column tiles not a multiple of 8
     (257, 64, 2048, "spiky", 6.0, True),      # one k tile; column tiles spread over the XCD bands
     (3, 64, 16, "normal", 0.0, True),         # every column an outlier
@@ -298,7 +299,7 @@ def test_gpu_llm_int8_linear_bit_exact(device, oracle, dt, case):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("N", [12288, 8192])  # 128x256 tiles (three rounds of the CUs), 256x256 tiles (one round)
+@pytest.mark.parametrize("N", [12288, 8192])  # one round of 256x256 tiles, at 12288 with one of 128x256 tiles behind it
 def test_gpu_llm_int8_linear_large_properties(device, oracle, N):
     """M = 2048, K = 4096, N = 12288 | 8192 (too large for the scalar oracle): rows
     checked against the oracle on a slice of the columns, and the whole result

@@ -1,8 +1,9 @@
 """Edges of llm_int8_linear's 128- and 256-row tiles, bit for bit against the CPU
 oracle: rows and columns on both sides of a tile, one to four 128-deep k tiles,
 ragged grids over the XCDs; sums that merge to zeros of either sign and to
-infinities, whose division by 127 takes the special cases.  And the activation
-stages of a few rows, on both sides of the one-launch form's limit."""
+infinities, whose division by 127 takes the special cases.  K in runs above 128
+rows.  And the activation stages of a few rows, on both sides of the one-launch
+form's limit."""
 import numpy as np
 import pytest
 
@@ -40,6 +41,34 @@ def test_tile_edges(device, oracle, dt, outliers, M, K, N):
     nan = np.isnan(H.bits_to_f32(want, dt))
     assert np.array_equal(np.isnan(H.bits_to_f32(g, dt)), nan)
     assert np.array_equal(g[~nan], want[~nan])
+
+
+@pytest.mark.parametrize("dt", [H.F16, H.BF16])
+@pytest.mark.parametrize("outliers", [0, 3, 40])
+@pytest.mark.parametrize("M,K,N,runs", [
+    (257, 1664, 528, 3),    # 13 k tiles in runs of 5: the last has 3; three row and three column tiles
+    (385, 2176, 272, 4),    # 17 in runs of 5: the last has 2
+    (129, 2688, 784, 5),    # 21 in runs of 5: the last has one
+    (300, 3968, 1040, 7),   # 31 in runs of 5; five column tiles, no multiple of the XCDs with three row tiles
+    (140, 8192, 272, 8),    # equal runs
+])
+def test_k_in_runs_above_128_rows(device, oracle, dt, outliers, M, K, N, runs):
+    import gpu_calls as G
+
+    rng = np.random.default_rng(M + K)
+    w = rng.integers(-127, 128, (N, K), dtype=np.int8)
+    ws = (rng.random(N, dtype=np.float32) * np.float32(1e-3) + np.float32(1e-4)).astype(np.float32)
+    ws[1::9] = -ws[1::9]
+    x = np.clip(rng.standard_normal((M, K), dtype=np.float32), -5, 5)
+    cols = np.r_[[0, K - 1, 639], 640 + rng.permutation(K - 641)][:outliers]  # ends of K, the end of a run of 5 tiles, behind it
+    x[rng.integers(0, M, cols.size), cols] = 20.0
+    xb = H.f32_to_bits(x, dt)
+    bb = H.make_bias(N, dt, seed=3, std=1.0) if M % 2 else None
+    o = oracle.llm_int8_linear(xb, w, bb, ws, 6.0, dt)
+    assert o["outlier"].sum() == outliers
+    got, st = G.llm_int8_linear(xb, w, bb, ws, 6.0, dt, stages=True)
+    assert st["runs"] == runs
+    assert np.array_equal(got, o["out"])
 
 
 @pytest.mark.parametrize("dt", [H.F16, H.BF16])
