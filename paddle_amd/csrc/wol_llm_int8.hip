@@ -343,12 +343,13 @@ struct Epi {
   const int32_t* list;
   uint16_t* out;          // [M,N] T
   int M, K, N;
-  // few outlier columns, collected by the outlier kernel for the GEMM's epilogue:
-  uint16_t* xo;           // [kOutCap][ldx] x of outlier column j, by row
-  uint16_t* wo;           // [kOutCap][ldw] T(w * wscale) of outlier column j, by output column
-  int ldx, ldw;           // M and N rounded up to whole tiles
+  // Few outlier columns, collected by the outlier kernel for the GEMM's epilogue (null: it picks them out of x and w):
+  // [kOutCap][M rounded up to whole tiles] x of outlier column j, by row, and behind them [kOutCap][N rounded up]
+  // T(w * wscale) of it, by output column.
+  uint16_t* cols;
 };
 constexpr int kOutCap = 32;
+__host__ __device__ constexpr int64_t align256(int64_t v) { return (v + 255) / 256 * 256; }  // also whole tiles, of any height and width
 
 // v / 127, correctly rounded, in four instructions instead of the dozen of the IEEE division sequence: q = v * RN(1/127),
 // r = v - 127 q (exact in an FMA), q + r * RN(1/127), and v_div_fixup for v = -0 and infinities, where q is already the
@@ -454,15 +455,20 @@ __device__ inline void load_ws_bias8(const Epi& e, int nn, float* ws, float* bia
 template <int DT>
 __global__ __launch_bounds__(256) void llm_outlier_kernel(Epi e, int fused_cap) {
   uint16_t* sub = e.out;  // the product waits where the output will go: whoever merges element (m, n) reads it first
+  const int per = e.M + e.N;  // elements of a collected column; kOutCap of them are below 2^30
+  const int64_t first = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
+  // the first element's column, fetched beside the count: if there is no such column, what stands there is not used
+  const bool may = e.cols != nullptr && first < static_cast<int64_t>(fused_cap) * per;
+  int k = may ? e.list[static_cast<int>(first) / per] : 0;
   const int cnt = *e.count;
   if (cnt <= fused_cap) {
-    const int per = e.M + e.N;
-    const int64_t total = static_cast<int64_t>(cnt) * per;
-    for (int64_t i = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x; i < total; i += static_cast<int64_t>(gridDim.x) * 256) {
-      const int j = static_cast<int>(i / per), r = static_cast<int>(i - static_cast<int64_t>(j) * per), k = e.list[j];
-      if (r < e.M) e.xo[static_cast<int64_t>(j) * e.ldx + r] = e.x[static_cast<int64_t>(r) * e.K + k];
+    if (e.cols == nullptr) return;  // the GEMM picks the columns itself
+    for (int64_t i = first; i < static_cast<int64_t>(cnt) * per; i += static_cast<int64_t>(gridDim.x) * 256) {
+      const int j = static_cast<int>(i) / per, r = static_cast<int>(i) - j * per;
+      if (i != first) k = e.list[j];
+      if (r < e.M) e.cols[j * align256(e.M) + r] = e.x[static_cast<int64_t>(r) * e.K + k];
       else
-        e.wo[static_cast<int64_t>(j) * e.ldw + (r - e.M)] =
+        e.cols[kOutCap * align256(e.M) + j * align256(e.N) + (r - e.M)] =
             cast_out<DT>(static_cast<float>(e.w[static_cast<int64_t>(r - e.M) * e.K + k]) * e.wscale[r - e.M]);
     }
     return;
@@ -471,6 +477,7 @@ __global__ __launch_bounds__(256) void llm_outlier_kernel(Epi e, int fused_cap) 
   const int tid = threadIdx.x;
   const int nbx = (e.N + 255) / 256;
   const int m0 = static_cast<int>(blockIdx.x / nbx) * 64;
+  if (m0 >= e.M) return;  // launched to collect
   const int n = static_cast<int>(blockIdx.x % nbx) * 256 + tid;
   const int nn = n < e.N ? n : e.N - 1;
   const float ws = e.wscale[nn];
@@ -522,8 +529,8 @@ __device__ inline void stage_outliers(const Epi& e, int cnt, int m0, int n0, int
       for (int q = 0; q < 8; ++q) dst[j * len + r + q] = to_f32<DT>(static_cast<uint16_t>(v[q >> 1] >> (16 * (q & 1))));
     }
   };
-  rows(e.xo + m0, e.ldx, BM, xs);
-  rows(e.wo + n0, e.ldw, BN, wd);
+  rows(e.cols + m0, align256(e.M), BM, xs);
+  rows(e.cols + kOutCap * align256(e.M) + n0, align256(e.N), BN, wd);
 }
 
 // ---------------------------------------------------------------------------
@@ -787,7 +794,18 @@ __global__ __launch_bounds__(WM* WN * 64) __attribute__((amdgpu_waves_per_eu(2))
     if (!fused) __syncthreads();
   }
   if (fused) {
-    stage_outliers<DT, BM, BN, NW * 64>(e, cnt, m0, n0, tid, xs, wdl);
+    if (e.cols != nullptr) {
+      stage_outliers<DT, BM, BN, NW * 64>(e, cnt, m0, n0, tid, xs, wdl);
+    } else {  // one row tile: this workgroup is the only one that needs its columns' weights
+      for (int i = tid; i < cnt * BM; i += NW * 64) {
+        const int j = i / BM, m = m0 + i % BM;
+        xs[i] = to_f32<DT>(e.x[static_cast<int64_t>(m < M ? m : M - 1) * K + e.list[j]]);
+      }
+      for (int i = tid; i < cnt * BN; i += NW * 64) {
+        const int j = i / BN, n = n0 + i % BN < N ? n0 + i % BN : N - 1;
+        wdl[i] = to_f32<DT>(cast_out<DT>(static_cast<float>(e.w[static_cast<int64_t>(n) * K + e.list[j]]) * e.wscale[n]));
+      }
+    }
     __syncthreads();
   }
 #pragma unroll
@@ -1165,8 +1183,6 @@ __global__ __launch_bounds__(64) void llm_merge_few_kernel(const int32_t* __rest
           merge_one<DT>(sum[m], to_f32<DT>(cast_out<DT>(sub[m])), e.ranges[m], ws, e.bias != nullptr, bias));
 }
 
-inline int64_t align256(int64_t v) { return (v + 255) / 256 * 256; }
-
 struct Plan {
   int bm, bn;     // tile
   int tk;         // k bytes per tile row
@@ -1258,9 +1274,7 @@ struct Workspace {
   int8_t* qx;
   int32_t* acc;
   int8_t* ow;
-  uint16_t* xo;
-  uint16_t* wo;
-  int ldx, ldw;
+  uint16_t* cols;
   int64_t bytes;
 };
 
@@ -1285,12 +1299,8 @@ Workspace carve(void* base, int64_t M, int64_t K, int64_t N, int runs) {
   off += align256(M * N * 4 * runs);
   w.ow = reinterpret_cast<int8_t*>(p + off);
   if (runs > 1 && M <= kFewRows) off += align256(kStash * N);
-  w.ldx = static_cast<int>(align256(M));  // whole tiles: 256 is a multiple of every tile's rows and columns
-  w.ldw = static_cast<int>(align256(N));
-  w.xo = reinterpret_cast<uint16_t*>(p + off);
-  if (runs == 0) off += static_cast<int64_t>(kOutCap) * w.ldx * 2;
-  w.wo = reinterpret_cast<uint16_t*>(p + off);
-  if (runs == 0) off += static_cast<int64_t>(kOutCap) * w.ldw * 2;
+  w.cols = reinterpret_cast<uint16_t*>(p + off);
+  if (runs == 0) off += kOutCap * (align256(M) + align256(N)) * 2;
   w.bytes = off;
   return w;
 }
@@ -1393,7 +1403,7 @@ int run_llm_int8(const void* x, const void* weight, const void* bias, const floa
   p.qx = ws.qx;
   p.e = Epi{xs, static_cast<const int8_t*>(weight), wscale, ws.ranges, static_cast<const uint16_t*>(bias),
             ws.count, ws.list, static_cast<uint16_t*>(out), static_cast<int>(M), static_cast<int>(K),
-            static_cast<int>(N), ws.xo, ws.wo, ws.ldx, ws.ldw};
+            static_cast<int>(N), ws.cols};
   p.acc = ws.acc;
   p.ow = pl.runs > 1 && M <= kFewRows ? ws.ow : nullptr;
   p.n_lo = 0;
@@ -1411,9 +1421,18 @@ int run_llm_int8(const void* x, const void* weight, const void* bias, const floa
   // up to four rows with K runs the merge kernel multiplies the outlier columns
   // itself (a launch costs more than that work)
   const bool direct = pl.runs > 1 && M <= kFewRows;
-  if (!direct)
-    hipLaunchKernelGGL(llm_outlier_kernel<DT>, dim3(static_cast<unsigned>(((N + 255) / 256) * ((M + 63) / 64))),
-                       dim3(256), 0, stream, p.e, p.cap);
+  if (!direct) {
+    // Few columns: collected once for all row tiles, by enough workgroups that no thread fetches many elements one after
+    // the other (300 x 4544 -> 4096, fp16, 20 columns, 90.0 us a call when every tile picks, 81 so).  Up to 128 rows
+    // there is one row tile, and the GEMM picks a column's weights exactly once (101 x 1024 -> 1024, bf16, 20 columns, us a
+    // call: collected on the workgroups of the product 38.5, on enough of them 33.1, picked 32.9; 3 columns 25.1 / 24.0 /
+    // 23.7).
+    int64_t blocks = ((N + 255) / 256) * ((M + 63) / 64);  // one per 64 x 256 piece of the product
+    if (M <= 128) p.e.cols = nullptr;
+    const int64_t collect = p.e.cols != nullptr ? (p.cap * (M + N) + 255) / 256 : 0;
+    if (blocks < collect) blocks = collect < 1024 ? collect : (blocks < 1024 ? 1024 : blocks);
+    hipLaunchKernelGGL(llm_outlier_kernel<DT>, dim3(static_cast<unsigned>(blocks)), dim3(256), 0, stream, p.e, p.cap);
+  }
   if (check_launch() != WOL_OK) return WOL_ERR_HIP;
   if (pl.runs == 1 && pl.bm == 256 && pl.bn == 256 && pl.whole_cols < N) {
     // 256x256 tiles on the first columns, 128x256 tiles on the rest

@@ -246,6 +246,9 @@ GPU_CASES = [  # M, K, N, kind, threshold, bias
     (4, 2048, 256, "normal", 2.0, False),     # four rows, K runs, most columns outliers
     (128, 2048, 272, "spiky", 6.0, True),     # 128-row tile, two runs
     (700, 512, 8192, "spiky", 6.0, True),     # 256x256 tiles
+    (200, 128, 65536, "spiky", 6.0, True),    # one row of 256x256 tiles
+    (100, 1024, 400, "spiky", 6.0, True),     # one row tile of 128 rows without K runs: the GEMM picks the outlier columns
+    (600, 192, 272, "normal", 4.0, True),     # K no multiple of 128, several row tiles: collected
 ]
 
 
