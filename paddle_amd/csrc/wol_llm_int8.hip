@@ -1226,12 +1226,14 @@ Plan make_plan(int64_t M, int64_t K, int64_t N) {
       if (best_c == 0) pl.bm = 128;
       // Few tiles leave CUs idle: half tiles with K cut into runs, by the estimate in us of a round (a k tile of a whole
       // tile takes 1.7, of a half one 1.0, their starts and ends 11 and 6, 4 with sums instead of results) and of the
-      // merge launch with the sums' way through memory.  The 0.9: with runs the outlier columns' product is a pass of its
-      // own, which the estimate cannot know.  Whole call, us, one run against this: 200 x 8192 x 3008 56.0 -> 34.7, with 5
-      // outlier columns 42.0; 1024 x 11008 x 4096 102 -> 79; 300 x 4096 x 4096 with 20 outlier columns 49.0 -> 51.3.
+      // merge launch with the sums' way through memory.  The 0.8: with runs the outlier columns' product is a pass of its
+      // own, which the estimate cannot know; where it promises less (ten problems between 0.8 and 0.9) one run is 1 / 5 / 11 /
+      // 19 % faster with 0 / 1 / 8 / 20 outlier columns.  Whole call, us, one run against this: 200 x 8192 x 3008
+      // 56.0 -> 34.7, with 5 outlier columns 42.0; 1024 x 11008 x 4096 102 -> 79; 300 x 4096 x 4096 with 20 outlier
+      // columns 49.0 -> 51.3.
       const double kt = static_cast<double>(ktiles);
       const double one = (best_c * rows256 + cus - 1) / cus * (1.7 * kt + 11) + ((cols - best_c) * rows128 + cus - 1) / cus * (1.0 * kt + 6);
-      double best = 0.9 * one;
+      double best = 0.8 * one;
       int64_t best_r = 1;
       for (int64_t r = 2; r <= 8 && ktiles / r >= 4; ++r) {
         const int64_t per = (ktiles + r - 1) / r, eff = (ktiles + per - 1) / per;

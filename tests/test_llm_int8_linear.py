@@ -236,8 +236,7 @@ GPU_CASES = [  # M, K, N, kind, threshold, bias
     (5, 128, 48, "normal", 2.0, True),        # many outlier columns
     (33, 192, 80, "spiky", 6.0, False),       # 64-row tile
     (100, 320, 400, "spiky", 6.0, True),      # 128-row tile, one run
-    (130, 1024, 144, "spiky", 6.0, True),     # 128-row tiles, two runs, ragged in M and N
-    (257, 384, 400, "spiky", 6.0, True),      # 128-row tiles, the outlier columns in the epilogue, ragged in M and N
+    (130, 1024, 144, "spiky", 6.0, True),     # 128-row tiles, the outlier columns in the epilogue, ragged in M and N
     (300, 512, 1040, "normal", 3.0, False),   # several row tiles, column tiles not a multiple of 8
     (257, 64, 2048, "spiky", 6.0, True),      # one k tile; column tiles spread over the XCD bands
     (3, 64, 16, "normal", 0.0, True),         # every column an outlier
