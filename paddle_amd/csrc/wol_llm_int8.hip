@@ -157,9 +157,12 @@ __device__ inline void build_list(int nwords, F word_at, int32_t* list, int32_t*
 // range on the way.  The mask lives in LDS (K / 32 words, dynamic).
 // Whole call, us, against three launches (one or two rows: one workgroup for
 // everything), K = 4096, N = 11008, 3 outlier columns: 1 row 20.1 -> 18.5, 4 rows
-// 23.4 -> 20.3, 8 rows 28.9 -> 26.8: the gain shrinks as every workgroup's look
-// through all rows grows, hence the limit.
+// 23.4 -> 20.3, 8 rows 28.9 -> 26.8.  Every workgroup's look through all rows grows
+// with M * K, so the gain shrinks: 8 rows K = 11008 31.7 -> 28.9, 28672 49.1 -> 48.3,
+// 32768 55.9 -> 56.6, 65536 79.7 -> 82.1; 7 rows 53.9 -> 52.4 and 77.7 -> 76.0.  Hence
+// eight rows up to K = 28672 and seven beyond.
 constexpr int kSmallRows = 8;
+constexpr int kSmallRowsMaxK = 28672;  // one row fewer beyond
 constexpr int kSmallThreads = 1024;
 constexpr int kSmallMaxK = 65536;
 
@@ -1373,7 +1376,7 @@ int run_llm_int8(const void* x, const void* weight, const void* bias, const floa
   const Plan pl = make_plan(M, K, N);
   const Workspace ws = carve(workspace, M, K, N, pl.runs);
   const uint16_t* xs = static_cast<const uint16_t*>(x);
-  const bool small = M <= kSmallRows && K <= kSmallMaxK;
+  const bool small = M <= kSmallRows - (K > kSmallRowsMaxK ? 1 : 0) && K <= kSmallMaxK;
   if (small) {
     hipLaunchKernelGGL(llm_act_small_kernel<DT>, dim3(static_cast<unsigned>(M + 1)), dim3(kSmallThreads), static_cast<size_t>(K / 32 * 4), stream,
                        xs, threshold, static_cast<int>(M), static_cast<int>(K), ws.ranges, ws.mask, ws.qx, ws.count,

@@ -73,7 +73,8 @@ def test_k_in_runs_above_128_rows(device, oracle, dt, outliers, M, K, N, runs):
 
 @pytest.mark.parametrize("dt", [H.F16, H.BF16])
 @pytest.mark.parametrize("M", [1, 2, 7, 8, 9])
-@pytest.mark.parametrize("K", [64, 2112, 8256])  # one, more than one and more than four rounds of the mask's 64 words
+@pytest.mark.parametrize("K", [64, 2112, 8256, 28736])  # one, more than one and more than four rounds of the mask's 64
+                                                       # words; past the K up to which eight rows take the one launch
 def test_few_rows(device, oracle, dt, M, K):
     import gpu_calls as G
 
