@@ -1085,13 +1085,16 @@ void launch_fast(const Args& a) {
 // own number, takes the limit with the shortest estimate:
 //   time of such a tile x rounds,
 // a round being what the CUs of an XCD take of its share of the tiles.  The
-// times of 64-, 128- and 192-row tiles against 256-row ones (0.46, 0.66, 0.85) and
-// of a 128-column tile against a 256-column one (0.7) come from 11 problems timed
-// under every pair of limits.  A limit of each product's own and these times
-// against one limit for both and the times of the former tiles, 22 problems, whole
-// call: 1.05 x on average, 0.97 to 1.25 (4 experts, hidden 4096, width 11008, 900
-// rows, int4 173 -> 138 us; 8 experts, 2048, 16384, 1500 rows, int4 228 -> 191; 8
-// experts, 4096, 28672, 4096 rows, int4 1311 -> 1283, 1024 rows int8 465 -> 477).
+// times of 64-, 128- and 192-row tiles against 256-row ones (0.54, 0.66, 0.84) and
+// of a 128-column tile against a 256-column one (0.7) are fitted to 200 problems
+// timed under every limit and tile width of either product (4 to 16 experts of 65
+// rows each up to 8192 in all, evenly and unequally loaded, hidden 1024 to 4096,
+// fc1 width 2816 to 28672, int4 and int8).  The choice is 0.5 % slower than the
+// best one on average (int4 0.3, int8 0.7) and 6 % at worst, on these and on 200
+// other problems alike; 256-row tiles always 24 %; 0.46, 0.66, 0.85, which came from
+// 11 problems, 0.9 and 10 %.  A limit of each product's own against one limit for
+// both: 4 experts, hidden 4096, width 11008, 900 rows, int4 173 -> 138 us; 8 experts,
+// 2048, 16384, 1500 rows, int4 228 -> 191.
 struct MoeHeights {
   int xcd_cus;      // CUs of an XCD
   int min_units;    // lowest limit the launch grid has room for; 4 = 256 rows, the highest
@@ -1540,7 +1543,7 @@ static MoeHeights plan_moe_heights(int64_t rows, int64_t cols, int bn, int num_e
   MoeHeights h;
   h.xcd_cus = cus / 8 > 0 ? cus / 8 : 1;
   h.nbx = static_cast<int>((cols + bn - 1) / bn);
-  const float times[kMaxUnits] = {0.46f, 0.66f, 0.85f, 1.0f};
+  const float times[kMaxUnits] = {0.54f, 0.66f, 0.84f, 1.0f};
   for (int u = 0; u < kMaxUnits; ++u) h.tile[u] = times[u] * column_cost;
   h.min_units = 1;
   while (h.min_units < kMaxUnits &&
