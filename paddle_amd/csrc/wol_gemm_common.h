@@ -35,7 +35,8 @@ struct DmaParams {
   const int* moe_table;
   int64_t moe_codes_stride;     // bytes between two experts' packed weights
   int moe_rows;                 // rows of the whole grouped problem (the partial sums' row count)
-  // STAMP instantiation only: six cycle counts per wavefront, [workgroup][wavefront][8] (see wol_prefill_phases)
+  // STAMP instantiation only: seven cycle counts and the number of k tiles of every wavefront, [workgroup][wavefront][8]
+  // (see wol_prefill_phases)
   unsigned long long* stamps;
 };
 

@@ -333,7 +333,7 @@ __device__ __forceinline__ void dma_tile(const DmaParams p) {
   constexpr int kGShift = G == 128 ? 7 : 6;
   static_assert(kGT * BN <= NW * 128, "the tile's scales must fit the wavefronts' 4-byte loads");
   // direct-to-LDS loads every lane issues per stage.  They are the only vector
-  // memory loads of the main loop, so they complete in issue order and
+  // memory loads of the main loop, and loads complete in issue order, so
   // s_waitcnt vmcnt(n) can tell which stages have landed.
   constexpr int kPerStage = kALoads + kBLoads + (G == 0 ? 0 : 1);
   static_assert(Q >= 2 && (Q - 2) % kFold != 0 && (Q - 2) % kFold != kFold - 1,
@@ -916,12 +916,20 @@ void launch_wide(const Args& a, int bits, int group, WideTile tile, int swi, int
 // Number of 256-column tiles given to the 256-row kernel; the remaining
 // columns run with half-size tiles.  Cost model: a workgroup owns its CU, so a
 // launch takes ceil(tiles / CUs) tile times; a half-size tile costs kSmall of a
-// full one (a little more than half).  int4 with group-wise scales: half-size
-// tiles cost more (their 128-deep k tiles run in two stages), and a last partial
-// round of them that plan_tail cuts into K runs costs the share of a round that
-// a run is plus the partial sums' way through memory (K = 4096, N = 12288, 700
-// rows, all on half-size tiles / all on full ones: bf16 g128 105 / 108 us, g64
-// 112 / 121; 1024 rows 129 / 113 and 137 / 125).
+// full one (a little more than half; 0.58 for int4 with group-wise scales, where
+// full tiles run on gemm_dma_kernel_tall).  int4 with group-wise scales also counts
+// a last partial round that plan_tail cuts into K runs as the share of a round that
+// a run is plus the partial sums' way through memory (kRuns).  480 problems (65 to
+// 8192 rows, K 1024 to 14336, N 1024 to 28672), timed with every number of
+// 256-column tiles that fills whole rounds: the choice is slower than the best of
+// them by 0.3 % (int4 with groups), 0.2 % (int8 with groups) and 0.3 % (per channel)
+// on average; at worst 11 % (1218 x 5120 -> 7104 int4 g64: half-size tiles with K
+// runs 128 us, whole ones 115), 17 % (3642 x 2432 -> 17824 int8 g64 374 against 320:
+// half-size tiles throughout, 68 of the 70 column tiles whole) and 15 % (3499 x 6528 -> 2592
+// int8 137 against 120: half-size tiles with K runs, which only int4 with groups
+// counts).  No other pair of constants was better everywhere: 0.62 with groups gains
+// 5 to 12 % on seven of the eleven problems it decides otherwise and loses 7 and 2 %
+// on two (360 x 13696 -> 25248 int4 g128 276 -> 296).
 inline int plan_big_columns(int M, int K, int N, int bits, int group) {
   const int cus = num_cus();
   const bool g4 = bits == 4 && group != 0;
@@ -1618,10 +1626,12 @@ int launch_moe_ffn(const void* x, const int64_t* rows_before_expert, const void*
 // ---- the prefill kernel's inner loop, one ingredient at a time (wol_mfma_probe) ----
 namespace {
 
-// The register tile and instruction mix of gemm_dma_kernel's 256 x 256
-// configuration (4 x 2 blocks of v_mfma_f32_32x32x16 per wavefront, k tiles of
-// four slices) with its ingredients switched on one by one, and no global
-// memory traffic other than what LOADS adds:
+// The register tile and instruction mix of a 256 x 256 tile of two by four
+// wavefronts (4 x 2 blocks of v_mfma_f32_32x32x16 each, k tiles of four
+// slices) with its ingredients switched on one by one, and no global memory
+// traffic other than what LOADS adds.  No product kernel has this form any more
+// (those of wol_linear_wide.hip put their wavefronts side by side); the ladder
+// says what each ingredient costs the matrix pipes of this machine:
 //   DQ     B fragments dequantised per slice (int8 -> bf16, exact) out of raw
 //          codes read from LDS once per tile (0 or 2)
 //   NA     A fragments read from LDS per slice (0 or 4)
