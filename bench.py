@@ -384,7 +384,7 @@ def bench_prefill_phases(torch, np, Q, _lib, dev):
         })
     return {"what": "wol_prefill_phases: per-wavefront cycle stamps in the 256 x 256 tile of the prefill GEMM "
                     "(int8 per-channel, bf16); 2048 cycles per k tile is what two wavefronts per SIMD need to issue "
-                    "their 2 x 32 MFMAs of 32 cycles back to back", "rows": rows}
+                    "their 2 x 64 MFMAs of 16 cycles back to back", "rows": rows}
 
 
 def bench_decode_phases(torch, np, Q, _lib, dev, c, x, copies, scales, steps):
@@ -544,7 +544,8 @@ def bench_moe_ffn(torch, np, Q, H, dev, quick, failures):
         failures.append("moe_ffn output differs from the oracle")
     return {"workload": "moe_ffn, 8 experts, hidden 4096, fc1 width 28672 (swiglu to 14336), int8 per-channel, bf16; "
                         "rows in expert order, the same number per expert",
-            "launches_per_call": "tile table, grouped GEMM, swiglu pass, grouped GEMM",
+            "launches_per_call": "tile table, grouped GEMM (swiglu in its epilogue, or a pass behind it up to 64 rows "
+                                  "per expert), grouped GEMM",
             "weight_bytes": wbytes, "rows": rows_out, "rel_l2_vs_oracle": err,
             "parity_sample": "two rows of expert 3 of the 4096-row call"}
 
@@ -780,7 +781,7 @@ def main():
     ceil_med, _ = time_graph(torch, ceil_step, 4, warm_launches=8, warm_ms=30.0, replays=5, eager=args.eager)
     ceil_tf = ceil_wgs * 8.0 * ceil_iters * 8 * 2 * 32 * 32 * 16 / (ceil_med / 4) / 1e12
 
-    # the prefill tile's inner loop with its ingredients switched on one at a time (wol_mfma_probe)
+    # a 256 x 256 tile's inner loop with its ingredients switched on one at a time (wol_mfma_probe)
     ladder = None
     if not args.no_ladder:
         probe_ops = torch.randn(12 * 1024 * 1024 + 65536, device=dev).to(torch.bfloat16)  # > WOL_MFMA_PROBE_OPERAND_BYTES
