@@ -346,6 +346,7 @@ struct Epi {
   const int32_t* list;
   uint16_t* out;          // [M,N] T
   int M, K, N;
+  int pick;               // outlier columns, up to which the GEMM picks them out of x and w although cols is there
   // Few outlier columns, collected by the outlier kernel for the GEMM's epilogue (null: it picks them out of x and w):
   // [kOutCap][M rounded up to whole tiles] x of outlier column j, by row, and behind them [kOutCap][N rounded up]
   // T(w * wscale) of it, by output column.
@@ -465,7 +466,7 @@ __global__ __launch_bounds__(256) void llm_outlier_kernel(Epi e, int fused_cap) 
   int k = may ? e.list[static_cast<int>(first) / per] : 0;
   const int cnt = *e.count;
   if (cnt <= fused_cap) {
-    if (e.cols == nullptr) return;  // the GEMM picks the columns itself
+    if (e.cols == nullptr || cnt <= e.pick) return;  // the GEMM picks the columns itself
     for (int64_t i = first; i < static_cast<int64_t>(cnt) * per; i += static_cast<int64_t>(gridDim.x) * 256) {
       const int j = static_cast<int>(i) / per, r = static_cast<int>(i) - j * per;
       if (i != first) k = e.list[j];
@@ -797,9 +798,9 @@ __global__ __launch_bounds__(WM* WN * 64) __attribute__((amdgpu_waves_per_eu(2))
     if (!fused) __syncthreads();
   }
   if (fused) {
-    if (e.cols != nullptr) {
+    if (e.cols != nullptr && cnt > e.pick) {
       stage_outliers<DT, BM, BN, NW * 64>(e, cnt, m0, n0, tid, xs, wdl);
-    } else {  // one row tile: this workgroup is the only one that needs its columns' weights
+    } else {  // one row tile, whose workgroup is the only one that needs its columns' weights, or one column
       for (int i = tid; i < cnt * BM; i += NW * 64) {
         const int j = i / BM, m = m0 + i % BM;
         xs[i] = to_f32<DT>(e.x[static_cast<int64_t>(m < M ? m : M - 1) * K + e.list[j]]);
@@ -1408,7 +1409,7 @@ int run_llm_int8(const void* x, const void* weight, const void* bias, const floa
   p.qx = ws.qx;
   p.e = Epi{xs, static_cast<const int8_t*>(weight), wscale, ws.ranges, static_cast<const uint16_t*>(bias),
             ws.count, ws.list, static_cast<uint16_t*>(out), static_cast<int>(M), static_cast<int>(K),
-            static_cast<int>(N), ws.cols};
+            static_cast<int>(N), pl.bn == 256 ? 0 : 1, ws.cols};  // 256 columns: llm_wide_kernel, which cannot pick
   p.acc = ws.acc;
   p.ow = pl.runs > 1 && M <= kFewRows ? ws.ow : nullptr;
   p.n_lo = 0;
@@ -1431,7 +1432,8 @@ int run_llm_int8(const void* x, const void* weight, const void* bias, const floa
     // the other (300 x 4544 -> 4096, fp16, 20 columns, 90.0 us a call when every tile picks, 81 so).  Up to 128 rows
     // there is one row tile, and the GEMM picks a column's weights exactly once (101 x 1024 -> 1024, bf16, 20 columns, us a
     // call: collected on the workgroups of the product 38.5, on enough of them 33.1, picked 32.9; 3 columns 25.1 / 24.0 /
-    // 23.7).
+    // 23.7).  Nor is a single column worth collecting for llm_gemm_kernel (Epi::pick): 129 x 2112 -> 12288, bf16, 39.4
+    // collected, 38.7 picked, 256 rows 41.1 / 40.1; with 3 columns collecting is level (41.7 / 41.6) and gains from there.
     int64_t blocks = ((N + 255) / 256) * ((M + 63) / 64);  // one per 64 x 256 piece of the product
     if (M <= 128) p.e.cols = nullptr;
     const int64_t collect = p.e.cols != nullptr ? (p.cap * (M + N) + 255) / 256 : 0;

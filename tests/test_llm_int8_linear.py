@@ -253,12 +253,13 @@ GPU_CASES = [  # M, K, N, kind, threshold, bias
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("dt", [H.F16, H.BF16])
-@pytest.mark.parametrize("cnt", [1, 8, 9, 32, 33])
+@pytest.mark.parametrize("cnt", [1, 2, 8, 9, 32, 33])
 @pytest.mark.parametrize("M,K,N", [(3, 1024, 400), (4, 576, 272), (130, 512, 400), (300, 576, 272)])
 def test_gpu_outlier_columns_out_of_the_gemm_tiles(device, oracle, dt, cnt, M, K, N):
     # with K runs and up to four rows the weight bytes of up to 32 outlier columns are picked out of
     # the GEMM's own tiles: columns at the ends of K, on both sides of a k tile and spread over the
     # runs; one more than the tiles' stash holds; and many rows, where the epilogue gathers them
+    # (a K that is 64 mod 128: one column picked by every tile, more collected ahead)
     _, w_nk, ws = _weights(K, N, dt, seed=K + N)
     rng = np.random.default_rng(cnt)
     cols = np.r_[[0, K - 1, 127, 128, 63, 64, 255, 256], rng.permutation(np.arange(300, K - 1))][:cnt]
